@@ -81,7 +81,6 @@ struct Block {
     Fields f;
     long arena_off = 0;     // doubles from the context's arena base
     double *geo = nullptr;  // acfd_grid_metrics: x, y, z, spci, spcj, spck (n each)
-    int tile_shape = -1;    // chosen by the autotuner on first use
     std::vector<acfd_subface> sub;
 };
 
@@ -137,20 +136,19 @@ struct acfd_ctx {
     unsigned int *d_nneg = nullptr;
     double *d_res = nullptr;       // 6 sums
     double *d_partial = nullptr;   // residual partials
-    LuWs lu{nullptr, nullptr, nullptr};  // tile-sweep workspace (lusgs_kernel 1, 2)
+    LuWs lu{nullptr, nullptr, nullptr, nullptr, {0, 0}};  // tile-sweep workspace (lusgs_kernel 1, 2)
     long lu_ex_n = 0;
-    LuBatch lub[4];          // lusgs_kernel 2: every block in one launch, per tile shape
-    LuBatch sab[4];          // the same for the SA model's scalar sweeps
-    int lub_shape = -1;      // chosen by the autotuner on first use
-    // what the sweep layout holds of the grid operands: the block of the last
-    // gather (-1: the batch, -2: nothing valid) and its tiling
-    int sl_block = -2, sl_shape = -1;
+    LuBatch lub;             // lusgs_kernel 2: every block in one launch
+    LuBatch sab;             // the same for the SA model's scalar sweeps
+    // whose grid operands the sweep layout holds: the block of the last
+    // gather (-1: the batch, -2: nothing valid)
+    int sl_block = -2;
     bool capturing = false;
     // the captured step gathers without the grid operands: it replays only
-    // onto the contents it was captured on (sl_block, sl_shape at its start)
+    // onto the contents it was captured on (sl_block at its start)
     // and leaves those of its end
     bool graph_geo_cached = false;
-    int graph_sl_in[2] = {-2, -1}, graph_sl_out[2] = {-2, -1};
+    int graph_sl_in = -2, graph_sl_out = -2;
     // pri_v holds getpri of the current q of every block: set by the closing
     // getpri of a step, cleared by every call that may write q or pri_v.
     // The next step's residual then starts without its getpri; a captured
@@ -593,8 +591,8 @@ int ensure_geo(acfd_ctx *ctx)
     return 0;
 }
 
-// Workspace of the tile sweeps, sized for the largest block and every tile
-// shape: the sweep-layout operand array (ordinary device memory), the
+// Workspace of the tile sweeps, sized for the largest block or the whole
+// batch: the sweep-layout operand array (ordinary device memory), the
 // exchange slots (uncached memory, filled with the sentinel; every sweep
 // leaves them that way) and an error word.  Nothing for hyperplane sweeps.
 int alloc_lu_ws(acfd_ctx *ctx)
@@ -612,14 +610,8 @@ int alloc_lu_ws(acfd_ctx *ctx)
     }
     long sl_n = 0, ex_n = 0;
     if (batch) {
-        // every block has its own part of the workspace; sized for the
-        // largest total over the tile shapes
-        for (int sh = 0; sh < lusgs_tile_shapes(); sh++) {
-            long a = 0, x = 0;
-            lusgs_batch_ws(nb, es.data(), sh, &a, &x);
-            sl_n = std::max(sl_n, a);
-            ex_n = std::max(ex_n, x);
-        }
+        // every block has its own part of the workspace
+        lusgs_batch_ws(nb, es.data(), &sl_n, &ex_n);
     } else {
         for (auto &b : ctx->blk) {
             long a = 0, x = 0;
@@ -630,15 +622,19 @@ int alloc_lu_ws(acfd_ctx *ctx)
     }
     if (sl_n <= 0) return 0;
     HIP_TRY(hipMalloc((void **)&ctx->lu.sl, (size_t)sl_n * sizeof(double)));
+    // idle lanes of the sweeps read the padding of the layout: defined values
+    HIP_TRY(hipMemsetAsync(ctx->lu.sl, 0, (size_t)sl_n * sizeof(double), ctx->stream));
     HIP_TRY(hipMalloc((void **)&ctx->lu.err, sizeof(int)));
     HIP_TRY(hipMemsetAsync(ctx->lu.err, 0, sizeof(int), ctx->stream));
     ctx->lu.ex = (double *)uc_acquire((size_t)ex_n * sizeof(double));
     if (!ctx->lu.ex) return fail(ACFD_EDEVICE, "uncached device memory for the tile exchange is unavailable");
     ctx->lu_ex_n = ex_n;
     KRN_TRY(launch_fill_sentinel(ctx->stream, ctx->lu.ex, ex_n));
+    HIP_TRY(hipMalloc((void **)&ctx->lu_ctr, 2 * sizeof(int)));
+    HIP_TRY(hipMemsetAsync(ctx->lu_ctr, 0, 2 * sizeof(int), ctx->stream));
+    ctx->lu.ctr = ctx->lu_ctr;
+    lusgs_resident(ctx->lu.resident);
     if (batch) {
-        HIP_TRY(hipMalloc((void **)&ctx->lu_ctr, 2 * sizeof(int)));
-        HIP_TRY(hipMemsetAsync(ctx->lu_ctr, 0, 2 * sizeof(int), ctx->stream));
         const bool sa = ctx->c.turb == 2 && ctx->c.solver == 0;
         const char *cc = std::getenv("ACFD_SA_CONCURRENT");
         ctx->sa_concurrent = sa && !(cc && std::atoi(cc) == 0);
@@ -661,14 +657,10 @@ int alloc_lu_ws(acfd_ctx *ctx)
             HIP_TRY(hipEventCreateWithFlags(&ctx->ev_rjoin, hipEventDisableTiming));
         }
         if (sa) {
-            // the SA sweep layout, sized for the largest tile shape, and
-            // the grid of the SA model's per-node passes
+            // the SA sweep layout and the grid of the SA model's per-node
+            // passes
             long sa_sl_n = 0;
-            for (int sh = 0; sh < lusgs_tile_shapes(); sh++) {
-                long a = 0;
-                sa_batch_sl(nb, es.data(), sh, &a);
-                sa_sl_n = std::max(sa_sl_n, a);
-            }
+            sa_batch_sl(nb, es.data(), &sa_sl_n);
             if (sa_sl_n > 0) HIP_TRY(hipMalloc((void **)&ctx->sa_sl, (size_t)sa_sl_n * sizeof(double)));
             std::vector<dim3> g;
             for (auto &b : ctx->blk) g.push_back(lin_grid(b.e));
@@ -676,18 +668,16 @@ int alloc_lu_ws(acfd_ctx *ctx)
             if (!rc) rc = make_grid(ctx->bg_sa, g);
             if (rc) return rc;
         }
-        for (int sh = 0; sh < lusgs_tile_shapes(); sh++) {
-            if (lusgs_batch_make(nb, es.data(), fs.data(), ctx->arena, sh, ctx->lu.sl, ctx->lu.ex, &ctx->lub[sh]))
-                return fail(ACFD_EDEVICE, "batched LU-SGS tables: device allocation failed");
-            if (sa && sa_batch_make(nb, es.data(), fs.data(), ctx->arena, sh, ctx->sa_concurrent ? ctx->sa_ex : ctx->lu.ex,
-                                    ctx->sa_sl, &ctx->sab[sh]))
-                return fail(ACFD_EDEVICE, "batched SA sweep tables: device allocation failed");
-            if (ctx->sa_concurrent) {
-                // two persistent launches share the device: tiles by ticket
-                // (each waits only on tiles that are already running)
-                ctx->lub[sh].resident[0] = ctx->lub[sh].resident[1] = 0;
-                ctx->sab[sh].resident[0] = ctx->sab[sh].resident[1] = 0;
-            }
+        if (lusgs_batch_make(nb, es.data(), fs.data(), ctx->arena, ctx->lu.sl, ctx->lu.ex, &ctx->lub))
+            return fail(ACFD_EDEVICE, "batched LU-SGS tables: device allocation failed");
+        if (sa && sa_batch_make(nb, es.data(), fs.data(), ctx->arena, ctx->sa_concurrent ? ctx->sa_ex : ctx->lu.ex,
+                                ctx->sa_sl, &ctx->sab))
+            return fail(ACFD_EDEVICE, "batched SA sweep tables: device allocation failed");
+        if (ctx->sa_concurrent) {
+            // two persistent launches share the device: tiles by ticket
+            // (each waits only on tiles that are already running)
+            ctx->lub.resident[0] = ctx->lub.resident[1] = 0;
+            ctx->sab.resident[0] = ctx->sab.resident[1] = 0;
         }
     }
     HIP_TRY(hipStreamSynchronize(ctx->stream));
@@ -881,10 +871,6 @@ bool sa_layout_on()
     return v == 1;
 }
 
-// Autotuner of the tile sweep: on a block's first update, time the gather
-// and forward sweep once per tile shape (they recompute dq* in the sweep
-// layout from unchanged inputs, so repeating them changes nothing) and keep
-// the fastest shape.
 bool geo_cache_on()
 {
     static const bool on = [] {
@@ -895,16 +881,15 @@ bool geo_cache_on()
 }
 
 // Whether the sweep layout already holds the grid operands (dxidx, inv_j)
-// of `block` (-1: the batch) in tiling `shape`, so that the gather about to
-// be launched may leave them in place; records that it holds them after.
+// of `block` (-1: the batch), so that the gather about to be launched may
+// leave them in place; records that it holds them after.
 // The sweeps write only the result fields, and the grid operands change
 // only through sl_invalidate's callers.  ACFD_SL_GEO_CACHE=0 gathers every
 // field every time.
-int sl_geo_cached(acfd_ctx *ctx, int block, int shape)
+int sl_geo_cached(acfd_ctx *ctx, int block)
 {
-    const bool same = ctx->sl_block == block && ctx->sl_shape == shape && geo_cache_on();
+    const bool same = ctx->sl_block == block && geo_cache_on();
     ctx->sl_block = block;
-    ctx->sl_shape = shape;
     if (same && ctx->capturing) ctx->graph_geo_cached = true;
     return same ? 1 : 0;
 }
@@ -913,45 +898,6 @@ int sl_geo_cached(acfd_ctx *ctx, int block, int shape)
 void sl_invalidate(acfd_ctx *ctx)
 {
     ctx->sl_block = -2;
-    ctx->sl_shape = -1;
-}
-
-int tune_tiles(acfd_ctx *ctx, Block &b)
-{
-    if (const char *fix = std::getenv("ACFD_TILE_SHAPE")) {
-        int s = std::atoi(fix);
-        if (s >= 0 && s < lusgs_tile_shapes()) {
-            b.tile_shape = s;
-            return 0;
-        }
-    }
-    hipEvent_t e0, e1;
-    HIP_TRY(hipEventCreate(&e0));
-    HIP_TRY(hipEventCreate(&e1));
-    float best = 1e30f;
-    int best_s = 0;
-    for (int s = 0; s < lusgs_tile_shapes(); s++) {
-        if (lusgs_tiles(b.e, s) <= 0) continue;
-        (void)hipEventRecord(e0, ctx->stream);
-        int rc = launch_lusgs_phase(ctx->stream, b.e, b.f, ctx->c, ctx->d_cfl, 1, &ctx->lu, 1, s,
-                                    sl_geo_cached(ctx, (int)(&b - ctx->blk.data()), s));
-        if (!rc) rc = launch_lusgs_phase(ctx->stream, b.e, b.f, ctx->c, ctx->d_cfl, 1, &ctx->lu, 2, s);
-        (void)hipEventRecord(e1, ctx->stream);
-        if (rc) return fail(ACFD_EDEVICE, "tile sweep launch failed during tuning");
-        HIP_TRY(hipEventSynchronize(e1));
-        float ms = 0.f;
-        (void)hipEventElapsedTime(&ms, e0, e1);
-        if (std::getenv("ACFD_VERBOSE"))
-            std::fprintf(stderr, "acfd: tile sweep shape %d (%ld tiles): %.3f ms\n", s, lusgs_tiles(b.e, s), ms);
-        if (ms < best) {
-            best = ms;
-            best_s = s;
-        }
-    }
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
-    b.tile_shape = best_s;
-    return 0;
 }
 
 int st_implicit(acfd_ctx *ctx, int m, const double *cfl)
@@ -960,58 +906,11 @@ int st_implicit(acfd_ctx *ctx, int m, const double *cfl)
     Block &b = ctx->blk[m];
     const int variant = ctx->cfg.lusgs_kernel;
     for (int ph = 0; ph < kLusgsPhases; ph++) {
-        if (ph == 1 && variant == 1 && b.tile_shape < 0) {
-            int rc = tune_tiles(ctx, b);
-            if (rc) return rc;
-        }
         StageTimer ts(ctx, ph == 2 ? kTimeLuForward : ph == 3 ? kTimeLuBackward
                            : ph == 1 ? kTimeLuGather : ph == 4 ? kTimeLuAdd : kTimeLuOther);
-        const int shape = b.tile_shape < 0 ? 0 : b.tile_shape;
-        KRN_TRY(launch_lusgs_phase(ctx->stream, b.e, b.f, ctx->c, cfl, variant, &ctx->lu, ph, shape,
-                                   ph == 1 && variant == 1 ? sl_geo_cached(ctx, m, shape) : 0));
+        KRN_TRY(launch_lusgs_phase(ctx->stream, b.e, b.f, ctx->c, cfl, variant, &ctx->lu, ph,
+                                   ph == 1 && variant == 1 ? sl_geo_cached(ctx, m) : 0));
     }
-    return 0;
-}
-
-// Autotuner of the batched sweep: the same timing as tune_tiles over the
-// whole batch, one shape for all blocks.
-int tune_batch(acfd_ctx *ctx)
-{
-    if (const char *fix = std::getenv("ACFD_TILE_SHAPE")) {
-        int s = std::atoi(fix);
-        if (s >= 0 && s < lusgs_tile_shapes()) {
-            ctx->lub_shape = s;
-            return 0;
-        }
-    }
-    hipEvent_t e0, e1;
-    HIP_TRY(hipEventCreate(&e0));
-    HIP_TRY(hipEventCreate(&e1));
-    float best = 1e30f;
-    int best_s = 0;
-    for (int s = 0; s < lusgs_tile_shapes(); s++) {
-        const LuBatch &lb = ctx->lub[s];
-        if (lb.total <= 0) continue;
-        (void)hipEventRecord(e0, ctx->stream);
-        int rc = launch_lusgs_batch(ctx->stream, lb, 1, ctx->c.gamma, ctx->lu.err, ctx->lu_ctr,
-                                    sl_geo_cached(ctx, -1, s));
-        if (!rc) rc = launch_lusgs_batch(ctx->stream, lb, 2, ctx->c.gamma, ctx->lu.err, ctx->lu_ctr);
-        (void)hipEventRecord(e1, ctx->stream);
-        if (rc) return fail(ACFD_EDEVICE, "batched tile sweep launch failed during tuning");
-        HIP_TRY(hipEventSynchronize(e1));
-        float ms = 0.f;
-        (void)hipEventElapsedTime(&ms, e0, e1);
-        if (std::getenv("ACFD_VERBOSE"))
-            std::fprintf(stderr, "acfd: batched sweep shape %d (%d tiles, %d blocks): %.3f ms\n", s, lb.total,
-                         lb.nent, ms);
-        if (ms < best) {
-            best = ms;
-            best_s = s;
-        }
-    }
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
-    ctx->lub_shape = best_s;
     return 0;
 }
 
@@ -1050,18 +949,14 @@ int st_implicit_all(acfd_ctx *ctx, const double *cfl_per_block)
         for (int m = 0; m < nb; m++) {
             const Block &b = ctx->blk[m];
             KRN_TRY(launch_lusgs_phase(ctx->stream, b.e, b.f, ctx->c, cfl_per_block ? cfl_per_block + m : ctx->d_cfl,
-                                       1, &ctx->lu, 0, 0));
+                                       1, &ctx->lu, 0));
         }
     }
-    if (ctx->lub_shape < 0) {
-        int rc = tune_batch(ctx);
-        if (rc) return rc;
-    }
-    const LuBatch &lb = ctx->lub[ctx->lub_shape];
+    const LuBatch &lb = ctx->lub;
     for (int ph = 1; ph < kLusgsPhases; ph++) {
         StageTimer ts(ctx, ph == 2 ? kTimeLuForward : ph == 3 ? kTimeLuBackward : ph == 1 ? kTimeLuGather : kTimeLuAdd);
         KRN_TRY(launch_lusgs_batch(ctx->stream, lb, ph, ctx->c.gamma, ctx->lu.err, ctx->lu_ctr,
-                                   ph == 1 ? sl_geo_cached(ctx, -1, ctx->lub_shape) : 0));
+                                   ph == 1 ? sl_geo_cached(ctx, -1) : 0));
     }
     return 0;
 }
@@ -1072,8 +967,7 @@ int st_sa(acfd_ctx *ctx, int m, const double *cfl)
     const Block &b = ctx->blk[m];
     if ((ctx->cfg.lusgs_kernel == 1 || ctx->cfg.lusgs_kernel == 2) && ctx->lu.ex) {
         // tile sweeps in the flow sweep's exchange slots (idle, sentinel-filled)
-        const int shape = b.tile_shape >= 0 ? b.tile_shape : ctx->lub_shape >= 0 ? ctx->lub_shape : 0;
-        const SaSweep sw{shape, ctx->sa_ex ? ctx->sa_ex : ctx->lu.ex, ctx->lu.err};
+        const SaSweep sw{ctx->sa_ex ? ctx->sa_ex : ctx->lu.ex, ctx->lu.err};
         KRN_TRY(launch_sa(ctx->stream, b.e, b.f, ctx->c, cfl, &sw));
     } else {
         KRN_TRY(launch_sa(ctx->stream, b.e, b.f, ctx->c, cfl));
@@ -1087,15 +981,7 @@ template <typename F>
 int st_sa_all(acfd_ctx *ctx, F cfl_of)
 {
     const int nb = (int)ctx->blk.size();
-    // the scalar SA sweeps run 8x8 tiles whatever the flow sweeps chose:
-    // measured the fastest of the four shapes on the channel (SA stage
-    // 32.2 ms against 34.0 at 16x8 and 36.4 at 16x16) and the flat plate
-    int shape = 2;
-    if (const char *v = std::getenv("ACFD_SA_TILE_SHAPE")) {
-        const int s = std::atoi(v);
-        if (s >= 0 && s < 4) shape = s;
-    }
-    if (ctx->cfg.lusgs_kernel != 2 || ctx->sab[shape].total <= 0) {
+    if (ctx->cfg.lusgs_kernel != 2 || ctx->sab.total <= 0) {
         for (int m = 0; m < nb; m++) {
             int rc = st_sa(ctx, m, cfl_of(m));
             if (rc) return rc;
@@ -1107,7 +993,7 @@ int st_sa_all(acfd_ctx *ctx, F cfl_of)
     if (ctx->sa_sl && ctx->bg_sa.total > 0 && sa_layout_on()) {
         // two per-node passes over all blocks, the operands into the SA
         // sweep layout, the two sweeps over it, nut += dnut
-        const LuBatch &sb = ctx->sab[shape];
+        const LuBatch &sb = ctx->sab;
         const double *c0 = cfl_of(0);
         const int stride = nb > 1 && cfl_of(1) != c0 ? 1 : 0;
         for (int part = ctx->timing ? 1 : 0; part <= (ctx->timing ? 2 : 0); part++) {
@@ -1140,12 +1026,12 @@ int st_sa_all(acfd_ctx *ctx, F cfl_of)
     if (ctx->timing) {
         {
             StageTimer ts(ctx, kTimeSaForward);
-            KRN_TRY(launch_sa_batch(ctx->stream, ctx->sab[shape], ctx->lu.err, ctr, 1));
+            KRN_TRY(launch_sa_batch(ctx->stream, ctx->sab, ctx->lu.err, ctr, 1));
         }
         StageTimer ts(ctx, kTimeSaBackward);
-        KRN_TRY(launch_sa_batch(ctx->stream, ctx->sab[shape], ctx->lu.err, ctr, -1));
+        KRN_TRY(launch_sa_batch(ctx->stream, ctx->sab, ctx->lu.err, ctr, -1));
     } else {
-        KRN_TRY(launch_sa_batch(ctx->stream, ctx->sab[shape], ctx->lu.err, ctr, 0));
+        KRN_TRY(launch_sa_batch(ctx->stream, ctx->sab, ctx->lu.err, ctr, 0));
     }
     StageTimer ts(ctx, kTimeSaAdd);
     for (int m = 0; m < nb; m++) KRN_TRY(launch_sa_post(ctx->stream, ctx->blk[m].e, ctx->blk[m].f));
@@ -1418,7 +1304,7 @@ int one_step(acfd_ctx *ctx)
     if (ctx->cfg.iflag_timeadvance == 2 && stagewise) {
         rc = residual_stage_all(ctx, aux, pri_ok);
         static_assert(!kBatchedUpdateWritesDq, "the concurrent SA update owns w_dqs / w_dq");
-        if (!rc && sa && ctx->sa_concurrent && ctx->lub_shape >= 0 && !ctx->timing) {
+        if (!rc && sa && ctx->sa_concurrent && !ctx->timing) {
             // sa_model reads nothing implicit1st writes (pri_v, amu, vor, dt
             // and the cfl are from the residual) and implicit1st reads no
             // SA field: the SA update runs on the second stream meanwhile
@@ -1525,16 +1411,14 @@ int capture_step(acfd_ctx *ctx)
     ctx->capturing = true;
     ctx->graph_geo_cached = false;
     ctx->graph_needs_pri = false;
-    ctx->graph_sl_in[0] = ctx->sl_block;
-    ctx->graph_sl_in[1] = ctx->sl_shape;
+    ctx->graph_sl_in = ctx->sl_block;
     const bool stale = ctx->rhsv_stale;
     ctx->rhsv_stale = false;
     const int rc = one_step(ctx);
     ctx->graph_rhsv = ctx->rhsv_stale;
     ctx->rhsv_stale = stale;  // nothing ran yet
     ctx->capturing = false;
-    ctx->graph_sl_out[0] = ctx->sl_block;
-    ctx->graph_sl_out[1] = ctx->sl_shape;
+    ctx->graph_sl_out = ctx->sl_block;
     hipGraph_t g = nullptr;
     const hipError_t ec = hipStreamEndCapture(ctx->stream, &g);
     ctx->timing = timing;
@@ -1622,8 +1506,8 @@ int acfd_destroy(acfd_ctx *ctx)
     if (ctx->lu.ex) uc_release(ctx->lu.ex);
     if (ctx->lu.sl) (void)hipFree(ctx->lu.sl);
     if (ctx->lu.err) (void)hipFree(ctx->lu.err);
-    for (auto &b : ctx->lub) lusgs_batch_free(&b);
-    for (auto &b : ctx->sab) lusgs_batch_free(&b);
+    lusgs_batch_free(&ctx->lub);
+    lusgs_batch_free(&ctx->sab);
     if (ctx->lu_ctr) (void)hipFree(ctx->lu_ctr);
     if (ctx->d_cfl_blk) (void)hipFree(ctx->d_cfl_blk);
     if (ctx->d_blocks) (void)hipFree(ctx->d_blocks);
@@ -1959,14 +1843,13 @@ int acfd_step(acfd_ctx *ctx, int nsteps)
     if (!ctx || !ctx->topo) return fail(ACFD_ESTATE, "acfd_step: no topology");
     if (nsteps > 0) ctx->res_current = false;
     int s = 0;
-    // graph mode: the first step runs eagerly (it also tunes the tile
-    // sweeps), the next one is captured, and every later step replays it;
+    // graph mode: the first step runs eagerly, the next one is
+    // captured, and every later step replays it;
     // audited sensor steps read results on the host, sensor steps that reuse
     // decisions alternate between two kernels, and steps under the
     // per-stage timers record events between launches: all stay eager
     const bool graph = ctx->cfg.use_graph && !ctx->timing && !(ctx->s_on && (ctx->s_audit > 0 || ctx->s_refresh > 1));
-    if (ctx->graph_exec && ctx->graph_geo_cached &&
-        (ctx->sl_block != ctx->graph_sl_in[0] || ctx->sl_shape != ctx->graph_sl_in[1]))
+    if (ctx->graph_exec && ctx->graph_geo_cached && ctx->sl_block != ctx->graph_sl_in)
         drop_graph(ctx);  // the sweep layout holds other grid operands than at capture
     if (ctx->graph_exec && ctx->graph_needs_pri && !ctx->pri_current)
         drop_graph(ctx);  // q or pri_v was written since the last step
@@ -1982,8 +1865,7 @@ int acfd_step(acfd_ctx *ctx, int nsteps)
     for (; s < nsteps; s++) {
         if (graph && ctx->graph_exec) {
             HIP_TRY(hipGraphLaunch(ctx->graph_exec, ctx->stream));
-            ctx->sl_block = ctx->graph_sl_out[0];
-            ctx->sl_shape = ctx->graph_sl_out[1];
+            ctx->sl_block = ctx->graph_sl_out;
             ctx->pri_current = true;
             if (ctx->graph_rhsv) ctx->rhsv_stale = true;
             continue;

@@ -12,16 +12,16 @@
 //   hyperplanes  one launch per plane l (2 (Li+Lj+Lk-2) launches per step),
 //                operands read in place.
 //
-//   tiles        one persistent launch per sweep.  Each workgroup owns a
-//                TJ x TK tile of (j,k) lines and marches along i on a skewed
-//                clock: thread (tj,tk) handles the node at sweep position
+//   tiles        one persistent launch per sweep.  Each workgroup owns an
+//                8 x 8 tile of (j,k) lines and marches along i on a skewed
+//                clock: lane (tj,tk) handles the node at sweep position
 //                s - tj - tk at step s.
 //                * Sweep layout.  Before the forward sweep the operands of
 //                  every node (metric rows, 1/J, q, sound speed, the time
 //                  term phi/dt, rhs: 22 values; the sweeps form the spectral
 //                  radii and the diagonal from them) are gathered into an
 //                  array ordered by (tile, step, field pair, lane), so at
-//                  every step a tile reads 11 contiguous rows of TJ*TK
+//                  every step a tile reads 11 contiguous rows of 64
 //                  16-byte pairs -- fully coalesced, where
 //                  the natural layout would have every lane on its own cache
 //                  line.  The sweeps write dq* and dq over the rhs slots and a
@@ -30,18 +30,16 @@
 //                  off-diagonal products 1/2 inv_j (A(q; grad xi_d) +- r_d I) dq
 //                  that its successors need, with its own operands: the i
 //                  product stays in registers, the j and k products go to the
-//                  next lanes through LDS, and the tile's last row/column
-//                  hand them to the neighbouring tile through exchange slots.
+//                  next lanes, and the tile's last row/column hand them to
+//                  the neighbouring tile through exchange slots.
 //                  Each product is the same expression of the same operands
 //                  as in the pull form, so both schedules give the same bits.
 //                * Exchange.  Slots live in uncached memory and hold a
 //                  sentinel bit pattern (a signalling NaN no arithmetic
 //                  produces) until the producer stores the value; the
-//                  consumer spins on the value itself and writes the sentinel
+//                  consumer polls the value itself and writes the sentinel
 //                  back.  No counters, no fences, no waits for store
-//                  acknowledgements on the per-step path; operands and
-//                  exchange values are loaded one step ahead, and a slot
-//                  found late is polled for all its late components at once.
+//                  acknowledgements between tiles.
 //
 // The flux Jacobian products use the closed form of A(q) v for the Euler
 // flux in generalised coordinates (one reciprocal of rho instead of the ~25
@@ -68,55 +66,93 @@ namespace acfd {
 //         a1 theta + U (dp + v5) ]
 // with u = mom/rho, U = m.u, theta = m.v_mom - U v1,
 // dp = (gamma-1)(|u|^2/2 v1 - u.v_mom + v5), a1 = gamma E/rho - (gamma-1)|u|^2/2.
-template <int SGN>
-__device__ inline void jac_mv_r(const double *qv, double mx, double my, double mz, double ij, double rr,
-                                double gamma, const double *v, double *out)
+// The factor s = 1/2 inv_j is taken into the metric row, U and r once per
+// node and direction, so that what depends on v -- all of a sweep's serial
+// chain -- is as short as it can be.
+
+// the part of a node's products that no direction changes
+struct LuState {
+    double u, v, w, q2h, a1;  // velocity, |u|^2/2, a1
+};
+// one direction: the metric row, U and +-r, each times s
+struct LuRow {
+    double x, y, z, U, r;
+};
+
+__device__ inline LuState lu_state(const double *qv, double ri, double gamma)
 {
-    const double rho = qv[0], mu = qv[1], mv = qv[2], mw = qv[3], E = qv[4];
-    const double ri = 1.0 / rho;
-    const double u = mu * ri, w2 = mv * ri, w3 = mw * ri;
-    const double U = fma(mz, w3, fma(my, w2, mx * u));
-    const double q2 = fma(w3, w3, fma(w2, w2, u * u));
-    const double g1 = gamma - 1.0;
-    const double a1 = fma(gamma * E, ri, -0.5 * g1 * q2);
-    const double mvm = fma(mz, v[3], fma(my, v[2], mx * v[1]));
-    const double theta = fma(-U, v[0], mvm);
-    const double uv = fma(w3, v[3], fma(w2, v[2], u * v[1]));
-    const double dp = g1 * (fma(0.5 * q2, v[0], -uv) + v[4]);
-    const double r = SGN > 0 ? rr : -rr;
-    const double s = 0.5 * ij;
-    out[0] = s * fma(r, v[0], mvm);
-    out[1] = s * fma(r, v[1], fma(mx, dp, fma(u, theta, U * v[1])));
-    out[2] = s * fma(r, v[2], fma(my, dp, fma(w2, theta, U * v[2])));
-    out[3] = s * fma(r, v[3], fma(mz, dp, fma(w3, theta, U * v[3])));
-    out[4] = s * fma(r, v[4], fma(U, dp + v[4], a1 * theta));
+    LuState t;
+    t.u = qv[1] * ri;
+    t.v = qv[2] * ri;
+    t.w = qv[3] * ri;
+    t.q2h = 0.5 * fma(t.w, t.w, fma(t.v, t.v, t.u * t.u));
+    t.a1 = fma(gamma * qv[4], ri, -(gamma - 1.0) * t.q2h);
+    return t;
 }
 
-// the same product with the operands of node n read from the SoA fields
+template <int SGN>
+__device__ inline LuRow lu_row(const LuState &t, double mx, double my, double mz, double s, double rr)
+{
+    LuRow m;
+    m.x = s * mx;
+    m.y = s * my;
+    m.z = s * mz;
+    m.U = fma(m.z, t.w, fma(m.y, t.v, m.x * t.u));
+    m.r = s * (SGN > 0 ? rr : -rr);
+    return m;
+}
+
+// dp of a solution vector v, shared by the three directions
+__device__ inline double lu_dp(const LuState &t, double gamma, const double *v)
+{
+    const double uv = fma(t.w, v[3], fma(t.v, v[2], t.u * v[1]));
+    return (gamma - 1.0) * (fma(t.q2h, v[0], -uv) + v[4]);
+}
+
+__device__ inline void lu_product(const LuState &t, const LuRow &m, double dp, const double *v, double *out)
+{
+    const double mvm = fma(m.z, v[3], fma(m.y, v[2], m.x * v[1]));
+    const double theta = fma(-m.U, v[0], mvm);
+    const double w = m.U + m.r;
+    out[0] = fma(m.r, v[0], mvm);
+    out[1] = fma(w, v[1], fma(m.x, dp, t.u * theta));
+    out[2] = fma(w, v[2], fma(m.y, dp, t.v * theta));
+    out[3] = fma(w, v[3], fma(m.z, dp, t.w * theta));
+    out[4] = fma(w, v[4], fma(m.U, dp, t.a1 * theta));
+}
+
+// the product with the operands of node n read from the SoA fields
 template <int SGN>
 __device__ inline void jac_mv(const double *__restrict__ q, const double *__restrict__ dxidx,
                               const double *__restrict__ inv_j, const double *__restrict__ rr, long N, long n,
                               int c0, double gamma, const double *v, double *out)
 {
     const double qv[5] = {q[n], q[N + n], q[2 * N + n], q[3 * N + n], q[4 * N + n]};
-    jac_mv_r<SGN>(qv, dxidx[c0 * N + n], dxidx[(c0 + 1) * N + n], dxidx[(c0 + 2) * N + n], inv_j[n], rr[n],
-                  gamma, v, out);
+    const LuState t = lu_state(qv, 1.0 / qv[0], gamma);
+    const LuRow m = lu_row<SGN>(t, dxidx[c0 * N + n], dxidx[(c0 + 1) * N + n], dxidx[(c0 + 2) * N + n],
+                                0.5 * inv_j[n], rr[n]);
+    lu_product(t, m, lu_dp(t, gamma, v), v, out);
 }
+
+// 1 / (diag inv_j): both sweeps divide by the two; one reciprocal per node,
+// formed before its neighbours' values arrive (the ten divisions of the
+// five components were on the sweeps' serial chain)
+__device__ inline double lu_rdiag(double dg, double ij) { return 1.0 / (dg * ij); }
 
 // forward node (:345-365): dq* = (rhs + A+ dq*_i-1 + B+ dq*_j-1 + C+ dq*_k-1)/diag/inv_j
 __device__ inline void lu_fwd_combine(const double *rhs, const double *ta, const double *tb, const double *tc,
-                                      double dg, double ij, double *res)
+                                      double rd, double *res)
 {
 #pragma unroll
-    for (int x = 0; x < 5; x++) res[x] = (rhs[x] + (ta[x] + tb[x] + tc[x])) / dg / ij;
+    for (int x = 0; x < 5; x++) res[x] = (rhs[x] + (ta[x] + tb[x] + tc[x])) * rd;
 }
 
 // backward node (:521-542): dq = dq* - (A- dq_i+1 + B- dq_j+1 + C- dq_k+1)/inv_j/diag
 __device__ inline void lu_bwd_combine(const double *dqs, const double *ta, const double *tb, const double *tc,
-                                      double dg, double ij, double *res)
+                                      double rd, double *res)
 {
 #pragma unroll
-    for (int x = 0; x < 5; x++) res[x] = dqs[x] - (ta[x] + tb[x] + tc[x]) / ij / dg;
+    for (int x = 0; x < 5; x++) res[x] = fma(-(ta[x] + tb[x] + tc[x]), rd, dqs[x]);
 }
 
 struct LuArgs {
@@ -136,7 +172,7 @@ __device__ inline void lu_forward(const LuArgs &a, long n, const double *vi, con
     jac_mv<1>(a.q, a.dxidx, a.inv_j, a.rr + 2 * N, N, n - sk, 6, a.gamma, vk, tc);
 #pragma unroll
     for (int x = 0; x < 5; x++) rhs[x] = a.rhs[x * N + n];
-    lu_fwd_combine(rhs, ta, tb, tc, a.diag[n], a.inv_j[n], res);
+    lu_fwd_combine(rhs, ta, tb, tc, lu_rdiag(a.diag[n], a.inv_j[n]), res);
 }
 
 __device__ inline void lu_backward(const LuArgs &a, long n, const double *vi, const double *vj,
@@ -149,7 +185,7 @@ __device__ inline void lu_backward(const LuArgs &a, long n, const double *vi, co
     jac_mv<-1>(a.q, a.dxidx, a.inv_j, a.rr + 2 * N, N, n + sk, 6, a.gamma, vk, tc);
 #pragma unroll
     for (int x = 0; x < 5; x++) dqs[x] = a.dqs[x * N + n];
-    lu_bwd_combine(dqs, ta, tb, tc, a.diag[n], a.inv_j[n], res);
+    lu_bwd_combine(dqs, ta, tb, tc, lu_rdiag(a.diag[n], a.inv_j[n]), res);
 }
 
 // rhs = rhsi + rhsv on the computed range (:72-78).  For the hyperplane
@@ -285,54 +321,31 @@ constexpr int kSlGeoPairs = 5;
 // only ever produces quiet NaNs
 constexpr unsigned long long kSentinel = 0xFFF5A5A5A5A5A5A5ull;
 
-// geometry of one tiling of a block's computed range
+// tile edge and lanes of a tile
+constexpr int kTile = 8, kLanes = 64;
+
+// geometry of the tiling of a block's computed range
 struct SlGeom {
-    int TJ, TK, TT, nbj, nbk, ntiles, nsteps, Li, Lj, Lk;
-    int lgTJ;  // TJ is a power of two
-    int refill;  // consumers leave exchange slots as they are; the region is refilled after each sweep
+    int nbj, nbk, ntiles, nsteps, Li, Lj, Lk;
     long exj_tile, exk_tile;  // doubles per tile of the j / k exchange regions
-    // fields are stored in pairs, so a lane's operands of one step are 12
+    // fields are stored in pairs, so a lane's operands of one step are 11
     // 16-byte loads; double index of field f of lane l at row t
     __host__ __device__ long slot(int tile, int t, int f, int l) const {
-        return ((((long)tile * nsteps + t) * (kSlF / 2) + (f >> 1)) * TT + l) * 2 + (f & 1);
+        return ((((long)tile * nsteps + t) * (kSlF / 2) + (f >> 1)) * kLanes + l) * 2 + (f & 1);
     }
 };
 
-// tile shapes the autotuner chooses from (TJ, TK)
-const int kTileShapes[][2] = {{16, 16}, {16, 8}, {8, 8}, {16, 4}};
-const int kNumTileShapes = 4;
-
-// Exchange slots are reset to the sentinel by one fill kernel after each
-// flow sweep rather than by their consumers, one store each: the per-step
-// stores were on the sweep's critical path.
-static int ex_refill()
-{
-    static int r = -1;
-    if (r < 0) {
-        const char *v = getenv("ACFD_EX_REFILL");
-        r = v && atoi(v) == 0 ? 0 : 1;
-    }
-    return r;
-}
-
-static SlGeom sl_geom(const Ext &e, int shape)
+static SlGeom sl_geom(const Ext &e)
 {
     SlGeom g;
-    g.refill = ex_refill();
-    g.TJ = kTileShapes[shape][0];
-    g.TK = kTileShapes[shape][1];
-    g.TT = g.TJ * g.TK;
-    g.lgTJ = 0;
-    while ((1 << g.lgTJ) < g.TJ) g.lgTJ++;
     g.Li = e.ie1 - e.is1 + 1;
     g.Lj = e.je1 - e.js1 + 1;
     g.Lk = e.ke1 - e.ks1 + 1;
-    g.nbj = (g.Lj + g.TJ - 1) / g.TJ;
-    g.nbk = (g.Lk + g.TK - 1) / g.TK;
+    g.nbj = (g.Lj + kTile - 1) / kTile;
+    g.nbk = (g.Lk + kTile - 1) / kTile;
     g.ntiles = g.nbj * g.nbk;
-    g.nsteps = g.Li + g.TJ + g.TK - 2;
-    g.exj_tile = (long)(g.Li + g.TK - 1) * g.TK * 5;
-    g.exk_tile = (long)(g.Li + g.TJ - 1) * g.TJ * 5;
+    g.nsteps = g.Li + 2 * kTile - 2;
+    g.exj_tile = g.exk_tile = (long)(g.Li + kTile - 1) * kTile * 5;
     return g;
 }
 
@@ -348,44 +361,6 @@ __device__ inline void xstore_bits(double *p, unsigned long long v)
 __device__ inline void xstore(double *p, double v)
 {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// Take the five values of one exchange slot (component x at slot + x *
-// stride): `pre` holds what was loaded a step earlier; components still at the sentinel are polled until the
-// producer's store arrives, each poll reloading the later components too,
-// so that a slot that was late costs one round trip more, not one per
-// component.  The wait is bounded: running out sets *err and every later
-// wait of the launch gives up at once, so the sweep always ends (the host
-// then reports the failure).  With `reset` the slot is set back to the
-// sentinel for the next sweep (otherwise the host refills the region).
-__device__ inline void ex_take(double *slot, int stride, const unsigned long long *pre, double *v, int *err,
-                               bool &failed, bool reset)
-{
-    unsigned long long cur[5];
-#pragma unroll
-    for (int x = 0; x < 5; x++) cur[x] = pre[x];
-#pragma unroll
-    for (int x = 0; x < 5; x++) {
-        unsigned long long b = cur[x];
-        if (b == kSentinel) {
-            for (long spins = 0; !failed; spins++) {
-                b = xload_bits(slot + x * stride);
-#pragma unroll
-                for (int y = x + 1; y < 5; y++)
-                    if (cur[y] == kSentinel) cur[y] = xload_bits(slot + y * stride);
-                if (b != kSentinel) break;
-                if ((spins & 1023) == 1023 &&
-                    (spins > (1L << 21) || __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) {
-                    atomicOr(err, 1);
-                    failed = true;
-                }
-                __builtin_amdgcn_s_sleep(1);
-            }
-            if (failed) b = 0;
-        }
-        v[x] = __longlong_as_double((long long)b);
-        if (reset) xstore_bits(slot + x * stride, kSentinel);
-    }
 }
 
 // LDS barrier that does not wait for outstanding global loads (the
@@ -410,25 +385,20 @@ __device__ inline void lds_barrier()
 // (CT = min(32, 4096/TT)).
 // Sweep side: thread x is lane x.  LDS holds [CT][TT] doubles per field
 // with the line index XOR-swizzled by ii (no bank conflicts either way).
-// steps a layout kernel transposes at a time: CT * TT <= kSlElems
-constexpr int kSlElems = 4096;
-constexpr int sl_ct_of(int tt) { return kSlElems / tt < 32 ? kSlElems / tt : 32; }
-// the SA return pass (one value per node) takes at most 16: measured on
-// 64-lane tiles, 0.86 against 1.25 ms (the two gathers and the flow add are
-// faster at 32)
-constexpr int sa_ret_ct_of(int tt) { return sl_ct_of(tt) < 16 ? sl_ct_of(tt) : 16; }
-// dynamic LDS of the flow layout kernels: [2][CT][TT] doubles
-constexpr size_t sl_lds_bytes(int tt) { return 2 * (size_t)sl_ct_of(tt) * tt * sizeof(double); }
+// steps a layout kernel transposes at a time
+constexpr int kSlCt = 32;
+// the SA return pass (one value per node) takes 16: measured 0.86 against
+// 1.25 ms (the two gathers and the flow add are faster at 32)
+constexpr int kSaRetCt = 16;
 
 // node index of (tile, line, li), li in range
 __device__ inline long sl_nat(const Ext &e, const SlGeom &g, int tile, int line, int li)
 {
-    const int tj = line & (g.TJ - 1), tk = line >> g.lgTJ;
-    return e.ix(e.is1 + li, e.js1 + (tile % g.nbj) * g.TJ + tj, e.ks1 + (tile / g.nbj) * g.TK + tk);
+    return e.ix(e.is1 + li, e.js1 + (tile % g.nbj) * kTile + line % kTile, e.ks1 + (tile / g.nbj) * kTile + line / kTile);
 }
 __device__ inline bool sl_line_ok(const SlGeom &g, int tile, int line)
 {
-    return (tile % g.nbj) * g.TJ + (line & (g.TJ - 1)) < g.Lj && (tile / g.nbj) * g.TK + (line >> g.lgTJ) < g.Lk;
+    return (tile % g.nbj) * kTile + line % kTile < g.Lj && (tile / g.nbj) * kTile + line / kTile < g.Lk;
 }
 
 // csnd: the sound speed (component 7 of pri_v), tterm: the time term
@@ -442,19 +412,17 @@ __device__ inline const double *gather_src(int f, long N, const double *q, const
 
 // Gather the operands of every node into the sweep layout, a field pair at
 // a time (each lane then stores whole 16-byte pairs), from pair fp0 on (0:
-// all kSlF fields, kSlGeoPairs: all but the grid's).  TT is a template
-// parameter so that a thread's CT loads are issued back to back.
-template <int TT>
+// all kSlF fields, kSlGeoPairs: all but the grid's).
 __device__ inline void sl_gather_tile(const Ext &e, const SlGeom &g, int tile, const double *__restrict__ q,
                                       const double *__restrict__ dxidx, const double *__restrict__ inv_j,
                                       const double *__restrict__ csnd, const double *__restrict__ tterm,
                                       const double *__restrict__ rhs, double *__restrict__ sl, int fp0,
                                       double *buf /* [2][CT][TT] LDS, swizzled */)
 {
-    constexpr int CT = sl_ct_of(TT), lstep = TT / CT;
+    constexpr int CT = kSlCt, TT = kLanes, lstep = TT / CT;
     const int x = threadIdx.x;
     const int ii_n = x % CT;
-    const int tj = x & (g.TJ - 1), tk = x >> g.lgTJ;
+    const int tj = x % kTile, tk = x / kTile;
     const bool me_ok = sl_line_ok(g, tile, x);
     const long N = e.n;
     double2 *sl2 = reinterpret_cast<double2 *>(sl);
@@ -465,7 +433,7 @@ __device__ inline void sl_gather_tile(const Ext &e, const SlGeom &g, int tile, c
 #pragma unroll
             for (int m = 0; m < CT; m++) {
                 const int line = m * lstep + x / CT;
-                const int li = t0 + ii_n - (line & (g.TJ - 1)) - (line >> g.lgTJ);
+                const int li = t0 + ii_n - (line % kTile) - (line / kTile);
                 nat[m] = (t0 + ii_n < g.nsteps && li >= 0 && li < g.Li && sl_line_ok(g, tile, line))
                              ? (int)sl_nat(e, g, tile, line, li) : -1;
             }
@@ -496,29 +464,27 @@ __device__ inline void sl_gather_tile(const Ext &e, const SlGeom &g, int tile, c
     }
 }
 
-template <int TT>
-__global__ void __launch_bounds__(TT) k_sl_gather(Ext e, SlGeom g, const double *__restrict__ q,
+__global__ void __launch_bounds__(kLanes) k_sl_gather(Ext e, SlGeom g, const double *__restrict__ q,
                                                   const double *__restrict__ dxidx,
                                                   const double *__restrict__ inv_j,
                                                   const double *__restrict__ csnd,
                                                   const double *__restrict__ tterm,
                                                   const double *__restrict__ rhs, double *__restrict__ sl, int fp0)
 {
-    extern __shared__ double buf[];
-    sl_gather_tile<TT>(e, g, (int)blockIdx.x, q, dxidx, inv_j, csnd, tterm, rhs, sl, fp0, buf);
+    __shared__ double buf[2 * kSlCt * kLanes];
+    sl_gather_tile(e, g, (int)blockIdx.x, q, dxidx, inv_j, csnd, tterm, rhs, sl, fp0, buf);
 }
 
 // q += dq (:568-574): the backward sweep left q + dq in the result slots of
 // the sweep layout; this pass moves it to q in the natural layout, same walk
 // as the gather, one field pair at a time.
-template <int TT>
 __device__ inline void sl_add_tile(const Ext &e, const SlGeom &g, int tile, const double *__restrict__ sl,
                                    double *__restrict__ q, double *buf /* [2][CT][TT] LDS, swizzled */)
 {
-    constexpr int CT = sl_ct_of(TT), lstep = TT / CT;
+    constexpr int CT = kSlCt, TT = kLanes, lstep = TT / CT;
     const int x = threadIdx.x;
     const int ii_n = x % CT;
-    const int tj = x & (g.TJ - 1), tk = x >> g.lgTJ;
+    const int tj = x % kTile, tk = x / kTile;
     const bool me_ok = sl_line_ok(g, tile, x);
     const long N = e.n;
     // the results are fields 19-23: the upper half of pair 9 (whose lower
@@ -530,7 +496,7 @@ __device__ inline void sl_add_tile(const Ext &e, const SlGeom &g, int tile, cons
 #pragma unroll
             for (int m = 0; m < CT; m++) {
                 const int line = m * lstep + x / CT;
-                const int li = t0 + ii_n - (line & (g.TJ - 1)) - (line >> g.lgTJ);
+                const int li = t0 + ii_n - (line % kTile) - (line / kTile);
                 nat[m] = (t0 + ii_n < g.nsteps && li >= 0 && li < g.Li && sl_line_ok(g, tile, line))
                              ? (int)sl_nat(e, g, tile, line, li) : -1;
             }
@@ -564,32 +530,21 @@ __device__ inline void sl_add_tile(const Ext &e, const SlGeom &g, int tile, cons
     }
 }
 
-template <int TT>
-__global__ void __launch_bounds__(TT) k_sl_add(Ext e, SlGeom g, const double *__restrict__ sl,
+__global__ void __launch_bounds__(kLanes) k_sl_add(Ext e, SlGeom g, const double *__restrict__ sl,
                                                double *__restrict__ q)
 {
-    extern __shared__ double buf[];
-    sl_add_tile<TT>(e, g, (int)blockIdx.x, sl, q, buf);
+    __shared__ double buf[2 * kSlCt * kLanes];
+    sl_add_tile(e, g, (int)blockIdx.x, sl, q, buf);
 }
 
-template <int TT>
-static void launch_layout(hipStream_t s, int which, const Ext &e, const SlGeom &g, const Fields &f,
-                          const LuWs &ws, int fp0)
+static void launch_layout(hipStream_t s, int which, const Ext &e, const SlGeom &g, const Fields &f, const LuWs &ws,
+                          int fp0 = 0)
 {
-    const size_t lds = sl_lds_bytes(TT);
     if (which == 0)
-        hipLaunchKernelGGL(k_sl_gather<TT>, dim3((unsigned)g.ntiles), dim3(TT), lds, s, e, g, f.q, f.dxidx,
-                           f.inv_j, f.pri + 6 * e.n, f.w_diag, f.rhs, ws.sl, fp0);
+        hipLaunchKernelGGL(k_sl_gather, dim3((unsigned)g.ntiles), dim3(kLanes), 0, s, e, g, f.q, f.dxidx, f.inv_j,
+                           f.pri + 6 * e.n, f.w_diag, f.rhs, ws.sl, fp0);
     else
-        hipLaunchKernelGGL(k_sl_add<TT>, dim3((unsigned)g.ntiles), dim3(TT), lds, s, e, g, ws.sl, f.q);
-}
-
-static void launch_layout_tt(hipStream_t s, int which, const Ext &e, const SlGeom &g, const Fields &f,
-                             const LuWs &ws, int fp0 = 0)
-{
-    if (g.TT == 256) launch_layout<256>(s, which, e, g, f, ws, fp0);
-    else if (g.TT == 128) launch_layout<128>(s, which, e, g, f, ws, fp0);
-    else launch_layout<64>(s, which, e, g, f, ws, fp0);
+        hipLaunchKernelGGL(k_sl_add, dim3((unsigned)g.ntiles), dim3(kLanes), 0, s, e, g, ws.sl, f.q);
 }
 
 // Fill exchange slots with the sentinel.
@@ -610,183 +565,445 @@ __device__ inline double lu_node_radii(const double *op, double *r)
     return lu_diag(op[kSlT], r);
 }
 
-// One step of a lane: combine, solve, push.  op = the node's operands, dg
-// and r its diagonal and spectral radii.
+// -------------------------------------------------- pipelined tile sweep
+// The sweep of one 8 x 8 tile by four wavefronts that run side by side.  The
+// dependency chain of a sweep is its sequence of steps (Li + Lj + Lk of
+// them from corner to corner of a block, and a hop through memory at every
+// tile edge), and a step done by one wavefront took 1.7 us: the operands'
+// loads, the radii and diagonal (square roots, divisions) and the wait for
+// the neighbours' slots all stood in the chain.  Here the chain keeps only
+// what depends on the neighbours:
+//   wave 0     solves: combine, three products, results out.  It reads
+//              prepared operands and neighbour values from LDS a step
+//              ahead; inside the tile a product passes to the next lane by
+//              ds_bpermute (k, formed first) and DPP (j), so no barrier is
+//              on its path.
+//   preparing  step s, s + 1, ... in turn: two steps' loads in flight
+//   waves      each, radii, 1/(diag inv_j) and the scaled metric rows
+//              written to a ring of kPipeRing steps.
+//   last wave  fetches the j and k neighbour tiles' products from the
+//              exchange slots, up to eight steps at a time, into a ring, and
+//              sets the slots back to the sentinel.
+// The waves meet only through counters in LDS (a wave's LDS operations
+// take effect in order): the others count what is ready, wave 0 what it has
+// used.  Every wait is on a wave that waits for less: preparing waves wait
+// for ring space (wave 0), wave 0 for operands and for slots, the slot
+// wave for the neighbouring tiles with a bounded poll; running out sets
+// *err and `stop`, at which every wait of the workgroup ends.
+// What bounds it: wave 0's instruction issue (about 215 instructions a step,
+// of which 80 are the FP64 arithmetic, at one per four cycles or more:
+// 0.57-0.65 us a step) and 2.6 us a hop; on large batches the HBM traffic.
+// Forward sweep, before (one wavefront a tile) and after: 33^3 184 -> 80 us,
+// 129^3 748 -> 330, 193^3 1218 -> 750, 12 blocks of 3.2 M nodes in all
+// 507 -> 350, 40 blocks of 98 M nodes 6.19 -> 6.10 ms (4.7 TB/s).  Tiles of
+// 16 x 16, 16 x 8 and 16 x 4 lines of the one-wavefront form were slower at
+// every one of these sizes and are gone.
+// A lane with nothing to do at a step takes part with rhs, 1/(diag inv_j)
+// and so its products zero (the padding of the sweep layout holds zeros or
+// another block's operands, finite either way), and no lane branches.
+constexpr int kPipeRing = 4;    // steps of prepared operands in LDS
+constexpr int kPipeXRing = 16;  // steps of neighbour values in LDS
+constexpr int kPipePrep = 2;    // preparing waves
+constexpr int kPipeThreads = 64 * (1 + kPipePrep + 1);
+
+// a prepared step, pairs of doubles per lane: rhs 0-4 (dq* in the backward
+// sweep), 1/(diag inv_j), then forward u, v, w, |u|^2/2, a1, the time term,
+// r of the i row, unused; backward q 0-4, 1/rho, |u|^2/2, a1, r of the i
+// row, the time term; then x, y, z, U of the three rows and r of the j and
+// the k row
 template <int DIR>
-__device__ inline void lu_node(const double *op, double dg, const double *r, const double *ta, const double *tb,
-                               const double *tc, double gamma, double *res, double *pa, double *pb, double *pc)
+struct PipeLds {
+    static constexpr int kRow0 = DIR > 0 ? 7 : 8;
+    static constexpr int kPairs = kRow0 + 7;
+    double2 op[kPipeRing][kPairs][64];
+    double x[kPipeXRing][2][5][kTile];
+    int prep[kPipePrep];  // first step each preparing wave has not finished
+    int xready;           // first step whose neighbour values are not there
+    int done;             // steps wave 0 has finished with
+    int stop;
+};
+
+__device__ inline int lds_get(const int *p)
 {
-    if (DIR > 0) lu_fwd_combine(op + kSlOut, ta, tb, tc, dg, op[9], res);
-    else lu_bwd_combine(op + kSlOut, ta, tb, tc, dg, op[9], res);
-    jac_mv_r<DIR>(op + kSlQ, op[0], op[1], op[2], op[9], r[0], gamma, res, pa);
-    jac_mv_r<DIR>(op + kSlQ, op[3], op[4], op[5], op[9], r[1], gamma, res, pb);
-    jac_mv_r<DIR>(op + kSlQ, op[6], op[7], op[8], op[9], r[2], gamma, res, pc);
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+// publish after the wave's earlier LDS operations (which take effect in
+// order; the barrier is for the compiler)
+__device__ inline void lds_post(int *p, int v)
+{
+    __asm__ volatile("" ::: "memory");
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    __asm__ volatile("" ::: "memory");
 }
 
-// Persistent tile sweep over the sweep layout.  The forward sweep numbers
-// tiles bj + nbj*bk and waits only on lower numbers; the backward sweep runs
-// the same tiles mirrored (lane (tj,tk) schedules as (TJ-1-tj, TK-1-tk)) and
-// is dispatched in reverse order.  Either way every wait is on a tile that
-// was dispatched earlier, so it is running or done.
-// With q (backward sweep only) the update q += dq is fused: each node's dq
-// is added to its q operand and stored into the natural layout (e: the
-// block's ranges), in place of writing dq to the sweep layout.
-template <int DIR, int TJ, int TK>
-__device__ inline void lu_tiles_body(const SlGeom &g, int tile, double *__restrict__ sl, double gamma, double *ex,
-                                     int *err, double (*pj)[5][TJ * TK], double (*pk)[5][TJ * TK],
-                                     const Ext *e = nullptr, double *__restrict__ q = nullptr)
+// wait until f() >= need (or the workgroup stops); the bound, some seconds,
+// is only there so that no mistake can hang the device
+template <typename F>
+__device__ inline int lds_wait(F f, int need, int *stop, int *err)
 {
-    constexpr int TT = TJ * TK;
-    const int bj = tile % g.nbj, bk = tile / g.nbj;
-    const int l = threadIdx.x, tj = l % TJ, tk = l / TJ;
-    const int lj = bj * TJ + tj, lk = bk * TK + tk;
-    const bool active = lj < g.Lj && lk < g.Lk;
-    const bool fuse_add = DIR < 0 && q != nullptr;
-    const long qN = fuse_add ? e->n : 0;
-    const long nat0 = fuse_add && active ? e->ix(e->is1, e->js1 + lj, e->ks1 + lk) : 0;
-    // schedule coordinates (mirrored for the backward sweep)
-    const int sj = DIR > 0 ? tj : TJ - 1 - tj, sk = DIR > 0 ? tk : TK - 1 - tk;
-    // the j / k predecessor: outside the computed range (0), in the
-    // neighbouring tile (exchange slot) or the previous lane (LDS)
-    const bool j_ring = DIR > 0 ? lj == 0 : lj + 1 >= g.Lj;
-    const bool k_ring = DIR > 0 ? lk == 0 : lk + 1 >= g.Lk;
-    const bool j_in = !j_ring && sj == 0, k_in = !k_ring && sk == 0;
-    const int lpj = l - DIR, lpk = l - DIR * TJ;
-    // this lane's products leave the tile when it is last in schedule and a
-    // neighbouring tile exists on that side
-    const bool j_out = sj == TJ - 1 && (DIR > 0 ? bj + 1 < g.nbj : bj > 0);
-    const bool k_out = sk == TK - 1 && (DIR > 0 ? bk + 1 < g.nbk : bk > 0);
-    double *exj = ex, *exk = ex + (long)g.ntiles * g.exj_tile;
-    // slots: j region [tile][d = pos + sk][5][tk], k region [tile][d = pos + sj][5][tj]:
-    // the lanes of a tile face store and load one component of their slots
-    // as one contiguous run (TK or TJ doubles)
-    double *jin = exj + (long)(DIR > 0 ? tile - 1 : tile + 1) * g.exj_tile + tk;
-    double *kin = exk + (long)(DIR > 0 ? tile - g.nbj : tile + g.nbj) * g.exk_tile + tj;
-    double *jout = exj + (long)tile * g.exj_tile + tk;
-    double *kout = exk + (long)tile * g.exk_tile + tj;
-    bool failed = false;
-    double ta[5] = {0, 0, 0, 0, 0};
-    double opA[kSlF], opB[kSlF];
-    unsigned long long xjA[5], xkA[5], xjB[5], xkB[5];
+    int v = __builtin_amdgcn_readfirstlane(f());
+    for (long n = 0; v < need && !__builtin_amdgcn_readfirstlane(lds_get(stop)); n++) {
+        if (n > (1L << 27)) {
+            atomicOr(err, 1);
+            lds_post(stop, 1);
+        }
+        v = __builtin_amdgcn_readfirstlane(f());
+    }
+    __asm__ volatile("" ::: "memory");
+    return v;
+}
 
+// the value of the lane one (j) or eight (k) behind in the sweep's order
+template <int DIR>
+__device__ inline double lane_behind_j(double v)
+{
+    const long long b = __double_as_longlong(v);
+    constexpr int ctrl = DIR > 0 ? 0x111 : 0x101;  // row_shr:1, row_shl:1
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, ctrl, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), ctrl, 0xf, 0xf, true);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+__device__ inline double lane_from(int addr, double v)
+{
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_ds_bpermute(addr, (int)b);
+    const int hi = __builtin_amdgcn_ds_bpermute(addr, (int)(b >> 32));
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+
+// preparing wave w: steps w, w + kPipePrep, ...
+template <int DIR>
+__device__ inline void pipe_prepare(const SlGeom &g, int tile, int w, const double *__restrict__ sl, double gamma,
+                                    PipeLds<DIR> &L, int *err)
+{
+    const int l = threadIdx.x & 63, tj = l % kTile, tk = l / kTile;
+    const bool active = (tile % g.nbj) * kTile + tj < g.Lj && (tile / g.nbj) * kTile + tk < g.Lk;
+    // row of the layout at which this lane's line starts
+    const int t0 = tj + tk;
     auto row = [&](int s) { return DIR > 0 ? s : g.nsteps - 1 - s; };
-    auto on_at = [&](int s) {
-        const int pos = s - sj - sk;
-        return active && pos >= 0 && pos < g.Li;
-    };
-    // Issue the loads of step s (operands and exchange values).  The loads
-    // are unconditional -- lanes with nothing to do at step s read a valid
-    // slot and ignore it -- so the compiler can count outstanding loads
-    // exactly and the prefetch stays in flight across the previous step.
-    const int xj_last = g.Li + TK - 2, xk_last = g.Li + TJ - 2;
-    // In a tile with a neighbour on that side every lane loads from the
-    // face lanes' slots of the step (so one load instruction touches one
-    // contiguous run); otherwise from the start of the region.  Only the
-    // face lanes use what they load.
-    const bool j_pred = DIR > 0 ? bj > 0 : bj + 1 < g.nbj;
-    const bool k_pred = DIR > 0 ? bk > 0 : bk + 1 < g.nbk;
-    const double *jsrc = j_pred ? jin : ex;
-    const double *ksrc = k_pred ? kin : ex;
-    auto fetch = [&](int s, double *op, unsigned long long *xj, unsigned long long *xk) {
-        const int sc = min(s, g.nsteps - 1);
-        const double2 *src = reinterpret_cast<const double2 *>(sl + g.slot(tile, row(sc), 0, l));
+    auto fetch = [&](int s, double *op) {
+        const double2 *src = reinterpret_cast<const double2 *>(sl + g.slot(tile, row(min(s, g.nsteps - 1)), 0, l));
 #pragma unroll
         for (int f = 0; f < kSlF / 2; f++) {
-            const double2 v = src[(long)f * TT];
+            const double2 v = src[f * 64];
             op[2 * f] = v.x;
             op[2 * f + 1] = v.y;
         }
-        // a face lane (sj == 0 / sk == 0) takes slot pos + sk = s / pos + sj = s
-        const int dj = j_pred ? min(max(s, 0), xj_last) : 0;
-        const int dk = k_pred ? min(max(s, 0), xk_last) : 0;
-#pragma unroll
-        for (int x = 0; x < 5; x++) xj[x] = xload_bits(jsrc + (long)dj * TK * 5 + x * TK);
-#pragma unroll
-        for (int x = 0; x < 5; x++) xk[x] = xload_bits(ksrc + (long)dk * TJ * 5 + x * TJ);
     };
-    auto step = [&](int s, const double *op, const unsigned long long *xj, const unsigned long long *xk) {
-        const int p = s & 1;
-        if (on_at(s)) {
-            const int pos = s - sj - sk;
-            // from the node's own operands, ahead of the waits on its
-            // neighbours' values
-            double rad[3];
-            const double dg = lu_node_radii(op, rad);
-            double tb[5], tc[5], res[5], pa[5], pb[5], pc[5];
-            if (j_ring) {
+    auto prepare = [&](int s, double *op) {
+        if (s >= g.nsteps) return;
+        const int li = row(s) - t0;
+        const bool on = active && li >= 0 && li < g.Li;
+        if (!on) {
+            op[kSlQ] = 1.0;
 #pragma unroll
-                for (int x = 0; x < 5; x++) tb[x] = 0.0;
-            } else if (j_in) {
-                ex_take(jin + (long)(pos + sk) * TK * 5, TK, xj, tb, err, failed, !g.refill);
-            } else {
-#pragma unroll
-                for (int x = 0; x < 5; x++) tb[x] = pj[p ^ 1][x][lpj];
-            }
-            if (k_ring) {
-#pragma unroll
-                for (int x = 0; x < 5; x++) tc[x] = 0.0;
-            } else if (k_in) {
-                ex_take(kin + (long)(pos + sj) * TJ * 5, TJ, xk, tc, err, failed, !g.refill);
-            } else {
-#pragma unroll
-                for (int x = 0; x < 5; x++) tc[x] = pk[p ^ 1][x][lpk];
-            }
-            lu_node<DIR>(op, dg, rad, ta, tb, tc, gamma, res, pa, pb, pc);
-            if (fuse_add) {
-                const long n = nat0 + (g.Li - 1 - pos);
-#pragma unroll
-                for (int x = 0; x < 5; x++) q[x * qN + n] = op[kSlQ + x] + res[x];
-            } else {
-                // the backward sweep leaves q + dq (its q operand plus the
-                // result, the update's one addition), the forward sweep dq*;
-                // stored as whole 16-byte pairs, the first one with the
-                // diagonal the lane read (its value unchanged)
-                double o[5];
-#pragma unroll
-                for (int x = 0; x < 5; x++) o[x] = DIR < 0 ? op[kSlQ + x] + res[x] : res[x];
-                double2 *dst = reinterpret_cast<double2 *>(sl + g.slot(tile, row(s), kSlT, l));
-                dst[0] = make_double2(op[kSlT], o[0]);
-                dst[TT] = make_double2(o[1], o[2]);
-                dst[2 * TT] = make_double2(o[3], o[4]);
-            }
-#pragma unroll
-            for (int x = 0; x < 5; x++) {
-                ta[x] = pa[x];
-                pj[p][x][l] = pb[x];
-                pk[p][x][l] = pc[x];
-            }
-            if (j_out) {
-#pragma unroll
-                for (int x = 0; x < 5; x++) xstore(jout + (long)(pos + sk) * TK * 5 + x * TK, pb[x]);
-            }
-            if (k_out) {
-#pragma unroll
-                for (int x = 0; x < 5; x++) xstore(kout + (long)(pos + sj) * TJ * 5 + x * TJ, pc[x]);
-            }
+            for (int x = 0; x < 5; x++) op[kSlOut + x] = 0.0;
         }
-        lds_barrier();
+        double rad[3];
+        const double ri = 1.0 / op[kSlQ], sc = 0.5 * op[9];
+        const LuState t = lu_state(op + kSlQ, ri, gamma);
+        const double dg = lu_node_radii(op, rad);
+        const double rd = on ? lu_rdiag(dg, op[9]) : 0.0;
+        LuRow m[3];
+#pragma unroll
+        for (int d = 0; d < 3; d++) m[d] = lu_row<DIR>(t, op[3 * d], op[3 * d + 1], op[3 * d + 2], sc, rad[d]);
+        lds_wait([&] { return lds_get(&L.done); }, s - kPipeRing + 1, &L.stop, err);
+        double2 *o = &L.op[s % kPipeRing][0][l];
+        const double *rhs = op + kSlOut;
+        o[0] = make_double2(rhs[0], rhs[1]);
+        o[64] = make_double2(rhs[2], rhs[3]);
+        o[2 * 64] = make_double2(rhs[4], rd);
+        if (DIR > 0) {
+            o[3 * 64] = make_double2(t.u, t.v);
+            o[4 * 64] = make_double2(t.w, t.q2h);
+            o[5 * 64] = make_double2(t.a1, op[kSlT]);
+            o[6 * 64] = make_double2(m[0].r, 0.0);
+        } else {
+            o[3 * 64] = make_double2(op[kSlQ], op[kSlQ + 1]);
+            o[4 * 64] = make_double2(op[kSlQ + 2], op[kSlQ + 3]);
+            o[5 * 64] = make_double2(op[kSlQ + 4], ri);
+            o[6 * 64] = make_double2(t.q2h, t.a1);
+            o[7 * 64] = make_double2(m[0].r, op[kSlT]);
+        }
+        double2 *r = o + PipeLds<DIR>::kRow0 * 64;
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            r[2 * d * 64] = make_double2(m[d].x, m[d].y);
+            r[(2 * d + 1) * 64] = make_double2(m[d].z, m[d].U);
+        }
+        r[6 * 64] = make_double2(m[1].r, m[2].r);
+        lds_post(&L.prep[w], s + kPipePrep);
     };
-
-    // operands are loaded one step ahead (two register sets in rotation):
-    // measured faster than two steps ahead with three sets (256^3 block,
-    // 16x8 tiles: 1.83 against 2.05 ms per forward sweep); steps past the
-    // end are no-ops that keep the barriers uniform
-    fetch(0, opA, xjA, xkA);
-    for (int s = 0; s < g.nsteps; s += 2) {
-        fetch(s + 1, opB, xjB, xkB);
-        step(s, opA, xjA, xkA);
-        fetch(s + 2, opA, xjA, xkA);
-        step(s + 1, opB, xjB, xkB);
+    double a[kSlF], b[kSlF];
+    fetch(w, a);
+    fetch(w + kPipePrep, b);
+    for (int s = w; s < g.nsteps; s += 2 * kPipePrep) {
+        prepare(s, a);
+        fetch(s + 2 * kPipePrep, a);
+        prepare(s + kPipePrep, b);
+        fetch(s + 3 * kPipePrep, b);
     }
 }
 
-template <int DIR, int TJ, int TK>
-__global__ void __launch_bounds__(TJ *TK) k_lu_tiles(SlGeom g, double *__restrict__ sl, double gamma,
-                                                      double *ex, int *err, Ext e, double *q)
+// last wave: the neighbour tiles' products on the j side (lanes 0-31) and
+// the k side (lanes 32-63).  Lane (face, r, f) loads steps d0 + r and
+// d0 + 4 + r of face line f; the leading steps whose lines have all arrived
+// go to the ring.  line_ok, src: of the lane's face line (no neighbour on
+// that side: false, the values are zeros).
+template <int DIR>
+__device__ inline void pipe_fetch(const SlGeom &g, bool line_ok, int skew, double *src, PipeLds<DIR> &L, int *err)
 {
-    __shared__ double pj[2][5][TJ * TK], pk[2][5][TJ * TK];
-    const int tile = DIR > 0 ? (int)blockIdx.x : g.ntiles - 1 - (int)blockIdx.x;
-    lu_tiles_body<DIR, TJ, TK>(g, tile, sl, gamma, ex, err, pj, pk, &e, q);
+    const int l = threadIdx.x & 63, face = l >> 5, r = (l >> 3) & 3, f = l & 7;
+    long spins = 0;
+    for (int d0 = 0; d0 < g.nsteps;) {
+        lds_wait([&] { return lds_get(&L.done); }, d0 + 8 - kPipeXRing, &L.stop, err);
+        if (__builtin_amdgcn_readfirstlane(lds_get(&L.stop))) return;
+        unsigned long long b[2][5];
+        bool need[2], ok[2];
+        double *p[2];
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const int d = d0 + 4 * h + r, pos = d - skew;
+            need[h] = line_ok && pos >= 0 && pos < g.Li;
+            p[h] = src + (long)(need[h] ? d : 0) * kTile * 5 + f;
+#pragma unroll
+            for (int x = 0; x < 5; x++) b[h][x] = xload_bits(p[h] + x * kTile);
+        }
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            ok[h] = true;
+#pragma unroll
+            for (int x = 0; x < 5; x++) ok[h] = ok[h] && b[h][x] != kSentinel;
+        }
+        // rows of lanes that wait, both faces: bits 8 r .. 8 r + 7
+        const unsigned long long m0 = __ballot(need[0] && !ok[0]), m1 = __ballot(need[1] && !ok[1]);
+        const unsigned late0 = (unsigned)m0 | (unsigned)(m0 >> 32), late1 = (unsigned)m1 | (unsigned)(m1 >> 32);
+        const int n = late0 ? __builtin_ctz(late0) >> 3 : late1 ? 4 + (__builtin_ctz(late1) >> 3) : 8;
+        if (n == 0) {
+            spins++;
+            if ((spins & 1023) == 0 &&
+                (spins > (1L << 21) || __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) {
+                atomicOr(err, 1);
+                lds_post(&L.stop, 1);
+            }
+            __builtin_amdgcn_s_sleep(1);
+            continue;
+        }
+        spins = 0;
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+            if (4 * h + r < n) {
+                double *o = &L.x[(d0 + 4 * h + r) % kPipeXRing][face][0][f];
+#pragma unroll
+                for (int x = 0; x < 5; x++) o[x * kTile] = need[h] ? __longlong_as_double((long long)b[h][x]) : 0.0;
+                if (need[h]) {
+#pragma unroll
+                    for (int x = 0; x < 5; x++) xstore_bits(p[h] + x * kTile, kSentinel);
+                }
+            }
+        d0 += n;
+        lds_post(&L.xready, d0);
+    }
+}
+
+// wave 0: the solve
+template <int DIR>
+__device__ inline void pipe_solve(const SlGeom &g, int tile, double *__restrict__ sl, double gamma, double *jout,
+                                  double *kout, bool pred, bool j_succ, bool k_succ, PipeLds<DIR> &L, int *err,
+                                  const Ext *e, double *__restrict__ q)
+{
+    const int bj = tile % g.nbj, bk = tile / g.nbj;
+    const int l = threadIdx.x & 63, tj = l % kTile, tk = l / kTile;
+    const int lj = bj * kTile + tj, lk = bk * kTile + tk;
+    const bool active = lj < g.Lj && lk < g.Lk;
+    const int sj = DIR > 0 ? tj : kTile - 1 - tj, sk = DIR > 0 ? tk : kTile - 1 - tk;
+    const bool fuse_add = DIR < 0 && q != nullptr;
+    const long qN = fuse_add ? e->n : 0;
+    const long nat0 = fuse_add && active ? e->ix(e->is1, e->js1 + lj, e->ks1 + lk) : 0;
+    const bool j_out = j_succ && sj == kTile - 1, k_out = k_succ && sk == kTile - 1;
+    const int behind_k = ((l - DIR * kTile) & 63) * 4;
+    double ta[5] = {0, 0, 0, 0, 0}, tb[5] = {0, 0, 0, 0, 0}, tc[5] = {0, 0, 0, 0, 0};
+    constexpr int kRow0 = PipeLds<DIR>::kRow0, kRows = PipeLds<DIR>::kPairs - kRow0;
+    double2 E[2][kRow0], R[2][kRows];
+    double fj[5], fk[5];
+    int have = 0, xhave = pred ? 0 : g.nsteps;
+    const int last = g.nsteps - 1;
+    // The LDS reads of a step, without a branch around any of them, so that
+    // the compiler's wait counts are exact and they stay in flight.  After
+    // the last step they read a slot that nobody uses.
+    auto wait_ops = [&](int s) {
+        if (have <= s)
+            have = lds_wait([&] {
+                int v = lds_get(&L.prep[0]);
+                for (int w = 1; w < kPipePrep; w++) v = min(v, lds_get(&L.prep[w]));
+                return v;
+            }, s + 1, &L.stop, err);
+    };
+    auto load_state = [&](int s, double2 *O) {
+        const double2 *o = &L.op[s % kPipeRing][0][l];
+#pragma unroll
+        for (int p = 0; p < kRow0; p++) O[p] = o[p * 64];
+    };
+    auto load_rows = [&](int s, double2 *O) {
+        const double2 *o = &L.op[s % kPipeRing][kRow0][l];
+#pragma unroll
+        for (int p = 0; p < kRows; p++) O[p] = o[p * 64];
+    };
+    auto wait_face = [&](int s) {
+        if (xhave <= s) xhave = lds_wait([&] { return lds_get(&L.xready); }, s + 1, &L.stop, err);
+    };
+    auto load_face = [&](int s) {
+        const double *v = &L.x[s % kPipeXRing][0][0][0];
+#pragma unroll
+        for (int x = 0; x < 5; x++) fj[x] = v[x * kTile + tk];
+#pragma unroll
+        for (int x = 0; x < 5; x++) fk[x] = v[(5 + x) * kTile + tj];
+    };
+    double2 *dst = reinterpret_cast<double2 *>(sl + g.slot(tile, DIR > 0 ? 0 : g.nsteps - 1, kSlT, l));
+    double *jo = jout - (kTile - 1) * kTile * 5 + tk, *ko = kout - (kTile - 1) * kTile * 5 + tj;
+    // step s with the operands E, R, while those of the next step are read
+    // into NE, NR
+    auto step = [&](int s, const double2 *E, const double2 *R, double2 *NE, double2 *NR) {
+        wait_ops(min(s + 1, last));
+        load_state(s + 1, NE);
+        const int pos = s - sj - sk;
+        const bool on = active && pos >= 0 && pos < g.Li;
+        const double rhs[5] = {E[0].x, E[0].y, E[1].x, E[1].y, E[2].x};
+        double res[5], qv[5], pb[5], pc[5];
+        LuState t;
+        double tterm, r0;
+#pragma unroll
+        for (int x = 0; x < 5; x++) {
+            tb[x] = sj == 0 ? fj[x] : tb[x];
+            tc[x] = sk == 0 ? fk[x] : tc[x];
+        }
+        if (DIR > 0) {
+            t = {E[3].x, E[3].y, E[4].x, E[4].y, E[5].x};
+            tterm = E[5].y;
+            r0 = E[6].x;
+            lu_fwd_combine(rhs, ta, tb, tc, E[2].y, res);
+        } else {
+            qv[0] = E[3].x; qv[1] = E[3].y; qv[2] = E[4].x; qv[3] = E[4].y; qv[4] = E[5].x;
+            const double ri = E[5].y;
+            t = {qv[1] * ri, qv[2] * ri, qv[3] * ri, E[6].x, E[6].y};
+            r0 = E[7 % kRow0].x;
+            tterm = E[7 % kRow0].y;
+            lu_bwd_combine(rhs, ta, tb, tc, E[2].y, res);
+        }
+        const double dp = lu_dp(t, gamma, res);
+        lu_product(t, {R[4].x, R[4].y, R[5].x, R[5].y, R[6].y}, dp, res, pc);
+#pragma unroll
+        for (int x = 0; x < 5; x++) tc[x] = lane_from(behind_k, pc[x]);
+        lu_product(t, {R[2].x, R[2].y, R[3].x, R[3].y, R[6].x}, dp, res, pb);
+#pragma unroll
+        for (int x = 0; x < 5; x++) tb[x] = lane_behind_j<DIR>(pb[x]);
+        wait_face(min(s + 1, last));
+        load_face(s + 1);
+        load_rows(s + 1, NR);
+        lds_post(&L.done, s + 1);
+        lu_product(t, {R[0].x, R[0].y, R[1].x, R[1].y, r0}, dp, res, ta);
+        // face lanes: slot pos + sk = s - (kTile - 1), and the same on the k side
+        if (k_out && on) {
+#pragma unroll
+            for (int x = 0; x < 5; x++) xstore(ko + x * kTile, pc[x]);
+        }
+        if (j_out && on) {
+#pragma unroll
+            for (int x = 0; x < 5; x++) xstore(jo + x * kTile, pb[x]);
+        }
+        jo += kTile * 5;
+        ko += kTile * 5;
+        if (on) {
+            if (fuse_add) {
+                const long n = nat0 + (g.Li - 1 - pos);
+#pragma unroll
+                for (int x = 0; x < 5; x++) q[x * qN + n] = qv[x] + res[x];
+            } else {
+                // the backward sweep leaves q + dq, the forward sweep dq*, as
+                // whole 16-byte pairs, the first one with the time term
+                double r[5];
+#pragma unroll
+                for (int x = 0; x < 5; x++) r[x] = DIR < 0 ? qv[x] + res[x] : res[x];
+                dst[0] = make_double2(tterm, r[0]);
+                dst[64] = make_double2(r[1], r[2]);
+                dst[2 * 64] = make_double2(r[3], r[4]);
+            }
+        }
+        dst += DIR * (kSlF / 2) * 64;
+    };
+    wait_ops(0);
+    load_state(0, E[0]);
+    load_rows(0, R[0]);
+    wait_face(0);
+    load_face(0);
+    for (int s = 0; s < g.nsteps; s += 2) {
+        step(s, E[0], R[0], E[1], R[1]);
+        if (s + 1 < g.nsteps) step(s + 1, E[1], R[1], E[0], R[0]);
+    }
+}
+
+template <int DIR>
+__device__ inline void pipe_body(const SlGeom &g, int tile, double *__restrict__ sl, double gamma, double *ex, int *err,
+                                 PipeLds<DIR> &L, const Ext *e, double *__restrict__ q)
+{
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    if (threadIdx.x < kPipePrep) L.prep[threadIdx.x] = threadIdx.x;
+    if (threadIdx.x == 64) L.xready = L.done = L.stop = 0;
+    for (int x = threadIdx.x; x < kPipeXRing * 10 * kTile; x += kPipeThreads) (&L.x[0][0][0][0])[x] = 0.0;
+    __syncthreads();
+    const int bj = tile % g.nbj, bk = tile / g.nbj;
+    const bool j_pred = DIR > 0 ? bj > 0 : bj + 1 < g.nbj, k_pred = DIR > 0 ? bk > 0 : bk + 1 < g.nbk;
+    const bool j_succ = DIR > 0 ? bj + 1 < g.nbj : bj > 0, k_succ = DIR > 0 ? bk + 1 < g.nbk : bk > 0;
+    double *exk = ex + (long)g.ntiles * g.exj_tile;
+    if (wave == 0) {
+        __builtin_amdgcn_s_setprio(3);
+        pipe_solve<DIR>(g, tile, sl, gamma, ex + (long)tile * g.exj_tile, exk + (long)tile * g.exk_tile,
+                        j_pred || k_pred, j_succ, k_succ, L, err, e, q);
+    } else if (wave <= kPipePrep) {
+        pipe_prepare<DIR>(g, tile, wave - 1, sl, gamma, L, err);
+    } else if (j_pred || k_pred) {
+        const bool k_face = (threadIdx.x & 32) != 0, has = k_face ? k_pred : j_pred;
+        const int f = threadIdx.x & 7;
+        const bool line_ok = has && (k_face ? bj : bk) * kTile + f < (k_face ? g.Lj : g.Lk);
+        double *src = !has ? ex : k_face ? exk + (long)(tile - DIR * g.nbj) * g.exk_tile
+                                         : ex + (long)(tile - DIR) * g.exj_tile;
+        pipe_fetch<DIR>(g, line_ok, DIR > 0 ? f : kTile - 1 - f, src, L, err);
+    }
+}
+
+// Tile numbers.  When every workgroup of the launch fits on the device at
+// once (ctr null), tile = workgroup index: all tiles run together and every
+// wait ends.  Otherwise the tiles are handed out in the order workgroups
+// start (a ticket counter): a tile then only ever waits on tiles whose
+// workgroups started before it, so the sweep progresses however the launch
+// is dispatched; the last workgroup to finish resets both counters for the
+// next launch.  (The first form is the faster one where it applies: the
+// hardware's placement of consecutive workgroups suits the sweep.)
+__device__ inline int pipe_ticket(int *ctr, int *ticket)
+{
+    if (!ctr) return (int)blockIdx.x;
+    if (threadIdx.x == 0) *ticket = __hip_atomic_fetch_add(ctr, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    return __builtin_amdgcn_readfirstlane(*ticket);
+}
+__device__ inline void pipe_ticket_done(int *ctr, int total)
+{
+    if (ctr && threadIdx.x == 0 &&
+        __hip_atomic_fetch_add(ctr + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == total - 1) {
+        __hip_atomic_store(ctr, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(ctr + 1, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+}
+
+template <int DIR>
+__global__ void __launch_bounds__(kPipeThreads, 2) k_lu_pipe(SlGeom g, double *__restrict__ sl, double gamma, double *ex,
+                                                             int *err, int *ctr, Ext e, double *q)
+{
+    __shared__ PipeLds<DIR> L;
+    __shared__ int ticket;
+    const int flat = pipe_ticket(ctr, &ticket);
+    pipe_body<DIR>(g, DIR > 0 ? flat : g.ntiles - 1 - flat, sl, gamma, ex, err, L, &e, q);
+    pipe_ticket_done(ctr, g.ntiles);
 }
 
 // ------------------------------------------------------------ batched tiles
@@ -807,67 +1024,49 @@ struct LuBatchEnt {
     int tile0;
 };
 
-template <int TT>
-__global__ void __launch_bounds__(TT) k_sl_gather_batch(const LuBatchEnt *__restrict__ ents,
+__global__ void __launch_bounds__(kLanes) k_sl_gather_batch(const LuBatchEnt *__restrict__ ents,
                                                         const int *__restrict__ tile_ent, double *arena,
                                                         double *slb, int fp0)
 {
-    extern __shared__ double buf[];
+    __shared__ double buf[2 * kSlCt * kLanes];
     const int flat = (int)blockIdx.x;
     const LuBatchEnt &b = ents[tile_ent[flat]];
     const Ext e = b.e;
     const SlGeom g = b.g;
-    sl_gather_tile<TT>(e, g, flat - b.tile0, arena + b.q, arena + b.dxidx, arena + b.inv_j, arena + b.csnd,
+    sl_gather_tile(e, g, flat - b.tile0, arena + b.q, arena + b.dxidx, arena + b.inv_j, arena + b.csnd,
                        arena + b.tterm, arena + b.rhs, slb + b.sl, fp0, buf);
 }
 
-template <int TT>
-__global__ void __launch_bounds__(TT) k_sl_add_batch(const LuBatchEnt *__restrict__ ents,
+__global__ void __launch_bounds__(kLanes) k_sl_add_batch(const LuBatchEnt *__restrict__ ents,
                                                      const int *__restrict__ tile_ent, double *arena,
                                                      const double *slb)
 {
-    extern __shared__ double buf[];
+    __shared__ double buf[2 * kSlCt * kLanes];
     const int flat = (int)blockIdx.x;
     const LuBatchEnt &b = ents[tile_ent[flat]];
     const Ext e = b.e;
     const SlGeom g = b.g;
-    sl_add_tile<TT>(e, g, flat - b.tile0, slb + b.sl, arena + b.q, buf);
+    sl_add_tile(e, g, flat - b.tile0, slb + b.sl, arena + b.q, buf);
 }
 
-// Flat tile numbers.  When every workgroup of the launch fits on the device
-// at once (`resident`), tile = workgroup index: all tiles run together and
-// every wait ends.  Otherwise the tiles are handed out in the order
-// workgroups start (a ticket counter): a tile then only ever waits on tiles
-// whose workgroups started before it, so the sweep progresses however the
-// launch is dispatched; the last workgroup to finish resets both counters
-// for the next launch.  (The first form is the faster one where it applies:
-// the hardware's placement of consecutive workgroups suits the sweep.)
-template <int DIR, int TJ, int TK>
-__global__ void __launch_bounds__(TJ *TK) k_lu_tiles_batch(const LuBatchEnt *__restrict__ ents,
-                                                            const int *__restrict__ tile_ent, int total,
-                                                            int resident, double *slb, double *exb,
-                                                            double gamma, int *err, int *ctr, double *arena,
-                                                            int fuse_add)
+template <int DIR>
+__global__ void __launch_bounds__(kPipeThreads, 2) k_lu_pipe_batch(const LuBatchEnt *__restrict__ ents,
+                                                                   const int *__restrict__ tile_ent, int total,
+                                                                   int resident, double *slb, double *exb,
+                                                                   double gamma, int *err, int *ctr, double *arena,
+                                                                   int fuse_add)
 {
-    __shared__ double pj[2][5][TJ * TK], pk[2][5][TJ * TK];
+    __shared__ PipeLds<DIR> L;
     __shared__ int ticket;
-    if (!resident) {
-        if (threadIdx.x == 0)
-            ticket = __hip_atomic_fetch_add(ctr, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __syncthreads();
-    }
-    const int flat = resident ? (int)blockIdx.x : __builtin_amdgcn_readfirstlane(ticket);
+    int *c = resident ? nullptr : ctr;
+    const int flat = pipe_ticket(c, &ticket);
     const LuBatchEnt &b = ents[tile_ent[flat]];
     const SlGeom g = b.g;
     const int local = flat - b.tile0;
     const Ext e = b.e;
-    lu_tiles_body<DIR, TJ, TK>(g, DIR > 0 ? local : g.ntiles - 1 - local, slb + b.sl, gamma, exb + b.ex, err, pj,
-                               pk, &e, fuse_add ? arena + b.q : nullptr);
-    if (!resident && threadIdx.x == 0 &&
-        __hip_atomic_fetch_add(ctr + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == total - 1) {
-        __hip_atomic_store(ctr, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(ctr + 1, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
+    pipe_body<DIR>(g, DIR > 0 ? local : g.ntiles - 1 - local, slb + b.sl, gamma, exb + b.ex, err, L, &e,
+                   fuse_add ? arena + b.q : nullptr);
+    pipe_ticket_done(c, total);
 }
 
 // ------------------------------------------------ scalar sweeps (SA model)
@@ -881,16 +1080,14 @@ __global__ void __launch_bounds__(TJ *TK) k_lu_tiles_batch(const LuBatchEnt *__r
 // dn*) are read in place, one i-line per lane (a cache line serves 16
 // consecutive steps), and one value per exchange slot crosses a tile edge.
 struct SaGeom {
-    int TJ, TK, nbj, nbk, ntiles, nsteps, Li, Lj, Lk;
+    int nbj, nbk, ntiles, nsteps, Li, Lj, Lk;
     long exj_tile, exk_tile;  // doubles per tile of the j / k exchange regions
 };
 
-static SaGeom sa_geom(const Ext &e, int shape)
+static SaGeom sa_geom(const Ext &e)
 {
-    const SlGeom s = sl_geom(e, shape);
+    const SlGeom s = sl_geom(e);
     SaGeom g;
-    g.TJ = s.TJ;
-    g.TK = s.TK;
     g.nbj = s.nbj;
     g.nbk = s.nbk;
     g.ntiles = s.ntiles;
@@ -898,8 +1095,7 @@ static SaGeom sa_geom(const Ext &e, int shape)
     g.Li = s.Li;
     g.Lj = s.Lj;
     g.Lk = s.Lk;
-    g.exj_tile = (long)(g.Li + g.TK - 1) * g.TK;
-    g.exk_tile = (long)(g.Li + g.TJ - 1) * g.TJ;
+    g.exj_tile = g.exk_tile = (long)(g.Li + kTile - 1) * kTile;
     return g;
 }
 
@@ -925,23 +1121,23 @@ __device__ inline double ex_take1(double *slot, unsigned long long pre, int *err
 
 // cu = a, b, c, diag (component stride N); fwd reads rhs and writes dns,
 // bwd reads dns and writes dn
-template <int DIR, int TJ, int TK>
+template <int DIR>
 __device__ inline void sa_tiles_body(const Ext &e, const SaGeom &g, int tile, const double *__restrict__ cu,
                                      const double *__restrict__ rhs, double *__restrict__ dns,
-                                     double *__restrict__ dn, double *ex, int *err, double (*pj)[TJ * TK],
-                                     double (*pk)[TJ * TK])
+                                     double *__restrict__ dn, double *ex, int *err, double (*pj)[kLanes],
+                                     double (*pk)[kLanes])
 {
     const int bj = tile % g.nbj, bk = tile / g.nbj;
-    const int l = threadIdx.x, tj = l % TJ, tk = l / TJ;
-    const int lj = bj * TJ + tj, lk = bk * TK + tk;
+    const int l = threadIdx.x, tj = l % kTile, tk = l / kTile;
+    const int lj = bj * kTile + tj, lk = bk * kTile + tk;
     const bool active = lj < g.Lj && lk < g.Lk;
-    const int sj = DIR > 0 ? tj : TJ - 1 - tj, sk = DIR > 0 ? tk : TK - 1 - tk;
+    const int sj = DIR > 0 ? tj : kTile - 1 - tj, sk = DIR > 0 ? tk : kTile - 1 - tk;
     const bool j_ring = DIR > 0 ? lj == 0 : lj + 1 >= g.Lj;
     const bool k_ring = DIR > 0 ? lk == 0 : lk + 1 >= g.Lk;
     const bool j_in = !j_ring && sj == 0, k_in = !k_ring && sk == 0;
-    const int lpj = l - DIR, lpk = l - DIR * TJ;
-    const bool j_out = sj == TJ - 1 && (DIR > 0 ? bj + 1 < g.nbj : bj > 0);
-    const bool k_out = sk == TK - 1 && (DIR > 0 ? bk + 1 < g.nbk : bk > 0);
+    const int lpj = l - DIR, lpk = l - DIR * kTile;
+    const bool j_out = sj == kTile - 1 && (DIR > 0 ? bj + 1 < g.nbj : bj > 0);
+    const bool k_out = sk == kTile - 1 && (DIR > 0 ? bk + 1 < g.nbk : bk > 0);
     double *exj = ex, *exk = ex + (long)g.ntiles * g.exj_tile;
     double *jin = exj + (long)(DIR > 0 ? tile - 1 : tile + 1) * g.exj_tile + tk;
     double *kin = exk + (long)(DIR > 0 ? tile - g.nbj : tile + g.nbj) * g.exk_tile + tj;
@@ -953,7 +1149,7 @@ __device__ inline void sa_tiles_body(const Ext &e, const SaGeom &g, int tile, co
     const bool k_pred = DIR > 0 ? bk > 0 : bk + 1 < g.nbk;
     const double *jsrc = j_pred ? jin : ex;
     const double *ksrc = k_pred ? kin : ex;
-    const int xj_last = g.Li + TK - 2, xk_last = g.Li + TJ - 2;
+    const int xj_last = g.Li + kTile - 2, xk_last = g.Li + kTile - 2;
     const long N = e.n;
     // first node of the lane's line in sweep order (inactive lanes read a
     // valid node and ignore it)
@@ -974,17 +1170,17 @@ __device__ inline void sa_tiles_body(const Ext &e, const SaGeom &g, int tile, co
         op[4] = src[n];
         const int dj = j_pred ? min(max(s, 0), xj_last) : 0;
         const int dk = k_pred ? min(max(s, 0), xk_last) : 0;
-        xj = xload_bits(jsrc + (long)dj * TK);
-        xk = xload_bits(ksrc + (long)dk * TJ);
+        xj = xload_bits(jsrc + (long)dj * kTile);
+        xk = xload_bits(ksrc + (long)dk * kTile);
     };
     auto step = [&](int s, const double *op, unsigned long long xj, unsigned long long xk) {
         const int par = s & 1;
         const int pos = s - sj - sk;
         if (active && pos >= 0 && pos < g.Li) {
             const long n = n0 + (DIR > 0 ? pos : g.Li - 1 - pos);
-            const double vj = j_ring ? 0.0 : j_in ? ex_take1(jin + (long)(pos + sk) * TK, xj, err, failed)
+            const double vj = j_ring ? 0.0 : j_in ? ex_take1(jin + (long)(pos + sk) * kTile, xj, err, failed)
                                                   : pj[par ^ 1][lpj];
-            const double vk = k_ring ? 0.0 : k_in ? ex_take1(kin + (long)(pos + sj) * TJ, xk, err, failed)
+            const double vk = k_ring ? 0.0 : k_in ? ex_take1(kin + (long)(pos + sj) * kTile, xk, err, failed)
                                                   : pk[par ^ 1][lpk];
             double res;
             if (DIR > 0) {
@@ -1002,8 +1198,8 @@ __device__ inline void sa_tiles_body(const Ext &e, const SaGeom &g, int tile, co
             vi = res;
             pj[par][l] = res;
             pk[par][l] = res;
-            if (j_out) xstore(jout + (long)(pos + sk) * TK, res);
-            if (k_out) xstore(kout + (long)(pos + sj) * TJ, res);
+            if (j_out) xstore(jout + (long)(pos + sk) * kTile, res);
+            if (k_out) xstore(kout + (long)(pos + sj) * kTile, res);
         }
         lds_barrier();
     };
@@ -1018,14 +1214,14 @@ __device__ inline void sa_tiles_body(const Ext &e, const SaGeom &g, int tile, co
     }
 }
 
-template <int DIR, int TJ, int TK>
-__global__ void __launch_bounds__(TJ *TK) k_sa_tiles(Ext e, SaGeom g, const double *__restrict__ cu,
+template <int DIR>
+__global__ void __launch_bounds__(kLanes) k_sa_tiles(Ext e, SaGeom g, const double *__restrict__ cu,
                                                       const double *__restrict__ rhs, double *__restrict__ dns,
                                                       double *__restrict__ dn, double *ex, int *err)
 {
-    __shared__ double pj[2][TJ * TK], pk[2][TJ * TK];
+    __shared__ double pj[2][kLanes], pk[2][kLanes];
     const int tile = DIR > 0 ? (int)blockIdx.x : g.ntiles - 1 - (int)blockIdx.x;
-    sa_tiles_body<DIR, TJ, TK>(e, g, tile, cu, rhs, dns, dn, ex, err, pj, pk);
+    sa_tiles_body<DIR>(e, g, tile, cu, rhs, dns, dn, ex, err, pj, pk);
 }
 
 struct SaBatchEnt {
@@ -1037,13 +1233,13 @@ struct SaBatchEnt {
     int tile0;
 };
 
-template <int DIR, int TJ, int TK>
-__global__ void __launch_bounds__(TJ *TK) k_sa_tiles_batch(const SaBatchEnt *__restrict__ ents,
+template <int DIR>
+__global__ void __launch_bounds__(kLanes) k_sa_tiles_batch(const SaBatchEnt *__restrict__ ents,
                                                             const int *__restrict__ tile_ent, int total,
                                                             int resident, double *arena, double *exb, int *err,
                                                             int *ctr)
 {
-    __shared__ double pj[2][TJ * TK], pk[2][TJ * TK];
+    __shared__ double pj[2][kLanes], pk[2][kLanes];
     __shared__ int ticket;
     if (!resident) {
         if (threadIdx.x == 0)
@@ -1055,7 +1251,7 @@ __global__ void __launch_bounds__(TJ *TK) k_sa_tiles_batch(const SaBatchEnt *__r
     const Ext e = b.e;
     const SaGeom g = b.g;
     const int local = flat - b.tile0;
-    sa_tiles_body<DIR, TJ, TK>(e, g, DIR > 0 ? local : g.ntiles - 1 - local, arena + b.cu, arena + b.rhs,
+    sa_tiles_body<DIR>(e, g, DIR > 0 ? local : g.ntiles - 1 - local, arena + b.cu, arena + b.rhs,
                                arena + b.dns, arena + b.dn, exb + b.ex, err, pj, pk);
     if (!resident && threadIdx.x == 0 &&
         __hip_atomic_fetch_add(ctr + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == total - 1) {
@@ -1076,20 +1272,20 @@ __global__ void __launch_bounds__(TJ *TK) k_sa_tiles_batch(const SaBatchEnt *__r
 // slot and the backward sweep dnut there; a last pass adds it to nut.
 constexpr int kSaOps = 5;
 
-__host__ __device__ inline long sa_slot(const SaGeom &g, int tt, int tile, int t, int f, int l)
+__host__ __device__ inline long sa_slot(const SaGeom &g, int tile, int t, int f, int l)
 {
-    return (((long)tile * g.nsteps + t) * kSaOps + f) * tt + l;
+    return (((long)tile * g.nsteps + t) * kSaOps + f) * kLanes + l;
 }
 
 // node of (tile, line, li) of a block and whether the line exists
 __device__ inline long sa_nat(const Ext &e, const SaGeom &g, int tile, int line, int li)
 {
-    const int tj = line % g.TJ, tk = line / g.TJ;
-    return e.ix(e.is1 + li, e.js1 + (tile % g.nbj) * g.TJ + tj, e.ks1 + (tile / g.nbj) * g.TK + tk);
+    const int tj = line % kTile, tk = line / kTile;
+    return e.ix(e.is1 + li, e.js1 + (tile % g.nbj) * kTile + tj, e.ks1 + (tile / g.nbj) * kTile + tk);
 }
 __device__ inline bool sa_line_ok(const SaGeom &g, int tile, int line)
 {
-    return (tile % g.nbj) * g.TJ + line % g.TJ < g.Lj && (tile / g.nbj) * g.TK + line / g.TJ < g.Lk;
+    return (tile % g.nbj) * kTile + line % kTile < g.Lj && (tile / g.nbj) * kTile + line / kTile < g.Lk;
 }
 
 // Natural layout <-> SA sweep layout for one tile (one workgroup of TT
@@ -1098,15 +1294,15 @@ __device__ inline bool sa_line_ok(const SaGeom &g, int tile, int line)
 // XOR-swizzled [CT][TT] LDS buffer in between.  TO_SL: cu (4 operands,
 // component stride N) and rhs into the layout; otherwise nut += the layout's
 // last operand.
-template <int TT, bool TO_SL>
+template <bool TO_SL>
 __device__ inline void sa_layout_tile(const Ext &e, const SaGeom &g, int tile, const double *__restrict__ cu,
                                       const double *__restrict__ rhs, double *__restrict__ nut, double *__restrict__ L,
                                       double *buf /* [CT][TT] */)
 {
-    constexpr int CT = TO_SL ? sl_ct_of(TT) : sa_ret_ct_of(TT), lstep = TT / CT;
+    constexpr int CT = TO_SL ? kSlCt : kSaRetCt, TT = kLanes, lstep = TT / CT;
     const int x = threadIdx.x;
     const int ii_n = x % CT;
-    const int tj = x % g.TJ, tk = x / g.TJ;
+    const int tj = x % kTile, tk = x / kTile;
     const bool me_ok = sa_line_ok(g, tile, x);
     const long N = e.n;
     for (int t0 = 0; t0 < g.nsteps; t0 += CT) {
@@ -1114,7 +1310,7 @@ __device__ inline void sa_layout_tile(const Ext &e, const SaGeom &g, int tile, c
 #pragma unroll
         for (int m = 0; m < CT; m++) {
             const int line = m * lstep + x / CT;
-            const int li = t0 + ii_n - line % g.TJ - line / g.TJ;
+            const int li = t0 + ii_n - line % kTile - line / kTile;
             nat[m] = (t0 + ii_n < g.nsteps && li >= 0 && li < g.Li && sa_line_ok(g, tile, line))
                          ? (int)sa_nat(e, g, tile, line, li) : -1;
         }
@@ -1134,7 +1330,7 @@ __device__ inline void sa_layout_tile(const Ext &e, const SaGeom &g, int tile, c
 #pragma unroll
                     for (int ii = 0; ii < CT; ii++) {
                         const int t = t0 + ii, li = t - tj - tk;
-                        if (t < g.nsteps && li >= 0 && li < g.Li) L[sa_slot(g, TT, tile, t, f, x)] = buf[ii * TT + (x ^ ii)];
+                        if (t < g.nsteps && li >= 0 && li < g.Li) L[sa_slot(g, tile, t, f, x)] = buf[ii * TT + (x ^ ii)];
                     }
                 }
                 __syncthreads();
@@ -1145,7 +1341,7 @@ __device__ inline void sa_layout_tile(const Ext &e, const SaGeom &g, int tile, c
                 for (int ii = 0; ii < CT; ii++) {
                     const int t = t0 + ii, li = t - tj - tk;
                     buf[ii * TT + (x ^ ii)] =
-                        (t < g.nsteps && li >= 0 && li < g.Li) ? L[sa_slot(g, TT, tile, t, kSaOps - 1, x)] : 0.0;
+                        (t < g.nsteps && li >= 0 && li < g.Li) ? L[sa_slot(g, tile, t, kSaOps - 1, x)] : 0.0;
                 }
             }
             __syncthreads();
@@ -1159,37 +1355,37 @@ __device__ inline void sa_layout_tile(const Ext &e, const SaGeom &g, int tile, c
     }
 }
 
-template <int TT, bool TO_SL>
-__global__ void __launch_bounds__(TT) k_sa_layout_batch(const SaBatchEnt *__restrict__ ents,
+template <bool TO_SL>
+__global__ void __launch_bounds__(kLanes) k_sa_layout_batch(const SaBatchEnt *__restrict__ ents,
                                                         const int *__restrict__ tile_ent, double *arena,
                                                         double *slbase)
 {
-    __shared__ double buf[(TO_SL ? sl_ct_of(TT) : sa_ret_ct_of(TT)) * TT];
+    __shared__ double buf[(TO_SL ? kSlCt : kSaRetCt) * kLanes];
     const int flat = (int)xcd_slab(blockIdx.x, gridDim.x);
     const SaBatchEnt &b = ents[tile_ent[flat]];
     const Ext e = b.e;
     const SaGeom g = b.g;
-    sa_layout_tile<TT, TO_SL>(e, g, flat - b.tile0, arena + b.cu, arena + b.rhs, arena + b.nut, slbase + b.sl, buf);
+    sa_layout_tile<TO_SL>(e, g, flat - b.tile0, arena + b.cu, arena + b.rhs, arena + b.nut, slbase + b.sl, buf);
 }
 
 // The scalar sweep of sa_tiles_body with its operands in the SA sweep
 // layout (the same expressions, the same exchange and skewed clock).
-template <int DIR, int TJ, int TK>
+template <int DIR>
 __device__ inline void sa_sl_body(const SaGeom &g, int tile, double *__restrict__ L, double *ex, int *err,
-                                  double (*pj)[TJ * TK], double (*pk)[TJ * TK])
+                                  double (*pj)[kLanes], double (*pk)[kLanes])
 {
-    constexpr int TT = TJ * TK;
+    constexpr int TT = kLanes;
     const int bj = tile % g.nbj, bk = tile / g.nbj;
-    const int l = threadIdx.x, tj = l % TJ, tk = l / TJ;
-    const int lj = bj * TJ + tj, lk = bk * TK + tk;
+    const int l = threadIdx.x, tj = l % kTile, tk = l / kTile;
+    const int lj = bj * kTile + tj, lk = bk * kTile + tk;
     const bool active = lj < g.Lj && lk < g.Lk;
-    const int sj = DIR > 0 ? tj : TJ - 1 - tj, sk = DIR > 0 ? tk : TK - 1 - tk;
+    const int sj = DIR > 0 ? tj : kTile - 1 - tj, sk = DIR > 0 ? tk : kTile - 1 - tk;
     const bool j_ring = DIR > 0 ? lj == 0 : lj + 1 >= g.Lj;
     const bool k_ring = DIR > 0 ? lk == 0 : lk + 1 >= g.Lk;
     const bool j_in = !j_ring && sj == 0, k_in = !k_ring && sk == 0;
-    const int lpj = l - DIR, lpk = l - DIR * TJ;
-    const bool j_out = sj == TJ - 1 && (DIR > 0 ? bj + 1 < g.nbj : bj > 0);
-    const bool k_out = sk == TK - 1 && (DIR > 0 ? bk + 1 < g.nbk : bk > 0);
+    const int lpj = l - DIR, lpk = l - DIR * kTile;
+    const bool j_out = sj == kTile - 1 && (DIR > 0 ? bj + 1 < g.nbj : bj > 0);
+    const bool k_out = sk == kTile - 1 && (DIR > 0 ? bk + 1 < g.nbk : bk > 0);
     double *exj = ex, *exk = ex + (long)g.ntiles * g.exj_tile;
     double *jin = exj + (long)(DIR > 0 ? tile - 1 : tile + 1) * g.exj_tile + tk;
     double *kin = exk + (long)(DIR > 0 ? tile - g.nbj : tile + g.nbj) * g.exk_tile + tj;
@@ -1202,7 +1398,7 @@ __device__ inline void sa_sl_body(const SaGeom &g, int tile, double *__restrict_
     const bool k_pred = DIR > 0 ? bk > 0 : bk + 1 < g.nbk;
     const double *jsrc = j_pred ? jin : ex;
     const double *ksrc = k_pred ? kin : ex;
-    const int xj_last = g.Li + TK - 2, xk_last = g.Li + TJ - 2;
+    const int xj_last = g.Li + kTile - 2, xk_last = g.Li + kTile - 2;
     bool failed = false;
     double vi = 0.0;
     auto row_of = [&](int s) -> long {
@@ -1215,16 +1411,16 @@ __device__ inline void sa_sl_body(const SaGeom &g, int tile, double *__restrict_
         for (int f = 0; f < kSaOps; f++) op[f] = p[f * TT];
         const int dj = j_pred ? min(max(s, 0), xj_last) : 0;
         const int dk = k_pred ? min(max(s, 0), xk_last) : 0;
-        xj = xload_bits(jsrc + (long)dj * TK);
-        xk = xload_bits(ksrc + (long)dk * TJ);
+        xj = xload_bits(jsrc + (long)dj * kTile);
+        xk = xload_bits(ksrc + (long)dk * kTile);
     };
     auto step = [&](int s, const double *op, unsigned long long xj, unsigned long long xk) {
         const int par = s & 1;
         const int pos = s - sj - sk;
         if (active && pos >= 0 && pos < g.Li) {
-            const double vj = j_ring ? 0.0 : j_in ? ex_take1(jin + (long)(pos + sk) * TK, xj, err, failed)
+            const double vj = j_ring ? 0.0 : j_in ? ex_take1(jin + (long)(pos + sk) * kTile, xj, err, failed)
                                                   : pj[par ^ 1][lpj];
-            const double vk = k_ring ? 0.0 : k_in ? ex_take1(kin + (long)(pos + sj) * TJ, xk, err, failed)
+            const double vk = k_ring ? 0.0 : k_in ? ex_take1(kin + (long)(pos + sj) * kTile, xk, err, failed)
                                                   : pk[par ^ 1][lpk];
             double res;
             if (DIR > 0) {
@@ -1242,8 +1438,8 @@ __device__ inline void sa_sl_body(const SaGeom &g, int tile, double *__restrict_
             vi = res;
             pj[par][l] = res;
             pk[par][l] = res;
-            if (j_out) xstore(jout + (long)(pos + sk) * TK, res);
-            if (k_out) xstore(kout + (long)(pos + sj) * TJ, res);
+            if (j_out) xstore(jout + (long)(pos + sk) * kTile, res);
+            if (k_out) xstore(kout + (long)(pos + sj) * kTile, res);
         }
         lds_barrier();
     };
@@ -1258,12 +1454,12 @@ __device__ inline void sa_sl_body(const SaGeom &g, int tile, double *__restrict_
     }
 }
 
-template <int DIR, int TJ, int TK>
-__global__ void __launch_bounds__(TJ *TK) k_sa_sl_batch(const SaBatchEnt *__restrict__ ents,
+template <int DIR>
+__global__ void __launch_bounds__(kLanes) k_sa_sl_batch(const SaBatchEnt *__restrict__ ents,
                                                          const int *__restrict__ tile_ent, int total, int resident,
                                                          double *slbase, double *exb, int *err, int *ctr)
 {
-    __shared__ double pj[2][TJ * TK], pk[2][TJ * TK];
+    __shared__ double pj[2][kLanes], pk[2][kLanes];
     __shared__ int ticket;
     if (!resident) {
         if (threadIdx.x == 0)
@@ -1274,7 +1470,7 @@ __global__ void __launch_bounds__(TJ *TK) k_sa_sl_batch(const SaBatchEnt *__rest
     const SaBatchEnt &b = ents[tile_ent[flat]];
     const SaGeom g = b.g;
     const int local = flat - b.tile0;
-    sa_sl_body<DIR, TJ, TK>(g, DIR > 0 ? local : g.ntiles - 1 - local, slbase + b.sl, exb + b.ex, err, pj, pk);
+    sa_sl_body<DIR>(g, DIR > 0 ? local : g.ntiles - 1 - local, slbase + b.sl, exb + b.ex, err, pj, pk);
     if (!resident && threadIdx.x == 0 &&
         __hip_atomic_fetch_add(ctr + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == total - 1) {
         __hip_atomic_store(ctr, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1282,25 +1478,18 @@ __global__ void __launch_bounds__(TJ *TK) k_sa_sl_batch(const SaBatchEnt *__rest
     }
 }
 
-int lusgs_tile_shapes() { return kNumTileShapes; }
-
-long lusgs_tiles(const Ext &e, int shape)
+static long lusgs_tiles(const Ext &e)
 {
-    SlGeom g = sl_geom(e, shape);
+    const SlGeom g = sl_geom(e);
     return g.Li > 0 && g.Lj > 0 && g.Lk > 0 ? g.ntiles : 0;
 }
 
 void lusgs_ws_sizes(const Ext &e, long *sl_n, long *ex_n)
 {
-    long a = 0, b = 0;
-    for (int s = 0; s < kNumTileShapes; s++) {
-        SlGeom g = sl_geom(e, s);
-        if (g.Li <= 0 || g.Lj <= 0 || g.Lk <= 0) continue;
-        a = std::max(a, (long)g.ntiles * g.nsteps * kSlF * g.TT);
-        b = std::max(b, (long)g.ntiles * (g.exj_tile + g.exk_tile));
-    }
-    *sl_n = a;
-    *ex_n = b;
+    const SlGeom g = sl_geom(e);
+    const bool any = lusgs_tiles(e) > 0;
+    *sl_n = any ? (long)g.ntiles * g.nsteps * kSlF * kLanes : 0;
+    *ex_n = any ? (long)g.ntiles * (g.exj_tile + g.exk_tile) : 0;
 }
 
 // Whether the backward sweep adds dq to q itself (and the add pass is
@@ -1328,38 +1517,38 @@ static long round_up32(long n) { return (n + 31) / 32 * 32; }
 static void batch_residency(LuBatch *b);
 
 // blocks of the batch in launch order: longest sweep first
-static std::vector<int> batch_order(int nblk, const Ext *e, int shape)
+static std::vector<int> batch_order(int nblk, const Ext *e)
 {
     std::vector<int> order;
     for (int m = 0; m < nblk; m++)
-        if (lusgs_tiles(e[m], shape) > 0) order.push_back(m);
+        if (lusgs_tiles(e[m]) > 0) order.push_back(m);
     std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
-        const SlGeom ga = sl_geom(e[a], shape), gb = sl_geom(e[b], shape);
+        const SlGeom ga = sl_geom(e[a]), gb = sl_geom(e[b]);
         return ga.nsteps + ga.nbj + ga.nbk > gb.nsteps + gb.nbj + gb.nbk;
     });
     return order;
 }
 
-void lusgs_batch_ws(int nblk, const Ext *e, int shape, long *sl_n, long *ex_n)
+void lusgs_batch_ws(int nblk, const Ext *e, long *sl_n, long *ex_n)
 {
     long a = 0, b = 0;
-    for (int m : batch_order(nblk, e, shape)) {
-        const SlGeom g = sl_geom(e[m], shape);
-        a += round_up32((long)g.ntiles * g.nsteps * kSlF * g.TT);
+    for (int m : batch_order(nblk, e)) {
+        const SlGeom g = sl_geom(e[m]);
+        a += round_up32((long)g.ntiles * g.nsteps * kSlF * kLanes);
         b += round_up32((long)g.ntiles * (g.exj_tile + g.exk_tile));
     }
     *sl_n = a;
     *ex_n = b;
 }
 
-int lusgs_batch_make(int nblk, const Ext *e, const Fields *f, double *arena, int shape, double *sl, double *ex,
+int lusgs_batch_make(int nblk, const Ext *e, const Fields *f, double *arena, double *sl, double *ex,
                      LuBatch *out)
 {
     std::vector<LuBatchEnt> ents;
     std::vector<int> te;
     long so = 0, xo = 0;
-    for (int m : batch_order(nblk, e, shape)) {
-        const SlGeom g = sl_geom(e[m], shape);
+    for (int m : batch_order(nblk, e)) {
+        const SlGeom g = sl_geom(e[m]);
         LuBatchEnt b;
         b.e = e[m];
         b.g = g;
@@ -1372,19 +1561,16 @@ int lusgs_batch_make(int nblk, const Ext *e, const Fields *f, double *arena, int
         b.sl = so;
         b.ex = xo;
         b.tile0 = (int)te.size();
-        so += round_up32((long)g.ntiles * g.nsteps * kSlF * g.TT);
+        so += round_up32((long)g.ntiles * g.nsteps * kSlF * kLanes);
         xo += round_up32((long)g.ntiles * (g.exj_tile + g.exk_tile));
         for (int t = 0; t < g.ntiles; t++) te.push_back((int)ents.size());
         ents.push_back(b);
     }
-    out->shape = shape;
     out->arena = arena;
     out->sl = sl;
     out->ex = ex;
     out->nent = (int)ents.size();
     out->total = (int)te.size();
-    out->ex_n = xo;
-    out->refill = ex_refill();
     if (ents.empty()) return 0;
     batch_residency(out);
     long total = 0;
@@ -1408,64 +1594,41 @@ void lusgs_batch_free(LuBatch *b)
 }
 
 // whether all `total` workgroups of the sweep kernel fit on the device at once
-template <int DIR, int TJ, int TK>
-static bool fits_resident(int total)
+// workgroups of the kernel that fit on the device at once (0: unknown)
+template <typename K>
+static int resident_wgs(K kernel, int threads)
 {
     int dev = 0, cus = 0, per_cu = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_lu_tiles_batch<DIR, TJ, TK>, TJ * TK, 0) !=
-            hipSuccess)
-        return false;
-    return (long)cus * per_cu >= total;
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, threads, 0) != hipSuccess)
+        return 0;
+    return cus * per_cu;
 }
 
-template <int DIR, int TJ, int TK>
-static void launch_tiles_batch(hipStream_t s, const LuBatch &b, double gamma, int *err, int *ctr)
+void lusgs_resident(int *tiles)
 {
-    hipLaunchKernelGGL((k_lu_tiles_batch<DIR, TJ, TK>), dim3((unsigned)b.total), dim3(TJ * TK), 0, s,
-                       (const LuBatchEnt *)b.ents, b.tile_ent, b.total, b.resident[DIR > 0 ? 0 : 1], b.sl, b.ex,
-                       gamma, err, ctr, b.arena, DIR < 0 && b.fuse_add ? 1 : 0);
+    const char *t = std::getenv("ACFD_LU_TICKETS");
+    const bool tickets = t && std::atoi(t) == 1;
+    tiles[0] = tickets ? 0 : resident_wgs(k_lu_pipe<1>, kPipeThreads);
+    tiles[1] = tickets ? 0 : resident_wgs(k_lu_pipe<-1>, kPipeThreads);
 }
 
 static void batch_residency(LuBatch *b)
 {
-    bool f = false, r = false;
-    switch (b->shape) {
-    case 0: f = fits_resident<1, 16, 16>(b->total); r = fits_resident<-1, 16, 16>(b->total); break;
-    case 1: f = fits_resident<1, 16, 8>(b->total); r = fits_resident<-1, 16, 8>(b->total); break;
-    case 2: f = fits_resident<1, 8, 8>(b->total); r = fits_resident<-1, 8, 8>(b->total); break;
-    default: f = fits_resident<1, 16, 4>(b->total); r = fits_resident<-1, 16, 4>(b->total); break;
-    }
     // ACFD_LU_TICKETS=1 hands tiles out by ticket even when all would fit
     const char *t = std::getenv("ACFD_LU_TICKETS");
     const bool tickets = t && std::atoi(t) == 1;
-    b->resident[0] = f && !tickets ? 1 : 0;
-    b->resident[1] = r && !tickets ? 1 : 0;
+    b->resident[0] = !tickets && resident_wgs(k_lu_pipe_batch<1>, kPipeThreads) >= b->total ? 1 : 0;
+    b->resident[1] = !tickets && resident_wgs(k_lu_pipe_batch<-1>, kPipeThreads) >= b->total ? 1 : 0;
 }
 
 template <int DIR>
-static void launch_tiles_batch_shape(hipStream_t s, const LuBatch &b, double gamma, int *err, int *ctr)
+static void launch_pipe_batch(hipStream_t s, const LuBatch &b, double gamma, int *err, int *ctr)
 {
-    switch (b.shape) {
-    case 0: launch_tiles_batch<DIR, 16, 16>(s, b, gamma, err, ctr); break;
-    case 1: launch_tiles_batch<DIR, 16, 8>(s, b, gamma, err, ctr); break;
-    case 2: launch_tiles_batch<DIR, 8, 8>(s, b, gamma, err, ctr); break;
-    default: launch_tiles_batch<DIR, 16, 4>(s, b, gamma, err, ctr); break;
-    }
-}
-
-template <int TT>
-static void launch_layout_batch(hipStream_t s, int which, const LuBatch &b, int fp0)
-{
-    const size_t lds = sl_lds_bytes(TT);
-    const LuBatchEnt *ents = (const LuBatchEnt *)b.ents;
-    if (which == 0)
-        hipLaunchKernelGGL(k_sl_gather_batch<TT>, dim3((unsigned)b.total), dim3(TT), lds, s, ents, b.tile_ent,
-                           b.arena, b.sl, fp0);
-    else
-        hipLaunchKernelGGL(k_sl_add_batch<TT>, dim3((unsigned)b.total), dim3(TT), lds, s, ents, b.tile_ent,
-                           b.arena, (const double *)b.sl);
+    hipLaunchKernelGGL((k_lu_pipe_batch<DIR>), dim3((unsigned)b.total), dim3(kPipeThreads), 0, s,
+                       (const LuBatchEnt *)b.ents, b.tile_ent, b.total, b.resident[DIR > 0 ? 0 : 1], b.sl, b.ex, gamma,
+                       err, ctr, b.arena, DIR < 0 && b.fuse_add ? 1 : 0);
 }
 
 // Phases 1-4 of the LU-SGS update for every block of the batch at once
@@ -1475,85 +1638,66 @@ static void launch_layout_batch(hipStream_t s, int which, const LuBatch &b, int 
 int launch_lusgs_batch(hipStream_t s, const LuBatch &b, int phase, double gamma, int *err, int *ctr, int geo_cached)
 {
     if (b.total <= 0 || phase < 1 || phase > 4) return 0;
-    const int tt = kTileShapes[b.shape][0] * kTileShapes[b.shape][1];
-    if (phase == 2 || phase == 3) {
-        if (phase == 2) launch_tiles_batch_shape<1>(s, b, gamma, err, ctr);
-        else launch_tiles_batch_shape<-1>(s, b, gamma, err, ctr);
-        if (b.refill)
-            hipLaunchKernelGGL(k_fill_sentinel, dim3((unsigned)((b.ex_n + 255) / 256)), dim3(256), 0, s, b.ex,
-                               b.ex_n);
-    } else if (phase == 4 && b.fuse_add) return 0;
-    else {
-        const int which = phase == 1 ? 0 : 1, fp0 = geo_cached ? kSlGeoPairs : 0;
-        if (tt == 256) launch_layout_batch<256>(s, which, b, fp0);
-        else if (tt == 128) launch_layout_batch<128>(s, which, b, fp0);
-        else launch_layout_batch<64>(s, which, b, fp0);
-    }
+    const LuBatchEnt *ents = (const LuBatchEnt *)b.ents;
+    if (phase == 1)
+        hipLaunchKernelGGL(k_sl_gather_batch, dim3((unsigned)b.total), dim3(kLanes), 0, s, ents, b.tile_ent, b.arena,
+                           b.sl, geo_cached ? kSlGeoPairs : 0);
+    else if (phase == 2) launch_pipe_batch<1>(s, b, gamma, err, ctr);
+    else if (phase == 3) launch_pipe_batch<-1>(s, b, gamma, err, ctr);
+    else if (!b.fuse_add)
+        hipLaunchKernelGGL(k_sl_add_batch, dim3((unsigned)b.total), dim3(kLanes), 0, s, ents, b.tile_ent, b.arena,
+                           (const double *)b.sl);
     ACFD_CHECK_LAUNCH();
     return 0;
 }
 
 // ---- scalar sweeps: host side
-template <int DIR, int TJ, int TK>
+template <int DIR>
 static bool sa_fits_resident(int total)
 {
     int dev = 0, cus = 0, per_cu = 0, per_cu_sl = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_sa_tiles_batch<DIR, TJ, TK>, TJ * TK, 0) !=
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_sa_tiles_batch<DIR>, kLanes, 0) !=
             hipSuccess ||
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu_sl, k_sa_sl_batch<DIR, TJ, TK>, TJ * TK, 0) !=
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu_sl, k_sa_sl_batch<DIR>, kLanes, 0) !=
             hipSuccess)
         return false;
     return (long)cus * std::min(per_cu, per_cu_sl) >= total;
 }
 
-template <int TJ, int TK>
-static void sa_sweeps_t(hipStream_t s, const Ext &e, const SaGeom &g, const double *cu, const double *rhs,
-                        double *dns, double *dn, double *ex, int *err)
-{
-    hipLaunchKernelGGL((k_sa_tiles<1, TJ, TK>), dim3((unsigned)g.ntiles), dim3(TJ * TK), 0, s, e, g, cu, rhs, dns,
-                       dn, ex, err);
-    hipLaunchKernelGGL((k_sa_tiles<-1, TJ, TK>), dim3((unsigned)g.ntiles), dim3(TJ * TK), 0, s, e, g, cu, rhs,
-                       dns, dn, ex, err);
-}
-
 // both SA sweeps of one block (ex: sentinel-filled, at least
 // ntiles * (exj_tile + exk_tile) doubles -- less than the flow sweep's)
-int launch_sa_sweeps(hipStream_t s, const Ext &e, int shape, const double *cu, const double *rhs, double *dns,
+int launch_sa_sweeps(hipStream_t s, const Ext &e, const double *cu, const double *rhs, double *dns,
                      double *dn, double *ex, int *err)
 {
-    const SaGeom g = sa_geom(e, shape);
+    const SaGeom g = sa_geom(e);
     if (g.Li <= 0 || g.Lj <= 0 || g.Lk <= 0) return 0;
-    switch (shape) {
-    case 0: sa_sweeps_t<16, 16>(s, e, g, cu, rhs, dns, dn, ex, err); break;
-    case 1: sa_sweeps_t<16, 8>(s, e, g, cu, rhs, dns, dn, ex, err); break;
-    case 2: sa_sweeps_t<8, 8>(s, e, g, cu, rhs, dns, dn, ex, err); break;
-    default: sa_sweeps_t<16, 4>(s, e, g, cu, rhs, dns, dn, ex, err); break;
-    }
+    hipLaunchKernelGGL((k_sa_tiles<1>), dim3((unsigned)g.ntiles), dim3(kLanes), 0, s, e, g, cu, rhs, dns, dn, ex, err);
+    hipLaunchKernelGGL((k_sa_tiles<-1>), dim3((unsigned)g.ntiles), dim3(kLanes), 0, s, e, g, cu, rhs, dns, dn, ex, err);
     ACFD_CHECK_LAUNCH();
     return 0;
 }
 
-void sa_batch_sl(int nblk, const Ext *e, int shape, long *sl_n)
+void sa_batch_sl(int nblk, const Ext *e, long *sl_n)
 {
     long so = 0;
     for (int m = 0; m < nblk; m++) {
-        const SaGeom g = sa_geom(e[m], shape);
+        const SaGeom g = sa_geom(e[m]);
         if (g.Li <= 0 || g.Lj <= 0 || g.Lk <= 0) continue;
-        so += round_up32((long)g.ntiles * g.nsteps * kSaOps * g.TJ * g.TK);
+        so += round_up32((long)g.ntiles * g.nsteps * kSaOps * kLanes);
     }
     *sl_n = so;
 }
 
-int sa_batch_make(int nblk, const Ext *e, const Fields *f, double *arena, int shape, double *ex, double *sl,
+int sa_batch_make(int nblk, const Ext *e, const Fields *f, double *arena, double *ex, double *sl,
                   LuBatch *out)
 {
     std::vector<SaBatchEnt> ents;
     std::vector<int> te;
     long xo = 0, so = 0;
-    for (int m : batch_order(nblk, e, shape)) {
-        const SaGeom g = sa_geom(e[m], shape);
+    for (int m : batch_order(nblk, e)) {
+        const SaGeom g = sa_geom(e[m]);
         if (!f[m].w_sa) continue;
         SaBatchEnt b;
         b.e = e[m];
@@ -1567,11 +1711,10 @@ int sa_batch_make(int nblk, const Ext *e, const Fields *f, double *arena, int sh
         b.sl = so;
         b.tile0 = (int)te.size();
         xo += round_up32((long)g.ntiles * (g.exj_tile + g.exk_tile));
-        so += round_up32((long)g.ntiles * g.nsteps * kSaOps * g.TJ * g.TK);
+        so += round_up32((long)g.ntiles * g.nsteps * kSaOps * kLanes);
         for (int t = 0; t < g.ntiles; t++) te.push_back((int)ents.size());
         ents.push_back(b);
     }
-    out->shape = shape;
     out->arena = arena;
     out->ex = ex;
     out->sl = sl;
@@ -1580,15 +1723,8 @@ int sa_batch_make(int nblk, const Ext *e, const Fields *f, double *arena, int sh
     if (ents.empty()) return 0;
     const char *t = std::getenv("ACFD_LU_TICKETS");
     const bool tickets = t && std::atoi(t) == 1;
-    bool fwd = false, bwd = false;
-    switch (shape) {
-    case 0: fwd = sa_fits_resident<1, 16, 16>(out->total); bwd = sa_fits_resident<-1, 16, 16>(out->total); break;
-    case 1: fwd = sa_fits_resident<1, 16, 8>(out->total); bwd = sa_fits_resident<-1, 16, 8>(out->total); break;
-    case 2: fwd = sa_fits_resident<1, 8, 8>(out->total); bwd = sa_fits_resident<-1, 8, 8>(out->total); break;
-    default: fwd = sa_fits_resident<1, 16, 4>(out->total); bwd = sa_fits_resident<-1, 16, 4>(out->total); break;
-    }
-    out->resident[0] = fwd && !tickets ? 1 : 0;
-    out->resident[1] = bwd && !tickets ? 1 : 0;
+    out->resident[0] = !tickets && sa_fits_resident<1>(out->total) ? 1 : 0;
+    out->resident[1] = !tickets && sa_fits_resident<-1>(out->total) ? 1 : 0;
     if (hipMalloc(&out->ents, ents.size() * sizeof(SaBatchEnt)) != hipSuccess) return 1;
     if (hipMalloc((void **)&out->tile_ent, te.size() * sizeof(int)) != hipSuccess) return 1;
     if (hipMemcpy(out->ents, ents.data(), ents.size() * sizeof(SaBatchEnt), hipMemcpyHostToDevice) != hipSuccess ||
@@ -1597,61 +1733,24 @@ int sa_batch_make(int nblk, const Ext *e, const Fields *f, double *arena, int sh
     return 0;
 }
 
-template <int TJ, int TK>
-static void sa_batch_t(hipStream_t s, const LuBatch &b, int *err, int *ctr, int dir)
-{
-    const SaBatchEnt *ents = (const SaBatchEnt *)b.ents;
-    if (dir >= 0)
-        hipLaunchKernelGGL((k_sa_tiles_batch<1, TJ, TK>), dim3((unsigned)b.total), dim3(TJ * TK), 0, s, ents,
-                           b.tile_ent, b.total, b.resident[0], b.arena, b.ex, err, ctr);
-    if (dir <= 0)
-        hipLaunchKernelGGL((k_sa_tiles_batch<-1, TJ, TK>), dim3((unsigned)b.total), dim3(TJ * TK), 0, s, ents,
-                           b.tile_ent, b.total, b.resident[1], b.arena, b.ex, err, ctr);
-}
-
-template <int TJ, int TK>
-static void sa_sl_batch_t(hipStream_t s, const LuBatch &b, int *err, int *ctr, int dir)
-{
-    const SaBatchEnt *ents = (const SaBatchEnt *)b.ents;
-    if (dir >= 0)
-        hipLaunchKernelGGL((k_sa_sl_batch<1, TJ, TK>), dim3((unsigned)b.total), dim3(TJ * TK), 0, s, ents,
-                           b.tile_ent, b.total, b.resident[0], b.sl, b.ex, err, ctr);
-    if (dir <= 0)
-        hipLaunchKernelGGL((k_sa_sl_batch<-1, TJ, TK>), dim3((unsigned)b.total), dim3(TJ * TK), 0, s, ents,
-                           b.tile_ent, b.total, b.resident[1], b.sl, b.ex, err, ctr);
-}
-
-template <int TT>
-static void sa_layout_batch_t(hipStream_t s, const LuBatch &b, bool to_sl)
-{
-    const SaBatchEnt *ents = (const SaBatchEnt *)b.ents;
-    if (to_sl)
-        hipLaunchKernelGGL((k_sa_layout_batch<TT, true>), dim3((unsigned)b.total), dim3(TT), 0, s, ents, b.tile_ent,
-                           b.arena, b.sl);
-    else
-        hipLaunchKernelGGL((k_sa_layout_batch<TT, false>), dim3((unsigned)b.total), dim3(TT), 0, s, ents,
-                           b.tile_ent, b.arena, b.sl);
-}
-
 // SA sweeps over the SA sweep layout: phase 0 moves a, b, c, diag and rhs
 // into the layout, 1 / -1 run the forward / backward sweep, 2 adds dnut
 // to nut
 int launch_sa_sl_batch(hipStream_t s, const LuBatch &b, int *err, int *ctr, int phase)
 {
     if (b.total <= 0 || !b.sl) return 0;
-    const int tt = kTileShapes[b.shape][0] * kTileShapes[b.shape][1];
-    if (phase == 0 || phase == 2) {
-        if (tt == 256) sa_layout_batch_t<256>(s, b, phase == 0);
-        else if (tt == 128) sa_layout_batch_t<128>(s, b, phase == 0);
-        else sa_layout_batch_t<64>(s, b, phase == 0);
-    } else {
-        switch (b.shape) {
-        case 0: sa_sl_batch_t<16, 16>(s, b, err, ctr, phase); break;
-        case 1: sa_sl_batch_t<16, 8>(s, b, err, ctr, phase); break;
-        case 2: sa_sl_batch_t<8, 8>(s, b, err, ctr, phase); break;
-        default: sa_sl_batch_t<16, 4>(s, b, err, ctr, phase); break;
-        }
-    }
+    const SaBatchEnt *ents = (const SaBatchEnt *)b.ents;
+    const dim3 gr((unsigned)b.total);
+    if (phase == 0)
+        hipLaunchKernelGGL((k_sa_layout_batch<true>), gr, dim3(kLanes), 0, s, ents, b.tile_ent, b.arena, b.sl);
+    else if (phase == 2)
+        hipLaunchKernelGGL((k_sa_layout_batch<false>), gr, dim3(kLanes), 0, s, ents, b.tile_ent, b.arena, b.sl);
+    else if (phase == 1)
+        hipLaunchKernelGGL((k_sa_sl_batch<1>), gr, dim3(kLanes), 0, s, ents, b.tile_ent, b.total, b.resident[0], b.sl,
+                           b.ex, err, ctr);
+    else
+        hipLaunchKernelGGL((k_sa_sl_batch<-1>), gr, dim3(kLanes), 0, s, ents, b.tile_ent, b.total, b.resident[1], b.sl,
+                           b.ex, err, ctr);
     ACFD_CHECK_LAUNCH();
     return 0;
 }
@@ -1660,12 +1759,14 @@ int launch_sa_sl_batch(hipStream_t s, const LuBatch &b, int *err, int *ctr, int 
 int launch_sa_batch(hipStream_t s, const LuBatch &b, int *err, int *ctr, int dir)
 {
     if (b.total <= 0) return 0;
-    switch (b.shape) {
-    case 0: sa_batch_t<16, 16>(s, b, err, ctr, dir); break;
-    case 1: sa_batch_t<16, 8>(s, b, err, ctr, dir); break;
-    case 2: sa_batch_t<8, 8>(s, b, err, ctr, dir); break;
-    default: sa_batch_t<16, 4>(s, b, err, ctr, dir); break;
-    }
+    const SaBatchEnt *ents = (const SaBatchEnt *)b.ents;
+    const dim3 gr((unsigned)b.total);
+    if (dir >= 0)
+        hipLaunchKernelGGL((k_sa_tiles_batch<1>), gr, dim3(kLanes), 0, s, ents, b.tile_ent, b.total, b.resident[0],
+                           b.arena, b.ex, err, ctr);
+    if (dir <= 0)
+        hipLaunchKernelGGL((k_sa_tiles_batch<-1>), gr, dim3(kLanes), 0, s, ents, b.tile_ent, b.total, b.resident[1],
+                           b.arena, b.ex, err, ctr);
     ACFD_CHECK_LAUNCH();
     return 0;
 }
@@ -1678,23 +1779,11 @@ int launch_fill_sentinel(hipStream_t s, double *p, long n)
     return 0;
 }
 
-template <int DIR, int TJ, int TK>
-static void launch_tiles(hipStream_t s, const SlGeom &g, const LuWs &ws, double gamma, const Ext &e, double *q)
-{
-    hipLaunchKernelGGL((k_lu_tiles<DIR, TJ, TK>), dim3((unsigned)g.ntiles), dim3(TJ * TK), 0, s, g, ws.sl, gamma,
-                       ws.ex, ws.err, e, q);
-}
-
 template <int DIR>
-static void launch_tiles_shape(hipStream_t s, int shape, const SlGeom &g, const LuWs &ws, double gamma,
-                               const Ext &e, double *q)
+static void launch_pipe(hipStream_t s, const SlGeom &g, const LuWs &ws, double gamma, const Ext &e, double *q)
 {
-    switch (shape) {
-    case 0: launch_tiles<DIR, 16, 16>(s, g, ws, gamma, e, q); break;
-    case 1: launch_tiles<DIR, 16, 8>(s, g, ws, gamma, e, q); break;
-    case 2: launch_tiles<DIR, 8, 8>(s, g, ws, gamma, e, q); break;
-    default: launch_tiles<DIR, 16, 4>(s, g, ws, gamma, e, q); break;
-    }
+    hipLaunchKernelGGL((k_lu_pipe<DIR>), dim3((unsigned)g.ntiles), dim3(kPipeThreads), 0, s, g, ws.sl, gamma, ws.ex,
+                       ws.err, g.ntiles > ws.resident[DIR > 0 ? 0 : 1] ? ws.ctr : nullptr, e, q);
 }
 
 // Phases of one LU-SGS update:
@@ -1706,9 +1795,9 @@ static void launch_tiles_shape(hipStream_t s, int shape, const SlGeom &g, const 
 //   2 forward sweep, 3 backward sweep,
 //   4 q += dq (tiles: from the sweep layout, or fused into the backward
 //     sweep, which then stores q + dq itself).
-// variant 0 = hyperplanes, 1 = tiles of the given shape index.
+// variant 0 = hyperplanes, 1 = tiles.
 int launch_lusgs_phase(hipStream_t s, const Ext &e, const Fields &f, const Consts &c, const double *cfl,
-                       int variant, const LuWs *ws, int phase, int shape, int geo_cached)
+                       int variant, const LuWs *ws, int phase, int geo_cached)
 {
     int Li = e.ie1 - e.is1 + 1, Lj = e.je1 - e.js1 + 1, Lk = e.ke1 - e.ks1 + 1;
     const bool tiles = variant == 1 && ws && ws->sl && ws->ex;
@@ -1719,18 +1808,12 @@ int launch_lusgs_phase(hipStream_t s, const Ext &e, const Fields &f, const Const
     } else if (empty) {
         return 0;
     } else if (tiles) {
-        const SlGeom g = sl_geom(e, shape);
-        if (phase == 1)
-            launch_layout_tt(s, 0, e, g, f, *ws, geo_cached ? kSlGeoPairs : 0);
-        else if (phase == 2 || phase == 3) {
-            if (phase == 2) launch_tiles_shape<1>(s, shape, g, *ws, c.gamma, e, nullptr);
-            else launch_tiles_shape<-1>(s, shape, g, *ws, c.gamma, e, fused_add(computed_nodes(e)) ? f.q : nullptr);
-            if (g.refill) {
-                const long n = (long)g.ntiles * (g.exj_tile + g.exk_tile);
-                hipLaunchKernelGGL(k_fill_sentinel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, ws->ex, n);
-            }
-        } else if (!fused_add(computed_nodes(e)))
-            launch_layout_tt(s, 1, e, g, f, *ws);
+        const SlGeom g = sl_geom(e);
+        const bool fuse = fused_add(computed_nodes(e));
+        if (phase == 1) launch_layout(s, 0, e, g, f, *ws, geo_cached ? kSlGeoPairs : 0);
+        else if (phase == 2) launch_pipe<1>(s, g, *ws, c.gamma, e, nullptr);
+        else if (phase == 3) launch_pipe<-1>(s, g, *ws, c.gamma, e, fuse ? f.q : nullptr);
+        else if (!fuse) launch_layout(s, 1, e, g, f, *ws);
     } else if (phase == 4) {
         Box b{e.is1, e.ie1, e.js1, e.je1, e.ks1, e.ke1};
         hipLaunchKernelGGL(k_add5, box_grid(b), dim3(64, 4, 1), 0, s, e, b, f.q, f.w_dq);
@@ -1747,16 +1830,6 @@ int launch_lusgs_phase(hipStream_t s, const Ext &e, const Fields &f, const Const
         }
     }
     ACFD_CHECK_LAUNCH();
-    return 0;
-}
-
-int launch_lusgs(hipStream_t s, const Ext &e, const Fields &f, const Consts &c, const double *cfl,
-                 int variant, const LuWs *ws, int shape)
-{
-    for (int ph = 0; ph < kLusgsPhases; ph++) {
-        int rc = launch_lusgs_phase(s, e, f, c, cfl, variant, ws, ph, shape);
-        if (rc) return rc;
-    }
     return 0;
 }
 

@@ -505,7 +505,7 @@ int launch_sa(hipStream_t s, const Ext &e, const Fields &f, const Consts &c, con
     int rc = launch_sa_pre(s, e, f, c, cfl);
     if (!rc) {
         if (sweep)
-            rc = launch_sa_sweeps(s, e, sweep->shape, f.w_dqs, f.sa_rhs, f.w_sa + 8 * e.n, f.w_dq, sweep->ex,
+            rc = launch_sa_sweeps(s, e, f.w_dqs, f.sa_rhs, f.w_sa + 8 * e.n, f.w_dq, sweep->ex,
                                   sweep->err);
         else
             rc = launch_sa_planes(s, e, f);

@@ -106,35 +106,34 @@ int launch_wall_forces(hipStream_t s, const BlockRec *blks, const WallCell *cell
 
 // k_lusgs.hip
 // workspace of the tile sweeps: sweep-layout operands (normal memory),
-// exchange slots (uncached memory, sentinel-filled) and an error word
+// exchange slots (uncached memory, sentinel-filled), an error word and the
+// ticket counters; resident: tiles of the forward / backward sweep of one
+// block that fit on the device at once (more are handed out by ticket)
 struct LuWs {
     double *sl;
     double *ex;
     int *err;
+    int *ctr = nullptr;
+    int resident[2] = {0, 0};
 };
+void lusgs_resident(int *tiles);
 constexpr int kLusgsPhases = 5;
-int launch_lusgs(hipStream_t s, const Ext &e, const Fields &f, const Consts &c, const double *cfl,
-                 int variant, const LuWs *ws, int shape);
 int launch_lusgs_phase(hipStream_t s, const Ext &e, const Fields &f, const Consts &c, const double *cfl,
-                       int variant, const LuWs *ws, int phase, int shape, int geo_cached = 0);
-int lusgs_tile_shapes();
-long lusgs_tiles(const Ext &e, int shape);
-// doubles of the sweep layout and of the exchange slots (max over shapes)
+                       int variant, const LuWs *ws, int phase, int geo_cached = 0);
+// doubles of the sweep layout and of the exchange slots
 void lusgs_ws_sizes(const Ext &e, long *sl_n, long *ex_n);
-// all blocks' tile sweeps in one launch per phase (one tile shape for all)
+// all blocks' tile sweeps in one launch per phase
 struct LuBatch {
     void *ents = nullptr;     // device table, one entry per block
     int *tile_ent = nullptr;  // device, entry of each flat tile number
     double *arena = nullptr, *sl = nullptr, *ex = nullptr;  // bases of the table's offsets
-    int nent = 0, total = 0, shape = 0;
+    int nent = 0, total = 0;
     int resident[2] = {0, 0};  // forward / backward sweep: every workgroup fits on the device at once
     int fuse_add = 0;          // the backward sweep stores q + dq (no add pass)
-    int refill = 0;            // the exchange region is refilled with the sentinel after each sweep
-    long ex_n = 0;             // doubles of the exchange region the batch uses
 };
-void lusgs_batch_ws(int nblk, const Ext *e, int shape, long *sl_n, long *ex_n);
+void lusgs_batch_ws(int nblk, const Ext *e, long *sl_n, long *ex_n);
 // f[m]'s fields must lie in the allocation starting at arena
-int lusgs_batch_make(int nblk, const Ext *e, const Fields *f, double *arena, int shape, double *sl, double *ex,
+int lusgs_batch_make(int nblk, const Ext *e, const Fields *f, double *arena, double *sl, double *ex,
                      LuBatch *out);
 void lusgs_batch_free(LuBatch *b);
 int launch_lusgs_batch(hipStream_t s, const LuBatch &b, int phase, double gamma, int *err, int *ctr,
@@ -142,11 +141,11 @@ int launch_lusgs_batch(hipStream_t s, const LuBatch &b, int phase, double gamma,
 
 int launch_fill_sentinel(hipStream_t s, double *p, long n);
 // tile sweeps of the SA model's scalar LU-SGS (cu = a, b, c, diag)
-int launch_sa_sweeps(hipStream_t s, const Ext &e, int shape, const double *cu, const double *rhs, double *dns,
+int launch_sa_sweeps(hipStream_t s, const Ext &e, const double *cu, const double *rhs, double *dns,
                      double *dn, double *ex, int *err);
-// sl: the SA sweep layout (sa_batch_sl doubles for this shape) or null
-void sa_batch_sl(int nblk, const Ext *e, int shape, long *sl_n);
-int sa_batch_make(int nblk, const Ext *e, const Fields *f, double *arena, int shape, double *ex, double *sl,
+// sl: the SA sweep layout (sa_batch_sl doubles) or null
+void sa_batch_sl(int nblk, const Ext *e, long *sl_n);
+int sa_batch_make(int nblk, const Ext *e, const Fields *f, double *arena, double *ex, double *sl,
                   LuBatch *out);
 // the batched SA sweeps over the SA sweep layout: phase 0 operands into
 // the layout, 1 forward sweep, -1 backward sweep, 2 nut += dnut
@@ -160,7 +159,6 @@ int launch_update_q0(hipStream_t s, const Ext &e, const Fields &f);
 
 // k_sa.hip
 struct SaSweep {
-    int shape;   // tile shape index
     double *ex;  // sentinel-filled exchange slots
     int *err;
 };
