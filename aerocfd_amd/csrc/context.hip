@@ -1039,17 +1039,38 @@ int st_sa_all(acfd_ctx *ctx, F cfl_of)
 }
 
 
+// crank2nd and update_q0 of every block: one launch per kernel with
+// batch_blocks, else block after block (the same kernels)
 int st_crank(acfd_ctx *ctx, int m)
 {
     StageTimer t(ctx, ACFD_STAGE_CRANK2ND);
-    KRN_TRY(launch_crank(ctx->stream, ctx->blk[m].e, ctx->blk[m].f, ctx->c));
+    const Ext *e = &ctx->blk[m].e;
+    KRN_TRY(launch_crank(ctx->stream, ctx->d_blocks, m, 1, &e, nullptr, ctx->arena, ctx->c));
     return 0;
 }
 
-int st_update_q0(acfd_ctx *ctx, int m)
+int st_crank_all(acfd_ctx *ctx)
 {
-    StageTimer t(ctx, ACFD_STAGE_UPDATE_Q0);
-    KRN_TRY(launch_update_q0(ctx->stream, ctx->blk[m].e, ctx->blk[m].f));
+    int rc = 0;
+    if (!batched(ctx)) {
+        for (int m = 0; m < (int)ctx->blk.size() && !rc; m++) rc = st_crank(ctx, m);
+        return rc;
+    }
+    StageTimer t(ctx, ACFD_STAGE_CRANK2ND);
+    std::vector<const Ext *> e;
+    for (auto &b : ctx->blk) e.push_back(&b.e);
+    KRN_TRY(launch_crank(ctx->stream, ctx->d_blocks, 0, (int)e.size(), e.data(), &ctx->bg_prep, ctx->arena, ctx->c));
+    return 0;
+}
+
+int st_update_q0_all(acfd_ctx *ctx)
+{
+    const bool all = batched(ctx);
+    for (int m = 0; m < (all ? 1 : (int)ctx->blk.size()); m++) {
+        StageTimer t(ctx, ACFD_STAGE_UPDATE_Q0);
+        KRN_TRY(launch_update_q0(ctx->stream, ctx->d_blocks, m, ctx->blk[m].e, all ? &ctx->bg_prep : nullptr,
+                                 ctx->arena));
+    }
     return 0;
 }
 
@@ -1328,9 +1349,9 @@ int one_step(acfd_ctx *ctx)
         for (int sub = 0; sub < 3 && !rc; sub++) {
             rc = refresh(ctx);
             if (!rc) rc = residual_stage_all(ctx, aux);
-            for (int m = 0; m < nb && !rc; m++) rc = st_crank(ctx, m);
+            if (!rc) rc = st_crank_all(ctx);
         }
-        for (int m = 0; m < nb && !rc; m++) rc = st_update_q0(ctx, m);
+        if (!rc) rc = st_update_q0_all(ctx);
         // after the sub-iterations the reference's cfl is the last block's
         for (int m = 0; m < nb && !rc && sa; m++) rc = st_sa(ctx, m, ctx->d_cfl);
         if (!rc) rc = refresh(ctx);
@@ -1351,7 +1372,7 @@ int one_step(acfd_ctx *ctx)
                 if (!rc) rc = st_crank(ctx, m);
             }
         }
-        for (int m = 0; m < nb && !rc; m++) rc = st_update_q0(ctx, m);
+        if (!rc) rc = st_update_q0_all(ctx);
         // after the sub-iterations the reference's cfl is the last block's
         for (int m = 0; m < nb && !rc && sa; m++) rc = st_sa(ctx, m, ctx->d_cfl);
         if (!rc) rc = refresh(ctx);
@@ -1701,6 +1722,7 @@ int acfd_set_topology(acfd_ctx *ctx, int nblk, const int *dims, const int *nsub,
         return rc;
     HIP_TRY(hipMalloc((void **)&ctx->d_partial, (size_t)parts * 6 * sizeof(double)));
     rc = alloc_lu_ws(ctx);
+    if (!rc && ctx->cfg.iflag_timeadvance == 3) rc = ensure_block_table(ctx);
     if (!rc) rc = build_batch(ctx);
     if (rc) return rc;
     HIP_TRY(hipStreamSynchronize(ctx->stream));
@@ -1814,11 +1836,11 @@ int acfd_run_stage(acfd_ctx *ctx, int stage)
     case ACFD_STAGE_AVERAGE: rc = st_average(ctx); break;
     case ACFD_STAGE_CRANK2ND:
         if (ctx->cfg.iflag_timeadvance != 3) return fail(ACFD_EINVAL, "crank stage needs iflag_timeadvance = 3");
-        for (int m = 0; m < nb && !rc; m++) rc = st_crank(ctx, m);
+        rc = st_crank_all(ctx);
         break;
     case ACFD_STAGE_UPDATE_Q0:
         if (ctx->cfg.iflag_timeadvance != 3) return fail(ACFD_EINVAL, "q0 stage needs iflag_timeadvance = 3");
-        for (int m = 0; m < nb && !rc; m++) rc = st_update_q0(ctx, m);
+        if (!rc) rc = st_update_q0_all(ctx);
         break;
     default: return fail(ACFD_EINVAL, "acfd_run_stage: unknown stage");
     }
@@ -2421,6 +2443,7 @@ int make_single(const acfd_config *cfg, const int *r, acfd_ctx **out)
     dev_upload(&ctx->d_ntab, nn);
     HIP_TRY(hipMalloc((void **)&ctx->d_partial, (size_t)residual_partials(e) * 6 * sizeof(double)));
     rc = alloc_lu_ws(ctx);
+    if (!rc && c.iflag_timeadvance == 3) rc = ensure_block_table(ctx);
     if (rc) return rc;
     ctx->totalnodes = (long)(e.ie0 - e.is0 + 1) * (e.je0 - e.js0 + 1) * (e.ke0 - e.ks0 + 1);
     ctx->topo = true;

@@ -154,8 +154,11 @@ int launch_sa_sl_batch(hipStream_t s, const LuBatch &b, int *err, int *ctr, int 
 int launch_sa_batch(hipStream_t s, const LuBatch &b, int *err, int *ctr, int dir = 0);
 
 // k_bdf2.hip
-int launch_crank(hipStream_t s, const Ext &e, const Fields &f, const Consts &c);
-int launch_update_q0(hipStream_t s, const Ext &e, const Fields &f);
+// blocks m0 .. m0 + nblk - 1 of the table (exts: their ranges); bg: the
+// linear-tile grid of all blocks, or null for one block
+int launch_crank(hipStream_t s, const BlockRec *blks, int m0, int nblk, const Ext *const *exts, const BatchGrid *bg,
+                 double *arena, const Consts &c);
+int launch_update_q0(hipStream_t s, const BlockRec *blks, int m0, const Ext &e, const BatchGrid *bg, double *arena);
 
 // k_sa.hip
 struct SaSweep {
