@@ -81,6 +81,11 @@ struct Block {
     Fields f;
     long arena_off = 0;     // doubles from the context's arena base
     double *geo = nullptr;  // acfd_grid_metrics: x, y, z, spci, spcj, spck (n each)
+    // rhsi is zero outside the computed range (the arena starts zeroed and
+    // the inviscid kernels store only inside it): the inviscid stage then
+    // skips clearing it.  An upload of rhsi clears the flag (and drops a
+    // captured step that relied on it).
+    bool rhsi_clean = true;
     std::vector<acfd_subface> sub;
 };
 
@@ -130,6 +135,7 @@ struct acfd_ctx {
     double *d_fwork = nullptr;
     long totalnodes = 0;
     bool topo = false;
+    int inv_run = 16;         // nodes per thread of the j / k inviscid kernels
     // device scalars
     double *d_cfl = nullptr;
     unsigned long long *d_stats = nullptr;
@@ -155,11 +161,6 @@ struct acfd_ctx {
     // step that did so replays only while it holds.
     bool pri_current = false;
     bool graph_needs_pri = false;
-    // rhsi is zero outside every block's computed range (the arena starts
-    // zeroed and the inviscid kernels store only inside it): the batched
-    // inviscid stage then skips clearing it.  An upload of rhsi clears the
-    // flag (and drops a captured step that relied on it).
-    bool rhsi_clean = true;
     // the last residual stage also formed implicit1st's rhs, spectral radii
     // and diagonal (batched, steady NS): the next batched update skips its
     // preparation pass
@@ -532,7 +533,7 @@ int build_batch(acfd_ctx *ctx)
     for (auto &b : ctx->blk) {
         g_pri.push_back(grid_1d(b.e.n));
         g_zero.push_back(grid_1d(5 * b.e.n));
-        for (int a = 0; a < 3; a++) g_inv[a].push_back(inviscid_grid(b.e, a));
+        for (int a = 0; a < 3; a++) g_inv[a].push_back(inviscid_grid(b.e, a, ctx->inv_run));
         g_visc.push_back(viscous_grid(b.e));
         g_prep.push_back(lu_prep_grid(b.e));
     }
@@ -771,14 +772,16 @@ int inviscid_with_sensor(acfd_ctx *ctx, int m)
     Block &b = ctx->blk[m];
     const long call = ctx->s_calls[m]++;
     SensorArgs sa{ctx->s_net, ctx->s_thr, ctx->s_stats, nullptr, 0};
+    const bool clear = !b.rhsi_clean;
+    b.rhsi_clean = true;
     if (ctx->s_refresh > 1) {
         sa.mask = ctx->s_mask[m];
         sa.replay = call % ctx->s_refresh != 0;
     }
     if (ctx->s_audit > 0 && call % ctx->s_audit == 0) {
-        KRN_TRY(launch_inviscid_ext(ctx->stream, b.e, b.f, ctx->c, ctx->cfg.precision, 2));
+        KRN_TRY(launch_inviscid_ext(ctx->stream, b.e, b.f, ctx->c, ctx->cfg.precision, 2, ctx->inv_run, clear));
         KRN_TRY(launch_copy(ctx->stream, b.f.rhsi, b.f.w_flux, 5 * b.e.n));
-        KRN_TRY(launch_inviscid_wcns_sensor(ctx->stream, b.e, b.f, ctx->c, ctx->cfg.precision, sa));
+        KRN_TRY(launch_inviscid_wcns_sensor(ctx->stream, b.e, b.f, ctx->c, ctx->cfg.precision, ctx->inv_run, clear, sa));
         const long np = diff_partials(b.e);
         if (ctx->s_dpart_n < 2 * np) {
             if (ctx->s_dpart) (void)hipFree(ctx->s_dpart);
@@ -804,7 +807,7 @@ int inviscid_with_sensor(acfd_ctx *ctx, int m)
         }
         return 0;
     }
-    KRN_TRY(launch_inviscid_wcns_sensor(ctx->stream, b.e, b.f, ctx->c, ctx->cfg.precision, sa));
+    KRN_TRY(launch_inviscid_wcns_sensor(ctx->stream, b.e, b.f, ctx->c, ctx->cfg.precision, ctx->inv_run, clear, sa));
     return 0;
 }
 
@@ -812,11 +815,14 @@ int st_inviscid(acfd_ctx *ctx, int m)
 {
     StageTimer t(ctx, ACFD_STAGE_INVISCID);
     if (ctx->s_on && ctx->cfg.inviscid_scheme == 2 && !ctx->s_off[m]) return inviscid_with_sensor(ctx, m);
+    Block &b = ctx->blk[m];
+    const bool clear = !b.rhsi_clean;
     if (ctx->cfg.inviscid_scheme == 0)
-        KRN_TRY(launch_inviscid(ctx->stream, ctx->blk[m].e, ctx->blk[m].f, ctx->c, ctx->cfg.precision));
+        KRN_TRY(launch_inviscid(ctx->stream, b.e, b.f, ctx->c, ctx->cfg.precision, ctx->inv_run, clear));
     else
-        KRN_TRY(launch_inviscid_ext(ctx->stream, ctx->blk[m].e, ctx->blk[m].f, ctx->c, ctx->cfg.precision,
-                                    ctx->cfg.inviscid_scheme));
+        KRN_TRY(launch_inviscid_ext(ctx->stream, b.e, b.f, ctx->c, ctx->cfg.precision, ctx->cfg.inviscid_scheme,
+                                    ctx->inv_run, clear));
+    b.rhsi_clean = true;
     return 0;
 }
 
@@ -1157,18 +1163,21 @@ int st_inviscid_all(acfd_ctx *ctx)
     }
     StageTimer t(ctx, ACFD_STAGE_INVISCID);
     // rhsi outside the computed ranges needs clearing only after an upload
-    const int first = ctx->rhsi_clean ? 1 : 0;
-    ctx->rhsi_clean = true;
+    int first = 1;
+    for (auto &b : ctx->blk) {
+        if (!b.rhsi_clean) first = 0;
+        b.rhsi_clean = true;
+    }
     if (ctx->timing) {
         for (int part = first; part < 4; part++) {
             StageTimer ts(ctx, kTimeInvZero + part);
             KRN_TRY(launch_inviscid_batch(ctx->stream, ctx->d_blocks, ctx->bg_inv, ctx->arena, ctx->c,
-                                          ctx->cfg.precision, part));
+                                          ctx->cfg.precision, ctx->inv_run, part));
         }
         return 0;
     }
     KRN_TRY(launch_inviscid_batch(ctx->stream, ctx->d_blocks, ctx->bg_inv, ctx->arena, ctx->c, ctx->cfg.precision,
-                                  first ? -2 : -1));
+                                  ctx->inv_run, first ? -2 : -1));
     return 0;
 }
 
@@ -1721,6 +1730,7 @@ int acfd_set_topology(acfd_ctx *ctx, int nblk, const int *dims, const int *nsub,
         (rc = dev_upload(&ctx->d_ntab, ntab)))
         return rc;
     HIP_TRY(hipMalloc((void **)&ctx->d_partial, (size_t)parts * 6 * sizeof(double)));
+    ctx->inv_run = inviscid_run(ctx->totalnodes, ctx->cfg.inviscid_scheme, ctx->cfg.precision);
     rc = alloc_lu_ws(ctx);
     if (!rc && ctx->cfg.iflag_timeadvance == 3) rc = ensure_block_table(ctx);
     if (!rc) rc = build_batch(ctx);
@@ -1770,7 +1780,7 @@ int acfd_upload(acfd_ctx *ctx, int m, int field, const double *host)
     }
     ctx->lu_prep_ready = false;
     if (field == ACFD_RHSI) {
-        ctx->rhsi_clean = false;
+        b.rhsi_clean = false;
         drop_graph(ctx);
     }
     int nc = kNcomp[field];
@@ -2442,6 +2452,7 @@ int make_single(const acfd_config *cfg, const int *r, acfd_ctx **out)
     dev_upload(&ctx->d_nuttab, nt);
     dev_upload(&ctx->d_ntab, nn);
     HIP_TRY(hipMalloc((void **)&ctx->d_partial, (size_t)residual_partials(e) * 6 * sizeof(double)));
+    ctx->inv_run = inviscid_run(e.n, c.inviscid_scheme, c.precision);
     rc = alloc_lu_ws(ctx);
     if (!rc && c.iflag_timeadvance == 3) rc = ensure_block_table(ctx);
     if (rc) return rc;

@@ -188,9 +188,30 @@ __global__ void __launch_bounds__(256) k_inviscid_i(Ext e, const double *__restr
 }
 
 // The j and k directions (:160-243): each thread marches along the axis
-// over kInvRun nodes, keeping the four-value window and the previous face
-// flux in registers, so each face is evaluated once.  rhsi -= (F+ - F-).
-constexpr int kInvRun = 16;
+// over `run` nodes, keeping the four-value window and the previous face
+// flux in registers, so a run evaluates run + 1 faces.  rhsi -= (F+ - F-).
+//
+// The run of a context comes from its nodes: long runs repeat fewer faces
+// at their ends (and, for the wide stencils, fewer node loads), short ones
+// put more wavefronts on a device that holds 2-3 thousand of them.  Inviscid
+// stage of WENO3 + Roe, us, at runs of 1 / 4 / 8 / 16: 33^3 26 / 38 / 57 /
+// 97, 65^3 50 / 47 / 63 / 101, 129^3 375 / 287 / 291 / 317, 193^3 1174 / 893
+// / 889 / 932, 256^3 - / 1814 / 1729 / 1732, 98 M nodes in 40 blocks best at
+// 16.  WENO5 splitting and WCNS (three evaluations) at 2 / 4 / 16 / 32:
+// 41^3 187 / 253 / 658 / 1156 and 172 / 211 / 464 / 772, 65^3 398 / 384 /
+// 778 / 1295 and 322 / 274 / 522 / 834, 129^3 2218 / 1998 / 1826 / 1998 and
+// 1948 / 1500 / 1222 / 1353, 193^3 WCNS 6265 / 4571 / 3764 / 3789.  A run's
+// first face of WENO3 + Roe is a second copy of the flux code, rounded in
+// its own way: the rule takes the context's nodes, not a launch's, so that
+// batched and per-block launches cut the same runs, and FP32 fluxes, where
+// an ulp is 1e-7, keep the run of 16 that they were measured with.
+constexpr int kInvRunF32 = 16;
+int inviscid_run(long nodes, int scheme, int precision)
+{
+    if (scheme != 0) return nodes < 150000 ? 2 : nodes < 1000000 ? 4 : 16;
+    if (precision == 1) return kInvRunF32;
+    return nodes < 100000 ? 1 : nodes < 4000000 ? 4 : nodes < 32000000 ? 8 : 16;
+}
 // Waves per SIMD asked of the k kernel: FP64 it needs 176 VGPRs (two
 // waves); held to 168 with a few values in scratch it runs three, and on
 // the 40-block channel takes 3.84 ms instead of 4.32.  The same bound on
@@ -198,12 +219,13 @@ constexpr int kInvRun = 16;
 // is slower by a third or more.
 constexpr int kInvKWaves = 3;
 template <typename R, int AXIS>
-__device__ inline void inviscid_jk_body(const Ext &e, int bx, int by, int bz, const double *__restrict__ q,
+__device__ inline void inviscid_jk_body(const Ext &e, int run_, int bx, int by, int bz, const double *__restrict__ q,
                                         const double *__restrict__ dxidx, const double *__restrict__ inv_j,
                                         double *__restrict__ rhsi, double gamma)
 {
-    const int a0 = e.lo1(AXIS) + bz * kInvRun;
-    const int a1 = min(a0 + kInvRun - 1, e.hi1(AXIS));
+    const int run = sizeof(R) == 4 ? kInvRunF32 : run_;  // a constant: see inviscid_run
+    const int a0 = e.lo1(AXIS) + bz * run;
+    const int a1 = min(a0 + run - 1, e.hi1(AXIS));
     int i, j, k;
     if (AXIS == 1) {
         i = e.is1 + (int)(bx * blockDim.x + threadIdx.x);
@@ -267,9 +289,9 @@ template <typename R, int AXIS>
 __global__ void __launch_bounds__(256, AXIS == 2 ? kInvKWaves : 1) k_inviscid_jk(Ext e, const double *__restrict__ q,
                                                     const double *__restrict__ dxidx,
                                                     const double *__restrict__ inv_j,
-                                                    double *__restrict__ rhsi, double gamma)
+                                                    double *__restrict__ rhsi, double gamma, int run)
 {
-    inviscid_jk_body<R, AXIS>(e, (int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z, q, dxidx, inv_j, rhsi, gamma);
+    inviscid_jk_body<R, AXIS>(e, run, (int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z, q, dxidx, inv_j, rhsi, gamma);
 }
 
 // AXIS 0 = the i kernel, 1 / 2 = the j / k kernels.  The k kernel runs at
@@ -277,7 +299,7 @@ __global__ void __launch_bounds__(256, AXIS == 2 ? kInvKWaves : 1) k_inviscid_jk
 template <typename R, int AXIS>
 __global__ void __launch_bounds__(256, AXIS == 2 ? kInvKWaves : 1) k_inviscid_batch(const BlockRec *__restrict__ blks,
                                                         const int *__restrict__ map,
-                                                        const KGrid *__restrict__ kg, double *arena, double gamma)
+                                                        const KGrid *__restrict__ kg, double *arena, double gamma, int run)
 {
     int bx, by, bz;
     const BlockRec &b = blks[batch_wg(map, kg, bx, by, bz)];
@@ -286,72 +308,72 @@ __global__ void __launch_bounds__(256, AXIS == 2 ? kInvKWaves : 1) k_inviscid_ba
         inviscid_i_body<R>(e, bx, by, bz, arena + b.o.q, arena + b.o.dxidx, arena + b.o.inv_j, arena + b.o.rhsi,
                            gamma);
     else
-        inviscid_jk_body<R, AXIS>(e, bx, by, bz, arena + b.o.q, arena + b.o.dxidx, arena + b.o.inv_j,
+        inviscid_jk_body<R, AXIS>(e, run, bx, by, bz, arena + b.o.q, arena + b.o.dxidx, arena + b.o.inv_j,
                                   arena + b.o.rhsi, gamma);
 }
 
 // per-block grids of the three inviscid kernels (64 x 4 threads)
-dim3 inviscid_grid(const Ext &e, int axis)
+dim3 inviscid_grid(const Ext &e, int axis, int run)
 {
     const int Li = e.ie1 - e.is1 + 1, Lj = e.je1 - e.js1 + 1, Lk = e.ke1 - e.ks1 + 1;
     if (Li <= 0 || Lj <= 0 || Lk <= 0) return dim3(0, 0, 0);
     if (axis == 0) return dim3((Li + kInvI - 1) / kInvI, (Lj + 3) / 4, Lk);
-    if (axis == 1) return dim3((Li + 63) / 64, (Lk + 3) / 4, (Lj + kInvRun - 1) / kInvRun);
+    if (axis == 1) return dim3((Li + 63) / 64, (Lk + 3) / 4, (Lj + run - 1) / run);
     // k: linear positions over the whole (extended) i-j plane
-    return dim3((unsigned)(((long)e.ni * e.nj + 255) / 256), 1, (Lk + kInvRun - 1) / kInvRun);
+    return dim3((unsigned)(((long)e.ni * e.nj + 255) / 256), 1, (Lk + run - 1) / run);
 }
 
 template <typename R>
-static void launch_inviscid_t(hipStream_t s, const Ext &e, const Fields &f, double gamma)
+static void launch_inviscid_t(hipStream_t s, const Ext &e, const Fields &f, double gamma, int run)
 {
     dim3 t(64, 4, 1);
-    hipLaunchKernelGGL((k_inviscid_i<R>), inviscid_grid(e, 0), t, 0, s, e, f.q, f.dxidx, f.inv_j, f.rhsi, gamma);
-    hipLaunchKernelGGL((k_inviscid_jk<R, 1>), inviscid_grid(e, 1), t, 0, s, e, f.q, f.dxidx, f.inv_j, f.rhsi,
-                       gamma);
-    hipLaunchKernelGGL((k_inviscid_jk<R, 2>), inviscid_grid(e, 2), t, 0, s, e, f.q, f.dxidx, f.inv_j, f.rhsi,
-                       gamma);
+    hipLaunchKernelGGL((k_inviscid_i<R>), inviscid_grid(e, 0, run), t, 0, s, e, f.q, f.dxidx, f.inv_j, f.rhsi, gamma);
+    hipLaunchKernelGGL((k_inviscid_jk<R, 1>), inviscid_grid(e, 1, run), t, 0, s, e, f.q, f.dxidx, f.inv_j, f.rhsi,
+                       gamma, run);
+    hipLaunchKernelGGL((k_inviscid_jk<R, 2>), inviscid_grid(e, 2, run), t, 0, s, e, f.q, f.dxidx, f.inv_j, f.rhsi,
+                       gamma, run);
 }
 
 // WENO3 + Roe residual of every block: bg[0] = rhsi zeroing (1-D over 5n),
 // bg[1..3] = the i, j, k kernels
 template <typename R>
 static void inviscid_batch_dirs(hipStream_t s, const BlockRec *blks, const BatchGrid *bg, double *arena, double gamma,
-                                int part)
+                                int part, int run)
 {
     const dim3 t(64, 4, 1);
     if (part < 0 || part == 1)
         hipLaunchKernelGGL((k_inviscid_batch<R, 0>), dim3((unsigned)bg[1].total), t, 0, s, blks, bg[1].map,
-                           bg[1].kg, arena, gamma);
+                           bg[1].kg, arena, gamma, run);
     if (part < 0 || part == 2)
         hipLaunchKernelGGL((k_inviscid_batch<R, 1>), dim3((unsigned)bg[2].total), t, 0, s, blks, bg[2].map,
-                           bg[2].kg, arena, gamma);
+                           bg[2].kg, arena, gamma, run);
     if (part < 0 || part == 3)
         hipLaunchKernelGGL((k_inviscid_batch<R, 2>), dim3((unsigned)bg[3].total), t, 0, s, blks, bg[3].map,
-                           bg[3].kg, arena, gamma);
+                           bg[3].kg, arena, gamma, run);
 }
 
 int launch_inviscid_batch(hipStream_t s, const BlockRec *blks, const BatchGrid *bg, double *arena,
-                          const Consts &c, int precision, int part)
+                          const Consts &c, int precision, int run, int part)
 {
     if (bg[0].total > 0 && (part == -1 || part == 0))
         hipLaunchKernelGGL(k_zero_rhsi_batch, dim3((unsigned)bg[0].total), dim3(256), 0, s, blks, bg[0].map,
                            bg[0].kg, arena);
     if (bg[1].total <= 0 || part == 0) return 0;
     const int dirs = part < 0 ? -1 : part;
-    if (precision == 1) inviscid_batch_dirs<float>(s, blks, bg, arena, c.gamma, dirs);
-    else inviscid_batch_dirs<double>(s, blks, bg, arena, c.gamma, dirs);
+    if (precision == 1) inviscid_batch_dirs<float>(s, blks, bg, arena, c.gamma, dirs, run);
+    else inviscid_batch_dirs<double>(s, blks, bg, arena, c.gamma, dirs, run);
     ACFD_CHECK_LAUNCH();
     return 0;
 }
 
-int launch_inviscid(hipStream_t s, const Ext &e, const Fields &f, const Consts &c, int precision)
+int launch_inviscid(hipStream_t s, const Ext &e, const Fields &f, const Consts &c, int precision, int run, bool clear)
 {
     // rhsi is zero outside the computed range (sub_inviscid1.f90:102)
-    int rc = launch_fill(s, f.rhsi, 5 * e.n, 0.0);
+    int rc = clear ? launch_fill(s, f.rhsi, 5 * e.n, 0.0) : 0;
     if (rc) return rc;
     if (e.ie1 < e.is1 || e.je1 < e.js1 || e.ke1 < e.ks1) return 0;
-    if (precision == 1) launch_inviscid_t<float>(s, e, f, c.gamma);
-    else launch_inviscid_t<double>(s, e, f, c.gamma);
+    if (precision == 1) launch_inviscid_t<float>(s, e, f, c.gamma, run);
+    else launch_inviscid_t<double>(s, e, f, c.gamma, run);
     ACFD_CHECK_LAUNCH();
     return 0;
 }

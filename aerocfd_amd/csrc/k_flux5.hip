@@ -213,9 +213,8 @@ __device__ inline double ext_diff(const R (*FR)[5], int x, int dord)
     return 75.0 / 64.0 * d1 - 25.0 / 384.0 * d3 + 3.0 / 640.0 * d5;
 }
 
-// j and k directions: each thread marches along the axis over kExtRun nodes
+// j and k directions: each thread marches along the axis over `run` nodes
 // with rolling windows of node quantities and face fluxes.
-constexpr int kExtRun = 32;
 // one wavefront's face counts into its slot (called by one lane)
 __device__ inline void sensor_count(unsigned long long *stats, unsigned long long ne, unsigned long long nl)
 {
@@ -230,13 +229,13 @@ template <typename R, int AXIS, int SCHEME, int SENS>
 __global__ void __launch_bounds__(256) k_ext_jk(Ext e, const double *__restrict__ q,
                                                const double *__restrict__ dxidx,
                                                const double *__restrict__ inv_j, double *__restrict__ rhsi,
-                                               double gamma_d, SensorArgs sa)
+                                               double gamma_d, SensorArgs sa, int run)
 {
     constexpr int NQ = SCHEME == 1 ? 10 : 5;
     const int ir = e.is1 + (int)(blockIdx.x * blockDim.x + threadIdx.x);
     const int orr = (int)(blockIdx.y * blockDim.y + threadIdx.y);
-    const int a0 = e.lo1(AXIS) + (int)blockIdx.z * kExtRun;
-    const int a1 = min(a0 + kExtRun - 1, e.hi1(AXIS));
+    const int a0 = e.lo1(AXIS) + (int)blockIdx.z * run;
+    const int a1 = min(a0 + run - 1, e.hi1(AXIS));
     const bool active = ir <= e.ie1 && (AXIS == 1 ? e.ks1 + orr <= e.ke1 : e.js1 + orr <= e.je1);
     // with the sensor every lane takes part (in the wavefront-wide network,
     // and in the wavefront's sum of its face counts); lanes outside the
@@ -418,47 +417,50 @@ __global__ void __launch_bounds__(256) k_ext_i(Ext e, const double *__restrict__
 }
 
 template <typename R, int SCHEME, int SENS = 0>
-static void launch_ext_t(hipStream_t s, const Ext &e, const Fields &f, double gamma, SensorArgs sa = {})
+static void launch_ext_t(hipStream_t s, const Ext &e, const Fields &f, double gamma, int run, SensorArgs sa = {})
 {
     const int Li = e.ie1 - e.is1 + 1, Lj = e.je1 - e.js1 + 1, Lk = e.ke1 - e.ks1 + 1;
     dim3 t(64, 4, 1);
     dim3 gi((Li + ExtI<SCHEME>::NPW - 1) / ExtI<SCHEME>::NPW, (Lj + 3) / 4, Lk);
     hipLaunchKernelGGL((k_ext_i<R, SCHEME, SENS>), gi, t, 0, s, e, f.q, f.dxidx, f.inv_j, f.rhsi, gamma, sa);
-    dim3 gj((Li + 63) / 64, (Lk + 3) / 4, (Lj + kExtRun - 1) / kExtRun);
-    hipLaunchKernelGGL((k_ext_jk<R, 1, SCHEME, SENS>), gj, t, 0, s, e, f.q, f.dxidx, f.inv_j, f.rhsi, gamma, sa);
-    dim3 gk((Li + 63) / 64, (Lj + 3) / 4, (Lk + kExtRun - 1) / kExtRun);
-    hipLaunchKernelGGL((k_ext_jk<R, 2, SCHEME, SENS>), gk, t, 0, s, e, f.q, f.dxidx, f.inv_j, f.rhsi, gamma, sa);
+    dim3 gj((Li + 63) / 64, (Lk + 3) / 4, (Lj + run - 1) / run);
+    hipLaunchKernelGGL((k_ext_jk<R, 1, SCHEME, SENS>), gj, t, 0, s, e, f.q, f.dxidx, f.inv_j, f.rhsi, gamma, sa,
+                       run);
+    dim3 gk((Li + 63) / 64, (Lj + 3) / 4, (Lk + run - 1) / run);
+    hipLaunchKernelGGL((k_ext_jk<R, 2, SCHEME, SENS>), gk, t, 0, s, e, f.q, f.dxidx, f.inv_j, f.rhsi, gamma, sa,
+                       run);
 }
 
 int launch_inviscid_wcns_sensor(hipStream_t s, const Ext &e, const Fields &f, const Consts &c, int precision,
-                                const SensorArgs &sa)
+                                int run, bool clear, const SensorArgs &sa)
 {
-    int rc = launch_fill(s, f.rhsi, 5 * e.n, 0.0);
+    int rc = clear ? launch_fill(s, f.rhsi, 5 * e.n, 0.0) : 0;
     if (rc) return rc;
     if (e.ie1 < e.is1 || e.je1 < e.js1 || e.ke1 < e.ks1) return 0;
     if (sa.replay) {
-        if (precision == 1) launch_ext_t<float, 2, 2>(s, e, f, c.gamma, sa);
-        else launch_ext_t<double, 2, 2>(s, e, f, c.gamma, sa);
+        if (precision == 1) launch_ext_t<float, 2, 2>(s, e, f, c.gamma, run, sa);
+        else launch_ext_t<double, 2, 2>(s, e, f, c.gamma, run, sa);
     } else {
-        if (precision == 1) launch_ext_t<float, 2, 1>(s, e, f, c.gamma, sa);
-        else launch_ext_t<double, 2, 1>(s, e, f, c.gamma, sa);
+        if (precision == 1) launch_ext_t<float, 2, 1>(s, e, f, c.gamma, run, sa);
+        else launch_ext_t<double, 2, 1>(s, e, f, c.gamma, run, sa);
     }
     ACFD_CHECK_LAUNCH();
     return 0;
 }
 
-int launch_inviscid_ext(hipStream_t s, const Ext &e, const Fields &f, const Consts &c, int precision, int scheme)
+int launch_inviscid_ext(hipStream_t s, const Ext &e, const Fields &f, const Consts &c, int precision, int scheme,
+                        int run, bool clear)
 {
     // rhsi is zero outside the computed range
-    int rc = launch_fill(s, f.rhsi, 5 * e.n, 0.0);
+    int rc = clear ? launch_fill(s, f.rhsi, 5 * e.n, 0.0) : 0;
     if (rc) return rc;
     if (e.ie1 < e.is1 || e.je1 < e.js1 || e.ke1 < e.ks1) return 0;
     if (scheme == 1) {
-        if (precision == 1) launch_ext_t<float, 1>(s, e, f, c.gamma);
-        else launch_ext_t<double, 1>(s, e, f, c.gamma);
+        if (precision == 1) launch_ext_t<float, 1>(s, e, f, c.gamma, run);
+        else launch_ext_t<double, 1>(s, e, f, c.gamma, run);
     } else {
-        if (precision == 1) launch_ext_t<float, 2>(s, e, f, c.gamma);
-        else launch_ext_t<double, 2>(s, e, f, c.gamma);
+        if (precision == 1) launch_ext_t<float, 2>(s, e, f, c.gamma, run);
+        else launch_ext_t<double, 2>(s, e, f, c.gamma, run);
     }
     ACFD_CHECK_LAUNCH();
     return 0;

@@ -8,7 +8,10 @@ namespace acfd {
 // k_flux.hip
 int launch_getpri(hipStream_t s, const Ext &e, const Fields &f, const Consts &c, unsigned int *nneg);
 int launch_fill(hipStream_t s, double *p, long n, double v);
-int launch_inviscid(hipStream_t s, const Ext &e, const Fields &f, const Consts &c, int precision);
+// run: nodes a thread of the j / k kernels marches over (inviscid_run);
+// clear: rhsi may not be zero outside the computed range
+int launch_inviscid(hipStream_t s, const Ext &e, const Fields &f, const Consts &c, int precision, int run, bool clear);
+int inviscid_run(long nodes, int scheme, int precision);
 int launch_viscous(hipStream_t s, const Ext &e, const Fields &f, const Consts &c, int precision,
                    int store_aux);
 // unsteady: the local cfl of the block's last node goes to *cfl and, when
@@ -19,7 +22,8 @@ int launch_reset_stats(hipStream_t s, unsigned long long *stats);
 
 // k_flux5.hip: schemes and time integration with no reference counterpart
 // (scheme 1 Steger-Warming + WENO5, 2 WCNS; Shu-Osher RK3)
-int launch_inviscid_ext(hipStream_t s, const Ext &e, const Fields &f, const Consts &c, int precision, int scheme);
+int launch_inviscid_ext(hipStream_t s, const Ext &e, const Fields &f, const Consts &c, int precision, int scheme,
+                        int run, bool clear);
 int launch_rk3_stage(hipStream_t s, const Ext &e, const Fields &f, const double *qn, int stage, bool viscous);
 int launch_copy(hipStream_t s, const double *a, double *b, long n);
 
@@ -52,11 +56,11 @@ size_t sensor_net_bytes();
 long diff_partials(const Ext &e);
 int launch_diff_partial(hipStream_t s, const Ext &e, const double *a, const double *b, double *part);
 int launch_inviscid_wcns_sensor(hipStream_t s, const Ext &e, const Fields &f, const Consts &c, int precision,
-                                const SensorArgs &sa);
+                                int run, bool clear, const SensorArgs &sa);
 
 // batched launches over every block (block table, per-kind grids)
 dim3 grid_1d(long n);                    // 256-thread workgroups over n items
-dim3 inviscid_grid(const Ext &e, int axis);
+dim3 inviscid_grid(const Ext &e, int axis, int run);
 dim3 viscous_grid(const Ext &e);
 dim3 lu_prep_grid(const Ext &e);
 int launch_getpri_batch(hipStream_t s, const BlockRec *blks, const BatchGrid &bg, double *arena, const Consts &c,
@@ -66,7 +70,7 @@ int launch_getpri_batch(hipStream_t s, const BlockRec *blks, const BatchGrid &bg
 // k directions; viscous: 1 node fluxes, 2 their difference), for per-kernel
 // timing
 int launch_inviscid_batch(hipStream_t s, const BlockRec *blks, const BatchGrid *bg, double *arena,
-                          const Consts &c, int precision, int part = -1);
+                          const Consts &c, int precision, int run, int part = -1);
 int launch_viscous_batch(hipStream_t s, const BlockRec *blks, const BatchGrid &bg, double *arena, const Consts &c,
                          int precision, int store_aux, int part = -1);
 // the viscous stage with the steady find_dt folded into its node pass
