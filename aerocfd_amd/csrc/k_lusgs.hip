@@ -66,20 +66,19 @@ namespace acfd {
 //         a1 theta + U (dp + v5) ]
 // with u = mom/rho, U = m.u, theta = m.v_mom - U v1,
 // dp = (gamma-1)(|u|^2/2 v1 - u.v_mom + v5), a1 = gamma E/rho - (gamma-1)|u|^2/2.
-// The factor s = 1/2 inv_j is taken into the metric row, U and r once per
-// node and direction, so that what depends on v -- all of a sweep's serial
-// chain -- is as short as it can be.
+// What depends on v is all of a sweep's serial chain; the rest of a node is
+// formed once, ahead of it: LuState, LuRow and LuDiag.
 
 // the part of a node's products that no direction changes
 struct LuState {
-    double u, v, w, q2h, a1;  // velocity, |u|^2/2, a1
+    double u, v, w, q2h, a1, s;  // velocity, |u|^2/2, a1, inv_j/2
 };
-// one direction: the metric row, U and +-r, each times s
+// one direction: the metric row, U and +-r
 struct LuRow {
     double x, y, z, U, r;
 };
 
-__device__ inline LuState lu_state(const double *qv, double ri, double gamma)
+__device__ inline LuState lu_state(const double *qv, double ri, double ij, double gamma)
 {
     LuState t;
     t.u = qv[1] * ri;
@@ -87,19 +86,14 @@ __device__ inline LuState lu_state(const double *qv, double ri, double gamma)
     t.w = qv[3] * ri;
     t.q2h = 0.5 * fma(t.w, t.w, fma(t.v, t.v, t.u * t.u));
     t.a1 = fma(gamma * qv[4], ri, -(gamma - 1.0) * t.q2h);
+    t.s = 0.5 * ij;
     return t;
 }
 
 template <int SGN>
-__device__ inline LuRow lu_row(const LuState &t, double mx, double my, double mz, double s, double rr)
+__device__ inline LuRow lu_row(const LuState &t, double mx, double my, double mz, double rr)
 {
-    LuRow m;
-    m.x = s * mx;
-    m.y = s * my;
-    m.z = s * mz;
-    m.U = fma(m.z, t.w, fma(m.y, t.v, m.x * t.u));
-    m.r = s * (SGN > 0 ? rr : -rr);
-    return m;
+    return {mx, my, mz, fma(mz, t.w, fma(my, t.v, mx * t.u)), SGN > 0 ? rr : -rr};
 }
 
 // dp of a solution vector v, shared by the three directions
@@ -113,12 +107,11 @@ __device__ inline void lu_product(const LuState &t, const LuRow &m, double dp, c
 {
     const double mvm = fma(m.z, v[3], fma(m.y, v[2], m.x * v[1]));
     const double theta = fma(-m.U, v[0], mvm);
-    const double w = m.U + m.r;
-    out[0] = fma(m.r, v[0], mvm);
-    out[1] = fma(w, v[1], fma(m.x, dp, t.u * theta));
-    out[2] = fma(w, v[2], fma(m.y, dp, t.v * theta));
-    out[3] = fma(w, v[3], fma(m.z, dp, t.w * theta));
-    out[4] = fma(w, v[4], fma(m.U, dp, t.a1 * theta));
+    out[0] = t.s * fma(m.r, v[0], mvm);
+    out[1] = t.s * fma(m.r, v[1], fma(m.x, dp, fma(t.u, theta, m.U * v[1])));
+    out[2] = t.s * fma(m.r, v[2], fma(m.y, dp, fma(t.v, theta, m.U * v[2])));
+    out[3] = t.s * fma(m.r, v[3], fma(m.z, dp, fma(t.w, theta, m.U * v[3])));
+    out[4] = t.s * fma(m.r, v[4], fma(m.U, dp + v[4], t.a1 * theta));
 }
 
 // the product with the operands of node n read from the SoA fields
@@ -128,31 +121,41 @@ __device__ inline void jac_mv(const double *__restrict__ q, const double *__rest
                               int c0, double gamma, const double *v, double *out)
 {
     const double qv[5] = {q[n], q[N + n], q[2 * N + n], q[3 * N + n], q[4 * N + n]};
-    const LuState t = lu_state(qv, 1.0 / qv[0], gamma);
-    const LuRow m = lu_row<SGN>(t, dxidx[c0 * N + n], dxidx[(c0 + 1) * N + n], dxidx[(c0 + 2) * N + n],
-                                0.5 * inv_j[n], rr[n]);
+    const LuState t = lu_state(qv, 1.0 / qv[0], inv_j[n], gamma);
+    const LuRow m = lu_row<SGN>(t, dxidx[c0 * N + n], dxidx[(c0 + 1) * N + n], dxidx[(c0 + 2) * N + n], rr[n]);
     lu_product(t, m, lu_dp(t, gamma, v), v, out);
 }
 
-// 1 / (diag inv_j): both sweeps divide by the two; one reciprocal per node,
-// formed before its neighbours' values arrive (the ten divisions of the
-// five components were on the sweeps' serial chain)
-__device__ inline double lu_rdiag(double dg, double ij) { return 1.0 / (dg * ij); }
+// A divisor known before its dividends: x / d from y = 1/d (rounded), the
+// quotient estimate x y and one correction by its remainder, in three
+// operations in place of a division's dozen.  The correction step rounds
+// the quotient as the division does (Markstein, IBM J. Res. Dev. 34, 1990),
+// so the sweeps' results are those of the reference's two divisions.  An
+// infinite d (dt = 0) has y = 0 and d held as 0: the quotient is 0.
+struct LuDivisor {
+    double d, y;
+};
+__device__ inline LuDivisor lu_divisor(double d) { return {isinf(d) ? 0.0 : d, 1.0 / d}; }
+__device__ inline double lu_over(double x, const LuDivisor &b)
+{
+    const double q = x * b.y;
+    return fma(fma(-q, b.d, x), b.y, q);
+}
 
 // forward node (:345-365): dq* = (rhs + A+ dq*_i-1 + B+ dq*_j-1 + C+ dq*_k-1)/diag/inv_j
 __device__ inline void lu_fwd_combine(const double *rhs, const double *ta, const double *tb, const double *tc,
-                                      double rd, double *res)
+                                      const LuDivisor &dg, const LuDivisor &ij, double *res)
 {
 #pragma unroll
-    for (int x = 0; x < 5; x++) res[x] = (rhs[x] + (ta[x] + tb[x] + tc[x])) * rd;
+    for (int x = 0; x < 5; x++) res[x] = lu_over(lu_over(rhs[x] + (ta[x] + tb[x] + tc[x]), dg), ij);
 }
 
 // backward node (:521-542): dq = dq* - (A- dq_i+1 + B- dq_j+1 + C- dq_k+1)/inv_j/diag
 __device__ inline void lu_bwd_combine(const double *dqs, const double *ta, const double *tb, const double *tc,
-                                      double rd, double *res)
+                                      const LuDivisor &dg, const LuDivisor &ij, double *res)
 {
 #pragma unroll
-    for (int x = 0; x < 5; x++) res[x] = fma(-(ta[x] + tb[x] + tc[x]), rd, dqs[x]);
+    for (int x = 0; x < 5; x++) res[x] = dqs[x] - lu_over(lu_over(ta[x] + tb[x] + tc[x], ij), dg);
 }
 
 struct LuArgs {
@@ -172,7 +175,7 @@ __device__ inline void lu_forward(const LuArgs &a, long n, const double *vi, con
     jac_mv<1>(a.q, a.dxidx, a.inv_j, a.rr + 2 * N, N, n - sk, 6, a.gamma, vk, tc);
 #pragma unroll
     for (int x = 0; x < 5; x++) rhs[x] = a.rhs[x * N + n];
-    lu_fwd_combine(rhs, ta, tb, tc, lu_rdiag(a.diag[n], a.inv_j[n]), res);
+    lu_fwd_combine(rhs, ta, tb, tc, lu_divisor(a.diag[n]), lu_divisor(a.inv_j[n]), res);
 }
 
 __device__ inline void lu_backward(const LuArgs &a, long n, const double *vi, const double *vj,
@@ -185,7 +188,7 @@ __device__ inline void lu_backward(const LuArgs &a, long n, const double *vi, co
     jac_mv<-1>(a.q, a.dxidx, a.inv_j, a.rr + 2 * N, N, n + sk, 6, a.gamma, vk, tc);
 #pragma unroll
     for (int x = 0; x < 5; x++) dqs[x] = a.dqs[x * N + n];
-    lu_bwd_combine(dqs, ta, tb, tc, lu_rdiag(a.diag[n], a.inv_j[n]), res);
+    lu_bwd_combine(dqs, ta, tb, tc, lu_divisor(a.diag[n]), lu_divisor(a.inv_j[n]), res);
 }
 
 // rhs = rhsi + rhsv on the computed range (:72-78).  For the hyperplane
@@ -607,13 +610,13 @@ constexpr int kPipePrep = 2;    // preparing waves
 constexpr int kPipeThreads = 64 * (1 + kPipePrep + 1);
 
 // a prepared step, pairs of doubles per lane: rhs 0-4 (dq* in the backward
-// sweep), 1/(diag inv_j), then forward u, v, w, |u|^2/2, a1, the time term,
-// r of the i row, unused; backward q 0-4, 1/rho, |u|^2/2, a1, r of the i
-// row, the time term; then x, y, z, U of the three rows and r of the j and
-// the k row
+// sweep), the divisors diag and inv_j (d, y, y, d), |u|^2/2, a1, the time
+// term, then forward u, v, w, r of the i row; backward q 0-4, 1/rho, r of the
+// i row, unused; then x, y, z, U of the three rows and r of the j and the k
+// row
 template <int DIR>
 struct PipeLds {
-    static constexpr int kRow0 = DIR > 0 ? 7 : 8;
+    static constexpr int kRow0 = DIR > 0 ? 8 : 10;
     static constexpr int kPairs = kRow0 + 7;
     double2 op[kPipeRing][kPairs][64];
     double x[kPipeXRing][2][5][kTile];
@@ -700,30 +703,30 @@ __device__ inline void pipe_prepare(const SlGeom &g, int tile, int w, const doub
             for (int x = 0; x < 5; x++) op[kSlOut + x] = 0.0;
         }
         double rad[3];
-        const double ri = 1.0 / op[kSlQ], sc = 0.5 * op[9];
-        const LuState t = lu_state(op + kSlQ, ri, gamma);
-        const double dg = lu_node_radii(op, rad);
-        const double rd = on ? lu_rdiag(dg, op[9]) : 0.0;
+        const double ri = 1.0 / op[kSlQ];
+        const LuState t = lu_state(op + kSlQ, ri, op[9], gamma);
+        LuDivisor dg = lu_divisor(lu_node_radii(op, rad)), ij = lu_divisor(op[9]);
+        if (!on) dg.d = dg.y = ij.d = ij.y = 0.0;
         LuRow m[3];
 #pragma unroll
-        for (int d = 0; d < 3; d++) m[d] = lu_row<DIR>(t, op[3 * d], op[3 * d + 1], op[3 * d + 2], sc, rad[d]);
+        for (int d = 0; d < 3; d++) m[d] = lu_row<DIR>(t, op[3 * d], op[3 * d + 1], op[3 * d + 2], rad[d]);
         lds_wait([&] { return lds_get(&L.done); }, s - kPipeRing + 1, &L.stop, err);
         double2 *o = &L.op[s % kPipeRing][0][l];
         const double *rhs = op + kSlOut;
         o[0] = make_double2(rhs[0], rhs[1]);
         o[64] = make_double2(rhs[2], rhs[3]);
-        o[2 * 64] = make_double2(rhs[4], rd);
+        o[2 * 64] = make_double2(rhs[4], dg.d);
+        o[3 * 64] = make_double2(dg.y, ij.y);
+        o[4 * 64] = make_double2(ij.d, t.q2h);
+        o[5 * 64] = make_double2(t.a1, op[kSlT]);
         if (DIR > 0) {
-            o[3 * 64] = make_double2(t.u, t.v);
-            o[4 * 64] = make_double2(t.w, t.q2h);
-            o[5 * 64] = make_double2(t.a1, op[kSlT]);
-            o[6 * 64] = make_double2(m[0].r, 0.0);
+            o[6 * 64] = make_double2(t.u, t.v);
+            o[7 * 64] = make_double2(t.w, m[0].r);
         } else {
-            o[3 * 64] = make_double2(op[kSlQ], op[kSlQ + 1]);
-            o[4 * 64] = make_double2(op[kSlQ + 2], op[kSlQ + 3]);
-            o[5 * 64] = make_double2(op[kSlQ + 4], ri);
-            o[6 * 64] = make_double2(t.q2h, t.a1);
-            o[7 * 64] = make_double2(m[0].r, op[kSlT]);
+            o[6 * 64] = make_double2(op[kSlQ], op[kSlQ + 1]);
+            o[7 * 64] = make_double2(op[kSlQ + 2], op[kSlQ + 3]);
+            o[8 * 64] = make_double2(op[kSlQ + 4], ri);
+            o[9 * 64] = make_double2(m[0].r, 0.0);
         }
         double2 *r = o + PipeLds<DIR>::kRow0 * 64;
 #pragma unroll
@@ -871,24 +874,24 @@ __device__ inline void pipe_solve(const SlGeom &g, int tile, double *__restrict_
         const double rhs[5] = {E[0].x, E[0].y, E[1].x, E[1].y, E[2].x};
         double res[5], qv[5], pb[5], pc[5];
         LuState t;
-        double tterm, r0;
+        const LuDivisor dg{E[2].y, E[3].x}, ij{E[4].x, E[3].y};
+        const double tterm = E[5].y;
+        double r0;
 #pragma unroll
         for (int x = 0; x < 5; x++) {
             tb[x] = sj == 0 ? fj[x] : tb[x];
             tc[x] = sk == 0 ? fk[x] : tc[x];
         }
         if (DIR > 0) {
-            t = {E[3].x, E[3].y, E[4].x, E[4].y, E[5].x};
-            tterm = E[5].y;
-            r0 = E[6].x;
-            lu_fwd_combine(rhs, ta, tb, tc, E[2].y, res);
+            t = {E[6].x, E[6].y, E[7].x, E[4].y, E[5].x, 0.5 * ij.d};
+            r0 = E[7].y;
+            lu_fwd_combine(rhs, ta, tb, tc, dg, ij, res);
         } else {
-            qv[0] = E[3].x; qv[1] = E[3].y; qv[2] = E[4].x; qv[3] = E[4].y; qv[4] = E[5].x;
-            const double ri = E[5].y;
-            t = {qv[1] * ri, qv[2] * ri, qv[3] * ri, E[6].x, E[6].y};
-            r0 = E[7 % kRow0].x;
-            tterm = E[7 % kRow0].y;
-            lu_bwd_combine(rhs, ta, tb, tc, E[2].y, res);
+            qv[0] = E[6].x; qv[1] = E[6].y; qv[2] = E[7].x; qv[3] = E[7].y; qv[4] = E[8 % kRow0].x;
+            const double ri = E[8 % kRow0].y;
+            t = {qv[1] * ri, qv[2] * ri, qv[3] * ri, E[4].y, E[5].x, 0.5 * ij.d};
+            r0 = E[9 % kRow0].x;
+            lu_bwd_combine(rhs, ta, tb, tc, dg, ij, res);
         }
         const double dp = lu_dp(t, gamma, res);
         lu_product(t, {R[4].x, R[4].y, R[5].x, R[5].y, R[6].y}, dp, res, pc);
