@@ -404,6 +404,17 @@ __device__ inline bool sl_line_ok(const SlGeom &g, int tile, int line)
     return (tile % g.nbj) * kTile + line % kTile < g.Lj && (tile / g.nbj) * kTile + line / kTile < g.Lk;
 }
 
+// the steps [t0, t1) of part `part` of `parts` of a tile's chunks of ct steps
+struct SlChunks {
+    int t0, t1;
+    __device__ SlChunks(int nsteps, int ct, int part, int parts)
+    {
+        const int n = (nsteps + ct - 1) / ct;
+        t0 = n * part / parts * ct;
+        t1 = min(n * (part + 1) / parts * ct, nsteps);
+    }
+};
+
 // csnd: the sound speed (component 7 of pri_v), tterm: the time term
 __device__ inline const double *gather_src(int f, long N, const double *q, const double *dxidx,
                                            const double *inv_j, const double *csnd, const double *tterm,
@@ -419,8 +430,8 @@ __device__ inline const double *gather_src(int f, long N, const double *q, const
 __device__ inline void sl_gather_tile(const Ext &e, const SlGeom &g, int tile, const double *__restrict__ q,
                                       const double *__restrict__ dxidx, const double *__restrict__ inv_j,
                                       const double *__restrict__ csnd, const double *__restrict__ tterm,
-                                      const double *__restrict__ rhs, double *__restrict__ sl, int fp0,
-                                      double *buf /* [2][CT][TT] LDS, swizzled */)
+                                      const double *__restrict__ rhs, double *__restrict__ sl, int fp,
+                                      int part, int parts, double *buf /* [2][CT][TT] LDS, swizzled */)
 {
     constexpr int CT = kSlCt, TT = kLanes, lstep = TT / CT;
     const int x = threadIdx.x;
@@ -429,41 +440,40 @@ __device__ inline void sl_gather_tile(const Ext &e, const SlGeom &g, int tile, c
     const bool me_ok = sl_line_ok(g, tile, x);
     const long N = e.n;
     double2 *sl2 = reinterpret_cast<double2 *>(sl);
-    for (int fp = fp0; fp < kSlF / 2; fp++) {
-        for (int t0 = 0; t0 < g.nsteps; t0 += CT) {
-            // natural-side node offsets of this thread's CT elements (-1: none)
-            int nat[CT];  // node offsets fit 32 bits (blocks below 2^31 nodes)
+    const SlChunks ch(g.nsteps, CT, part, parts);
+    for (int t0 = ch.t0; t0 < ch.t1; t0 += CT) {
+        // natural-side node offsets of this thread's CT elements (-1: none)
+        int nat[CT];  // node offsets fit 32 bits (blocks below 2^31 nodes)
+#pragma unroll
+        for (int m = 0; m < CT; m++) {
+            const int line = m * lstep + x / CT;
+            const int li = t0 + ii_n - (line % kTile) - (line / kTile);
+            nat[m] = (t0 + ii_n < g.nsteps && li >= 0 && li < g.Li && sl_line_ok(g, tile, line))
+                         ? (int)sl_nat(e, g, tile, line, li) : -1;
+        }
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const double *src = gather_src(2 * fp + h, N, q, dxidx, inv_j, csnd, tterm, rhs);
+            double v[CT];
+#pragma unroll
+            for (int m = 0; m < CT; m++) v[m] = nat[m] >= 0 ? src[nat[m]] : 0.0;
 #pragma unroll
             for (int m = 0; m < CT; m++) {
                 const int line = m * lstep + x / CT;
-                const int li = t0 + ii_n - (line % kTile) - (line / kTile);
-                nat[m] = (t0 + ii_n < g.nsteps && li >= 0 && li < g.Li && sl_line_ok(g, tile, line))
-                             ? (int)sl_nat(e, g, tile, line, li) : -1;
+                buf[(h * CT + ii_n) * TT + (line ^ ii_n)] = v[m];
             }
-#pragma unroll
-            for (int h = 0; h < 2; h++) {
-                const double *src = gather_src(2 * fp + h, N, q, dxidx, inv_j, csnd, tterm, rhs);
-                double v[CT];
-#pragma unroll
-                for (int m = 0; m < CT; m++) v[m] = nat[m] >= 0 ? src[nat[m]] : 0.0;
-#pragma unroll
-                for (int m = 0; m < CT; m++) {
-                    const int line = m * lstep + x / CT;
-                    buf[(h * CT + ii_n) * TT + (line ^ ii_n)] = v[m];
-                }
-            }
-            __syncthreads();
-            if (me_ok) {
-#pragma unroll
-                for (int ii = 0; ii < CT; ii++) {
-                    const int t = t0 + ii, li = t - tj - tk;
-                    if (t < g.nsteps && li >= 0 && li < g.Li)
-                        sl2[g.slot(tile, t, 2 * fp, x) >> 1] =
-                            make_double2(buf[ii * TT + (x ^ ii)], buf[(CT + ii) * TT + (x ^ ii)]);
-                }
-            }
-            __syncthreads();
         }
+        __syncthreads();
+        if (me_ok) {
+#pragma unroll
+            for (int ii = 0; ii < CT; ii++) {
+                const int t = t0 + ii, li = t - tj - tk;
+                if (t < g.nsteps && li >= 0 && li < g.Li)
+                    sl2[g.slot(tile, t, 2 * fp, x) >> 1] =
+                        make_double2(buf[ii * TT + (x ^ ii)], buf[(CT + ii) * TT + (x ^ ii)]);
+            }
+        }
+        __syncthreads();
     }
 }
 
@@ -472,17 +482,20 @@ __global__ void __launch_bounds__(kLanes) k_sl_gather(Ext e, SlGeom g, const dou
                                                   const double *__restrict__ inv_j,
                                                   const double *__restrict__ csnd,
                                                   const double *__restrict__ tterm,
-                                                  const double *__restrict__ rhs, double *__restrict__ sl, int fp0)
+                                                  const double *__restrict__ rhs, double *__restrict__ sl, int fp0,
+                                                  int parts)
 {
     __shared__ double buf[2 * kSlCt * kLanes];
-    sl_gather_tile(e, g, (int)blockIdx.x, q, dxidx, inv_j, csnd, tterm, rhs, sl, fp0, buf);
+    sl_gather_tile(e, g, (int)blockIdx.x, q, dxidx, inv_j, csnd, tterm, rhs, sl, fp0 + (int)blockIdx.y / parts,
+                   (int)blockIdx.y % parts, parts, buf);
 }
 
 // q += dq (:568-574): the backward sweep left q + dq in the result slots of
 // the sweep layout; this pass moves it to q in the natural layout, same walk
 // as the gather, one field pair at a time.
 __device__ inline void sl_add_tile(const Ext &e, const SlGeom &g, int tile, const double *__restrict__ sl,
-                                   double *__restrict__ q, double *buf /* [2][CT][TT] LDS, swizzled */)
+                                   double *__restrict__ q, int fp, int part, int parts,
+                                   double *buf /* [2][CT][TT] LDS, swizzled */)
 {
     constexpr int CT = kSlCt, TT = kLanes, lstep = TT / CT;
     const int x = threadIdx.x;
@@ -490,64 +503,80 @@ __device__ inline void sl_add_tile(const Ext &e, const SlGeom &g, int tile, cons
     const int tj = x % kTile, tk = x / kTile;
     const bool me_ok = sl_line_ok(g, tile, x);
     const long N = e.n;
-    // the results are fields 19-23: the upper half of pair 9 (whose lower
-    // half, diag, is not written) and pairs 10 and 11, read as whole
-    // 16-byte pairs
-    for (int fp = kSlOut / 2; fp < kSlF / 2; fp++) {
-        for (int t0 = 0; t0 < g.nsteps; t0 += CT) {
-            int nat[CT];  // node offsets fit 32 bits (blocks below 2^31 nodes)
+    const SlChunks ch(g.nsteps, CT, part, parts);
+    for (int t0 = ch.t0; t0 < ch.t1; t0 += CT) {
+        int nat[CT];  // node offsets fit 32 bits (blocks below 2^31 nodes)
 #pragma unroll
-            for (int m = 0; m < CT; m++) {
-                const int line = m * lstep + x / CT;
-                const int li = t0 + ii_n - (line % kTile) - (line / kTile);
-                nat[m] = (t0 + ii_n < g.nsteps && li >= 0 && li < g.Li && sl_line_ok(g, tile, line))
-                             ? (int)sl_nat(e, g, tile, line, li) : -1;
-            }
-            const int v0 = 2 * fp - kSlOut;  // component of the pair's lower field (-1: diag)
-            if (me_ok) {
-                const double2 *sl2 = reinterpret_cast<const double2 *>(sl);
-                double2 d[CT];
-#pragma unroll
-                for (int ii = 0; ii < CT; ii++) {
-                    const int t = t0 + ii, li = t - tj - tk;
-                    d[ii] = (t < g.nsteps && li >= 0 && li < g.Li) ? sl2[g.slot(tile, t, 2 * fp, x) >> 1]
-                                                                   : make_double2(0.0, 0.0);
-                }
-#pragma unroll
-                for (int ii = 0; ii < CT; ii++) {
-                    buf[ii * TT + (x ^ ii)] = d[ii].x;
-                    buf[(CT + ii) * TT + (x ^ ii)] = d[ii].y;
-                }
-            }
-            __syncthreads();
-#pragma unroll
-            for (int m = 0; m < CT; m++) {
-                const int line = m * lstep + x / CT;
-                if (nat[m] >= 0) {
-                    if (v0 >= 0) q[v0 * N + nat[m]] = buf[ii_n * TT + (line ^ ii_n)];
-                    q[(v0 + 1) * N + nat[m]] = buf[(CT + ii_n) * TT + (line ^ ii_n)];
-                }
-            }
-            __syncthreads();
+        for (int m = 0; m < CT; m++) {
+            const int line = m * lstep + x / CT;
+            const int li = t0 + ii_n - (line % kTile) - (line / kTile);
+            nat[m] = (t0 + ii_n < g.nsteps && li >= 0 && li < g.Li && sl_line_ok(g, tile, line))
+                         ? (int)sl_nat(e, g, tile, line, li) : -1;
         }
+        const int v0 = 2 * fp - kSlOut;  // component of the pair's lower field (-1: diag)
+        if (me_ok) {
+            const double2 *sl2 = reinterpret_cast<const double2 *>(sl);
+            double2 d[CT];
+#pragma unroll
+            for (int ii = 0; ii < CT; ii++) {
+                const int t = t0 + ii, li = t - tj - tk;
+                d[ii] = (t < g.nsteps && li >= 0 && li < g.Li) ? sl2[g.slot(tile, t, 2 * fp, x) >> 1]
+                                                               : make_double2(0.0, 0.0);
+            }
+#pragma unroll
+            for (int ii = 0; ii < CT; ii++) {
+                buf[ii * TT + (x ^ ii)] = d[ii].x;
+                buf[(CT + ii) * TT + (x ^ ii)] = d[ii].y;
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int m = 0; m < CT; m++) {
+            const int line = m * lstep + x / CT;
+            if (nat[m] >= 0) {
+                if (v0 >= 0) q[v0 * N + nat[m]] = buf[ii_n * TT + (line ^ ii_n)];
+                q[(v0 + 1) * N + nat[m]] = buf[(CT + ii_n) * TT + (line ^ ii_n)];
+            }
+        }
+        __syncthreads();
     }
 }
 
+// the results are fields 17-21: the upper half of pair 8 (whose lower half
+// is the time term) and pairs 9 and 10, read as whole 16-byte pairs
 __global__ void __launch_bounds__(kLanes) k_sl_add(Ext e, SlGeom g, const double *__restrict__ sl,
-                                               double *__restrict__ q)
+                                               double *__restrict__ q, int parts)
 {
     __shared__ double buf[2 * kSlCt * kLanes];
-    sl_add_tile(e, g, (int)blockIdx.x, sl, q, buf);
+    sl_add_tile(e, g, (int)blockIdx.x, sl, q, kSlOut / 2 + (int)blockIdx.y / parts, (int)blockIdx.y % parts, parts, buf);
+}
+
+// Parts of a layout pass: a workgroup takes one field pair of one tile, and
+// where the tiles are few, one of `parts` runs of its chunks, so that about
+// kSlWgs workgroups come together (one workgroup per tile, all pairs in
+// turn, left most of the device idle).  More parts split more cache lines
+// between workgroups, so a launch that has enough tiles takes one.  Gather
+// before and after: 33^3 75 -> 12 us, 129^3 231 -> 114, 12 blocks of 3.2 M
+// nodes 233 -> 158, 98 M nodes 4.81 -> 4.52 ms; add 129^3 114 -> 55 us; SA
+// gather and return of the 12 blocks 111 -> 94 and 128 -> 60 us.
+constexpr int kSlWgs = 2048;
+static int sl_parts(int ntiles, int fields, int nsteps, int ct)
+{
+    const long wgs = (long)ntiles * fields;
+    return (int)std::max(1L, std::min((long)(nsteps + ct - 1) / ct, (kSlWgs + wgs - 1) / wgs));
 }
 
 static void launch_layout(hipStream_t s, int which, const Ext &e, const SlGeom &g, const Fields &f, const LuWs &ws,
                           int fp0 = 0)
 {
+    const int pairs = which == 0 ? kSlF / 2 - fp0 : kSlF / 2 - kSlOut / 2;
+    const int parts = sl_parts(g.ntiles, pairs, g.nsteps, kSlCt);
+    const dim3 gr((unsigned)g.ntiles, (unsigned)(pairs * parts));
     if (which == 0)
-        hipLaunchKernelGGL(k_sl_gather, dim3((unsigned)g.ntiles), dim3(kLanes), 0, s, e, g, f.q, f.dxidx, f.inv_j,
-                           f.pri + 6 * e.n, f.w_diag, f.rhs, ws.sl, fp0);
+        hipLaunchKernelGGL(k_sl_gather, gr, dim3(kLanes), 0, s, e, g, f.q, f.dxidx, f.inv_j, f.pri + 6 * e.n, f.w_diag,
+                           f.rhs, ws.sl, fp0, parts);
     else
-        hipLaunchKernelGGL(k_sl_add, dim3((unsigned)g.ntiles), dim3(kLanes), 0, s, e, g, ws.sl, f.q);
+        hipLaunchKernelGGL(k_sl_add, gr, dim3(kLanes), 0, s, e, g, ws.sl, f.q, parts);
 }
 
 // Fill exchange slots with the sentinel.
@@ -593,11 +622,11 @@ __device__ inline double lu_node_radii(const double *op, double *r)
 // for ring space (wave 0), wave 0 for operands and for slots, the slot
 // wave for the neighbouring tiles with a bounded poll; running out sets
 // *err and `stop`, at which every wait of the workgroup ends.
-// What bounds it: wave 0's instruction issue (about 215 instructions a step,
-// of which 80 are the FP64 arithmetic, at one per four cycles or more:
-// 0.57-0.65 us a step) and 2.6 us a hop; on large batches the HBM traffic.
-// Forward sweep, before (one wavefront a tile) and after: 33^3 184 -> 80 us,
-// 129^3 748 -> 330, 193^3 1218 -> 750, 12 blocks of 3.2 M nodes in all
+// What bounds it: wave 0's instruction issue (about 260 instructions a step,
+// of which 127 are the FP64 arithmetic, at one per four cycles or more:
+// about 0.65 us a step) and 2.6 us a hop; on large batches the HBM traffic.
+// Forward sweep, before (one wavefront a tile) and after: 33^3 184 -> 88 us,
+// 129^3 748 -> 346, 193^3 1218 -> 740, 12 blocks of 3.2 M nodes in all
 // 507 -> 350, 40 blocks of 98 M nodes 6.19 -> 6.10 ms (4.7 TB/s).  Tiles of
 // 16 x 16, 16 x 8 and 16 x 4 lines of the one-wavefront form were slower at
 // every one of these sizes and are gone.
@@ -1029,7 +1058,7 @@ struct LuBatchEnt {
 
 __global__ void __launch_bounds__(kLanes) k_sl_gather_batch(const LuBatchEnt *__restrict__ ents,
                                                         const int *__restrict__ tile_ent, double *arena,
-                                                        double *slb, int fp0)
+                                                        double *slb, int fp0, int parts)
 {
     __shared__ double buf[2 * kSlCt * kLanes];
     const int flat = (int)blockIdx.x;
@@ -1037,19 +1066,21 @@ __global__ void __launch_bounds__(kLanes) k_sl_gather_batch(const LuBatchEnt *__
     const Ext e = b.e;
     const SlGeom g = b.g;
     sl_gather_tile(e, g, flat - b.tile0, arena + b.q, arena + b.dxidx, arena + b.inv_j, arena + b.csnd,
-                       arena + b.tterm, arena + b.rhs, slb + b.sl, fp0, buf);
+                       arena + b.tterm, arena + b.rhs, slb + b.sl, fp0 + (int)blockIdx.y / parts, (int)blockIdx.y % parts,
+                   parts, buf);
 }
 
 __global__ void __launch_bounds__(kLanes) k_sl_add_batch(const LuBatchEnt *__restrict__ ents,
                                                      const int *__restrict__ tile_ent, double *arena,
-                                                     const double *slb)
+                                                     const double *slb, int parts)
 {
     __shared__ double buf[2 * kSlCt * kLanes];
     const int flat = (int)blockIdx.x;
     const LuBatchEnt &b = ents[tile_ent[flat]];
     const Ext e = b.e;
     const SlGeom g = b.g;
-    sl_add_tile(e, g, flat - b.tile0, slb + b.sl, arena + b.q, buf);
+    sl_add_tile(e, g, flat - b.tile0, slb + b.sl, arena + b.q, kSlOut / 2 + (int)blockIdx.y / parts,
+                (int)blockIdx.y % parts, parts, buf);
 }
 
 template <int DIR>
@@ -1300,7 +1331,7 @@ __device__ inline bool sa_line_ok(const SaGeom &g, int tile, int line)
 template <bool TO_SL>
 __device__ inline void sa_layout_tile(const Ext &e, const SaGeom &g, int tile, const double *__restrict__ cu,
                                       const double *__restrict__ rhs, double *__restrict__ nut, double *__restrict__ L,
-                                      double *buf /* [CT][TT] */)
+                                      int f, int part, int parts, double *buf /* [CT][TT] */)
 {
     constexpr int CT = TO_SL ? kSlCt : kSaRetCt, TT = kLanes, lstep = TT / CT;
     const int x = threadIdx.x;
@@ -1308,7 +1339,8 @@ __device__ inline void sa_layout_tile(const Ext &e, const SaGeom &g, int tile, c
     const int tj = x % kTile, tk = x / kTile;
     const bool me_ok = sa_line_ok(g, tile, x);
     const long N = e.n;
-    for (int t0 = 0; t0 < g.nsteps; t0 += CT) {
+    const SlChunks ch(g.nsteps, CT, part, parts);
+    for (int t0 = ch.t0; t0 < ch.t1; t0 += CT) {
         int nat[CT];  // node offsets fit 32 bits (blocks below 2^31 nodes)
 #pragma unroll
         for (int m = 0; m < CT; m++) {
@@ -1318,26 +1350,24 @@ __device__ inline void sa_layout_tile(const Ext &e, const SaGeom &g, int tile, c
                          ? (int)sa_nat(e, g, tile, line, li) : -1;
         }
         if (TO_SL) {
-            for (int f = 0; f < kSaOps; f++) {
-                const double *src = f < 4 ? cu + f * N : rhs;
-                double v[CT];
+            const double *src = f < 4 ? cu + f * N : rhs;
+            double v[CT];
 #pragma unroll
-                for (int m = 0; m < CT; m++) v[m] = nat[m] >= 0 ? src[nat[m]] : 0.0;
+            for (int m = 0; m < CT; m++) v[m] = nat[m] >= 0 ? src[nat[m]] : 0.0;
 #pragma unroll
-                for (int m = 0; m < CT; m++) {
-                    const int line = m * lstep + x / CT;
-                    buf[ii_n * TT + (line ^ ii_n)] = v[m];
-                }
-                __syncthreads();
-                if (me_ok) {
-#pragma unroll
-                    for (int ii = 0; ii < CT; ii++) {
-                        const int t = t0 + ii, li = t - tj - tk;
-                        if (t < g.nsteps && li >= 0 && li < g.Li) L[sa_slot(g, tile, t, f, x)] = buf[ii * TT + (x ^ ii)];
-                    }
-                }
-                __syncthreads();
+            for (int m = 0; m < CT; m++) {
+                const int line = m * lstep + x / CT;
+                buf[ii_n * TT + (line ^ ii_n)] = v[m];
             }
+            __syncthreads();
+            if (me_ok) {
+#pragma unroll
+                for (int ii = 0; ii < CT; ii++) {
+                    const int t = t0 + ii, li = t - tj - tk;
+                    if (t < g.nsteps && li >= 0 && li < g.Li) L[sa_slot(g, tile, t, f, x)] = buf[ii * TT + (x ^ ii)];
+                }
+            }
+            __syncthreads();
         } else {
             if (me_ok) {
 #pragma unroll
@@ -1361,14 +1391,15 @@ __device__ inline void sa_layout_tile(const Ext &e, const SaGeom &g, int tile, c
 template <bool TO_SL>
 __global__ void __launch_bounds__(kLanes) k_sa_layout_batch(const SaBatchEnt *__restrict__ ents,
                                                         const int *__restrict__ tile_ent, double *arena,
-                                                        double *slbase)
+                                                        double *slbase, int parts)
 {
     __shared__ double buf[(TO_SL ? kSlCt : kSaRetCt) * kLanes];
     const int flat = (int)xcd_slab(blockIdx.x, gridDim.x);
     const SaBatchEnt &b = ents[tile_ent[flat]];
     const Ext e = b.e;
     const SaGeom g = b.g;
-    sa_layout_tile<TO_SL>(e, g, flat - b.tile0, arena + b.cu, arena + b.rhs, arena + b.nut, slbase + b.sl, buf);
+    sa_layout_tile<TO_SL>(e, g, flat - b.tile0, arena + b.cu, arena + b.rhs, arena + b.nut, slbase + b.sl,
+                          (int)blockIdx.y / parts, (int)blockIdx.y % parts, parts, buf);
 }
 
 // The scalar sweep of sa_tiles_body with its operands in the SA sweep
@@ -1497,14 +1528,13 @@ void lusgs_ws_sizes(const Ext &e, long *sl_n, long *ex_n)
 
 // Whether the backward sweep adds dq to q itself (and the add pass is
 // skipped).  Its stores then go to the natural layout, one line per lane.
-// On one block's launch that is free up to a few million computed nodes
-// (128^3: 0.644 against 0.642 ms per sweep, 0.1 ms of add pass saved) and
-// dearer on larger ones (256^3: +1.0 ms in the sweep against 0.64 ms
-// saved).  In the batched sweeps it costs more than the pass it saves
-// (flat plate, 12 blocks: +0.25 ms against 0.10 ms; 128^3 in 64 blocks:
-// +0.16 ms against 0.12 ms), so batched launches never fuse.
+// On one block's launch that is the faster form up to about a million
+// computed nodes (step of 33^3 0.256 against 0.264 ms, 65^3 0.531 / 0.537,
+// 97^3 0.892 / 0.896) and dearer on larger ones (129^3 1.576 / 1.560).  In
+// the batched sweeps it costs more than the pass it saves (12 blocks of 3.2
+// M nodes: +0.25 ms against 0.10 ms), so batched launches never fuse.
 // ACFD_LU_FUSED_ADD=0/1 forces either form.
-constexpr long kFuseAddMaxNodes = 1L << 22;
+constexpr long kFuseAddMaxNodes = 1L << 20;
 static bool fused_add(long launch_nodes, bool batched = false)
 {
     const char *v = std::getenv("ACFD_LU_FUSED_ADD");
@@ -1574,6 +1604,7 @@ int lusgs_batch_make(int nblk, const Ext *e, const Fields *f, double *arena, dou
     out->ex = ex;
     out->nent = (int)ents.size();
     out->total = (int)te.size();
+    for (const LuBatchEnt &b : ents) out->nsteps = std::max(out->nsteps, b.g.nsteps);
     if (ents.empty()) return 0;
     batch_residency(out);
     long total = 0;
@@ -1642,14 +1673,16 @@ int launch_lusgs_batch(hipStream_t s, const LuBatch &b, int phase, double gamma,
 {
     if (b.total <= 0 || phase < 1 || phase > 4) return 0;
     const LuBatchEnt *ents = (const LuBatchEnt *)b.ents;
+    const int fp0 = geo_cached ? kSlGeoPairs : 0, pairs = phase == 1 ? kSlF / 2 - fp0 : kSlF / 2 - kSlOut / 2;
+    const int parts = sl_parts(b.total, pairs, b.nsteps, kSlCt);
     if (phase == 1)
-        hipLaunchKernelGGL(k_sl_gather_batch, dim3((unsigned)b.total), dim3(kLanes), 0, s, ents, b.tile_ent, b.arena,
-                           b.sl, geo_cached ? kSlGeoPairs : 0);
+        hipLaunchKernelGGL(k_sl_gather_batch, dim3((unsigned)b.total, (unsigned)(pairs * parts)), dim3(kLanes), 0, s, ents,
+                           b.tile_ent, b.arena, b.sl, fp0, parts);
     else if (phase == 2) launch_pipe_batch<1>(s, b, gamma, err, ctr);
     else if (phase == 3) launch_pipe_batch<-1>(s, b, gamma, err, ctr);
     else if (!b.fuse_add)
-        hipLaunchKernelGGL(k_sl_add_batch, dim3((unsigned)b.total), dim3(kLanes), 0, s, ents, b.tile_ent, b.arena,
-                           (const double *)b.sl);
+        hipLaunchKernelGGL(k_sl_add_batch, dim3((unsigned)b.total, (unsigned)(pairs * parts)), dim3(kLanes), 0, s, ents,
+                           b.tile_ent, b.arena, (const double *)b.sl, parts);
     ACFD_CHECK_LAUNCH();
     return 0;
 }
@@ -1723,6 +1756,7 @@ int sa_batch_make(int nblk, const Ext *e, const Fields *f, double *arena, double
     out->sl = sl;
     out->nent = (int)ents.size();
     out->total = (int)te.size();
+    for (const SaBatchEnt &b : ents) out->nsteps = std::max(out->nsteps, b.g.nsteps);
     if (ents.empty()) return 0;
     const char *t = std::getenv("ACFD_LU_TICKETS");
     const bool tickets = t && std::atoi(t) == 1;
@@ -1744,10 +1778,12 @@ int launch_sa_sl_batch(hipStream_t s, const LuBatch &b, int *err, int *ctr, int 
     if (b.total <= 0 || !b.sl) return 0;
     const SaBatchEnt *ents = (const SaBatchEnt *)b.ents;
     const dim3 gr((unsigned)b.total);
+    const int fields = phase == 0 ? kSaOps : 1, parts = sl_parts(b.total, fields, b.nsteps, phase == 0 ? kSlCt : kSaRetCt);
+    const dim3 gl((unsigned)b.total, (unsigned)(fields * parts));
     if (phase == 0)
-        hipLaunchKernelGGL((k_sa_layout_batch<true>), gr, dim3(kLanes), 0, s, ents, b.tile_ent, b.arena, b.sl);
+        hipLaunchKernelGGL((k_sa_layout_batch<true>), gl, dim3(kLanes), 0, s, ents, b.tile_ent, b.arena, b.sl, parts);
     else if (phase == 2)
-        hipLaunchKernelGGL((k_sa_layout_batch<false>), gr, dim3(kLanes), 0, s, ents, b.tile_ent, b.arena, b.sl);
+        hipLaunchKernelGGL((k_sa_layout_batch<false>), gl, dim3(kLanes), 0, s, ents, b.tile_ent, b.arena, b.sl, parts);
     else if (phase == 1)
         hipLaunchKernelGGL((k_sa_sl_batch<1>), gr, dim3(kLanes), 0, s, ents, b.tile_ent, b.total, b.resident[0], b.sl,
                            b.ex, err, ctr);

@@ -131,7 +131,7 @@ struct LuBatch {
     void *ents = nullptr;     // device table, one entry per block
     int *tile_ent = nullptr;  // device, entry of each flat tile number
     double *arena = nullptr, *sl = nullptr, *ex = nullptr;  // bases of the table's offsets
-    int nent = 0, total = 0;
+    int nent = 0, total = 0, nsteps = 0;  // nsteps: of the longest sweep
     int resident[2] = {0, 0};  // forward / backward sweep: every workgroup fits on the device at once
     int fuse_add = 0;          // the backward sweep stores q + dq (no add pass)
 };

@@ -86,9 +86,9 @@ SA_PRE_DERIVED = BYTES_PER_NODE["sa_pre"] - 72 + 8
 # formed: no dist, spacing in, no length out
 SA_PRE_LENGTH_KEPT = 24
 # the tile sweep backward pass adds dq to q itself on one block's launch
-# under 2^22 computed nodes (never in the batched sweeps): q in and q out
+# under 2^20 computed nodes (never in the batched sweeps): q in and q out
 # instead of dq out (the add pass is skipped)
-FUSED_ADD_MAX_NODES = 1 << 22
+FUSED_ADD_MAX_NODES = 1 << 20
 FUSED_BACKWARD_BYTES = 24 * 8 + 40 + 40
 # scheme -> (inviscid_scheme, iflag_timeadvance, workload suffix)
 SCHEMES = {
@@ -380,7 +380,7 @@ def roofline_of(args, tm, rr, sa, derived=False, length_kept=False):
         table.update(HYPERPLANE_BYTES)
     else:
         env = os.environ.get("ACFD_LU_FUSED_ADD")
-        # batched sweeps never fuse; a block's own launch does under 2^22
+        # batched sweeps never fuse; a block's own launch does under 2^20
         # computed nodes
         launch = max((r[13] - r[12] + 1) * (r[15] - r[14] + 1) * (r[17] - r[16] + 1) for r in rr)
         if (int(env) != 0) if env is not None else (args.lusgs != 2 and launch < FUSED_ADD_MAX_NODES):
