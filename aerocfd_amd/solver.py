@@ -167,7 +167,7 @@ class Solver:
 
     def download(self, m, name):
         fid, nc = FIELDS[name]
-        a = np.zeros(self.shape(m, name))
+        a = np.empty(self.shape(m, name))  # every value is written
         _lib.check(self.lib.acfd_download(self.h, C.c_int(m), C.c_int(fid), _dp(a)))
         return a
 
