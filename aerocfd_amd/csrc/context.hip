@@ -99,9 +99,11 @@ struct UcChunk {
     bool used;
 };
 std::vector<UcChunk> g_uc;
+std::mutex g_uc_mu;
 
 void *uc_acquire(size_t n)
 {
+    std::lock_guard<std::mutex> lock(g_uc_mu);
     for (auto &c : g_uc)
         if (!c.used && c.n >= n) {
             c.used = true;
@@ -115,6 +117,7 @@ void *uc_acquire(size_t n)
 
 void uc_release(void *p)
 {
+    std::lock_guard<std::mutex> lock(g_uc_mu);
     for (auto &c : g_uc)
         if (c.p == p) c.used = false;
 }
@@ -143,7 +146,10 @@ struct acfd_ctx {
     unsigned int *d_nneg = nullptr;
     double *d_res = nullptr;       // 6 sums
     double *d_partial = nullptr;   // residual partials
-    LuWs lu{nullptr, nullptr, nullptr, nullptr, {0, 0}};  // tile-sweep workspace (lusgs_kernel 1, 2)
+    LuWs lu{nullptr, nullptr, nullptr, nullptr, {0, 0}};  // tile-sweep workspace
+    // the sweeps' schedule: cfg.lusgs_kernel, except that a resident context
+    // with 0 takes the tiles per block where their workspace is to be had
+    int lu_variant = 0;
     long lu_ex_n = 0;
     LuBatch lub;             // lusgs_kernel 2: every block in one launch
     LuBatch sab;             // the same for the SA model's scalar sweeps
@@ -602,13 +608,24 @@ int ensure_geo(acfd_ctx *ctx)
 // batch: the sweep-layout operand array (ordinary device memory), the
 // exchange slots (uncached memory, filled with the sentinel; every sweep
 // leaves them that way) and an error word.  Nothing for hyperplane sweeps.
-int alloc_lu_ws(acfd_ctx *ctx)
+//
+// lusgs_kernel 0 of a resident context (may_pick) takes the tile sweeps per
+// block, with the same results, if their workspace is at most a quarter of
+// the free device memory and can be allocated; else, and with
+// ACFD_LU_HYPERPLANES=1, hyperplane launches, two per plane and 3 (Li + Lj +
+// Lk) of them a step, each of some 9 us: one step of a 65^3 Euler block
+// 3.44 -> 0.43 ms.  A stateless call's context does not repay the workspace.
+int alloc_lu_ws(acfd_ctx *ctx, bool may_pick)
 {
     const int nb = (int)ctx->blk.size();
     HIP_TRY(hipMalloc((void **)&ctx->d_cfl_blk, nb * sizeof(double)));
     for (int m = 0; m < nb; m++) HIP_TRY(hipMemcpy(ctx->d_cfl_blk + m, &ctx->cfg.cfl, sizeof(double), hipMemcpyHostToDevice));
-    if (ctx->cfg.lusgs_kernel != 1 && ctx->cfg.lusgs_kernel != 2) return 0;
-    const bool batch = ctx->cfg.lusgs_kernel == 2;
+    const char *hp = std::getenv("ACFD_LU_HYPERPLANES");
+    const bool pick = ctx->cfg.lusgs_kernel == 0 && may_pick && ctx->cfg.iflag_timeadvance == 2 &&
+                      !(hp && std::atoi(hp) == 1);
+    ctx->lu_variant = ctx->cfg.lusgs_kernel;
+    if (ctx->lu_variant == 0 && !pick) return 0;
+    const bool batch = ctx->lu_variant == 2;
     std::vector<Ext> es;
     std::vector<Fields> fs;
     for (auto &b : ctx->blk) {
@@ -628,13 +645,27 @@ int alloc_lu_ws(acfd_ctx *ctx)
         }
     }
     if (sl_n <= 0) return 0;
-    HIP_TRY(hipMalloc((void **)&ctx->lu.sl, (size_t)sl_n * sizeof(double)));
+    if (pick) {
+        size_t avail = 0, total = 0;
+        const size_t need = (size_t)(sl_n + ex_n) * sizeof(double);
+        if (hipMemGetInfo(&avail, &total) != hipSuccess || need > avail / 4 ||
+            hipMalloc((void **)&ctx->lu.sl, (size_t)sl_n * sizeof(double)) != hipSuccess ||
+            !(ctx->lu.ex = (double *)uc_acquire((size_t)ex_n * sizeof(double)))) {
+            (void)hipGetLastError();
+            if (ctx->lu.sl) (void)hipFree(ctx->lu.sl);
+            ctx->lu.sl = nullptr;
+            return 0;
+        }
+        ctx->lu_variant = 1;
+    } else {
+        HIP_TRY(hipMalloc((void **)&ctx->lu.sl, (size_t)sl_n * sizeof(double)));
+        ctx->lu.ex = (double *)uc_acquire((size_t)ex_n * sizeof(double));
+        if (!ctx->lu.ex) return fail(ACFD_EDEVICE, "uncached device memory for the tile exchange is unavailable");
+    }
     // idle lanes of the sweeps read the padding of the layout: defined values
     HIP_TRY(hipMemsetAsync(ctx->lu.sl, 0, (size_t)sl_n * sizeof(double), ctx->stream));
     HIP_TRY(hipMalloc((void **)&ctx->lu.err, sizeof(int)));
     HIP_TRY(hipMemsetAsync(ctx->lu.err, 0, sizeof(int), ctx->stream));
-    ctx->lu.ex = (double *)uc_acquire((size_t)ex_n * sizeof(double));
-    if (!ctx->lu.ex) return fail(ACFD_EDEVICE, "uncached device memory for the tile exchange is unavailable");
     ctx->lu_ex_n = ex_n;
     KRN_TRY(launch_fill_sentinel(ctx->stream, ctx->lu.ex, ex_n));
     HIP_TRY(hipMalloc((void **)&ctx->lu_ctr, 2 * sizeof(int)));
@@ -916,7 +947,7 @@ int st_implicit(acfd_ctx *ctx, int m, const double *cfl)
 {
     StageTimer t(ctx, ACFD_STAGE_IMPLICIT1ST);
     Block &b = ctx->blk[m];
-    const int variant = ctx->cfg.lusgs_kernel;
+    const int variant = ctx->lu_variant;
     for (int ph = 0; ph < kLusgsPhases; ph++) {
         StageTimer ts(ctx, ph == 2 ? kTimeLuForward : ph == 3 ? kTimeLuBackward
                            : ph == 1 ? kTimeLuGather : ph == 4 ? kTimeLuAdd : kTimeLuOther);
@@ -940,7 +971,7 @@ constexpr bool kBatchedUpdateWritesDq = false;
 int st_implicit_all(acfd_ctx *ctx, const double *cfl_per_block)
 {
     const int nb = (int)ctx->blk.size();
-    if (ctx->cfg.lusgs_kernel != 2) {
+    if (ctx->lu_variant != 2) {
         for (int m = 0; m < nb; m++) {
             int rc = st_implicit(ctx, m, cfl_per_block ? cfl_per_block + m : ctx->d_cfl);
             if (rc) return rc;
@@ -977,7 +1008,7 @@ int st_sa(acfd_ctx *ctx, int m, const double *cfl)
 {
     StageTimer t(ctx, ACFD_STAGE_SA);
     const Block &b = ctx->blk[m];
-    if ((ctx->cfg.lusgs_kernel == 1 || ctx->cfg.lusgs_kernel == 2) && ctx->lu.ex) {
+    if (ctx->lu_variant != 0 && ctx->lu.ex) {
         // tile sweeps in the flow sweep's exchange slots (idle, sentinel-filled)
         const SaSweep sw{ctx->sa_ex ? ctx->sa_ex : ctx->lu.ex, ctx->lu.err};
         KRN_TRY(launch_sa(ctx->stream, b.e, b.f, ctx->c, cfl, &sw));
@@ -1498,7 +1529,7 @@ int acfd_create(const acfd_config *cfg, acfd_ctx **out)
         return fail(ACFD_EINVAL, "acfd_create: inviscid_scheme must be 0 (WENO3 + Roe), 1 (Steger-Warming + WENO5) "
                                  "or 2 (WCNS)");
     if (cfg->lusgs_kernel < 0 || cfg->lusgs_kernel > 2)
-        return fail(ACFD_EINVAL, "acfd_create: lusgs_kernel must be 0 (hyperplanes), 1 (tile sweep per block) or 2 "
+        return fail(ACFD_EINVAL, "acfd_create: lusgs_kernel must be 0 (the library's choice), 1 (tile sweep per block) or 2 "
                                  "(tile sweeps of all blocks in one launch)");
     if (cfg->iflag_timeadvance == 4 && cfg->iflag_turbulence == 2 && cfg->iflag_solver == 0)
         return fail(ACFD_EINVAL, "acfd_create: the explicit RK3 advance is for laminar or Euler flow");
@@ -1737,7 +1768,7 @@ int acfd_set_topology(acfd_ctx *ctx, int nblk, const int *dims, const int *nsub,
         return rc;
     HIP_TRY(hipMalloc((void **)&ctx->d_partial, (size_t)parts * 6 * sizeof(double)));
     ctx->inv_run = inviscid_run(ctx->totalnodes, ctx->cfg.inviscid_scheme, ctx->cfg.precision);
-    rc = alloc_lu_ws(ctx);
+    rc = alloc_lu_ws(ctx, true);
     if (!rc && ctx->cfg.iflag_timeadvance == 3) rc = ensure_block_table(ctx);
     if (!rc) rc = build_batch(ctx);
     if (rc) return rc;
@@ -2465,7 +2496,7 @@ int make_single(const acfd_config *cfg, const int *r, acfd_ctx **out)
     dev_upload(&ctx->d_ntab, nn);
     HIP_TRY(hipMalloc((void **)&ctx->d_partial, (size_t)residual_partials(e) * 6 * sizeof(double)));
     ctx->inv_run = inviscid_run(e.n, c.inviscid_scheme, c.precision);
-    rc = alloc_lu_ws(ctx);
+    rc = alloc_lu_ws(ctx, false);
     if (!rc && c.iflag_timeadvance == 3) rc = ensure_block_table(ctx);
     if (rc) return rc;
     ctx->totalnodes = (long)(e.ie0 - e.is0 + 1) * (e.je0 - e.js0 + 1) * (e.ke0 - e.ks0 + 1);

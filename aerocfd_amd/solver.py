@@ -69,7 +69,7 @@ class FlowConfig:
     iflag_des: int = 0
     iflag_timeadvance: int = 2   # 2 LU-SGS, 3 BDF2, 4 explicit RK3 (no reference counterpart)
     precision: int = 0           # 0 FP64, 1 FP32 flux / FP64 update
-    lusgs_kernel: int = 0        # 0 hyperplane launches, 1 pipelined tiles
+    lusgs_kernel: int = 0        # 0 the library's choice of 1 or hyperplane launches, 1 pipelined tiles
     inviscid_scheme: int = 0     # 0 WENO3 + Roe (reference); 1 Steger-Warming + WENO5, 2 WCNS
     use_graph: int = 0           # 1 replay one captured HIP graph per step
     batch_blocks: int = 0        # 1 one launch per stage over all blocks

@@ -315,6 +315,8 @@ def timed_run(args, case, fields, coords, precision):
     cfg = case.cfg
     cfg.precision = precision
     cfg.lusgs_kernel = args.lusgs
+    if args.lusgs == 0:
+        os.environ["ACFD_LU_HYPERPLANES"] = "1"
     cfg.use_graph = 1 if args.graph else 0
     cfg.batch_blocks = 1 if args.batch else 0
     sol = Solver(cfg, case.dims, case.subfaces)

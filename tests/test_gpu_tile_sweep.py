@@ -36,6 +36,9 @@ def run(case, kernel, batch=0, tickets=False):
     case.cfg.lusgs_kernel, case.cfg.batch_blocks = kernel, batch
     if tickets:
         os.environ["ACFD_LU_TICKETS"] = "1"
+    if kernel == "hyperplanes":
+        os.environ["ACFD_LU_HYPERPLANES"] = "1"
+        case.cfg.lusgs_kernel = 0
     try:
         sol = Solver(case.cfg, case.dims, case.subfaces)
         try:
@@ -47,6 +50,7 @@ def run(case, kernel, batch=0, tickets=False):
             sol.close()
     finally:
         os.environ.pop("ACFD_LU_TICKETS", None)
+        os.environ.pop("ACFD_LU_HYPERPLANES", None)
 
 
 @pytest.mark.parametrize("solver", [0, 1])
@@ -55,9 +59,9 @@ def run(case, kernel, batch=0, tickets=False):
 def test_tiles_equal_hyperplanes(dims, solver):
     print("test_tiles_equal_hyperplanes", dims, solver, flush=True)
     sys.stdout.flush()
-    ref = run(box(dims, solver), 0)
+    ref = run(box(dims, solver), "hyperplanes")
     assert np.isfinite(ref[0]).all()
-    for kernel, batch, tickets in ((1, 0, False), (1, 0, True), (2, 1, False), (2, 0, True)):
+    for kernel, batch, tickets in ((0, 0, False), (1, 0, False), (1, 0, True), (2, 1, False), (2, 0, True)):
         got = run(box(dims, solver), kernel, batch, tickets)
         assert np.array_equal(ref[0], got[0]), (dims, kernel, tickets, np.abs(ref[0] - got[0]).max())
         assert np.array_equal(ref[1], got[1])
@@ -68,6 +72,6 @@ def test_more_tiles_than_fit():
     of the sweep's workgroups)."""
     dims = (8, 802, 58)
     print("test_more_tiles_than_fit", dims, flush=True)
-    ref = run(box(dims, 1), 0)
+    ref = run(box(dims, 1), "hyperplanes")
     got = run(box(dims, 1), 1)
     assert np.array_equal(ref[0], got[0])
