@@ -139,7 +139,7 @@ struct acfd_ctx {
     double *d_fwork = nullptr;
     long totalnodes = 0;
     bool topo = false;
-    int inv_run = 16;         // nodes per thread of the j / k inviscid kernels
+    int inv_run = 16;         // nodes per thread of the j / k kernels of scheme 0
     // device scalars
     double *d_cfl = nullptr;
     unsigned long long *d_stats = nullptr;
@@ -816,9 +816,9 @@ int inviscid_with_sensor(acfd_ctx *ctx, int m)
         sa.replay = call % ctx->s_refresh != 0;
     }
     if (ctx->s_audit > 0 && call % ctx->s_audit == 0) {
-        KRN_TRY(launch_inviscid_ext(ctx->stream, b.e, b.f, ctx->c, ctx->cfg.precision, 2, ctx->inv_run, clear));
+        KRN_TRY(launch_inviscid_ext(ctx->stream, b.e, b.f, ctx->c, ctx->cfg.precision, 2, clear));
         KRN_TRY(launch_copy(ctx->stream, b.f.rhsi, b.f.w_flux, 5 * b.e.n));
-        KRN_TRY(launch_inviscid_wcns_sensor(ctx->stream, b.e, b.f, ctx->c, ctx->cfg.precision, ctx->inv_run, clear, sa));
+        KRN_TRY(launch_inviscid_wcns_sensor(ctx->stream, b.e, b.f, ctx->c, ctx->cfg.precision, clear, sa));
         const long np = diff_partials(b.e);
         if (ctx->s_dpart_n < 2 * np) {
             if (ctx->s_dpart) (void)hipFree(ctx->s_dpart);
@@ -844,7 +844,7 @@ int inviscid_with_sensor(acfd_ctx *ctx, int m)
         }
         return 0;
     }
-    KRN_TRY(launch_inviscid_wcns_sensor(ctx->stream, b.e, b.f, ctx->c, ctx->cfg.precision, ctx->inv_run, clear, sa));
+    KRN_TRY(launch_inviscid_wcns_sensor(ctx->stream, b.e, b.f, ctx->c, ctx->cfg.precision, clear, sa));
     return 0;
 }
 
@@ -858,7 +858,7 @@ int st_inviscid(acfd_ctx *ctx, int m)
         KRN_TRY(launch_inviscid(ctx->stream, b.e, b.f, ctx->c, ctx->cfg.precision, ctx->inv_run, clear));
     else
         KRN_TRY(launch_inviscid_ext(ctx->stream, b.e, b.f, ctx->c, ctx->cfg.precision, ctx->cfg.inviscid_scheme,
-                                    ctx->inv_run, clear));
+                                    clear));
     b.rhsi_clean = true;
     return 0;
 }
@@ -1767,7 +1767,7 @@ int acfd_set_topology(acfd_ctx *ctx, int nblk, const int *dims, const int *nsub,
         (rc = dev_upload(&ctx->d_ntab, ntab)))
         return rc;
     HIP_TRY(hipMalloc((void **)&ctx->d_partial, (size_t)parts * 6 * sizeof(double)));
-    ctx->inv_run = inviscid_run(ctx->totalnodes, ctx->cfg.inviscid_scheme, ctx->cfg.precision);
+    ctx->inv_run = inviscid_run(ctx->totalnodes, ctx->cfg.precision);
     rc = alloc_lu_ws(ctx, true);
     if (!rc && ctx->cfg.iflag_timeadvance == 3) rc = ensure_block_table(ctx);
     if (!rc) rc = build_batch(ctx);
@@ -2495,7 +2495,7 @@ int make_single(const acfd_config *cfg, const int *r, acfd_ctx **out)
     dev_upload(&ctx->d_nuttab, nt);
     dev_upload(&ctx->d_ntab, nn);
     HIP_TRY(hipMalloc((void **)&ctx->d_partial, (size_t)residual_partials(e) * 6 * sizeof(double)));
-    ctx->inv_run = inviscid_run(e.n, c.inviscid_scheme, c.precision);
+    ctx->inv_run = inviscid_run(e.n, c.precision);
     rc = alloc_lu_ws(ctx, false);
     if (!rc && c.iflag_timeadvance == 3) rc = ensure_block_table(ctx);
     if (rc) return rc;

@@ -192,23 +192,18 @@ __global__ void __launch_bounds__(256) k_inviscid_i(Ext e, const double *__restr
 // flux in registers, so a run evaluates run + 1 faces.  rhsi -= (F+ - F-).
 //
 // The run of a context comes from its nodes: long runs repeat fewer faces
-// at their ends (and, for the wide stencils, fewer node loads), short ones
-// put more wavefronts on a device that holds 2-3 thousand of them.  Inviscid
-// stage of WENO3 + Roe, us, at runs of 1 / 4 / 8 / 16: 33^3 26 / 38 / 57 /
-// 97, 65^3 50 / 47 / 63 / 101, 129^3 375 / 287 / 291 / 317, 193^3 1174 / 893
-// / 889 / 932, 256^3 - / 1814 / 1729 / 1732, 98 M nodes in 40 blocks best at
-// 16.  WENO5 splitting and WCNS (three evaluations) at 2 / 4 / 16 / 32:
-// 41^3 187 / 253 / 658 / 1156 and 172 / 211 / 464 / 772, 65^3 398 / 384 /
-// 778 / 1295 and 322 / 274 / 522 / 834, 129^3 2218 / 1998 / 1826 / 1998 and
-// 1948 / 1500 / 1222 / 1353, 193^3 WCNS 6265 / 4571 / 3764 / 3789.  A run's
-// first face of WENO3 + Roe is a second copy of the flux code, rounded in
-// its own way: the rule takes the context's nodes, not a launch's, so that
-// batched and per-block launches cut the same runs, and FP32 fluxes, where
-// an ulp is 1e-7, keep the run of 16 that they were measured with.
+// at their ends, short ones put more wavefronts on a device that holds 2-3
+// thousand of them.  Inviscid stage, us, at runs of 1 / 4 / 8 / 16: 33^3 26 /
+// 38 / 57 / 97, 65^3 50 / 47 / 63 / 101, 129^3 375 / 287 / 291 / 317, 193^3
+// 1174 / 893 / 889 / 932, 256^3 - / 1814 / 1729 / 1732, 98 M nodes in 40
+// blocks best at 16.  A run's first face is a second copy of the flux code,
+// rounded in its own way: the rule takes the context's nodes, not a
+// launch's, so that batched and per-block launches cut the same runs, and
+// FP32 fluxes, where an ulp is 1e-7, keep the run of 16 that they were
+// measured with.
 constexpr int kInvRunF32 = 16;
-int inviscid_run(long nodes, int scheme, int precision)
+int inviscid_run(long nodes, int precision)
 {
-    if (scheme != 0) return nodes < 150000 ? 2 : nodes < 1000000 ? 4 : 16;
     if (precision == 1) return kInvRunF32;
     return nodes < 100000 ? 1 : nodes < 4000000 ? 4 : nodes < 32000000 ? 8 : 16;
 }

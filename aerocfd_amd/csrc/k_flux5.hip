@@ -21,22 +21,34 @@
 
 namespace acfd {
 
+// x / y for a positive normal y: FP64 through rcp_pos, FP32 divides
+template <typename R>
+__device__ inline R over_pos(R x, R y)
+{
+    return x / y;
+}
+template <>
+__device__ inline double over_pos<double>(double x, double y)
+{
+    return x * rcp_pos<double>(y);
+}
+
 // Steger-Warming split fluxes through the node metric M = grad xi / J.
 template <typename R>
 __device__ inline void sw_split(const R *q, R mx, R my, R mz, R gamma, R *fp, R *fm)
 {
-    const R rho = q[0], ri = (R)1.0 / rho;
+    const R rho = q[0], ri = rcp_pos<R>(rho);
     const R u = q[1] * ri, v = q[2] * ri, w = q[3] * ri;
     const R v2 = u * u + v * v + w * w;
     const R p = (gamma - (R)1.0) * (q[4] - (R)0.5 * rho * v2);
     const R c = sqrt(gamma * p * ri);
     const R mm = sqrt(mx * mx + my * my + mz * mz);
-    const R rm = (R)1.0 / mm;
+    const R rm = rcp_pos<R>(mm);
     const R nx = mx * rm, ny = my * rm, nz = mz * rm;
     const R ut = u * nx + v * ny + w * nz;
-    const R h = c * c / (gamma - (R)1.0) + (R)0.5 * v2;
+    const R h = over_pos<R>(c * c, gamma - (R)1.0) + (R)0.5 * v2;
     const R l[3] = {mm * ut, mm * (ut + c), mm * (ut - c)};
-    const R s = rho / ((R)2.0 * gamma);
+    const R s = over_pos<R>(rho, (R)2.0 * gamma);
 #pragma unroll
     for (int side = 0; side < 2; side++) {
         R lp[3];
@@ -85,6 +97,51 @@ __device__ inline R weno5_rec(R a, R b, R c, R d, R e5)
     return weno_combine3(q0, q1, q2, b0, b1, b2, (R)0.1, (R)0.6, (R)0.3);
 }
 
+// The FP64 form of both fifth-order states at a face, from the first and
+// second differences of the values: with c the value next to the face on
+// the state's side, ea = c - b, eb = d - c and the second differences D0,
+// D1, D2 of the three stencils, the candidates are c + ea/2 + al D0,
+// c + eb/2 - be D1 and c + eb/2 - be D2 (al, be = 1/3, 1/6 of the flux
+// reconstruction, 3/8, 1/8 of the interpolation), and the smoothness
+// indicators 13/12 D^2 + g^2 with g = ea + D0/2, ea + D1/2, eb - D2/2.  The
+// kernels below are bound by the FP64 instructions they issue; this takes
+// 40 to a state and no division, where the written-out sums take about 65,
+// with the quotients by 3 and 6 of the reconstruction 170.  A WCNS face's
+// two states share the differences.  The value is a correction to c, so its
+// rounding is that of the differences, which is the smaller.
+struct Weno5Diff {
+    double D, P;  // a second difference, eps + 13/12 D^2
+    __device__ inline void set(double ea, double eb)
+    {
+        D = eb - ea;
+        P = fma(13.0 / 12.0 * D, D, 1.0e-6);
+    }
+};
+
+// linear weights 1 : C1 : C2; AL2, BE2 twice the al, be above
+__device__ inline double weno5_state(double c, double ea, double eb, const Weno5Diff &d0, const Weno5Diff &d1,
+                                     const Weno5Diff &d2, double C1, double C2, double AL2, double BE2)
+{
+    const double g0 = fma(0.5, d0.D, ea), g1 = fma(0.5, d1.D, ea), g2 = fma(-0.5, d2.D, eb);
+    const double s0 = fma(g0, g0, d0.P), s1 = fma(g1, g1, d1.P), s2 = fma(g2, g2, d2.P);
+    const double t0 = s0 * s0, t1 = s1 * s1, t2 = s2 * s2;
+    const double w0 = t1 * t2, w1 = C1 * (t0 * t2), w2 = C2 * (t0 * t1);
+    const double r0 = fma(AL2, d0.D, ea), r1 = fma(-BE2, d1.D, eb), r2 = fma(-BE2, d2.D, eb);
+    const double num = fma(w2, r2, fma(w1, r1, w0 * r0));
+    return fma(0.5 * num, rcp_pos<double>(w0 + w1 + w2), c);
+}
+
+template <>
+__device__ inline double weno5_rec<double>(double a, double b, double c, double d, double e5)
+{
+    const double ea = c - b, eb = d - c;
+    Weno5Diff d0, d1, d2;
+    d0.set(b - a, ea);
+    d1.set(ea, eb);
+    d2.set(eb, e5 - d);
+    return weno5_state(c, ea, eb, d0, d1, d2, 6.0, 3.0, 2.0 / 3.0, 1.0 / 3.0);
+}
+
 // WENO3 flux reconstruction at i+1/2 from f(i-1..i+1) (linear weights 1/3, 2/3)
 template <typename R>
 __device__ inline R weno3_rec(R a, R b, R c)
@@ -106,6 +163,27 @@ __device__ inline R weno5_interp(R a, R b, R c, R d, R e5)
     R b0, b1, b2;
     js_beta(a, b, c, d, e5, b0, b1, b2);
     return weno_combine3(q0, q1, q2, b0, b1, b2, (R)1.0 / (R)16.0, (R)10.0 / (R)16.0, (R)5.0 / (R)16.0);
+}
+
+// left and right midpoint states of a face from the six values around it
+template <typename R>
+__device__ inline void weno5_interp2(R a, R b, R c, R d, R e5, R f, R &l, R &r)
+{
+    l = weno5_interp<R>(a, b, c, d, e5);
+    r = weno5_interp<R>(f, e5, d, c, b);
+}
+template <>
+__device__ inline void weno5_interp2<double>(double a, double b, double c, double d, double e5, double f, double &l,
+                                             double &r)
+{
+    const double x1 = c - b, x2 = d - c, x3 = e5 - d;
+    Weno5Diff d0, d1, d2, d3;
+    d0.set(b - a, x1);
+    d1.set(x1, x2);
+    d2.set(x2, x3);
+    d3.set(x3, f - e5);
+    l = weno5_state(c, x1, x2, d0, d1, d2, 10.0, 5.0, 0.75, 0.25);
+    r = weno5_state(d, -x3, -x2, d3, d2, d1, 10.0, 5.0, 0.75, 0.25);
 }
 
 __device__ inline int face_order(int a, int lo, int hi)
@@ -141,7 +219,10 @@ __device__ inline void node_quantity(const double *__restrict__ q, const double 
     }
 }
 
-// face flux at a+1/2 from node quantities W[0..5] at a-2..a+3 (order ord);
+// face flux at a+1/2 from node quantities W[0..5] at a-2..a+3 (order ord;
+// one branch on ord around all five variables instead of one each is 1 %
+// faster, but the compiler then contracts FP32's sums in another way, which
+// moves the FP32 results by their rounding);
 // scheme 2 also needs the face metric m
 template <typename R, int SCHEME, int NQ>
 __device__ inline void ext_face(const R (*W)[NQ], int ord, const R *m, R gamma, R *F, bool lin = false)
@@ -173,8 +254,7 @@ __device__ inline void ext_face(const R (*W)[NQ], int ord, const R *m, R gamma, 
                 ur[x] = ((R)3.0 * W[5][x] - (R)20.0 * W[4][x] + (R)90.0 * W[3][x] + (R)60.0 * W[2][x] -
                          (R)5.0 * W[1][x]) / (R)128.0;
             } else if (ord == 5) {
-                ul[x] = weno5_interp<R>(W[0][x], W[1][x], W[2][x], W[3][x], W[4][x]);
-                ur[x] = weno5_interp<R>(W[5][x], W[4][x], W[3][x], W[2][x], W[1][x]);
+                weno5_interp2<R>(W[0][x], W[1][x], W[2][x], W[3][x], W[4][x], W[5][x], ul[x], ur[x]);
             } else if (ord == 3) {
                 ul[x] = weno3<R>(W[1][x], W[2][x], W[3][x]);
                 ur[x] = weno3<R>(W[4][x], W[3][x], W[2][x]);
@@ -213,8 +293,6 @@ __device__ inline double ext_diff(const R (*FR)[5], int x, int dord)
     return 75.0 / 64.0 * d1 - 25.0 / 384.0 * d3 + 3.0 / 640.0 * d5;
 }
 
-// j and k directions: each thread marches along the axis over `run` nodes
-// with rolling windows of node quantities and face fluxes.
 // one wavefront's face counts into its slot (called by one lane)
 __device__ inline void sensor_count(unsigned long long *stats, unsigned long long ne, unsigned long long nl)
 {
@@ -223,6 +301,13 @@ __device__ inline void sensor_count(unsigned long long *stats, unsigned long lon
     atomicAdd(&stats[slot * kSensorStatStride + 1], nl);
 }
 
+// j and k directions: each thread marches along the axis over `run` nodes
+// with rolling windows of node quantities and face fluxes.  Bound by FP64
+// instructions and, on small blocks, by their latency.  81^3, all three
+// directions, a stage: WENO5 splitting 230 us with the written-out
+// candidates (100 divisions a face) and 64-wide tiles of 81-node rows, 91
+// now; WCNS on 1024 x 512 x 4 226, now 191.  Reading the next node a step
+// ahead gave scheme 1 2 % and took 2 % from scheme 2: not done.
 // SENS: 0 plain; 1 the network decides per face (and records the decisions
 // in sa.mask when given); 2 the decisions are read from sa.mask
 template <typename R, int AXIS, int SCHEME, int SENS>
@@ -232,11 +317,13 @@ __global__ void __launch_bounds__(256) k_ext_jk(Ext e, const double *__restrict_
                                                double gamma_d, SensorArgs sa, int run)
 {
     constexpr int NQ = SCHEME == 1 ? 10 : 5;
-    const int ir = e.is1 + (int)(blockIdx.x * blockDim.x + threadIdx.x);
-    const int orr = (int)(blockIdx.y * blockDim.y + threadIdx.y);
-    const int a0 = e.lo1(AXIS) + (int)blockIdx.z * run;
+    // the lines of this axis, counted through the rows of the computed
+    // range: full wavefronts whatever the row length
+    const int Li = e.ie1 - e.is1 + 1, Lo = AXIS == 1 ? e.ke1 - e.ks1 + 1 : e.je1 - e.js1 + 1;
+    const int lr = (int)(blockIdx.x * 256 + threadIdx.y * 64 + threadIdx.x);
+    const int a0 = e.lo1(AXIS) + (int)blockIdx.y * run;
     const int a1 = min(a0 + run - 1, e.hi1(AXIS));
-    const bool active = ir <= e.ie1 && (AXIS == 1 ? e.ks1 + orr <= e.ke1 : e.js1 + orr <= e.je1);
+    const bool active = lr < Li * Lo;
     // with the sensor every lane takes part (in the wavefront-wide network,
     // and in the wavefront's sum of its face counts); lanes outside the
     // range work on a valid line and store nothing
@@ -247,8 +334,8 @@ __global__ void __launch_bounds__(256) k_ext_jk(Ext e, const double *__restrict_
     } else if constexpr (SENS == 0) {
         if (!active) return;
     }
-    const int i = min(ir, e.ie1);
-    const int o = min(orr, AXIS == 1 ? e.ke1 - e.ks1 : e.je1 - e.js1);
+    const int l = min(lr, Li * Lo - 1);
+    const int o = l / Li, i = e.is1 + (l - o * Li);
     const int j = AXIS == 1 ? e.lo(1) : e.js1 + o;
     const int k = AXIS == 2 ? e.lo(2) : e.ks1 + o;
     unsigned n_eval = 0, n_lin = 0;
@@ -344,17 +431,26 @@ __global__ void __launch_bounds__(256) k_ext_i(Ext e, const double *__restrict__
                                               double gamma_d, SensorArgs sa)
 {
     constexpr int NQ = SCHEME == 1 ? 10 : 5;
-    __shared__ R nq[4][NQ][64];
-    __shared__ R fq[4][5][64];
+    // a lane's neighbours at constant distances: rows of 64 with a margin (a
+    // margin's values reach only faces that no node of the wavefront uses)
+    __shared__ R nq[4][NQ][2 + 64 + 3];
+    __shared__ R fq[4][5][3 + 64 + 2];
     __shared__ typename std::conditional<SENS == 1, SensorLds, char>::type slds;
     if constexpr (SENS == 1) sensor_load_net(sa.net, slds);
     const int lane = threadIdx.x, row = threadIdx.y;
-    const int jr = e.js1 + (int)(blockIdx.y * blockDim.y + threadIdx.y);
-    const bool row_ok = jr <= e.je1;
-    const int j = row_ok ? jr : e.je1;
-    const int k = e.ks1 + (int)blockIdx.z;
-    const int i0 = e.is1 + (int)blockIdx.x * ExtI<SCHEME>::NPW;
-    const int p = i0 - ExtI<SCHEME>::OFF + lane;  // position of this lane
+    // Plain: the rows of the computed range end to end, each with the OFF
+    // positions that its end nodes read beyond it; wavefronts take 64
+    // positions, NPW apart, also across the end of a row.  With the sensor
+    // a wavefront stays in its row, in whose wavefronts the faces are
+    // counted.
+    constexpr int OFF = ExtI<SCHEME>::OFF, NPW = ExtI<SCHEME>::NPW;
+    const int Li = e.ie1 - e.is1 + 1, Lj = e.je1 - e.js1 + 1, rows = Lj * (e.ke1 - e.ks1 + 1);
+    const int pitch = SENS ? (Li + NPW - 1) / NPW * NPW : Li + 2 * OFF;
+    const int g0 = (int)(blockIdx.x * 4 + row) * NPW, g = SENS ? g0 : g0 + lane;
+    const int rr = g / pitch, rc = min(rr, rows - 1);
+    const bool row_ok = rr < rows;
+    const int j = e.js1 + rc % Lj, k = e.ks1 + rc / Lj;
+    const int p = e.is1 - OFF + (g - rr * pitch) + (SENS ? lane : 0);  // position of this lane
     const int lo = e.is, hi = e.ie;
     const R gamma = (R)gamma_d;
     const long N = e.n;
@@ -364,7 +460,7 @@ __global__ void __launch_bounds__(256) k_ext_i(Ext e, const double *__restrict__
         R v[NQ];
         node_quantity<R, SCHEME>(q, dxidx, inv_j, N, n, 0, gamma, v);
 #pragma unroll
-        for (int x = 0; x < NQ; x++) nq[row][x][lane] = v[x];
+        for (int x = 0; x < NQ; x++) nq[row][x][2 + lane] = v[x];
     }
     __syncthreads();
     {
@@ -374,7 +470,7 @@ __global__ void __launch_bounds__(256) k_ext_i(Ext e, const double *__restrict__
 #pragma unroll
         for (int w = 0; w < 6; w++)
 #pragma unroll
-            for (int x = 0; x < NQ; x++) W[w][x] = nq[row][x][min(max(lane - 2 + w, 0), 63)];
+            for (int x = 0; x < NQ; x++) W[w][x] = nq[row][x][lane + w];
         const int ord = face_order(p, lo, hi);
         bool lin = false;
         if constexpr (SENS == 1) {
@@ -397,70 +493,88 @@ __global__ void __launch_bounds__(256) k_ext_i(Ext e, const double *__restrict__
             ext_face<R, SCHEME, NQ>(W, ord, m, gamma, F, lin);
         }
 #pragma unroll
-        for (int x = 0; x < 5; x++) fq[row][x][lane] = F[x];
+        for (int x = 0; x < 5; x++) fq[row][x][3 + lane] = F[x];
     }
     __syncthreads();
-    if (row_ok && lane >= ExtI<SCHEME>::OFF && lane < ExtI<SCHEME>::OFF + ExtI<SCHEME>::NPW && p >= e.is1 &&
-        p <= e.ie1) {
+    if (row_ok && lane >= OFF && lane < OFF + ExtI<SCHEME>::NPW && p >= e.is1 && p <= e.ie1) {
         R FR[6][5];
 #pragma unroll
         for (int f = 0; f < 6; f++)
 #pragma unroll
-            for (int x = 0; x < 5; x++) {
-                const int l = lane - 3 + f;
-                FR[f][x] = (l >= 0 && l < 64) ? fq[row][x][l] : (R)0;
-            }
+            for (int x = 0; x < 5; x++) FR[f][x] = fq[row][x][lane + f];
         const int dord = SCHEME == 2 ? wcns_order(p, lo, hi) : 2;
 #pragma unroll
         for (int x = 0; x < 5; x++) rhsi[x * N + n] = -ext_diff<R, SCHEME, 3>(FR, x, dord);
     }
 }
 
+// Nodes a thread of k_ext_jk marches over.  A run of r nodes evaluates r + 1
+// faces and r + 5 split fluxes (scheme 1) or r + 5 faces (scheme 2), so
+// short ones repeat work; long ones leave SIMDs idle, and a wavefront alone
+// on its SIMD needs 3 us a node for its chain of dependent FP64 operations
+// (two share a SIMD at 0.7 us a node).  RK3 step, us, at runs of 1 / 2 / 4 /
+// 8 / 16: WENO5 splitting 33^3 232 / 249 / 289 / 365 / 496, 65^3 398 / 355 /
+// 359 / 423 / 566, 81^3 644 / 551 / 496 / 518 / 657, 113^3 1407 / 1159 /
+// 1056 / 1027 / 1060, 169^3 4590 / 3687 / 3267 / 3116 / 3193; WCNS 33^3 262 /
+// 275 / 314 / 387 / 514, 65^3 510 / 411 / 383 / 455 / 605, 81^3 839 / 642 /
+// 565 / 558 / 699, 169^3 6276 / 4548 / 3752 / 3404 / 3430, 1024 x 512 x 4
+// 1344 / 1059 / 993 / 951 / 976; FP32 has its best runs at the same sizes.
+// A face's value does not depend on the run that holds it.  With the
+// sensor the faces counted are those of the runs, which stay at 16.
+static int ext_run(long nodes, bool sensor)
+{
+    if (sensor) return 16;
+    return nodes < 80000 ? 1 : nodes < 200000 ? 2 : nodes < 1000000 ? 4 : 8;
+}
+
 template <typename R, int SCHEME, int SENS = 0>
-static void launch_ext_t(hipStream_t s, const Ext &e, const Fields &f, double gamma, int run, SensorArgs sa = {})
+static void launch_ext_t(hipStream_t s, const Ext &e, const Fields &f, double gamma, SensorArgs sa = {})
 {
     const int Li = e.ie1 - e.is1 + 1, Lj = e.je1 - e.js1 + 1, Lk = e.ke1 - e.ks1 + 1;
+    const int run = ext_run((long)Li * Lj * Lk, SENS != 0);
     dim3 t(64, 4, 1);
-    dim3 gi((Li + ExtI<SCHEME>::NPW - 1) / ExtI<SCHEME>::NPW, (Lj + 3) / 4, Lk);
+    constexpr int OFF = ExtI<SCHEME>::OFF, NPW = ExtI<SCHEME>::NPW;
+    const long pitch = SENS ? (Li + NPW - 1) / NPW * NPW : Li + 2 * OFF;
+    dim3 gi((unsigned)((pitch * Lj * Lk + 4 * NPW - 1) / (4 * NPW)));
     hipLaunchKernelGGL((k_ext_i<R, SCHEME, SENS>), gi, t, 0, s, e, f.q, f.dxidx, f.inv_j, f.rhsi, gamma, sa);
-    dim3 gj((Li + 63) / 64, (Lk + 3) / 4, (Lj + run - 1) / run);
+    dim3 gj((unsigned)(((long)Li * Lk + 255) / 256), (Lj + run - 1) / run);
     hipLaunchKernelGGL((k_ext_jk<R, 1, SCHEME, SENS>), gj, t, 0, s, e, f.q, f.dxidx, f.inv_j, f.rhsi, gamma, sa,
                        run);
-    dim3 gk((Li + 63) / 64, (Lj + 3) / 4, (Lk + run - 1) / run);
+    dim3 gk((unsigned)(((long)Li * Lj + 255) / 256), (Lk + run - 1) / run);
     hipLaunchKernelGGL((k_ext_jk<R, 2, SCHEME, SENS>), gk, t, 0, s, e, f.q, f.dxidx, f.inv_j, f.rhsi, gamma, sa,
                        run);
 }
 
 int launch_inviscid_wcns_sensor(hipStream_t s, const Ext &e, const Fields &f, const Consts &c, int precision,
-                                int run, bool clear, const SensorArgs &sa)
+                                bool clear, const SensorArgs &sa)
 {
     int rc = clear ? launch_fill(s, f.rhsi, 5 * e.n, 0.0) : 0;
     if (rc) return rc;
     if (e.ie1 < e.is1 || e.je1 < e.js1 || e.ke1 < e.ks1) return 0;
     if (sa.replay) {
-        if (precision == 1) launch_ext_t<float, 2, 2>(s, e, f, c.gamma, run, sa);
-        else launch_ext_t<double, 2, 2>(s, e, f, c.gamma, run, sa);
+        if (precision == 1) launch_ext_t<float, 2, 2>(s, e, f, c.gamma, sa);
+        else launch_ext_t<double, 2, 2>(s, e, f, c.gamma, sa);
     } else {
-        if (precision == 1) launch_ext_t<float, 2, 1>(s, e, f, c.gamma, run, sa);
-        else launch_ext_t<double, 2, 1>(s, e, f, c.gamma, run, sa);
+        if (precision == 1) launch_ext_t<float, 2, 1>(s, e, f, c.gamma, sa);
+        else launch_ext_t<double, 2, 1>(s, e, f, c.gamma, sa);
     }
     ACFD_CHECK_LAUNCH();
     return 0;
 }
 
 int launch_inviscid_ext(hipStream_t s, const Ext &e, const Fields &f, const Consts &c, int precision, int scheme,
-                        int run, bool clear)
+                        bool clear)
 {
     // rhsi is zero outside the computed range
     int rc = clear ? launch_fill(s, f.rhsi, 5 * e.n, 0.0) : 0;
     if (rc) return rc;
     if (e.ie1 < e.is1 || e.je1 < e.js1 || e.ke1 < e.ks1) return 0;
     if (scheme == 1) {
-        if (precision == 1) launch_ext_t<float, 1>(s, e, f, c.gamma, run);
-        else launch_ext_t<double, 1>(s, e, f, c.gamma, run);
+        if (precision == 1) launch_ext_t<float, 1>(s, e, f, c.gamma);
+        else launch_ext_t<double, 1>(s, e, f, c.gamma);
     } else {
-        if (precision == 1) launch_ext_t<float, 2>(s, e, f, c.gamma, run);
-        else launch_ext_t<double, 2>(s, e, f, c.gamma, run);
+        if (precision == 1) launch_ext_t<float, 2>(s, e, f, c.gamma);
+        else launch_ext_t<double, 2>(s, e, f, c.gamma);
     }
     ACFD_CHECK_LAUNCH();
     return 0;

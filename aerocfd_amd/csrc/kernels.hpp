@@ -11,7 +11,7 @@ int launch_fill(hipStream_t s, double *p, long n, double v);
 // run: nodes a thread of the j / k kernels marches over (inviscid_run);
 // clear: rhsi may not be zero outside the computed range
 int launch_inviscid(hipStream_t s, const Ext &e, const Fields &f, const Consts &c, int precision, int run, bool clear);
-int inviscid_run(long nodes, int scheme, int precision);
+int inviscid_run(long nodes, int precision);
 int launch_viscous(hipStream_t s, const Ext &e, const Fields &f, const Consts &c, int precision,
                    int store_aux);
 // unsteady: the local cfl of the block's last node goes to *cfl and, when
@@ -23,7 +23,7 @@ int launch_reset_stats(hipStream_t s, unsigned long long *stats);
 // k_flux5.hip: schemes and time integration with no reference counterpart
 // (scheme 1 Steger-Warming + WENO5, 2 WCNS; Shu-Osher RK3)
 int launch_inviscid_ext(hipStream_t s, const Ext &e, const Fields &f, const Consts &c, int precision, int scheme,
-                        int run, bool clear);
+                        bool clear);
 int launch_rk3_stage(hipStream_t s, const Ext &e, const Fields &f, const double *qn, int stage, bool viscous);
 int launch_copy(hipStream_t s, const double *a, double *b, long n);
 
@@ -56,7 +56,7 @@ size_t sensor_net_bytes();
 long diff_partials(const Ext &e);
 int launch_diff_partial(hipStream_t s, const Ext &e, const double *a, const double *b, double *part);
 int launch_inviscid_wcns_sensor(hipStream_t s, const Ext &e, const Fields &f, const Consts &c, int precision,
-                                int run, bool clear, const SensorArgs &sa);
+                                bool clear, const SensorArgs &sa);
 
 // batched launches over every block (block table, per-kind grids)
 dim3 grid_1d(long n);                    // 256-thread workgroups over n items
