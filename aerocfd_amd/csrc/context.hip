@@ -537,6 +537,42 @@ int ensure_block_table(acfd_ctx *ctx)
     return dev_upload(&ctx->d_blocks, block_records(ctx));
 }
 
+// Rounds of the physical boundary subfaces, each one launch over all blocks:
+// a subface goes to the first round behind every earlier subface of its
+// block that it shares nodes with (either writes what the other reads or
+// writes), so the values are those of the reference's order.  The six faces
+// of a box take three rounds, each launch 5-10 us for a few thousand nodes
+// whatever it holds: 81^3 RK3 step 131 -> 65 us of boundary conditions.
+int build_bc_rounds(acfd_ctx *ctx)
+{
+    for (size_t r = 0; r < ctx->bg_bc.size(); r++) {
+        if (ctx->d_bc_round[r]) (void)hipFree(ctx->d_bc_round[r]);
+        free_grid(ctx->bg_bc[r]);
+    }
+    ctx->d_bc_round.clear();
+    ctx->bg_bc.clear();
+    std::vector<std::vector<BcTask>> rounds;
+    std::vector<int> round_of(ctx->bc.size());
+    for (size_t x = 0; x < ctx->bc.size(); x++) {
+        const BcTask &t = ctx->bc[x];
+        for (size_t y = x; y-- > 0 && ctx->bc[y].block == t.block;)
+            if (bc_overlap(ctx->bc[y], t)) round_of[x] = std::max(round_of[x], round_of[y] + 1);
+        if ((int)rounds.size() <= round_of[x]) rounds.resize(round_of[x] + 1);
+        rounds[round_of[x]].push_back(t);
+    }
+    int rc = rounds.empty() ? 0 : ensure_block_table(ctx);
+    for (auto &tasks : rounds) {
+        if (rc) break;
+        std::vector<dim3> g;
+        for (const BcTask &t : tasks) g.push_back(dim3((unsigned)((std::max(bc_nodes(t), 0L) + 255) / 256)));
+        ctx->d_bc_round.push_back(nullptr);
+        ctx->bg_bc.push_back(BatchGrid());
+        rc = dev_upload(&ctx->d_bc_round.back(), tasks);
+        if (!rc) rc = make_grid(ctx->bg_bc.back(), g);
+    }
+    return rc;
+}
+
 // Block table and grids of the batched stage launches (batch_blocks).
 int build_batch(acfd_ctx *ctx)
 {
@@ -556,30 +592,6 @@ int build_batch(acfd_ctx *ctx)
     if (!rc) rc = make_grid(ctx->bg_visc, g_visc);
     if (!rc) rc = make_grid(ctx->bg_dt, g_pri);
     if (!rc) rc = make_grid(ctx->bg_prep, g_prep);
-    // physical boundary rounds; a block's subfaces keep the order of ctx->bc
-    for (size_t r = 0; r < ctx->bg_bc.size(); r++) {
-        if (ctx->d_bc_round[r]) (void)hipFree(ctx->d_bc_round[r]);
-        free_grid(ctx->bg_bc[r]);
-    }
-    ctx->d_bc_round.clear();
-    ctx->bg_bc.clear();
-    std::vector<std::vector<BcTask>> per(ctx->blk.size());
-    for (const BcTask &t : ctx->bc) per[t.block].push_back(t);
-    size_t rounds = 0;
-    for (auto &v : per) rounds = std::max(rounds, v.size());
-    for (size_t r = 0; r < rounds && !rc; r++) {
-        std::vector<BcTask> tasks;
-        std::vector<dim3> g;
-        for (auto &v : per)
-            if (r < v.size()) {
-                tasks.push_back(v[r]);
-                g.push_back(dim3((unsigned)((std::max(bc_nodes(v[r]), 0L) + 255) / 256)));
-            }
-        ctx->d_bc_round.push_back(nullptr);
-        ctx->bg_bc.push_back(BatchGrid());
-        rc = dev_upload(&ctx->d_bc_round.back(), tasks);
-        if (!rc) rc = make_grid(ctx->bg_bc.back(), g);
-    }
     ctx->batch_ready = rc == 0;
     return rc;
 }
@@ -1120,20 +1132,14 @@ int st_update_q0_all(acfd_ctx *ctx)
 int st_physical_bc(acfd_ctx *ctx)
 {
     StageTimer t(ctx, ACFD_STAGE_PHYSICAL_BC);
+    for (size_t r = 0; r < ctx->bg_bc.size(); r++)
+        KRN_TRY(launch_bc_batch(ctx->stream, ctx->d_bc_round[r], ctx->bg_bc[r], ctx->d_blocks, ctx->arena, ctx->c));
+    if (ctx->c.turb != 2 || ctx->c.solver != 0) return 0;
     if (batched(ctx)) {
-        for (size_t r = 0; r < ctx->bg_bc.size(); r++)
-            KRN_TRY(launch_bc_batch(ctx->stream, ctx->d_bc_round[r], ctx->bg_bc[r], ctx->d_blocks, ctx->arena,
-                                    ctx->c));
-        if (ctx->c.turb == 2 && ctx->c.solver == 0)
-            KRN_TRY(launch_sa_clamp_batch(ctx->stream, ctx->d_blocks, ctx->bg_getpri, ctx->arena));
+        KRN_TRY(launch_sa_clamp_batch(ctx->stream, ctx->d_blocks, ctx->bg_getpri, ctx->arena));
         return 0;
     }
-    for (const BcTask &task : ctx->bc) {
-        Block &b = ctx->blk[task.block];
-        KRN_TRY(launch_bc(ctx->stream, b.e, b.f, ctx->c, task));
-    }
-    if (ctx->c.turb == 2 && ctx->c.solver == 0)
-        for (auto &b : ctx->blk) KRN_TRY(launch_sa_clamp(ctx->stream, b.e, b.f));
+    for (auto &b : ctx->blk) KRN_TRY(launch_sa_clamp(ctx->stream, b.e, b.f));
     return 0;
 }
 
@@ -1424,11 +1430,8 @@ int one_step(acfd_ctx *ctx)
         if (!rc) rc = refresh(ctx);
         for (int m = 0; m < nb && !rc; m++) rc = st_getpri(ctx, m);
     } else if (ctx->cfg.iflag_timeadvance == 4) {
-        // explicit Shu-Osher RK3: q^n is kept in w_dqs (free in this mode)
-        for (int m = 0; m < nb; m++) {
-            const Block &b = ctx->blk[m];
-            KRN_TRY(launch_copy(ctx->stream, b.f.q, b.f.w_dqs, 5 * b.e.n));
-        }
+        // explicit Shu-Osher RK3: the first stage keeps q^n of the computed
+        // range in w_dqs (free in this mode)
         for (int stage = 0; stage < 3 && !rc; stage++) {
             if (stage > 0) rc = refresh(ctx);
             if (stagewise) {
@@ -1770,6 +1773,7 @@ int acfd_set_topology(acfd_ctx *ctx, int nblk, const int *dims, const int *nsub,
     ctx->inv_run = inviscid_run(ctx->totalnodes, ctx->cfg.precision);
     rc = alloc_lu_ws(ctx, true);
     if (!rc && ctx->cfg.iflag_timeadvance == 3) rc = ensure_block_table(ctx);
+    if (!rc) rc = build_bc_rounds(ctx);
     if (!rc) rc = build_batch(ctx);
     if (rc) return rc;
     HIP_TRY(hipStreamSynchronize(ctx->stream));

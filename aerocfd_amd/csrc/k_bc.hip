@@ -120,16 +120,9 @@ __device__ inline void bc_node(const Ext &e, const Consts &c, const BcTask &t, l
     }
 }
 
-__global__ void __launch_bounds__(256) k_bc(Ext e, Consts c, BcTask t, double *__restrict__ q,
-                                            double *__restrict__ nut, const double *__restrict__ dxidx)
-{
-    bc_node(e, c, t, (long)blockIdx.x * blockDim.x + threadIdx.x, q, nut, dxidx);
-}
-
-// One subface of each of several blocks in one launch (tasks[m] for the
-// workgroups of entry m of the grid).  Blocks touch only their own arrays,
-// so the subfaces of different blocks are independent; the subfaces of one
-// block go to successive launches, in the reference's order.
+// Independent subfaces in one launch (tasks[m] for the workgroups of entry m
+// of the grid): those of different blocks, which touch only their own
+// arrays, and those of one block that share no nodes.
 __global__ void __launch_bounds__(256) k_bc_batch(const BcTask *__restrict__ tasks, const int *__restrict__ map,
                                                   const KGrid *__restrict__ kg, const BlockRec *__restrict__ blks,
                                                   double *arena, Consts c)
@@ -149,14 +142,28 @@ long bc_nodes(const BcTask &t)
     return (long)(hi[0] - lo[0] + 1) * (hi[1] - lo[1] + 1) * (hi[2] - lo[2] + 1);
 }
 
-int launch_bc(hipStream_t s, const Ext &e, const Fields &f, const Consts &c, const BcTask &t)
+// whether two subfaces of a block have to keep their order: one writes (its
+// face) what the other reads (up to three nodes inwards) or writes
+bool bc_overlap(const BcTask &a, const BcTask &b)
 {
-    const long cnt = bc_nodes(t);
-    if (cnt <= 0) return 0;
-    int bs = 256;
-    hipLaunchKernelGGL(k_bc, dim3((unsigned)((cnt + bs - 1) / bs)), dim3(bs), 0, s, e, c, t, f.q, f.nut, f.dxidx);
-    ACFD_CHECK_LAUNCH();
-    return 0;
+    int w[2][6], r[2][6];
+    const BcTask *t[2] = {&a, &b};
+    for (int x = 0; x < 2; x++) {
+        const int axis = (t[x]->face - 1) / 2;
+        const bool minus = (t[x]->face & 1) == 1;
+        const int box[6] = {t[x]->is, t[x]->ie, t[x]->js, t[x]->je, t[x]->ks, t[x]->ke};
+        for (int d = 0; d < 6; d++) w[x][d] = r[x][d] = box[d];
+        const int fix = minus ? box[2 * axis] : box[2 * axis + 1];
+        w[x][2 * axis] = w[x][2 * axis + 1] = fix;
+        r[x][2 * axis] = minus ? fix : fix - 3;
+        r[x][2 * axis + 1] = minus ? fix + 3 : fix;
+    }
+    auto meet = [](const int *u, const int *v) {
+        for (int d = 0; d < 3; d++)
+            if (u[2 * d] > v[2 * d + 1] || v[2 * d] > u[2 * d + 1]) return false;
+        return true;
+    };
+    return meet(w[0], r[1]) || meet(r[0], w[1]);  // r holds w
 }
 
 int launch_bc_batch(hipStream_t s, const BcTask *tasks, const BatchGrid &bg, const BlockRec *blks, double *arena,

@@ -584,9 +584,9 @@ int launch_inviscid_ext(hipStream_t s, const Ext &e, const Fields &f, const Cons
 // Stage s of the Shu-Osher scheme on the computed range:
 // q = a_s qn + b_s (q + dt (rhsi + rhsv) / inv_j), (a,b) = (0,1), (3/4,1/4),
 // (1/3,2/3); the first stage also stores rhs = rhsi + rhsv (the step's
-// residual).
+// residual) and qn = q.
 __global__ void __launch_bounds__(256) k_rk3_stage(Ext e, Box b, double *__restrict__ q,
-                                                  const double *__restrict__ qn,
+                                                  double *__restrict__ qn, bool first,
                                                   const double *__restrict__ rhsi,
                                                   const double *__restrict__ rhsv, double *__restrict__ rhs,
                                                   const double *__restrict__ dt, const double *__restrict__ inv_j,
@@ -600,8 +600,10 @@ __global__ void __launch_bounds__(256) k_rk3_stage(Ext e, Box b, double *__restr
     for (int x = 0; x < 5; x++) {
         const double r = rhsv ? rhsi[x * N + n] + rhsv[x * N + n] : rhsi[x * N + n] + 0.0;
         if (rhs) rhs[x * N + n] = r;
-        const double upd = q[x * N + n] + dtn * r / ij;
-        q[x * N + n] = A * qn[x * N + n] + B * upd;
+        const double qv = q[x * N + n], upd = qv + dtn * r / ij;
+        if (first) qn[x * N + n] = qv;
+        const double q0 = first ? qv : qn[x * N + n];
+        q[x * N + n] = fma(A, q0, B * upd);
     }
 }
 
@@ -619,12 +621,12 @@ int launch_copy(hipStream_t s, const double *a, double *b, long n)
     return 0;
 }
 
-int launch_rk3_stage(hipStream_t s, const Ext &e, const Fields &f, const double *qn, int stage, bool viscous)
+int launch_rk3_stage(hipStream_t s, const Ext &e, const Fields &f, double *qn, int stage, bool viscous)
 {
     static const double A[3] = {0.0, 0.75, 1.0 / 3.0}, B[3] = {1.0, 0.25, 2.0 / 3.0};
     Box b{e.is1, e.ie1, e.js1, e.je1, e.ks1, e.ke1};
     if (b.i1 < b.i0 || b.j1 < b.j0 || b.k1 < b.k0) return 0;
-    hipLaunchKernelGGL(k_rk3_stage, box_grid(b), dim3(64, 4, 1), 0, s, e, b, f.q, qn, f.rhsi,
+    hipLaunchKernelGGL(k_rk3_stage, box_grid(b), dim3(64, 4, 1), 0, s, e, b, f.q, qn, stage == 0, f.rhsi,
                        viscous ? f.rhsv : nullptr, stage == 0 ? f.rhs : nullptr, f.dt, f.inv_j, A[stage],
                        B[stage]);
     ACFD_CHECK_LAUNCH();

@@ -24,7 +24,7 @@ int launch_reset_stats(hipStream_t s, unsigned long long *stats);
 // (scheme 1 Steger-Warming + WENO5, 2 WCNS; Shu-Osher RK3)
 int launch_inviscid_ext(hipStream_t s, const Ext &e, const Fields &f, const Consts &c, int precision, int scheme,
                         bool clear);
-int launch_rk3_stage(hipStream_t s, const Ext &e, const Fields &f, const double *qn, int stage, bool viscous);
+int launch_rk3_stage(hipStream_t s, const Ext &e, const Fields &f, double *qn, int stage, bool viscous);
 int launch_copy(hipStream_t s, const double *a, double *b, long n);
 
 // k_sensor.hip: learned WCNS sensor (training, data, inference)
@@ -190,9 +190,9 @@ struct BcTask {       // one physical subface
     int face, kind;   // kind = blk_t (-10 .. -50)
     int is, ie, js, je, ks, ke;  // loop range actually used (farfield js quirk applied)
 };
-int launch_bc(hipStream_t s, const Ext &e, const Fields &f, const Consts &c, const BcTask &t);
 int launch_sa_clamp(hipStream_t s, const Ext &e, const Fields &f);
 long bc_nodes(const BcTask &t);  // face nodes of a subface
+bool bc_overlap(const BcTask &a, const BcTask &b);  // of one block: the second has to follow the first
 // tasks[m]: one subface of block tasks[m].block, m over the grid's entries
 int launch_bc_batch(hipStream_t s, const BcTask *tasks, const BatchGrid &bg, const BlockRec *blks, double *arena,
                     const Consts &c);
