@@ -168,9 +168,8 @@ struct acfd_ctx {
     // step that did so replays only while it holds.
     bool pri_current = false;
     bool graph_needs_pri = false;
-    // the last residual stage also formed implicit1st's rhs, spectral radii
-    // and diagonal (batched, steady NS): the next batched update skips its
-    // preparation pass
+    // the last residual stage also formed implicit1st's rhs and time term
+    // (lu_fold): the update that follows skips its preparation pass
     bool lu_prep_ready = false;
     // the last residual stage formed rhs = rhsi + rhsv without storing rhsv
     // (the same fold): rhsv_refresh forms it from the node fluxes, which
@@ -875,10 +874,14 @@ int st_inviscid(acfd_ctx *ctx, int m)
     return 0;
 }
 
-int st_viscous(acfd_ctx *ctx, int m, int store_aux)
+// part 1: the node pass, 2: the difference pass, with prep_cfl also
+// implicit1st's rhs and time term (lu_fold)
+int st_viscous(acfd_ctx *ctx, int m, int store_aux, int part = -1, const double *prep_cfl = nullptr)
 {
     StageTimer t(ctx, ACFD_STAGE_VISCOUS);
-    KRN_TRY(launch_viscous(ctx->stream, ctx->blk[m].e, ctx->blk[m].f, ctx->c, ctx->cfg.precision, store_aux));
+    KRN_TRY(launch_viscous(ctx->stream, ctx->blk[m].e, ctx->blk[m].f, ctx->c, ctx->cfg.precision, store_aux, part,
+                           prep_cfl));
+    if (prep_cfl) ctx->lu_prep_ready = ctx->rhsv_stale = true;
     return 0;
 }
 
@@ -911,6 +914,23 @@ bool viscous_dt_fused_on()
         v = e && std::atoi(e) == 0 ? 0 : 1;
     }
     return v == 1;
+}
+
+// With NS and the tile sweeps the viscous difference pass of a step also
+// forms what implicit1st starts from, rhs = rhsi + rhsv and the time term,
+// and leaves rhsv out (ACFD_VISCOUS_DT_FUSED=0: passes of their own; the
+// same results either way).  find_dt, which reads the viscosity that the
+// node pass stores, then runs between the two viscous passes.
+bool lu_fold(const acfd_ctx *ctx)
+{
+    return ctx->c.solver == 0 && ctx->cfg.iflag_timeadvance == 2 && ctx->lu_variant != 0 && viscous_dt_fused_on();
+}
+
+// the cfl that block m's update reads: the one its own find_dt left (the
+// reference runs each block's find_dt, implicit1st and sa_model back to back)
+const double *update_cfl(const acfd_ctx *ctx, int m)
+{
+    return ctx->c.itime == 0 ? ctx->d_cfl : ctx->d_cfl_blk + m;
 }
 
 // The batched SA update moves its sweep operands into a sweep layout
@@ -955,12 +975,12 @@ void sl_invalidate(acfd_ctx *ctx)
     ctx->sl_block = -2;
 }
 
-int st_implicit(acfd_ctx *ctx, int m, const double *cfl)
+int st_implicit(acfd_ctx *ctx, int m, const double *cfl, bool prep_ready = false)
 {
     StageTimer t(ctx, ACFD_STAGE_IMPLICIT1ST);
     Block &b = ctx->blk[m];
     const int variant = ctx->lu_variant;
-    for (int ph = 0; ph < kLusgsPhases; ph++) {
+    for (int ph = prep_ready ? 1 : 0; ph < kLusgsPhases; ph++) {
         StageTimer ts(ctx, ph == 2 ? kTimeLuForward : ph == 3 ? kTimeLuBackward
                            : ph == 1 ? kTimeLuGather : ph == 4 ? kTimeLuAdd : kTimeLuOther);
         KRN_TRY(launch_lusgs_phase(ctx->stream, b.e, b.f, ctx->c, cfl, variant, &ctx->lu, ph,
@@ -983,16 +1003,16 @@ constexpr bool kBatchedUpdateWritesDq = false;
 int st_implicit_all(acfd_ctx *ctx, const double *cfl_per_block)
 {
     const int nb = (int)ctx->blk.size();
+    const bool prep_ready = ctx->lu_prep_ready;
+    ctx->lu_prep_ready = false;
     if (ctx->lu_variant != 2) {
         for (int m = 0; m < nb; m++) {
-            int rc = st_implicit(ctx, m, cfl_per_block ? cfl_per_block + m : ctx->d_cfl);
+            int rc = st_implicit(ctx, m, cfl_per_block ? cfl_per_block + m : ctx->d_cfl, prep_ready);
             if (rc) return rc;
         }
         return 0;
     }
     StageTimer t(ctx, ACFD_STAGE_IMPLICIT1ST);
-    const bool prep_ready = ctx->lu_prep_ready;
-    ctx->lu_prep_ready = false;
     if (prep_ready) {
         // formed by the residual's viscous passes
     } else if (batched(ctx)) {
@@ -1170,9 +1190,11 @@ int refresh(acfd_ctx *ctx)
 int residual_stage(acfd_ctx *ctx, int m, int store_aux, bool pri_ok = false)
 {
     int rc = pri_ok ? 0 : st_getpri(ctx, m);
+    const bool fold = lu_fold(ctx);
     if (!rc) rc = st_inviscid(ctx, m);
-    if (!rc && ctx->c.solver == 0) rc = st_viscous(ctx, m, store_aux);
+    if (!rc && ctx->c.solver == 0) rc = st_viscous(ctx, m, store_aux, fold ? 1 : -1);
     if (!rc) rc = st_find_dt(ctx, m);
+    if (!rc && fold) rc = st_viscous(ctx, m, store_aux, 2, update_cfl(ctx, m));
     return rc;
 }
 
@@ -1224,26 +1246,30 @@ int st_inviscid_all(acfd_ctx *ctx)
     return 0;
 }
 
-int st_viscous_all(acfd_ctx *ctx, int store_aux)
+int st_viscous_all(acfd_ctx *ctx, int store_aux, int only = -1, bool fold = false)
 {
     if (!batched(ctx)) {
         for (int m = 0; m < (int)ctx->blk.size(); m++) {
-            int rc = st_viscous(ctx, m, store_aux);
+            int rc = st_viscous(ctx, m, store_aux, only, fold ? update_cfl(ctx, m) : nullptr);
             if (rc) return rc;
         }
         return 0;
     }
     StageTimer t(ctx, ACFD_STAGE_VISCOUS);
+    // (steady: the fold is st_viscous_dt_all's)
+    const double *prep_cfl = fold ? ctx->d_cfl_blk : nullptr;
+    if (fold) ctx->lu_prep_ready = ctx->rhsv_stale = true;
     if (ctx->timing) {
         for (int part = 1; part <= 2; part++) {
+            if (only > 0 && part != only) continue;
             StageTimer ts(ctx, part == 1 ? kTimeViscNode : kTimeViscDiff);
             KRN_TRY(launch_viscous_batch(ctx->stream, ctx->d_blocks, ctx->bg_visc, ctx->arena, ctx->c,
-                                         ctx->cfg.precision, store_aux, part));
+                                         ctx->cfg.precision, store_aux, part, prep_cfl));
         }
         return 0;
     }
     KRN_TRY(launch_viscous_batch(ctx->stream, ctx->d_blocks, ctx->bg_visc, ctx->arena, ctx->c, ctx->cfg.precision,
-                                 store_aux));
+                                 store_aux, only, prep_cfl));
     return 0;
 }
 
@@ -1273,7 +1299,7 @@ int st_viscous_dt_all(acfd_ctx *ctx, int store_aux, int parts = -1)
     const int nb = (int)ctx->blk.size();
     // the batched LU-SGS update's time term and rhs come from these two
     // passes too (implicit1st then skips its own preparation)
-    const int prep = ctx->cfg.lusgs_kernel == 2 && ctx->cfg.iflag_timeadvance == 2 ? 1 : 0;
+    const int prep = lu_fold(ctx) ? 1 : 0;
     if (parts >= 0) {
         if (parts == 1) KRN_TRY(launch_reset_stats(ctx->stream, ctx->d_stats));
         KRN_TRY(launch_viscous_dt_batch(ctx->stream, ctx->d_blocks, nb, ctx->bg_visc, ctx->arena, ctx->c,
@@ -1305,6 +1331,10 @@ int rhsv_refresh(acfd_ctx *ctx)
 {
     if (!ctx->rhsv_stale) return 0;
     ctx->rhsv_stale = false;
+    if (!batched(ctx)) {
+        for (auto &b : ctx->blk) KRN_TRY(launch_viscous(ctx->stream, b.e, b.f, ctx->c, ctx->cfg.precision, 0, 2));
+        return 0;
+    }
     KRN_TRY(launch_viscous_batch(ctx->stream, ctx->d_blocks, ctx->bg_visc, ctx->arena, ctx->c, ctx->cfg.precision, 0,
                                  2));
     return 0;
@@ -1331,8 +1361,10 @@ int residual_stage_all(acfd_ctx *ctx, int store_aux, bool pri_ok = false)
     }
     if (!rc) rc = st_inviscid_all(ctx);
     if (!rc && fused) return st_viscous_dt_all(ctx, store_aux);
-    if (!rc && ctx->c.solver == 0) rc = st_viscous_all(ctx, store_aux);
+    const bool fold = lu_fold(ctx);
+    if (!rc && ctx->c.solver == 0) rc = st_viscous_all(ctx, store_aux, fold ? 1 : -1);
     if (!rc) rc = st_find_dt_all(ctx);
+    if (!rc && fold) rc = st_viscous_all(ctx, store_aux, 2, true);
     return rc;
 }
 
@@ -1362,10 +1394,9 @@ int one_step(acfd_ctx *ctx)
     const int aux = sa ? (ctx->c.des == 2 ? 2 : 1) : 0;
     const int nb = (int)ctx->blk.size();
     int rc = 0;
-    // block m's update reads the cfl its own find_dt left (the reference
-    // runs each block's find_dt, implicit1st and sa_model back to back)
-    const double *cfl = ctx->c.itime == 0 ? nullptr : ctx->d_cfl_blk;
-    auto cfl_of = [&](int m) { return cfl ? cfl + m : ctx->d_cfl; };
+    const double *cfl = ctx->c.itime == 0 ? nullptr : ctx->d_cfl_blk;  // one a block (update_cfl)
+    auto cfl_of = [&](int m) { return update_cfl(ctx, m); };
+    ctx->lu_prep_ready = false;
     const bool stagewise = ctx->cfg.batch_blocks || ctx->cfg.lusgs_kernel == 2;
     // pri_v of every block is getpri of its q when the last step's closing
     // getpri is the latest write (a block's q changes only in its own update,
@@ -1411,7 +1442,9 @@ int one_step(acfd_ctx *ctx)
     } else if (ctx->cfg.iflag_timeadvance == 2) {
         for (int m = 0; m < nb && !rc; m++) {
             rc = residual_stage(ctx, m, aux, pri_ok);
-            if (!rc) rc = st_implicit(ctx, m, cfl_of(m));
+            const bool ready = ctx->lu_prep_ready;
+            ctx->lu_prep_ready = false;
+            if (!rc) rc = st_implicit(ctx, m, cfl_of(m), ready);
             if (!rc && sa) rc = st_sa(ctx, m, cfl_of(m));
         }
         if (!rc) rc = refresh(ctx);

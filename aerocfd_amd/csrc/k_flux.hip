@@ -505,11 +505,17 @@ __global__ void __launch_bounds__(256) k_viscous_node(Ext e, Consts c, const dou
 // Stage 2 (sub_viscous.f90:296-365): rhsv = (d/dxi fv + d/deta gv + d/dzeta hv)/re;
 // with rhsi given, also rhs = rhsi + rhsv on the computed range (the
 // first line of implicit1st, sub_timeadvancement_1stimplicit.f90:72-78),
-// and with rhsv null only rhs
+// and with rhsv null only rhs; with diag given, implicit1st's time term
+// phi*1/dt there too (:98-102,151, as lu_prep_body forms it for the tile
+// sweeps).  Bound by memory: for a context that updates with the tile sweeps
+// this replaces storing rhsv, and a pass (lu_prep) that read it and rhsi and
+// wrote rhs and the time term.  Viscous stage and that pass, before and
+// after: 33^3 26.7 -> 23.2 us, 129^3 294 -> 268, 193^3 910 -> 809.
 template <typename S>
 __device__ inline void viscous_diff_body(const Ext &e, long wg, const S *__restrict__ w,
                                          double *__restrict__ rhsv, double re, const double *__restrict__ rhsi = nullptr,
-                                         double *__restrict__ rhs = nullptr)
+                                         double *__restrict__ rhs = nullptr, const double *__restrict__ dt = nullptr,
+                                         double *__restrict__ diag = nullptr, const double *cfl = nullptr)
 {
     const Box b{e.is0, e.ie0, e.js0, e.je0, e.ks0, e.ke0};
     int i, j, k;
@@ -522,6 +528,10 @@ __device__ inline void viscous_diff_body(const Ext &e, long wg, const S *__restr
     const double v0 = (0.0 + 0.0 + 0.0) / re;
     if (rhsv) st_out(rhsv + n, v0);
     if (inner) st_out(rhs + n, ld_once(rhsi + n) + v0);
+    if (inner && diag) {
+        const double phi = *cfl >= 1.0e3 ? 0.0 : 1.0;
+        diag[n] = phi * 1.0 / dt[n];
+    }
 #pragma unroll
     for (int c = 0; c < 4; c++) {
         double a = ndiff(w + (0 + c) * N, n, 1, i, e.is0, e.ie0);
@@ -541,6 +551,17 @@ __global__ void __launch_bounds__(256) k_viscous_diff(Ext e, const double *__res
     viscous_diff_body<S>(e, xcd_slab(blockIdx.x, gridDim.x), reinterpret_cast<const S *>(w), rhsv, re);
 }
 
+// with implicit1st's rhs and time term, rhsv not stored
+template <typename S>
+__global__ void __launch_bounds__(256) k_viscous_diff_prep(Ext e, const double *__restrict__ w, double re,
+                                                           const double *__restrict__ rhsi, double *__restrict__ rhs,
+                                                           const double *__restrict__ dt, double *__restrict__ diag,
+                                                           const double *cfl)
+{
+    viscous_diff_body<S>(e, xcd_slab(blockIdx.x, gridDim.x), reinterpret_cast<const S *>(w), nullptr, re, rhsi, rhs, dt,
+                         diag, cfl);
+}
+
 template <typename R>
 __global__ void __launch_bounds__(256) k_viscous_node_batch(const BlockRec *__restrict__ blks,
                                                             const int *__restrict__ map,
@@ -555,21 +576,23 @@ __global__ void __launch_bounds__(256) k_viscous_node_batch(const BlockRec *__re
                          store_aux);
 }
 
-// with_rhs 1: also rhs = rhsi + rhsv on the computed range; 2: rhs only
-// (rhsv not stored); S: the storage type of the node fluxes
+// with_rhs 2: rhs = rhsi + rhsv on the computed range instead of rhsv; 3:
+// and the time term, block m with cfl[m]; S: the storage type of the node
+// fluxes
 template <typename S>
 __global__ void __launch_bounds__(256) k_viscous_diff_batch(const BlockRec *__restrict__ blks,
                                                             const int *__restrict__ map,
                                                             const KGrid *__restrict__ kg, double *arena, double re,
-                                                            int with_rhs = 0)
+                                                            int with_rhs, const double *cfl)
 {
     int bx, by, bz;
-    const BlockRec &b = blks[batch_wg(map, kg, bx, by, bz)];
+    const int m = batch_wg(map, kg, bx, by, bz);
+    const BlockRec &b = blks[m];
     const Ext e = b.e;
     const S *w = reinterpret_cast<const S *>(arena + b.o.w_flux);
     if (with_rhs)
-        viscous_diff_body<S>(e, bx, w, with_rhs == 2 ? nullptr : arena + b.o.rhsv, re, arena + b.o.rhsi,
-                             arena + b.o.rhs);
+        viscous_diff_body<S>(e, bx, w, nullptr, re, arena + b.o.rhsi, arena + b.o.rhs, arena + b.o.dt,
+                             with_rhs == 3 ? arena + b.o.w_diag : nullptr, cfl + m);
     else viscous_diff_body<S>(e, bx, w, arena + b.o.rhsv, re);
 }
 
@@ -578,26 +601,35 @@ __global__ void __launch_bounds__(256) k_viscous_diff_batch(const BlockRec *__re
 dim3 viscous_grid(const Ext &e) { return lin_grid(e); }
 
 int launch_viscous(hipStream_t s, const Ext &e, const Fields &f, const Consts &c, int precision,
-                   int store_aux)
+                   int store_aux, int part, const double *prep_cfl)
 {
     dim3 g = viscous_grid(e), t(64, 4, 1);
-    if (precision == 1)
+    if (part == 2) {
+    } else if (precision == 1)
         hipLaunchKernelGGL((k_viscous_node<float>), g, t, 0, s, e, c, f.pri, f.amu, f.dxidx, f.inv_j, f.w_flux,
                            f.vor, f.dudx, f.tao, store_aux);
     else
         hipLaunchKernelGGL((k_viscous_node<double>), g, t, 0, s, e, c, f.pri, f.amu, f.dxidx, f.inv_j, f.w_flux,
                            f.vor, f.dudx, f.tao, store_aux);
-    if (precision == 1) hipLaunchKernelGGL(k_viscous_diff<float>, g, t, 0, s, e, f.w_flux, f.rhsv, c.re);
+    if (part == 1) {
+    } else if (prep_cfl && precision == 1)
+        hipLaunchKernelGGL(k_viscous_diff_prep<float>, g, t, 0, s, e, f.w_flux, c.re, f.rhsi, f.rhs, f.dt, f.w_diag,
+                           prep_cfl);
+    else if (prep_cfl)
+        hipLaunchKernelGGL(k_viscous_diff_prep<double>, g, t, 0, s, e, f.w_flux, c.re, f.rhsi, f.rhs, f.dt, f.w_diag,
+                           prep_cfl);
+    else if (precision == 1) hipLaunchKernelGGL(k_viscous_diff<float>, g, t, 0, s, e, f.w_flux, f.rhsv, c.re);
     else hipLaunchKernelGGL(k_viscous_diff<double>, g, t, 0, s, e, f.w_flux, f.rhsv, c.re);
     ACFD_CHECK_LAUNCH();
     return 0;
 }
 
 int launch_viscous_batch(hipStream_t s, const BlockRec *blks, const BatchGrid &bg, double *arena, const Consts &c,
-                         int precision, int store_aux, int part)
+                         int precision, int store_aux, int part, const double *prep_cfl)
 {
     if (bg.total <= 0) return 0;
     dim3 g((unsigned)bg.total), t(64, 4, 1);
+    const int with_rhs = prep_cfl ? 3 : 0;
     if (part < 0 || part == 1) {
         if (precision == 1)
             hipLaunchKernelGGL((k_viscous_node_batch<float>), g, t, 0, s, blks, bg.map, bg.kg, arena, c, store_aux);
@@ -606,9 +638,11 @@ int launch_viscous_batch(hipStream_t s, const BlockRec *blks, const BatchGrid &b
     }
     if (part < 0 || part == 2) {
         if (precision == 1)
-            hipLaunchKernelGGL(k_viscous_diff_batch<float>, g, t, 0, s, blks, bg.map, bg.kg, arena, c.re, 0);
+            hipLaunchKernelGGL(k_viscous_diff_batch<float>, g, t, 0, s, blks, bg.map, bg.kg, arena, c.re, with_rhs,
+                               prep_cfl);
         else
-            hipLaunchKernelGGL(k_viscous_diff_batch<double>, g, t, 0, s, blks, bg.map, bg.kg, arena, c.re, 0);
+            hipLaunchKernelGGL(k_viscous_diff_batch<double>, g, t, 0, s, blks, bg.map, bg.kg, arena, c.re, with_rhs,
+                               prep_cfl);
     }
     ACFD_CHECK_LAUNCH();
     return 0;
@@ -822,9 +856,11 @@ int launch_viscous_dt_batch(hipStream_t s, const BlockRec *blks, int nblk, const
     }
     if (part < 0 || part == 2) {
         if (precision == 1)
-            hipLaunchKernelGGL(k_viscous_diff_batch<float>, g, t, 0, s, blks, bg.map, bg.kg, arena, c.re, 2 * prep);
+            hipLaunchKernelGGL(k_viscous_diff_batch<float>, g, t, 0, s, blks, bg.map, bg.kg, arena, c.re, 2 * prep,
+                               nullptr);
         else
-            hipLaunchKernelGGL(k_viscous_diff_batch<double>, g, t, 0, s, blks, bg.map, bg.kg, arena, c.re, 2 * prep);
+            hipLaunchKernelGGL(k_viscous_diff_batch<double>, g, t, 0, s, blks, bg.map, bg.kg, arena, c.re, 2 * prep,
+                               nullptr);
     }
     ACFD_CHECK_LAUNCH();
     return 0;

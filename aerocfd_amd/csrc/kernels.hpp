@@ -12,8 +12,10 @@ int launch_fill(hipStream_t s, double *p, long n, double v);
 // clear: rhsi may not be zero outside the computed range
 int launch_inviscid(hipStream_t s, const Ext &e, const Fields &f, const Consts &c, int precision, int run, bool clear);
 int inviscid_run(long nodes, int precision);
+// part 1, 2: only the node, the difference pass; prep_cfl: that pass forms implicit1st's
+// rhs and (with the cfl it points to) time term and stores no rhsv
 int launch_viscous(hipStream_t s, const Ext &e, const Fields &f, const Consts &c, int precision,
-                   int store_aux);
+                   int store_aux, int part = -1, const double *prep_cfl = nullptr);
 // unsteady: the local cfl of the block's last node goes to *cfl and, when
 // not null, *cfl_blk
 int launch_find_dt(hipStream_t s, const Ext &e, const Fields &f, const Consts &c, double *cfl, double *cfl_blk,
@@ -72,7 +74,7 @@ int launch_getpri_batch(hipStream_t s, const BlockRec *blks, const BatchGrid &bg
 int launch_inviscid_batch(hipStream_t s, const BlockRec *blks, const BatchGrid *bg, double *arena,
                           const Consts &c, int precision, int run, int part = -1);
 int launch_viscous_batch(hipStream_t s, const BlockRec *blks, const BatchGrid &bg, double *arena, const Consts &c,
-                         int precision, int store_aux, int part = -1);
+                         int precision, int store_aux, int part = -1, const double *prep_cfl = nullptr);
 // the viscous stage with the steady find_dt folded into its node pass
 // (statistics into stats from the last block; reset them first); with
 // prep, also what launch_lu_prep_batch forms for the tile sweeps: the time
