@@ -366,13 +366,6 @@ __device__ inline void xstore(double *p, double v)
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// LDS barrier that does not wait for outstanding global loads (the
-// prefetched operands stay in flight across it)
-__device__ inline void lds_barrier()
-{
-    __asm__ volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
-
 // The layout passes move data between the natural layout (i fastest) and
 // the sweep layout through LDS.  One workgroup per tile walks the tile's
 // steps in chunks of CT steps, one field pair at a time through all the
@@ -1133,33 +1126,39 @@ static SaGeom sa_geom(const Ext &e)
     return g;
 }
 
-__device__ inline double ex_take1(double *slot, unsigned long long pre, int *err, bool &failed)
+// a node's new value from the neighbours' (every product and sum rounded by
+// itself, as the published sweep's results have them)
+template <int DIR>
+__device__ inline double sa_node(const double *op, double vi, double vj, double vk)
 {
-    unsigned long long b = pre;
-    if (b == kSentinel) {
-        for (long spins = 0; !failed; spins++) {
-            b = xload_bits(slot);
-            if (b != kSentinel) break;
-            if ((spins & 1023) == 1023 &&
-                (spins > (1L << 21) || __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) {
-                atomicOr(err, 1);
-                failed = true;
-            }
-            __builtin_amdgcn_s_sleep(1);
-        }
-        if (failed) b = 0;
-    }
-    xstore_bits(slot, kSentinel);
-    return __longlong_as_double((long long)b);
+#pragma clang fp contract(off)
+    const LuDivisor dg = lu_divisor(op[3]);
+    const double a = DIR > 0 ? fabs(op[0]) : -fabs(op[0]), b = DIR > 0 ? fabs(op[1]) : -fabs(op[1]),
+                 c = DIR > 0 ? fabs(op[2]) : -fabs(op[2]);
+    const double ta = 0.5 * (op[0] + a) * vi, tb = 0.5 * (op[1] + b) * vj, tc = 0.5 * (op[2] + c) * vk;
+    const double t = ta + tb + tc;
+    return DIR > 0 ? lu_over(op[4] + t, dg) : op[4] - lu_over(t, dg);
 }
 
-// cu = a, b, c, diag (component stride N); fwd reads rhs and writes dns,
-// bwd reads dns and writes dn
-template <int DIR>
-__device__ inline void sa_tiles_body(const Ext &e, const SaGeom &g, int tile, const double *__restrict__ cu,
-                                     const double *__restrict__ rhs, double *__restrict__ dns,
-                                     double *__restrict__ dn, double *ex, int *err, double (*pj)[kLanes],
-                                     double (*pk)[kLanes])
+// The scalar sweep of one tile by one wavefront.  IO gives the operands a,
+// b, c, diag and rhs / dn* of a step and takes its result.
+//
+// What bounds it: the steps in a row (Li + Lj + Lk of them from corner to
+// corner of a block, a hop through memory at every tile edge).  A step used
+// to take 0.64 us, its operands' latency, as they were read one step ahead
+// and the lanes met through LDS; now they are read kSaAhead steps ahead,
+// the exchange slots kSaSlotAhead (a slot read earlier than the neighbour
+// writes it is polled for), values pass to the next lanes by DPP (j) and
+// ds_bpermute (k), and the one division is a product and two fused
+// operations on the chain (the quotient is the same).  Forward / backward
+// sweep, 12 blocks of 3.2 M nodes in all: 206 / 182 us before, 173 / 154
+// now; 24 blocks of 8 M nodes 234 / 203, now 216 / 186.  Steps and slots
+// ahead, the 12 blocks: 4, 2 182 / 156; 4, 4 176 / 160; 6, 6 185 / 170; 8, 4
+// 175 / 160.
+constexpr int kSaOps = 5;  // a, b, c, diag, rhs / dn*
+constexpr int kSaAhead = 6, kSaSlotAhead = 3;
+template <int DIR, class IO>
+__device__ inline void sa_sweep_body(const SaGeom &g, int tile, const IO &io, double *ex, int *err)
 {
     const int bj = tile % g.nbj, bk = tile / g.nbj;
     const int l = threadIdx.x, tj = l % kTile, tk = l / kTile;
@@ -1168,94 +1167,117 @@ __device__ inline void sa_tiles_body(const Ext &e, const SaGeom &g, int tile, co
     const int sj = DIR > 0 ? tj : kTile - 1 - tj, sk = DIR > 0 ? tk : kTile - 1 - tk;
     const bool j_ring = DIR > 0 ? lj == 0 : lj + 1 >= g.Lj;
     const bool k_ring = DIR > 0 ? lk == 0 : lk + 1 >= g.Lk;
-    const bool j_in = !j_ring && sj == 0, k_in = !k_ring && sk == 0;
-    const int lpj = l - DIR, lpk = l - DIR * kTile;
-    const bool j_out = sj == kTile - 1 && (DIR > 0 ? bj + 1 < g.nbj : bj > 0);
-    const bool k_out = sk == kTile - 1 && (DIR > 0 ? bk + 1 < g.nbk : bk > 0);
+    const bool j_in = active && !j_ring && sj == 0, k_in = active && !k_ring && sk == 0;
+    const bool j_out = active && sj == kTile - 1 && (DIR > 0 ? bj + 1 < g.nbj : bj > 0);
+    const bool k_out = active && sk == kTile - 1 && (DIR > 0 ? bk + 1 < g.nbk : bk > 0);
     double *exj = ex, *exk = ex + (long)g.ntiles * g.exj_tile;
-    double *jin = exj + (long)(DIR > 0 ? tile - 1 : tile + 1) * g.exj_tile + tk;
-    double *kin = exk + (long)(DIR > 0 ? tile - g.nbj : tile + g.nbj) * g.exk_tile + tj;
-    double *jout = exj + (long)tile * g.exj_tile + tk;
-    double *kout = exk + (long)tile * g.exk_tile + tj;
     // every lane of a tile with a neighbour on that side loads the face
-    // lanes' slot run of the step; only the face lanes use it
+    // lanes' slot run of the step (one contiguous run per load); only the
+    // face lanes use it
     const bool j_pred = DIR > 0 ? bj > 0 : bj + 1 < g.nbj;
     const bool k_pred = DIR > 0 ? bk > 0 : bk + 1 < g.nbk;
-    const double *jsrc = j_pred ? jin : ex;
-    const double *ksrc = k_pred ? kin : ex;
-    const int xj_last = g.Li + kTile - 2, xk_last = g.Li + kTile - 2;
-    const long N = e.n;
-    // first node of the lane's line in sweep order (inactive lanes read a
-    // valid node and ignore it)
-    const int cj = min(lj, g.Lj - 1), ck = min(lk, g.Lk - 1);
-    const long n0 = e.ix(e.is1, e.js1 + cj, e.ks1 + ck);
-    const double *src = DIR > 0 ? rhs : dns;
-    double *out = DIR > 0 ? dns : dn;
+    double *jin = j_pred ? exj + (long)(DIR > 0 ? tile - 1 : tile + 1) * g.exj_tile + tk : ex;
+    double *kin = k_pred ? exk + (long)(DIR > 0 ? tile - g.nbj : tile + g.nbj) * g.exk_tile + tj : ex;
+    double *jout = exj + (long)tile * g.exj_tile + tk;
+    double *kout = exk + (long)tile * g.exk_tile + tj;
+    const int x_last = g.Li + kTile - 2;
+    const int behind_k = 4 * (l - DIR * kTile);
     bool failed = false;
     double vi = 0.0;
-    // operands of step s: a, b, c, diag, rhs / dn*, and the exchange bits
-    auto fetch = [&](int s, double *op, unsigned long long &xj, unsigned long long &xk) {
-        const int pos = min(max(s - sj - sk, 0), g.Li - 1);
-        const long n = n0 + (DIR > 0 ? pos : g.Li - 1 - pos);
-        op[0] = cu[n];
-        op[1] = cu[N + n];
-        op[2] = cu[2 * N + n];
-        op[3] = cu[3 * N + n];
-        op[4] = src[n];
-        const int dj = j_pred ? min(max(s, 0), xj_last) : 0;
-        const int dk = k_pred ? min(max(s, 0), xk_last) : 0;
-        xj = xload_bits(jsrc + (long)dj * kTile);
-        xk = xload_bits(ksrc + (long)dk * kTile);
+    auto fetch_slots = [&](int s, unsigned long long &xj, unsigned long long &xk) {
+        const long d = (long)min(s, x_last) * kTile;
+        xj = xload_bits(jin + (j_pred ? d : 0));
+        xk = xload_bits(kin + (k_pred ? d : 0));
     };
     auto step = [&](int s, const double *op, unsigned long long xj, unsigned long long xk) {
-        const int par = s & 1;
         const int pos = s - sj - sk;
-        if (active && pos >= 0 && pos < g.Li) {
-            const long n = n0 + (DIR > 0 ? pos : g.Li - 1 - pos);
-            const double vj = j_ring ? 0.0 : j_in ? ex_take1(jin + (long)(pos + sk) * kTile, xj, err, failed)
-                                                  : pj[par ^ 1][lpj];
-            const double vk = k_ring ? 0.0 : k_in ? ex_take1(kin + (long)(pos + sj) * kTile, xk, err, failed)
-                                                  : pk[par ^ 1][lpk];
-            double res;
-            if (DIR > 0) {
-                const double ta = 0.5 * (op[0] + fabs(op[0])) * vi;
-                const double tb = 0.5 * (op[1] + fabs(op[1])) * vj;
-                const double tc = 0.5 * (op[2] + fabs(op[2])) * vk;
-                res = (op[4] + (ta + tb + tc)) / op[3];
-            } else {
-                const double ta = 0.5 * (op[0] - fabs(op[0])) * vi;
-                const double tb = 0.5 * (op[1] - fabs(op[1])) * vj;
-                const double tc = 0.5 * (op[2] - fabs(op[2])) * vk;
-                res = op[4] - (ta + tb + tc) / op[3];
+        const bool on = active && pos >= 0 && pos < g.Li;
+        const bool take_j = on && j_in, take_k = on && k_in;
+        bool wait_j = take_j && xj == kSentinel, wait_k = take_k && xk == kSentinel;
+        if (__builtin_amdgcn_ballot_w64(wait_j || wait_k)) {
+            for (long spins = 0; !failed; spins++) {
+                if (wait_j) xj = xload_bits(jin + (long)s * kTile);
+                if (wait_k) xk = xload_bits(kin + (long)s * kTile);
+                wait_j = wait_j && xj == kSentinel;
+                wait_k = wait_k && xk == kSentinel;
+                if (!__builtin_amdgcn_ballot_w64(wait_j || wait_k)) break;
+                if ((spins & 1023) == 1023 &&
+                    (spins > (1L << 21) || __builtin_amdgcn_readfirstlane(__hip_atomic_load(
+                                               err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)))) {
+                    if (l == 0) atomicOr(err, 1);
+                    failed = true;
+                }
+                __builtin_amdgcn_s_sleep(1);
             }
-            out[n] = res;
-            vi = res;
-            pj[par][l] = res;
-            pk[par][l] = res;
+            if (wait_j) xj = 0;
+            if (wait_k) xk = 0;
+        }
+        if (take_j) xstore_bits(jin + (long)s * kTile, kSentinel);
+        if (take_k) xstore_bits(kin + (long)s * kTile, kSentinel);
+        const double nj = lane_behind_j<DIR>(vi), nk = lane_from(behind_k, vi);
+        const double vj = j_ring ? 0.0 : j_in ? __longlong_as_double((long long)xj) : nj;
+        const double vk = k_ring ? 0.0 : k_in ? __longlong_as_double((long long)xk) : nk;
+        const double res = sa_node<DIR>(op, vi, vj, vk);
+        vi = on ? res : 0.0;
+        if (on) {
+            io.store(s, pos, res);
             if (j_out) xstore(jout + (long)(pos + sk) * kTile, res);
             if (k_out) xstore(kout + (long)(pos + sj) * kTile, res);
         }
-        lds_barrier();
     };
-    double opA[5], opB[5];
-    unsigned long long xjA, xkA, xjB, xkB;
-    fetch(0, opA, xjA, xkA);
-    for (int s = 0; s < g.nsteps; s += 2) {
-        fetch(s + 1, opB, xjB, xkB);
-        step(s, opA, xjA, xkA);
-        fetch(s + 2, opA, xjA, xkA);
-        step(s + 1, opB, xjB, xkB);
+    double op[kSaAhead][kSaOps];
+    unsigned long long xj[kSaAhead], xk[kSaAhead];
+#pragma unroll
+    for (int u = 0; u < kSaAhead; u++) io.load(u, u - sj - sk, op[u]);
+#pragma unroll
+    for (int u = 0; u < kSaSlotAhead; u++) fetch_slots(u, xj[u], xk[u]);
+    // (steps past the last find every lane off)
+    for (int s = 0; s < g.nsteps; s += kSaAhead) {
+#pragma unroll
+        for (int u = 0; u < kSaAhead; u++) {
+            constexpr int A = kSaAhead;
+            fetch_slots(s + u + kSaSlotAhead, xj[(u + kSaSlotAhead) % A], xk[(u + kSaSlotAhead) % A]);
+            step(s + u, op[u], xj[u], xk[u]);
+            io.load(s + u + A, s + u + A - sj - sk, op[u]);
+        }
     }
 }
+
+// operands and results in place, one i-line of a block per lane: cu = a, b,
+// c, diag (component stride N); forward reads rhs and writes dns, backward
+// reads dns and writes dn
+template <int DIR>
+struct SaInPlace {
+    const double *cu, *src;
+    double *out;
+    long N, n0;  // n0: the lane's first node in storage (a valid one on inactive lanes)
+    int Li;
+    __device__ SaInPlace(const Ext &e, const SaGeom &g, int tile, const double *c, const double *rhs, double *dns,
+                         double *dn)
+        : cu(c), src(DIR > 0 ? rhs : dns), out(DIR > 0 ? dns : dn), N(e.n), Li(g.Li)
+    {
+        const int l = threadIdx.x;
+        n0 = e.ix(e.is1, e.js1 + min(tile % g.nbj * kTile + l % kTile, g.Lj - 1),
+                  e.ks1 + min(tile / g.nbj * kTile + l / kTile, g.Lk - 1));
+    }
+    __device__ long node(int pos) const { return n0 + (DIR > 0 ? pos : Li - 1 - pos); }
+    __device__ void load(int, int pos, double *op) const
+    {
+        const long n = node(min(max(pos, 0), Li - 1));
+#pragma unroll
+        for (int f = 0; f < 4; f++) op[f] = cu[f * N + n];
+        op[4] = src[n];
+    }
+    __device__ void store(int, int pos, double v) const { out[node(pos)] = v; }
+};
 
 template <int DIR>
 __global__ void __launch_bounds__(kLanes) k_sa_tiles(Ext e, SaGeom g, const double *__restrict__ cu,
                                                       const double *__restrict__ rhs, double *__restrict__ dns,
                                                       double *__restrict__ dn, double *ex, int *err)
 {
-    __shared__ double pj[2][kLanes], pk[2][kLanes];
     const int tile = DIR > 0 ? (int)blockIdx.x : g.ntiles - 1 - (int)blockIdx.x;
-    sa_tiles_body<DIR>(e, g, tile, cu, rhs, dns, dn, ex, err, pj, pk);
+    sa_sweep_body<DIR>(g, tile, SaInPlace<DIR>(e, g, tile, cu, rhs, dns, dn), ex, err);
 }
 
 struct SaBatchEnt {
@@ -1273,7 +1295,6 @@ __global__ void __launch_bounds__(kLanes) k_sa_tiles_batch(const SaBatchEnt *__r
                                                             int resident, double *arena, double *exb, int *err,
                                                             int *ctr)
 {
-    __shared__ double pj[2][kLanes], pk[2][kLanes];
     __shared__ int ticket;
     if (!resident) {
         if (threadIdx.x == 0)
@@ -1284,9 +1305,10 @@ __global__ void __launch_bounds__(kLanes) k_sa_tiles_batch(const SaBatchEnt *__r
     const SaBatchEnt &b = ents[tile_ent[flat]];
     const Ext e = b.e;
     const SaGeom g = b.g;
-    const int local = flat - b.tile0;
-    sa_tiles_body<DIR>(e, g, DIR > 0 ? local : g.ntiles - 1 - local, arena + b.cu, arena + b.rhs,
-                               arena + b.dns, arena + b.dn, exb + b.ex, err, pj, pk);
+    const int local = flat - b.tile0, tile = DIR > 0 ? local : g.ntiles - 1 - local;
+    sa_sweep_body<DIR>(g, tile,
+                       SaInPlace<DIR>(e, g, tile, arena + b.cu, arena + b.rhs, arena + b.dns, arena + b.dn),
+                       exb + b.ex, err);
     if (!resident && threadIdx.x == 0 &&
         __hip_atomic_fetch_add(ctr + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == total - 1) {
         __hip_atomic_store(ctr, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1304,8 +1326,6 @@ __global__ void __launch_bounds__(kLanes) k_sa_tiles_batch(const SaBatchEnt *__r
 // s reads row nsteps-1-s for every lane (its skewed clock runs the same
 // rows in reverse).  The forward sweep leaves dnut* in the rhs operand's
 // slot and the backward sweep dnut there; a last pass adds it to nut.
-constexpr int kSaOps = 5;
-
 __host__ __device__ inline long sa_slot(const SaGeom &g, int tile, int t, int f, int l)
 {
     return (((long)tile * g.nsteps + t) * kSaOps + f) * kLanes + l;
@@ -1402,98 +1422,31 @@ __global__ void __launch_bounds__(kLanes) k_sa_layout_batch(const SaBatchEnt *__
                           (int)blockIdx.y / parts, (int)blockIdx.y % parts, parts, buf);
 }
 
-// The scalar sweep of sa_tiles_body with its operands in the SA sweep
-// layout (the same expressions, the same exchange and skewed clock).
+// operands and results in the SA sweep layout; rows: the tile's row 0 at
+// this lane
 template <int DIR>
-__device__ inline void sa_sl_body(const SaGeom &g, int tile, double *__restrict__ L, double *ex, int *err,
-                                  double (*pj)[kLanes], double (*pk)[kLanes])
-{
-    constexpr int TT = kLanes;
-    const int bj = tile % g.nbj, bk = tile / g.nbj;
-    const int l = threadIdx.x, tj = l % kTile, tk = l / kTile;
-    const int lj = bj * kTile + tj, lk = bk * kTile + tk;
-    const bool active = lj < g.Lj && lk < g.Lk;
-    const int sj = DIR > 0 ? tj : kTile - 1 - tj, sk = DIR > 0 ? tk : kTile - 1 - tk;
-    const bool j_ring = DIR > 0 ? lj == 0 : lj + 1 >= g.Lj;
-    const bool k_ring = DIR > 0 ? lk == 0 : lk + 1 >= g.Lk;
-    const bool j_in = !j_ring && sj == 0, k_in = !k_ring && sk == 0;
-    const int lpj = l - DIR, lpk = l - DIR * kTile;
-    const bool j_out = sj == kTile - 1 && (DIR > 0 ? bj + 1 < g.nbj : bj > 0);
-    const bool k_out = sk == kTile - 1 && (DIR > 0 ? bk + 1 < g.nbk : bk > 0);
-    double *exj = ex, *exk = ex + (long)g.ntiles * g.exj_tile;
-    double *jin = exj + (long)(DIR > 0 ? tile - 1 : tile + 1) * g.exj_tile + tk;
-    double *kin = exk + (long)(DIR > 0 ? tile - g.nbj : tile + g.nbj) * g.exk_tile + tj;
-    double *jout = exj + (long)tile * g.exj_tile + tk;
-    double *kout = exk + (long)tile * g.exk_tile + tj;
-    // every lane of a tile with a neighbour on that side loads the face
-    // lanes' slot run of the step (one contiguous run per load); only the
-    // face lanes use it
-    const bool j_pred = DIR > 0 ? bj > 0 : bj + 1 < g.nbj;
-    const bool k_pred = DIR > 0 ? bk > 0 : bk + 1 < g.nbk;
-    const double *jsrc = j_pred ? jin : ex;
-    const double *ksrc = k_pred ? kin : ex;
-    const int xj_last = g.Li + kTile - 2, xk_last = g.Li + kTile - 2;
-    bool failed = false;
-    double vi = 0.0;
-    auto row_of = [&](int s) -> long {
-        const int sc = min(s, g.nsteps - 1);
-        return ((long)tile * g.nsteps + (DIR > 0 ? sc : g.nsteps - 1 - sc)) * kSaOps * TT + l;
-    };
-    auto fetch = [&](int s, double *op, unsigned long long &xj, unsigned long long &xk) {
-        const double *p = L + row_of(s);
-#pragma unroll
-        for (int f = 0; f < kSaOps; f++) op[f] = p[f * TT];
-        const int dj = j_pred ? min(max(s, 0), xj_last) : 0;
-        const int dk = k_pred ? min(max(s, 0), xk_last) : 0;
-        xj = xload_bits(jsrc + (long)dj * kTile);
-        xk = xload_bits(ksrc + (long)dk * kTile);
-    };
-    auto step = [&](int s, const double *op, unsigned long long xj, unsigned long long xk) {
-        const int par = s & 1;
-        const int pos = s - sj - sk;
-        if (active && pos >= 0 && pos < g.Li) {
-            const double vj = j_ring ? 0.0 : j_in ? ex_take1(jin + (long)(pos + sk) * kTile, xj, err, failed)
-                                                  : pj[par ^ 1][lpj];
-            const double vk = k_ring ? 0.0 : k_in ? ex_take1(kin + (long)(pos + sj) * kTile, xk, err, failed)
-                                                  : pk[par ^ 1][lpk];
-            double res;
-            if (DIR > 0) {
-                const double ta = 0.5 * (op[0] + fabs(op[0])) * vi;
-                const double tb = 0.5 * (op[1] + fabs(op[1])) * vj;
-                const double tc = 0.5 * (op[2] + fabs(op[2])) * vk;
-                res = (op[4] + (ta + tb + tc)) / op[3];
-            } else {
-                const double ta = 0.5 * (op[0] - fabs(op[0])) * vi;
-                const double tb = 0.5 * (op[1] - fabs(op[1])) * vj;
-                const double tc = 0.5 * (op[2] - fabs(op[2])) * vk;
-                res = op[4] - (ta + tb + tc) / op[3];
-            }
-            L[row_of(s) + (kSaOps - 1) * TT] = res;
-            vi = res;
-            pj[par][l] = res;
-            pk[par][l] = res;
-            if (j_out) xstore(jout + (long)(pos + sk) * kTile, res);
-            if (k_out) xstore(kout + (long)(pos + sj) * kTile, res);
-        }
-        lds_barrier();
-    };
-    double opA[kSaOps], opB[kSaOps];
-    unsigned long long xjA, xkA, xjB, xkB;
-    fetch(0, opA, xjA, xkA);
-    for (int s = 0; s < g.nsteps; s += 2) {
-        fetch(s + 1, opB, xjB, xkB);
-        step(s, opA, xjA, xkA);
-        fetch(s + 2, opA, xjA, xkA);
-        step(s + 1, opB, xjB, xkB);
+struct SaRows {
+    double *rows;
+    int nsteps;
+    __device__ double *row(int s) const
+    {
+        const int sc = min(s, nsteps - 1);
+        return rows + (long)(DIR > 0 ? sc : nsteps - 1 - sc) * kSaOps * kLanes;
     }
-}
+    __device__ void load(int s, int, double *op) const
+    {
+        const double *p = row(s);
+#pragma unroll
+        for (int f = 0; f < kSaOps; f++) op[f] = p[f * kLanes];
+    }
+    __device__ void store(int s, int, double v) const { row(s)[(kSaOps - 1) * kLanes] = v; }
+};
 
 template <int DIR>
 __global__ void __launch_bounds__(kLanes) k_sa_sl_batch(const SaBatchEnt *__restrict__ ents,
                                                          const int *__restrict__ tile_ent, int total, int resident,
                                                          double *slbase, double *exb, int *err, int *ctr)
 {
-    __shared__ double pj[2][kLanes], pk[2][kLanes];
     __shared__ int ticket;
     if (!resident) {
         if (threadIdx.x == 0)
@@ -1503,8 +1456,9 @@ __global__ void __launch_bounds__(kLanes) k_sa_sl_batch(const SaBatchEnt *__rest
     const int flat = resident ? (int)blockIdx.x : __builtin_amdgcn_readfirstlane(ticket);
     const SaBatchEnt &b = ents[tile_ent[flat]];
     const SaGeom g = b.g;
-    const int local = flat - b.tile0;
-    sa_sl_body<DIR>(g, DIR > 0 ? local : g.ntiles - 1 - local, slbase + b.sl, exb + b.ex, err, pj, pk);
+    const int local = flat - b.tile0, tile = DIR > 0 ? local : g.ntiles - 1 - local;
+    sa_sweep_body<DIR>(g, tile, SaRows<DIR>{slbase + b.sl + sa_slot(g, tile, 0, 0, (int)threadIdx.x), g.nsteps},
+                       exb + b.ex, err);
     if (!resident && threadIdx.x == 0 &&
         __hip_atomic_fetch_add(ctr + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == total - 1) {
         __hip_atomic_store(ctr, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
