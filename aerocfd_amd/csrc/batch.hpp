@@ -54,9 +54,9 @@ __device__ inline long xcd_slab(long w, long total)
 // workgroup numbers in XCD slabs, so that each XCD walks contiguous parts
 // of the blocks).
 __device__ inline int batch_wg(const int *__restrict__ map, const KGrid *__restrict__ kg, int &bx, int &by,
-                               int &bz)
+                               int &bz, unsigned total = 0)
 {
-    const int flat = (int)xcd_slab(blockIdx.x, gridDim.x);
+    const int flat = (int)xcd_slab(blockIdx.x, total ? total : gridDim.x);
     const int m = map[flat];
     const KGrid g = kg[m];
     int local = flat - g.wg0;

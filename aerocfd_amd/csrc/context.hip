@@ -168,8 +168,8 @@ struct acfd_ctx {
     // step that did so replays only while it holds.
     bool pri_current = false;
     bool graph_needs_pri = false;
-    // the last residual stage also formed implicit1st's rhs and time term
-    // (lu_fold): the update that follows skips its preparation pass
+    // the last residual stage also formed implicit1st's rhs (lu_fold): the
+    // update that follows skips its preparation pass
     bool lu_prep_ready = false;
     // the last residual stage formed rhs = rhsi + rhsv without storing rhsv
     // (the same fold): rhsv_refresh forms it from the node fluxes, which
@@ -224,6 +224,7 @@ struct acfd_ctx {
     long *d_ntab = nullptr;
     // halo copy list
     int halo_n = 0;
+    bool refresh_one = false;  // halo fill and average1's gather in one launch
     int *d_h_sb = nullptr, *d_h_db = nullptr;
     long *d_h_sn = nullptr, *d_h_dn = nullptr;
     std::vector<int> h_sb, h_db;
@@ -874,14 +875,14 @@ int st_inviscid(acfd_ctx *ctx, int m)
     return 0;
 }
 
-// part 1: the node pass, 2: the difference pass, with prep_cfl also
-// implicit1st's rhs and time term (lu_fold)
-int st_viscous(acfd_ctx *ctx, int m, int store_aux, int part = -1, const double *prep_cfl = nullptr)
+// part 1: the node pass, 2: the difference pass; prep: that pass forms
+// implicit1st's rhs (lu_fold), find_dt: and does the unsteady find_dt
+int st_viscous(acfd_ctx *ctx, int m, int store_aux, int part = -1, bool prep = false, bool find_dt = false)
 {
     StageTimer t(ctx, ACFD_STAGE_VISCOUS);
     KRN_TRY(launch_viscous(ctx->stream, ctx->blk[m].e, ctx->blk[m].f, ctx->c, ctx->cfg.precision, store_aux, part,
-                           prep_cfl));
-    if (prep_cfl) ctx->lu_prep_ready = ctx->rhsv_stale = true;
+                           prep, find_dt ? ctx->d_cfl : nullptr, find_dt ? ctx->d_cfl_blk + m : nullptr));
+    if (prep) ctx->lu_prep_ready = ctx->rhsv_stale = true;
     return 0;
 }
 
@@ -917,14 +918,17 @@ bool viscous_dt_fused_on()
 }
 
 // With NS and the tile sweeps the viscous difference pass of a step also
-// forms what implicit1st starts from, rhs = rhsi + rhsv and the time term,
-// and leaves rhsv out (ACFD_VISCOUS_DT_FUSED=0: passes of their own; the
-// same results either way).  find_dt, which reads the viscosity that the
-// node pass stores, then runs between the two viscous passes.
+// forms what implicit1st starts from, rhs = rhsi + rhsv, and leaves rhsv out
+// (ACFD_VISCOUS_DT_FUSED=0: passes of their own; the same results either
+// way).  The unsteady find_dt, one node a block, which reads the viscosity
+// that the node pass stores, is a workgroup of that pass (a launch of its own
+// under the stage timers: 5 us).
 bool lu_fold(const acfd_ctx *ctx)
 {
     return ctx->c.solver == 0 && ctx->cfg.iflag_timeadvance == 2 && ctx->lu_variant != 0 && viscous_dt_fused_on();
 }
+
+bool dt_in_diff(const acfd_ctx *ctx) { return lu_fold(ctx) && ctx->c.itime != 0 && !ctx->timing; }
 
 // the cfl that block m's update reads: the one its own find_dt left (the
 // reference runs each block's find_dt, implicit1st and sa_model back to back)
@@ -1031,6 +1035,7 @@ int st_implicit_all(acfd_ctx *ctx, const double *cfl_per_block)
     for (int ph = 1; ph < kLusgsPhases; ph++) {
         StageTimer ts(ctx, ph == 2 ? kTimeLuForward : ph == 3 ? kTimeLuBackward : ph == 1 ? kTimeLuGather : kTimeLuAdd);
         KRN_TRY(launch_lusgs_batch(ctx->stream, lb, ph, ctx->c.gamma, ctx->lu.err, ctx->lu_ctr,
+                                   cfl_per_block ? cfl_per_block : ctx->d_cfl, cfl_per_block ? 1 : 0,
                                    ph == 1 ? sl_geo_cached(ctx, -1) : 0));
     }
     return 0;
@@ -1179,9 +1184,19 @@ int st_average(acfd_ctx *ctx)
     return 0;
 }
 
+// The halo fill writes nodes outside every block's physical range only and
+// average1's gather reads nodes inside only (refresh_one, checked over the
+// lists when they are made), so the two are one launch (not under the stage
+// timers).
 int refresh(acfd_ctx *ctx)
 {
     int rc = st_physical_bc(ctx);
+    if (!rc && ctx->refresh_one && !ctx->timing) {
+        CopyList cl{ctx->halo_n, ctx->d_h_sb, ctx->d_h_db, ctx->d_h_sn, ctx->d_h_dn};
+        KRN_TRY(launch_halo_average(ctx->stream, cl, ctx->avg, ctx->d_qtab, ctx->d_nuttab, ctx->d_ntab, ctx->d_a_buf,
+                                    ctx->c.turb == 2));
+        return 0;
+    }
     if (!rc) rc = st_update_buffer(ctx);
     if (!rc) rc = st_average(ctx);
     return rc;
@@ -1190,11 +1205,10 @@ int refresh(acfd_ctx *ctx)
 int residual_stage(acfd_ctx *ctx, int m, int store_aux, bool pri_ok = false)
 {
     int rc = pri_ok ? 0 : st_getpri(ctx, m);
-    const bool fold = lu_fold(ctx);
+    const bool fold = lu_fold(ctx), dt_in = dt_in_diff(ctx);
     if (!rc) rc = st_inviscid(ctx, m);
-    if (!rc && ctx->c.solver == 0) rc = st_viscous(ctx, m, store_aux, fold ? 1 : -1);
-    if (!rc) rc = st_find_dt(ctx, m);
-    if (!rc && fold) rc = st_viscous(ctx, m, store_aux, 2, update_cfl(ctx, m));
+    if (!rc && ctx->c.solver == 0) rc = st_viscous(ctx, m, store_aux, -1, fold, dt_in);
+    if (!rc && !dt_in) rc = st_find_dt(ctx, m);
     return rc;
 }
 
@@ -1246,30 +1260,28 @@ int st_inviscid_all(acfd_ctx *ctx)
     return 0;
 }
 
-int st_viscous_all(acfd_ctx *ctx, int store_aux, int only = -1, bool fold = false)
+int st_viscous_all(acfd_ctx *ctx, int store_aux, bool fold = false, bool dt_in = false)
 {
+    const int nb = (int)ctx->blk.size();
     if (!batched(ctx)) {
-        for (int m = 0; m < (int)ctx->blk.size(); m++) {
-            int rc = st_viscous(ctx, m, store_aux, only, fold ? update_cfl(ctx, m) : nullptr);
+        for (int m = 0; m < nb; m++) {
+            int rc = st_viscous(ctx, m, store_aux, -1, fold, dt_in);
             if (rc) return rc;
         }
         return 0;
     }
     StageTimer t(ctx, ACFD_STAGE_VISCOUS);
-    // (steady: the fold is st_viscous_dt_all's)
-    const double *prep_cfl = fold ? ctx->d_cfl_blk : nullptr;
     if (fold) ctx->lu_prep_ready = ctx->rhsv_stale = true;
     if (ctx->timing) {
         for (int part = 1; part <= 2; part++) {
-            if (only > 0 && part != only) continue;
             StageTimer ts(ctx, part == 1 ? kTimeViscNode : kTimeViscDiff);
             KRN_TRY(launch_viscous_batch(ctx->stream, ctx->d_blocks, ctx->bg_visc, ctx->arena, ctx->c,
-                                         ctx->cfg.precision, store_aux, part, prep_cfl));
+                                         ctx->cfg.precision, store_aux, part, fold));
         }
         return 0;
     }
     KRN_TRY(launch_viscous_batch(ctx->stream, ctx->d_blocks, ctx->bg_visc, ctx->arena, ctx->c, ctx->cfg.precision,
-                                 store_aux, only, prep_cfl));
+                                 store_aux, -1, fold, nb, dt_in ? ctx->d_cfl : nullptr, ctx->d_cfl_blk));
     return 0;
 }
 
@@ -1297,8 +1309,8 @@ int st_viscous_dt_all(acfd_ctx *ctx, int store_aux, int parts = -1)
 {
     StageTimer t(ctx, ACFD_STAGE_VISCOUS);
     const int nb = (int)ctx->blk.size();
-    // the batched LU-SGS update's time term and rhs come from these two
-    // passes too (implicit1st then skips its own preparation)
+    // implicit1st's rhs comes from the difference pass too (and its own
+    // preparation is skipped)
     const int prep = lu_fold(ctx) ? 1 : 0;
     if (parts >= 0) {
         if (parts == 1) KRN_TRY(launch_reset_stats(ctx->stream, ctx->d_stats));
@@ -1361,10 +1373,9 @@ int residual_stage_all(acfd_ctx *ctx, int store_aux, bool pri_ok = false)
     }
     if (!rc) rc = st_inviscid_all(ctx);
     if (!rc && fused) return st_viscous_dt_all(ctx, store_aux);
-    const bool fold = lu_fold(ctx);
-    if (!rc && ctx->c.solver == 0) rc = st_viscous_all(ctx, store_aux, fold ? 1 : -1);
-    if (!rc) rc = st_find_dt_all(ctx);
-    if (!rc && fold) rc = st_viscous_all(ctx, store_aux, 2, true);
+    const bool dt_in = dt_in_diff(ctx);
+    if (!rc && ctx->c.solver == 0) rc = st_viscous_all(ctx, store_aux, lu_fold(ctx), dt_in);
+    if (!rc && !dt_in) rc = st_find_dt_all(ctx);
     return rc;
 }
 
@@ -1775,6 +1786,15 @@ int acfd_set_topology(acfd_ctx *ctx, int nblk, const int *dims, const int *nsub,
     ctx->avg.grp_blk = ctx->d_a_gb;
     ctx->avg.grp_dst = ctx->d_a_gd;
     ctx->avg.grp_start = ctx->d_a_gs;
+    auto physical = [&](int m, long n) {
+        const Ext &e = ctx->blk[m].e;
+        const int i = e.is + (int)(n % e.ni), j = e.js + (int)(n / e.ni % e.nj), k = e.ks + (int)(n / e.ni / e.nj);
+        return i >= e.is0 && i <= e.ie0 && j >= e.js0 && j <= e.je0 && k >= e.ks0 && k <= e.ke0;
+    };
+    ctx->refresh_one = ctx->halo_n > 0 && !e_sb.empty();
+    for (size_t x = 0; x < ctx->h_db.size() && ctx->refresh_one; x++)
+        ctx->refresh_one = !physical(ctx->h_db[x], ctx->h_dn[x]);
+    for (size_t x = 0; x < e_sb.size() && ctx->refresh_one; x++) ctx->refresh_one = physical(e_sb[x], e_sn[x]);
     // physical boundary tasks in block/subface order (sub_bc.f90:26-62);
     // farfield runs with the block's js in place of the subface's js
     // (sub_bc.f90:57-59)

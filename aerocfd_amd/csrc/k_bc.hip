@@ -229,12 +229,11 @@ int launch_sa_clamp(hipStream_t s, const Ext &e, const Fields &f)
 
 // Halo fill: a pure gather over a precomputed list of (source node,
 // destination halo node) pairs covering every interface, both layers.
-__global__ void k_halo_copy(int count, const int *__restrict__ sb, const long *__restrict__ sn,
-                            const int *__restrict__ db, const long *__restrict__ dn,
-                            double *const *__restrict__ qtab, double *const *__restrict__ nuttab,
-                            const long *__restrict__ ntab, int with_nut)
+__device__ inline void halo_copy_at(int x, int count, const int *__restrict__ sb, const long *__restrict__ sn,
+                                    const int *__restrict__ db, const long *__restrict__ dn,
+                                    double *const *__restrict__ qtab, double *const *__restrict__ nuttab,
+                                    const long *__restrict__ ntab, int with_nut)
 {
-    int x = blockIdx.x * blockDim.x + threadIdx.x;
     if (x >= count) return;
     int b0 = sb[x], b1 = db[x];
     long s = sn[x], d = dn[x];
@@ -244,6 +243,14 @@ __global__ void k_halo_copy(int count, const int *__restrict__ sb, const long *_
 #pragma unroll
     for (int v = 0; v < 5; v++) qd[v * Nd + d] = qs[v * Ns + s];
     if (with_nut) nuttab[b1][d] = nuttab[b0][s];
+}
+
+__global__ void k_halo_copy(int count, const int *__restrict__ sb, const long *__restrict__ sn,
+                            const int *__restrict__ db, const long *__restrict__ dn,
+                            double *const *__restrict__ qtab, double *const *__restrict__ nuttab,
+                            const long *__restrict__ ntab, int with_nut)
+{
+    halo_copy_at(blockIdx.x * blockDim.x + threadIdx.x, count, sb, sn, db, dn, qtab, nuttab, ntab, with_nut);
 }
 
 int launch_halo_copy(hipStream_t s, const CopyList &cl, double *const *q_tab, double *const *nut_tab,
@@ -258,11 +265,10 @@ int launch_halo_copy(hipStream_t s, const CopyList &cl, double *const *q_tab, do
 }
 
 // average1: gather the neighbour's face node of every pairing entry.
-__global__ void k_avg_gather(int count, const int *__restrict__ sb, const long *__restrict__ sn,
-                             double *const *__restrict__ qtab, double *const *__restrict__ nuttab,
-                             const long *__restrict__ ntab, double *__restrict__ buf, int with_nut)
+__device__ inline void avg_gather_at(int x, int count, const int *__restrict__ sb, const long *__restrict__ sn,
+                                     double *const *__restrict__ qtab, double *const *__restrict__ nuttab,
+                                     const long *__restrict__ ntab, double *__restrict__ buf, int with_nut)
 {
-    int x = blockIdx.x * blockDim.x + threadIdx.x;
     if (x >= count) return;
     int b0 = sb[x];
     long s = sn[x];
@@ -271,6 +277,29 @@ __global__ void k_avg_gather(int count, const int *__restrict__ sb, const long *
 #pragma unroll
     for (int v = 0; v < 5; v++) buf[(long)6 * x + v] = qs[v * Ns + s];
     buf[(long)6 * x + 5] = with_nut ? nuttab[b0][s] : 0.0;
+}
+
+__global__ void k_avg_gather(int count, const int *__restrict__ sb, const long *__restrict__ sn,
+                             double *const *__restrict__ qtab, double *const *__restrict__ nuttab,
+                             const long *__restrict__ ntab, double *__restrict__ buf, int with_nut)
+{
+    avg_gather_at(blockIdx.x * blockDim.x + threadIdx.x, count, sb, sn, qtab, nuttab, ntab, buf, with_nut);
+}
+
+// The halo fill by the first hwg workgroups and average1's gather by the
+// rest, where neither writes what the other reads (a launch of a few
+// thousand nodes takes 5 us whatever it holds)
+__global__ void k_halo_avg_gather(int hwg, int hcount, const int *__restrict__ hsb, const long *__restrict__ hsn,
+                                  const int *__restrict__ hdb, const long *__restrict__ hdn, int acount,
+                                  const int *__restrict__ asb, const long *__restrict__ asn,
+                                  double *const *__restrict__ qtab, double *const *__restrict__ nuttab,
+                                  const long *__restrict__ ntab, double *__restrict__ buf, int with_nut)
+{
+    if ((int)blockIdx.x < hwg)
+        halo_copy_at(blockIdx.x * blockDim.x + threadIdx.x, hcount, hsb, hsn, hdb, hdn, qtab, nuttab, ntab, with_nut);
+    else
+        avg_gather_at(((int)blockIdx.x - hwg) * blockDim.x + threadIdx.x, acount, asb, asn, qtab, nuttab, ntab, buf,
+                      with_nut);
 }
 
 // average2: for each destination node, apply q = (q + buf)*0.5 for its
@@ -306,6 +335,26 @@ __global__ void k_avg_apply(int ngroups, const int *__restrict__ gb, const long 
     if (with_nut) nuttab[b][d] = vn;
 }
 
+static void launch_avg_apply(hipStream_t s, const AvgList &al, double *const *q_tab, double *const *nut_tab,
+                             const long *n_tab, double *buf, int with_nut)
+{
+    const int bs = 256;
+    hipLaunchKernelGGL(k_avg_apply, dim3((al.ngroups + bs - 1) / bs), dim3(bs), 0, s, al.ngroups, al.grp_blk,
+                       al.grp_dst, al.grp_start, q_tab, nut_tab, n_tab, buf, with_nut);
+}
+
+int launch_halo_average(hipStream_t s, const CopyList &cl, const AvgList &al, double *const *q_tab,
+                        double *const *nut_tab, const long *n_tab, double *buf, int with_nut)
+{
+    const int bs = 256, hwg = (cl.count + bs - 1) / bs, awg = (al.count + bs - 1) / bs;
+    if (hwg + awg <= 0) return 0;
+    hipLaunchKernelGGL(k_halo_avg_gather, dim3(hwg + awg), dim3(bs), 0, s, hwg, cl.count, cl.src_blk, cl.src,
+                       cl.dst_blk, cl.dst, al.count, al.src_blk, al.src, q_tab, nut_tab, n_tab, buf, with_nut);
+    if (al.count > 0) launch_avg_apply(s, al, q_tab, nut_tab, n_tab, buf, with_nut);
+    ACFD_CHECK_LAUNCH();
+    return 0;
+}
+
 int launch_average(hipStream_t s, const AvgList &al, double *const *q_tab, double *const *nut_tab,
                    const long *n_tab, double *buf, int with_nut)
 {
@@ -313,8 +362,7 @@ int launch_average(hipStream_t s, const AvgList &al, double *const *q_tab, doubl
     int bs = 256;
     hipLaunchKernelGGL(k_avg_gather, dim3((al.count + bs - 1) / bs), dim3(bs), 0, s, al.count, al.src_blk, al.src,
                        q_tab, nut_tab, n_tab, buf, with_nut);
-    hipLaunchKernelGGL(k_avg_apply, dim3((al.ngroups + bs - 1) / bs), dim3(bs), 0, s, al.ngroups, al.grp_blk,
-                       al.grp_dst, al.grp_start, q_tab, nut_tab, n_tab, buf, with_nut);
+    launch_avg_apply(s, al, q_tab, nut_tab, n_tab, buf, with_nut);
     ACFD_CHECK_LAUNCH();
     return 0;
 }

@@ -502,20 +502,22 @@ __global__ void __launch_bounds__(256) k_viscous_node(Ext e, Consts c, const dou
                          vor, dudx, tao, store_aux);
 }
 
+__device__ inline void find_dt_unsteady_block(const Ext &e, const double *pri, const double *amu, const double *dxidx,
+                                              const double *dt, double re, double *cfl, double *cfl_blk);
+__device__ inline void find_dt_unsteady_rec(const BlockRec &b, const double *arena, double re, double *cfl,
+                                            double *cfl_blk);
+
 // Stage 2 (sub_viscous.f90:296-365): rhsv = (d/dxi fv + d/deta gv + d/dzeta hv)/re;
 // with rhsi given, also rhs = rhsi + rhsv on the computed range (the
 // first line of implicit1st, sub_timeadvancement_1stimplicit.f90:72-78),
-// and with rhsv null only rhs; with diag given, implicit1st's time term
-// phi*1/dt there too (:98-102,151, as lu_prep_body forms it for the tile
-// sweeps).  Bound by memory: for a context that updates with the tile sweeps
-// this replaces storing rhsv, and a pass (lu_prep) that read it and rhsi and
-// wrote rhs and the time term.  Viscous stage and that pass, before and
-// after: 33^3 26.7 -> 23.2 us, 129^3 294 -> 268, 193^3 910 -> 809.
+// and with rhsv null only rhs.  Bound by memory: for a context that updates
+// with the tile sweeps this replaces storing rhsv, and a pass (lu_prep) that
+// read it and rhsi and wrote rhs.  Viscous stage and that pass, before and
+// after: 33^3 26.7 -> 20.0 us, 129^3 294 -> 257, 193^3 910 -> 782.
 template <typename S>
 __device__ inline void viscous_diff_body(const Ext &e, long wg, const S *__restrict__ w,
                                          double *__restrict__ rhsv, double re, const double *__restrict__ rhsi = nullptr,
-                                         double *__restrict__ rhs = nullptr, const double *__restrict__ dt = nullptr,
-                                         double *__restrict__ diag = nullptr, const double *cfl = nullptr)
+                                         double *__restrict__ rhs = nullptr)
 {
     const Box b{e.is0, e.ie0, e.js0, e.je0, e.ks0, e.ke0};
     int i, j, k;
@@ -528,10 +530,6 @@ __device__ inline void viscous_diff_body(const Ext &e, long wg, const S *__restr
     const double v0 = (0.0 + 0.0 + 0.0) / re;
     if (rhsv) st_out(rhsv + n, v0);
     if (inner) st_out(rhs + n, ld_once(rhsi + n) + v0);
-    if (inner && diag) {
-        const double phi = *cfl >= 1.0e3 ? 0.0 : 1.0;
-        diag[n] = phi * 1.0 / dt[n];
-    }
 #pragma unroll
     for (int c = 0; c < 4; c++) {
         double a = ndiff(w + (0 + c) * N, n, 1, i, e.is0, e.ie0);
@@ -551,15 +549,23 @@ __global__ void __launch_bounds__(256) k_viscous_diff(Ext e, const double *__res
     viscous_diff_body<S>(e, xcd_slab(blockIdx.x, gridDim.x), reinterpret_cast<const S *>(w), rhsv, re);
 }
 
-// with implicit1st's rhs and time term, rhsv not stored
+// with implicit1st's rhs, rhsv not stored; with dt given one workgroup more
+// than the tiles, which does the unsteady find_dt (a node of the block; it
+// reads the viscosity that the node pass has stored)
 template <typename S>
 __global__ void __launch_bounds__(256) k_viscous_diff_prep(Ext e, const double *__restrict__ w, double re,
                                                            const double *__restrict__ rhsi, double *__restrict__ rhs,
-                                                           const double *__restrict__ dt, double *__restrict__ diag,
-                                                           const double *cfl)
+                                                           const double *__restrict__ pri,
+                                                           const double *__restrict__ amu,
+                                                           const double *__restrict__ dxidx,
+                                                           const double *__restrict__ dt, double *cfl, double *cfl_blk)
 {
-    viscous_diff_body<S>(e, xcd_slab(blockIdx.x, gridDim.x), reinterpret_cast<const S *>(w), nullptr, re, rhsi, rhs, dt,
-                         diag, cfl);
+    const unsigned tiles = gridDim.x - (dt ? 1 : 0);
+    if (blockIdx.x == tiles) {
+        if (threadIdx.x + threadIdx.y == 0) find_dt_unsteady_block(e, pri, amu, dxidx, dt, re, cfl, cfl_blk);
+        return;
+    }
+    viscous_diff_body<S>(e, xcd_slab(blockIdx.x, tiles), reinterpret_cast<const S *>(w), nullptr, re, rhsi, rhs);
 }
 
 template <typename R>
@@ -576,23 +582,26 @@ __global__ void __launch_bounds__(256) k_viscous_node_batch(const BlockRec *__re
                          store_aux);
 }
 
-// with_rhs 2: rhs = rhsi + rhsv on the computed range instead of rhsv; 3:
-// and the time term, block m with cfl[m]; S: the storage type of the node
-// fluxes
+// with_rhs: rhs = rhsi + rhsv on the computed range instead of rhsv; with
+// cfl given one workgroup more than the tiles, which does every block's
+// unsteady find_dt; S: the storage type of the node fluxes
 template <typename S>
 __global__ void __launch_bounds__(256) k_viscous_diff_batch(const BlockRec *__restrict__ blks,
                                                             const int *__restrict__ map,
                                                             const KGrid *__restrict__ kg, double *arena, double re,
-                                                            int with_rhs, const double *cfl)
+                                                            int with_rhs, int nblk, double *cfl, double *cfl_blk)
 {
+    const unsigned tiles = gridDim.x - (cfl ? 1 : 0);
+    if (blockIdx.x == tiles) {
+        for (int m = (int)(threadIdx.x + blockDim.x * threadIdx.y); m < nblk; m += 256)
+            find_dt_unsteady_rec(blks[m], arena, re, m == nblk - 1 ? cfl : nullptr, cfl_blk + m);
+        return;
+    }
     int bx, by, bz;
-    const int m = batch_wg(map, kg, bx, by, bz);
-    const BlockRec &b = blks[m];
+    const BlockRec &b = blks[batch_wg(map, kg, bx, by, bz, tiles)];
     const Ext e = b.e;
     const S *w = reinterpret_cast<const S *>(arena + b.o.w_flux);
-    if (with_rhs)
-        viscous_diff_body<S>(e, bx, w, nullptr, re, arena + b.o.rhsi, arena + b.o.rhs, arena + b.o.dt,
-                             with_rhs == 3 ? arena + b.o.w_diag : nullptr, cfl + m);
+    if (with_rhs) viscous_diff_body<S>(e, bx, w, nullptr, re, arena + b.o.rhsi, arena + b.o.rhs);
     else viscous_diff_body<S>(e, bx, w, arena + b.o.rhsv, re);
 }
 
@@ -601,9 +610,11 @@ __global__ void __launch_bounds__(256) k_viscous_diff_batch(const BlockRec *__re
 dim3 viscous_grid(const Ext &e) { return lin_grid(e); }
 
 int launch_viscous(hipStream_t s, const Ext &e, const Fields &f, const Consts &c, int precision,
-                   int store_aux, int part, const double *prep_cfl)
+                   int store_aux, int part, bool prep, double *cfl, double *cfl_blk)
 {
     dim3 g = viscous_grid(e), t(64, 4, 1);
+    const dim3 gp(g.x + (cfl ? 1 : 0));
+    const double *dt = cfl ? f.dt : nullptr;
     if (part == 2) {
     } else if (precision == 1)
         hipLaunchKernelGGL((k_viscous_node<float>), g, t, 0, s, e, c, f.pri, f.amu, f.dxidx, f.inv_j, f.w_flux,
@@ -612,12 +623,12 @@ int launch_viscous(hipStream_t s, const Ext &e, const Fields &f, const Consts &c
         hipLaunchKernelGGL((k_viscous_node<double>), g, t, 0, s, e, c, f.pri, f.amu, f.dxidx, f.inv_j, f.w_flux,
                            f.vor, f.dudx, f.tao, store_aux);
     if (part == 1) {
-    } else if (prep_cfl && precision == 1)
-        hipLaunchKernelGGL(k_viscous_diff_prep<float>, g, t, 0, s, e, f.w_flux, c.re, f.rhsi, f.rhs, f.dt, f.w_diag,
-                           prep_cfl);
-    else if (prep_cfl)
-        hipLaunchKernelGGL(k_viscous_diff_prep<double>, g, t, 0, s, e, f.w_flux, c.re, f.rhsi, f.rhs, f.dt, f.w_diag,
-                           prep_cfl);
+    } else if (prep && precision == 1)
+        hipLaunchKernelGGL(k_viscous_diff_prep<float>, gp, t, 0, s, e, f.w_flux, c.re, f.rhsi, f.rhs, f.pri, f.amu,
+                           f.dxidx, dt, cfl, cfl_blk);
+    else if (prep)
+        hipLaunchKernelGGL(k_viscous_diff_prep<double>, gp, t, 0, s, e, f.w_flux, c.re, f.rhsi, f.rhs, f.pri, f.amu,
+                           f.dxidx, dt, cfl, cfl_blk);
     else if (precision == 1) hipLaunchKernelGGL(k_viscous_diff<float>, g, t, 0, s, e, f.w_flux, f.rhsv, c.re);
     else hipLaunchKernelGGL(k_viscous_diff<double>, g, t, 0, s, e, f.w_flux, f.rhsv, c.re);
     ACFD_CHECK_LAUNCH();
@@ -625,11 +636,12 @@ int launch_viscous(hipStream_t s, const Ext &e, const Fields &f, const Consts &c
 }
 
 int launch_viscous_batch(hipStream_t s, const BlockRec *blks, const BatchGrid &bg, double *arena, const Consts &c,
-                         int precision, int store_aux, int part, const double *prep_cfl)
+                         int precision, int store_aux, int part, bool prep, int nblk, double *cfl, double *cfl_blk)
 {
     if (bg.total <= 0) return 0;
     dim3 g((unsigned)bg.total), t(64, 4, 1);
-    const int with_rhs = prep_cfl ? 3 : 0;
+    const dim3 gp(g.x + (cfl ? 1 : 0));
+    const int with_rhs = prep ? 1 : 0;
     if (part < 0 || part == 1) {
         if (precision == 1)
             hipLaunchKernelGGL((k_viscous_node_batch<float>), g, t, 0, s, blks, bg.map, bg.kg, arena, c, store_aux);
@@ -638,11 +650,11 @@ int launch_viscous_batch(hipStream_t s, const BlockRec *blks, const BatchGrid &b
     }
     if (part < 0 || part == 2) {
         if (precision == 1)
-            hipLaunchKernelGGL(k_viscous_diff_batch<float>, g, t, 0, s, blks, bg.map, bg.kg, arena, c.re, with_rhs,
-                               prep_cfl);
+            hipLaunchKernelGGL(k_viscous_diff_batch<float>, gp, t, 0, s, blks, bg.map, bg.kg, arena, c.re, with_rhs,
+                               nblk, cfl, cfl_blk);
         else
-            hipLaunchKernelGGL(k_viscous_diff_batch<double>, g, t, 0, s, blks, bg.map, bg.kg, arena, c.re, with_rhs,
-                               prep_cfl);
+            hipLaunchKernelGGL(k_viscous_diff_batch<double>, gp, t, 0, s, blks, bg.map, bg.kg, arena, c.re, with_rhs,
+                               nblk, cfl, cfl_blk);
     }
     ACFD_CHECK_LAUNCH();
     return 0;
@@ -744,14 +756,27 @@ __global__ void __launch_bounds__(256) k_find_dt_steady_batch(const BlockRec *__
                         m == nblk - 1 ? stats : nullptr);
 }
 
+// the local CFL of node (ie, je, ke) of a block
+__device__ inline void find_dt_unsteady_block(const Ext &e, const double *pri, const double *amu, const double *dxidx,
+                                              const double *dt, double re, double *cfl, double *cfl_blk)
+{
+    const long n = e.n - 1;
+    const double v = dt[n] * local_rate(e, n, pri, amu, dxidx, re);
+    if (cfl) *cfl = v;
+    if (cfl_blk) *cfl_blk = v;
+}
+__device__ inline void find_dt_unsteady_rec(const BlockRec &b, const double *arena, double re, double *cfl,
+                                            double *cfl_blk)
+{
+    const Ext e = b.e;
+    find_dt_unsteady_block(e, arena + b.o.pri, arena + b.o.amu, arena + b.o.dxidx, arena + b.o.dt, re, cfl, cfl_blk);
+}
+
 __global__ void k_find_dt_unsteady(Ext e, const double *__restrict__ pri, const double *__restrict__ amu,
                                    const double *__restrict__ dxidx, const double *__restrict__ dt,
                                    double *cfl, double *cfl_blk, double re)
 {
-    long n = e.n - 1;  // node (ie, je, ke)
-    const double v = dt[n] * local_rate(e, n, pri, amu, dxidx, re);
-    *cfl = v;
-    if (cfl_blk) *cfl_blk = v;
+    find_dt_unsteady_block(e, pri, amu, dxidx, dt, re, cfl, cfl_blk);
 }
 
 // unsteady, every block: thread m writes block m's cfl to cfl_blk[m]; the
@@ -761,12 +786,7 @@ __global__ void k_find_dt_unsteady_batch(const BlockRec *__restrict__ blks, doub
 {
     const int m = (int)(blockIdx.x * blockDim.x + threadIdx.x);
     if (m >= nblk) return;
-    const BlockRec &b = blks[m];
-    const Ext e = b.e;
-    const long n = e.n - 1;
-    const double v = arena[b.o.dt + n] * local_rate(e, n, arena + b.o.pri, arena + b.o.amu, arena + b.o.dxidx, re);
-    cfl_blk[m] = v;
-    if (m == nblk - 1) *cfl = v;
+    find_dt_unsteady_rec(blks[m], arena, re, m == nblk - 1 ? cfl : nullptr, cfl_blk + m);
 }
 
 __global__ void k_reset_stats(unsigned long long *st)
@@ -781,12 +801,7 @@ __global__ void k_reset_stats(unsigned long long *st)
 // formed; every other node of the extended block only dt (k_find_dt_steady
 // reads the stored viscosity there).  The same expressions as the two
 // kernels; the dt statistics from the last block.
-//
-// With PREP, the node also forms implicit1st's time term phi*1/dt
-// (sub_timeadvancement_1stimplicit.f90:98-102,151, as lu_prep_body forms it
-// for the tile sweeps, which add the spectral radii themselves) from its
-// dt; the difference pass then forms rhs.
-template <typename R, bool PREP>
+template <typename R>
 __global__ void __launch_bounds__(256) k_viscous_node_dt_batch(const BlockRec *__restrict__ blks,
                                                                const int *__restrict__ map,
                                                                const KGrid *__restrict__ kg, double *arena,
@@ -823,25 +838,8 @@ __global__ void __launch_bounds__(256) k_viscous_node_dt_batch(const BlockRec *_
         }
         v = *cfl / local_rate_a3(e, n, pri, a3, dxidx, c.re);
         st_out(arena + b.o.dt + n, v);
-        if (PREP) {
-            const double phi = *cfl >= 1.0e3 ? 0.0 : 1.0;  // implicit1st :98-102
-            st_out(arena + b.o.w_diag + n, phi * 1.0 / v);
-        }
     }
     dt_stats(ok, v, m == nblk - 1 ? stats : nullptr);
-}
-
-template <bool PREP>
-static void viscous_dt_node(hipStream_t s, const BlockRec *blks, int nblk, const BatchGrid &bg, double *arena,
-                            const Consts &c, int precision, int store_aux, const double *cfl, unsigned long long *stats)
-{
-    const dim3 g((unsigned)bg.total), t(64, 4, 1);
-    if (precision == 1)
-        hipLaunchKernelGGL((k_viscous_node_dt_batch<float, PREP>), g, t, 0, s, blks, bg.map, bg.kg, arena, c,
-                           store_aux, nblk, cfl, stats);
-    else
-        hipLaunchKernelGGL((k_viscous_node_dt_batch<double, PREP>), g, t, 0, s, blks, bg.map, bg.kg, arena, c,
-                           store_aux, nblk, cfl, stats);
 }
 
 int launch_viscous_dt_batch(hipStream_t s, const BlockRec *blks, int nblk, const BatchGrid &bg, double *arena,
@@ -851,16 +849,20 @@ int launch_viscous_dt_batch(hipStream_t s, const BlockRec *blks, int nblk, const
     if (bg.total <= 0) return 0;
     const dim3 g((unsigned)bg.total), t(64, 4, 1);
     if (part < 0 || part == 1) {
-        if (prep) viscous_dt_node<true>(s, blks, nblk, bg, arena, c, precision, store_aux, cfl, stats);
-        else viscous_dt_node<false>(s, blks, nblk, bg, arena, c, precision, store_aux, cfl, stats);
+        if (precision == 1)
+            hipLaunchKernelGGL(k_viscous_node_dt_batch<float>, g, t, 0, s, blks, bg.map, bg.kg, arena, c, store_aux,
+                               nblk, cfl, stats);
+        else
+            hipLaunchKernelGGL(k_viscous_node_dt_batch<double>, g, t, 0, s, blks, bg.map, bg.kg, arena, c, store_aux,
+                               nblk, cfl, stats);
     }
     if (part < 0 || part == 2) {
         if (precision == 1)
-            hipLaunchKernelGGL(k_viscous_diff_batch<float>, g, t, 0, s, blks, bg.map, bg.kg, arena, c.re, 2 * prep,
-                               nullptr);
+            hipLaunchKernelGGL(k_viscous_diff_batch<float>, g, t, 0, s, blks, bg.map, bg.kg, arena, c.re, prep, 0,
+                               nullptr, nullptr);
         else
-            hipLaunchKernelGGL(k_viscous_diff_batch<double>, g, t, 0, s, blks, bg.map, bg.kg, arena, c.re, 2 * prep,
-                               nullptr);
+            hipLaunchKernelGGL(k_viscous_diff_batch<double>, g, t, 0, s, blks, bg.map, bg.kg, arena, c.re, prep, 0,
+                               nullptr, nullptr);
     }
     ACFD_CHECK_LAUNCH();
     return 0;

@@ -194,8 +194,8 @@ __device__ inline void lu_backward(const LuArgs &a, long n, const double *vi, co
 // rhs = rhsi + rhsv on the computed range (:72-78).  For the hyperplane
 // sweeps (tiles = 0): spectral radii ra, rb, rc and diag on the ring
 // is1-1..ie1+1 (:98-156), and dq* and dq cleared on the ring so that
-// out-of-range neighbours read 0 (:105-106).  For the tile sweeps, which
-// form radii and diagonal themselves: only the time term phi*1/dt into diag.
+// out-of-range neighbours read 0 (:105-106).  The tile sweeps form radii and
+// diagonal themselves, and their gather the time term phi*1/dt: only rhs.
 __device__ inline void lu_prep_body(const Ext &e, long wg, const double *__restrict__ pri,
                                     const double *__restrict__ dxidx, const double *__restrict__ dt,
                                     const double *__restrict__ rhsi, const double *__restrict__ rhsv,
@@ -209,8 +209,7 @@ __device__ inline void lu_prep_body(const Ext &e, long wg, const double *__restr
     if (!lin_node_at(e, ring, wg, i, j, k, n)) return;
     const long N = e.n;
     const double phi = *cfl >= 1.0e3 ? 0.0 : 1.0;  // :98-102
-    if (tiles) diag[n] = phi * 1.0 / dt[n];
-    else diag[n] = lu_radii_diag(pri, dxidx, N, n, dt[n], phi, rr);
+    if (!tiles) diag[n] = lu_radii_diag(pri, dxidx, N, n, dt[n], phi, rr);
     bool inner = i >= e.is1 && i <= e.ie1 && j >= e.js1 && j <= e.je1 && k >= e.ks1 && k <= e.ke1;
 #pragma unroll
     for (int x = 0; x < 5; x++) {
@@ -233,8 +232,8 @@ __global__ void __launch_bounds__(256) k_lu_prep(Ext e, const double *__restrict
                  tiles);
 }
 
-// every block, for the batched tile sweeps (rhs and the time term; dq*
-// and dq are never touched); block m reads cfl[m * cfl_stride]
+// every block, for the batched tile sweeps (rhs only; dq* and dq are never
+// touched); block m reads cfl[m * cfl_stride]
 __global__ void __launch_bounds__(256) k_lu_prep_batch(const BlockRec *__restrict__ blks,
                                                        const int *__restrict__ map, const KGrid *__restrict__ kg,
                                                        double *arena, const double *cfl, int cfl_stride)
@@ -408,23 +407,27 @@ struct SlChunks {
     }
 };
 
-// csnd: the sound speed (component 7 of pri_v), tterm: the time term
+// csnd: the sound speed (component 7 of pri_v); dt: of which the time term
+// is formed
 __device__ inline const double *gather_src(int f, long N, const double *q, const double *dxidx,
-                                           const double *inv_j, const double *csnd, const double *tterm,
+                                           const double *inv_j, const double *csnd, const double *dt,
                                            const double *rhs)
 {
     return f < 9 ? dxidx + f * N : f == 9 ? inv_j : f < kSlC ? q + (f - kSlQ) * N
-         : f == kSlC ? csnd : f == kSlT ? tterm : rhs + (f - kSlOut) * N;
+         : f == kSlC ? csnd : f == kSlT ? dt : rhs + (f - kSlOut) * N;
 }
+
+// phi of sub_timeadvancement_1stimplicit.f90:98-102
+__device__ inline double lu_phi(const double *cfl) { return *cfl >= 1.0e3 ? 0.0 : 1.0; }
 
 // Gather the operands of every node into the sweep layout, a field pair at
 // a time (each lane then stores whole 16-byte pairs), from pair fp0 on (0:
 // all kSlF fields, kSlGeoPairs: all but the grid's).
 __device__ inline void sl_gather_tile(const Ext &e, const SlGeom &g, int tile, const double *__restrict__ q,
                                       const double *__restrict__ dxidx, const double *__restrict__ inv_j,
-                                      const double *__restrict__ csnd, const double *__restrict__ tterm,
-                                      const double *__restrict__ rhs, double *__restrict__ sl, int fp,
-                                      int part, int parts, double *buf /* [2][CT][TT] LDS, swizzled */)
+                                      const double *__restrict__ csnd, const double *__restrict__ dt,
+                                      const double *cfl, const double *__restrict__ rhs, double *__restrict__ sl,
+                                      int fp, int part, int parts, double *buf /* [2][CT][TT] LDS, swizzled */)
 {
     constexpr int CT = kSlCt, TT = kLanes, lstep = TT / CT;
     const int x = threadIdx.x;
@@ -446,10 +449,15 @@ __device__ inline void sl_gather_tile(const Ext &e, const SlGeom &g, int tile, c
         }
 #pragma unroll
         for (int h = 0; h < 2; h++) {
-            const double *src = gather_src(2 * fp + h, N, q, dxidx, inv_j, csnd, tterm, rhs);
+            const double *src = gather_src(2 * fp + h, N, q, dxidx, inv_j, csnd, dt, rhs);
             double v[CT];
 #pragma unroll
             for (int m = 0; m < CT; m++) v[m] = nat[m] >= 0 ? src[nat[m]] : 0.0;
+            if (2 * fp + h == kSlT) {
+                const double phi = lu_phi(cfl);
+#pragma unroll
+                for (int m = 0; m < CT; m++) v[m] = nat[m] >= 0 ? phi * 1.0 / v[m] : 0.0;
+            }
 #pragma unroll
             for (int m = 0; m < CT; m++) {
                 const int line = m * lstep + x / CT;
@@ -474,12 +482,12 @@ __global__ void __launch_bounds__(kLanes) k_sl_gather(Ext e, SlGeom g, const dou
                                                   const double *__restrict__ dxidx,
                                                   const double *__restrict__ inv_j,
                                                   const double *__restrict__ csnd,
-                                                  const double *__restrict__ tterm,
+                                                  const double *__restrict__ dt, const double *cfl,
                                                   const double *__restrict__ rhs, double *__restrict__ sl, int fp0,
                                                   int parts)
 {
     __shared__ double buf[2 * kSlCt * kLanes];
-    sl_gather_tile(e, g, (int)blockIdx.x, q, dxidx, inv_j, csnd, tterm, rhs, sl, fp0 + (int)blockIdx.y / parts,
+    sl_gather_tile(e, g, (int)blockIdx.x, q, dxidx, inv_j, csnd, dt, cfl, rhs, sl, fp0 + (int)blockIdx.y / parts,
                    (int)blockIdx.y % parts, parts, buf);
 }
 
@@ -560,14 +568,14 @@ static int sl_parts(int ntiles, int fields, int nsteps, int ct)
 }
 
 static void launch_layout(hipStream_t s, int which, const Ext &e, const SlGeom &g, const Fields &f, const LuWs &ws,
-                          int fp0 = 0)
+                          const double *cfl = nullptr, int fp0 = 0)
 {
     const int pairs = which == 0 ? kSlF / 2 - fp0 : kSlF / 2 - kSlOut / 2;
     const int parts = sl_parts(g.ntiles, pairs, g.nsteps, kSlCt);
     const dim3 gr((unsigned)g.ntiles, (unsigned)(pairs * parts));
     if (which == 0)
-        hipLaunchKernelGGL(k_sl_gather, gr, dim3(kLanes), 0, s, e, g, f.q, f.dxidx, f.inv_j, f.pri + 6 * e.n, f.w_diag,
-                           f.rhs, ws.sl, fp0, parts);
+        hipLaunchKernelGGL(k_sl_gather, gr, dim3(kLanes), 0, s, e, g, f.q, f.dxidx, f.inv_j, f.pri + 6 * e.n, f.dt,
+                           cfl, f.rhs, ws.sl, fp0, parts);
     else
         hipLaunchKernelGGL(k_sl_add, gr, dim3(kLanes), 0, s, e, g, ws.sl, f.q, parts);
 }
@@ -1044,14 +1052,15 @@ __global__ void __launch_bounds__(kPipeThreads, 2) k_lu_pipe(SlGeom g, double *_
 struct LuBatchEnt {
     Ext e;
     SlGeom g;
-    long q, dxidx, inv_j, csnd, tterm, rhs;
+    long q, dxidx, inv_j, csnd, dt, rhs;
     long sl, ex;
-    int tile0;
+    int tile0, blk;  // first tile number, block of the context
 };
 
 __global__ void __launch_bounds__(kLanes) k_sl_gather_batch(const LuBatchEnt *__restrict__ ents,
                                                         const int *__restrict__ tile_ent, double *arena,
-                                                        double *slb, int fp0, int parts)
+                                                        const double *cfl, int cfl_stride, double *slb, int fp0,
+                                                        int parts)
 {
     __shared__ double buf[2 * kSlCt * kLanes];
     const int flat = (int)blockIdx.x;
@@ -1059,8 +1068,8 @@ __global__ void __launch_bounds__(kLanes) k_sl_gather_batch(const LuBatchEnt *__
     const Ext e = b.e;
     const SlGeom g = b.g;
     sl_gather_tile(e, g, flat - b.tile0, arena + b.q, arena + b.dxidx, arena + b.inv_j, arena + b.csnd,
-                       arena + b.tterm, arena + b.rhs, slb + b.sl, fp0 + (int)blockIdx.y / parts, (int)blockIdx.y % parts,
-                   parts, buf);
+                   arena + b.dt, cfl + (long)b.blk * cfl_stride, arena + b.rhs, slb + b.sl,
+                   fp0 + (int)blockIdx.y / parts, (int)blockIdx.y % parts, parts, buf);
 }
 
 __global__ void __launch_bounds__(kLanes) k_sl_add_batch(const LuBatchEnt *__restrict__ ents,
@@ -1543,7 +1552,8 @@ int lusgs_batch_make(int nblk, const Ext *e, const Fields *f, double *arena, dou
         b.dxidx = f[m].dxidx - arena;
         b.inv_j = f[m].inv_j - arena;
         b.csnd = f[m].pri + 6 * e[m].n - arena;
-        b.tterm = f[m].w_diag - arena;
+        b.dt = f[m].dt - arena;
+        b.blk = m;
         b.rhs = f[m].rhs - arena;
         b.sl = so;
         b.ex = xo;
@@ -1623,7 +1633,8 @@ static void launch_pipe_batch(hipStream_t s, const LuBatch &b, double gamma, int
 // (phase 0, the per-node preparation, stays per block).  geo_cached: the
 // sweep layout already holds this batch's grid operands (phase 1 then
 // gathers the other fields only).
-int launch_lusgs_batch(hipStream_t s, const LuBatch &b, int phase, double gamma, int *err, int *ctr, int geo_cached)
+int launch_lusgs_batch(hipStream_t s, const LuBatch &b, int phase, double gamma, int *err, int *ctr, const double *cfl,
+                       int cfl_stride, int geo_cached)
 {
     if (b.total <= 0 || phase < 1 || phase > 4) return 0;
     const LuBatchEnt *ents = (const LuBatchEnt *)b.ents;
@@ -1631,7 +1642,7 @@ int launch_lusgs_batch(hipStream_t s, const LuBatch &b, int phase, double gamma,
     const int parts = sl_parts(b.total, pairs, b.nsteps, kSlCt);
     if (phase == 1)
         hipLaunchKernelGGL(k_sl_gather_batch, dim3((unsigned)b.total, (unsigned)(pairs * parts)), dim3(kLanes), 0, s, ents,
-                           b.tile_ent, b.arena, b.sl, fp0, parts);
+                           b.tile_ent, b.arena, cfl, cfl_stride, b.sl, fp0, parts);
     else if (phase == 2) launch_pipe_batch<1>(s, b, gamma, err, ctr);
     else if (phase == 3) launch_pipe_batch<-1>(s, b, gamma, err, ctr);
     else if (!b.fuse_add)
@@ -1781,8 +1792,9 @@ static void launch_pipe(hipStream_t s, const SlGeom &g, const LuWs &ws, double g
 
 // Phases of one LU-SGS update:
 //   0 rhs and, for hyperplanes, spectral radii and diag (and dq* and dq
-//     cleared), for tiles the time term phi/dt,
-//   1 tiles: gather the operands into the sweep layout (with geo_cached,
+//     cleared),
+//   1 tiles: gather the operands, with the time term phi/dt, into the
+//     sweep layout (with geo_cached,
 //     which says that it already holds this block's grid operands in this
 //     tiling, all but those),
 //   2 forward sweep, 3 backward sweep,
@@ -1803,7 +1815,7 @@ int launch_lusgs_phase(hipStream_t s, const Ext &e, const Fields &f, const Const
     } else if (tiles) {
         const SlGeom g = sl_geom(e);
         const bool fuse = fused_add(computed_nodes(e));
-        if (phase == 1) launch_layout(s, 0, e, g, f, *ws, geo_cached ? kSlGeoPairs : 0);
+        if (phase == 1) launch_layout(s, 0, e, g, f, *ws, cfl, geo_cached ? kSlGeoPairs : 0);
         else if (phase == 2) launch_pipe<1>(s, g, *ws, c.gamma, e, nullptr);
         else if (phase == 3) launch_pipe<-1>(s, g, *ws, c.gamma, e, fuse ? f.q : nullptr);
         else if (!fuse) launch_layout(s, 1, e, g, f, *ws);

@@ -12,10 +12,11 @@ int launch_fill(hipStream_t s, double *p, long n, double v);
 // clear: rhsi may not be zero outside the computed range
 int launch_inviscid(hipStream_t s, const Ext &e, const Fields &f, const Consts &c, int precision, int run, bool clear);
 int inviscid_run(long nodes, int precision);
-// part 1, 2: only the node, the difference pass; prep_cfl: that pass forms implicit1st's
-// rhs and (with the cfl it points to) time term and stores no rhsv
+// part 1, 2: only the node, the difference pass; prep: that pass forms
+// implicit1st's rhs and stores no rhsv, and with cfl given it also does the
+// unsteady find_dt
 int launch_viscous(hipStream_t s, const Ext &e, const Fields &f, const Consts &c, int precision,
-                   int store_aux, int part = -1, const double *prep_cfl = nullptr);
+                   int store_aux, int part = -1, bool prep = false, double *cfl = nullptr, double *cfl_blk = nullptr);
 // unsteady: the local cfl of the block's last node goes to *cfl and, when
 // not null, *cfl_blk
 int launch_find_dt(hipStream_t s, const Ext &e, const Fields &f, const Consts &c, double *cfl, double *cfl_blk,
@@ -74,19 +75,19 @@ int launch_getpri_batch(hipStream_t s, const BlockRec *blks, const BatchGrid &bg
 int launch_inviscid_batch(hipStream_t s, const BlockRec *blks, const BatchGrid *bg, double *arena,
                           const Consts &c, int precision, int run, int part = -1);
 int launch_viscous_batch(hipStream_t s, const BlockRec *blks, const BatchGrid &bg, double *arena, const Consts &c,
-                         int precision, int store_aux, int part = -1, const double *prep_cfl = nullptr);
+                         int precision, int store_aux, int part = -1, bool prep = false, int nblk = 0,
+                         double *cfl = nullptr, double *cfl_blk = nullptr);
 // the viscous stage with the steady find_dt folded into its node pass
 // (statistics into stats from the last block; reset them first); with
-// prep, also what launch_lu_prep_batch forms for the tile sweeps: the time
-// term phi/dt (node pass) and rhs = rhsi + rhsv (difference pass, which
-// then does not store rhsv: launch_viscous_batch part 2 forms it again from
-// the node fluxes)
+// prep, also what launch_lu_prep_batch forms for the tile sweeps: rhs = rhsi
+// + rhsv (difference pass, which then does not store rhsv:
+// launch_viscous_batch part 2 forms it again from the node fluxes)
 int launch_viscous_dt_batch(hipStream_t s, const BlockRec *blks, int nblk, const BatchGrid &bg, double *arena,
                             const Consts &c, int precision, int store_aux, const double *cfl,
                             unsigned long long *stats, int part = -1, int prep = 0);
 int launch_find_dt_batch(hipStream_t s, const BlockRec *blks, int nblk, const BatchGrid &bg, double *arena,
                          const Consts &c, double *cfl, double *cfl_blk, unsigned long long *stats);
-// rhs and the time term phi/dt of the batched tile sweeps
+// rhs of the batched tile sweeps
 int launch_lu_prep_batch(hipStream_t s, const BlockRec *blks, const BatchGrid &bg, double *arena, const double *cfl,
                          int cfl_stride);
 int launch_residual_batch(hipStream_t s, const BlockRec *blks, int nblk, double *arena, double *partial,
@@ -142,8 +143,9 @@ void lusgs_batch_ws(int nblk, const Ext *e, long *sl_n, long *ex_n);
 int lusgs_batch_make(int nblk, const Ext *e, const Fields *f, double *arena, double *sl, double *ex,
                      LuBatch *out);
 void lusgs_batch_free(LuBatch *b);
-int launch_lusgs_batch(hipStream_t s, const LuBatch &b, int phase, double gamma, int *err, int *ctr,
-                       int geo_cached = 0);
+// block m's gather reads its cfl at cfl[m * cfl_stride]
+int launch_lusgs_batch(hipStream_t s, const LuBatch &b, int phase, double gamma, int *err, int *ctr, const double *cfl,
+                       int cfl_stride, int geo_cached = 0);
 
 int launch_fill_sentinel(hipStream_t s, double *p, long n);
 // tile sweeps of the SA model's scalar LU-SGS (cu = a, b, c, diag)
@@ -220,6 +222,10 @@ struct AvgList {
 };
 int launch_average(hipStream_t s, const AvgList &al, double *const *q_tab, double *const *nut_tab,
                    const long *n_tab, double *buf, int with_nut);
+// both in one launch and average2 (the caller knows that neither list writes
+// what the other reads)
+int launch_halo_average(hipStream_t s, const CopyList &cl, const AvgList &al, double *const *q_tab,
+                        double *const *nut_tab, const long *n_tab, double *buf, int with_nut);
 
 int launch_residual(hipStream_t s, const Ext &e, const Fields &f, double *partial, int with_sa);
 int residual_partials(const Ext &e);

@@ -1,5 +1,6 @@
-"""A step whose viscous difference pass forms implicit1st's rhs and time term
-against the same step taken stage by stage: the flow, rhs, rhsv (which
+"""A step whose viscous difference pass forms implicit1st's rhs and does the
+unsteady find_dt, and whose halo fill and average1 share a launch, against
+the same step taken stage by stage: the flow, rhs, rhsv (which
 the step leaves out and a download forms), dt and its statistics are equal bit for bit."""
 import numpy as np
 import pytest
