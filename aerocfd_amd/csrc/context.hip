@@ -542,7 +542,7 @@ int ensure_block_table(acfd_ctx *ctx)
 // block that it shares nodes with (either writes what the other reads or
 // writes), so the values are those of the reference's order.  The six faces
 // of a box take three rounds, each launch 5-10 us for a few thousand nodes
-// whatever it holds: 81^3 RK3 step 131 -> 65 us of boundary conditions.
+// whatever it holds: 81^3 RK3 step 132 -> 82 us of boundary conditions.
 int build_bc_rounds(acfd_ctx *ctx)
 {
     for (size_t r = 0; r < ctx->bg_bc.size(); r++) {

@@ -306,7 +306,7 @@ __device__ inline void sensor_count(unsigned long long *stats, unsigned long lon
 // instructions and, on small blocks, by their latency.  81^3, all three
 // directions, a stage: WENO5 splitting 230 us with the written-out
 // candidates (100 divisions a face) and 64-wide tiles of 81-node rows, 91
-// now; WCNS on 1024 x 512 x 4 226, now 191.  Reading the next node a step
+// now; WCNS on 1024 x 512 x 4 226, now 182.  Reading the next node a step
 // ahead gave scheme 1 2 % and took 2 % from scheme 2: not done.
 // SENS: 0 plain; 1 the network decides per face (and records the decisions
 // in sa.mask when given); 2 the decisions are read from sa.mask

@@ -50,11 +50,12 @@ BYTES_PER_NODE = {
     # tile sweeps over the sweep layout: 22 operands in, 5 results out
     "lusgs_forward": 22 * 8 + 40,                   # dxidx, inv_j, q, c, phi/dt, rhs -> dq*
     "lusgs_backward": 22 * 8 + 40,                  # dxidx, inv_j, q, c, phi/dt, dq* -> q + dq
-    # 12 operands in (natural) and out (sweep layout): the 10 grid operands
-    # stay in the sweep layout from one update of a block to the next
+    # 12 operands in (natural; dt for phi/dt) and out (sweep layout): the 10
+    # grid operands stay in the sweep layout from one update of a block to
+    # the next
     "lusgs_gather": 2 * 12 * 8,
     "lusgs_add": 40 + 40,                           # q + dq (sweep layout) -> q
-    "lusgs_other": 8 + 80 + 40 + 8,                 # dt, rhsi+rhsv -> rhs, phi/dt (tile sweeps)
+    "lusgs_other": 80 + 40,                         # rhsi+rhsv -> rhs (tile sweeps)
     # SA scalar sweeps: a, b, c, diag and rhs (forward) / dnut* (backward)
     # in, dnut* / dnut out
     "sa_forward": 5 * 8 + 8,
@@ -114,34 +115,32 @@ HYPERPLANE_BYTES = {  # the hyperplane sweeps read the operands in place
 # HBM bytes per launch of the timed kernels, from two rocprofv3 --pmc runs
 # (FETCH_SIZE, WRITE_SIZE) scaled by a 1 GiB copy read through the same
 # counters.  The channel with bump at FP64, batched stages and sweeps
-# (profiles/channel_bump_fp64_hbm_traffic.md); the sweeps' figures include
-# the refill of the exchange slots that shares their timer.
+# (profiles/channel_bump_fp64_hbm_traffic.md).
 MEASURED_TRAFFIC_CHANNEL = {
-    "getpri": 10.033e9,
-    "inviscid_i": 11.021e9,
-    "inviscid_j": 17.097e9,
-    "inviscid_k": 17.817e9,
-    "viscous_node_dt": 30.728e9,
-    "viscous_diff": 20.763e9,
-    "lusgs_gather": 23.392e9,
-    "lusgs_forward": 28.469e9,
-    "lusgs_backward": 28.466e9,
-    "lusgs_add": 9.256e9,
-    "sa_pre": 17.185e9,
-    "sa_pre_b": 24.725e9,
-    "sa_gather": 9.872e9,
-    "sa_forward": 6.167e9,
-    "sa_backward": 6.158e9,
+    "getpri": 10.035e9,
+    "inviscid_i": 11.019e9,
+    "inviscid_j": 17.098e9,
+    "inviscid_k": 17.812e9,
+    "viscous_node_dt": 29.872e9,
+    "viscous_diff": 20.764e9,
+    "lusgs_gather": 23.470e9,
+    "lusgs_forward": 28.875e9,
+    "lusgs_backward": 28.883e9,
+    "lusgs_add": 9.261e9,
+    "sa_pre": 17.184e9,
+    "sa_pre_b": 24.719e9,
+    "sa_gather": 9.829e9,
+    "sa_forward": 6.183e9,
+    "sa_backward": 6.181e9,
     "sa_add": 3.286e9,
 }
 # The TGV 256^3 block, FP64, tile sweeps (profiles/tgv256_fp64_hbm_traffic.md).
 MEASURED_TRAFFIC_256 = {
     "getpri": 1.687e9,
-    "lusgs_other": 2.322e9,
-    "lusgs_gather": 4.092e9,
-    "lusgs_forward": 4.456e9,
-    "lusgs_backward": 4.456e9,
-    "lusgs_add": 1.576e9,
+    "lusgs_gather": 4.090e9,
+    "lusgs_forward": 4.569e9,
+    "lusgs_backward": 4.574e9,
+    "lusgs_add": 1.578e9,
 }
 
 
@@ -370,12 +369,11 @@ def roofline_of(args, tm, rr, sa, derived=False, length_kept=False):
         table["sa_pre"] = SA_PRE_DERIVED
     if sa and length_kept and args.lusgs == 2:
         table["sa_pre"] -= SA_PRE_LENGTH_KEPT
-    # the viscous node pass with the steady find_dt: + rho, c in, dt out;
-    # when it also forms implicit1st's preparation (batched sweeps, no
-    # separate preparation timed): + the time term phi/dt out, and the
-    # difference pass + rhsi in, rhs out, rhsv not stored
-    folded = args.lusgs == 2 and tm.get("lusgs_other", (0, 0))[1] == 0 and tm.get("viscous_node_dt", (0, 0))[1] > 0
-    table["viscous_node_dt"] = table["viscous_node"] + 16 + 8 + (8 if folded else 0)
+    # the viscous node pass with the steady find_dt: + rho, c in, dt out; the
+    # difference pass when it forms implicit1st's rhs (tile sweeps, no
+    # separate preparation timed): + rhsi in, rhs out, rhsv not stored
+    folded = args.lusgs != 0 and tm.get("lusgs_other", (0, 0))[1] == 0 and tm.get("lusgs_forward", (0, 0))[1] > 0
+    table["viscous_node_dt"] = table["viscous_node"] + 16 + 8
     if folded:
         table["viscous_diff"] = BYTES_PER_NODE["viscous_diff"] + 40
     if args.lusgs == 0:
