@@ -33,6 +33,20 @@ __device__ inline R weno3(R far, R near, R other)
     return w1 * ((R)1.5 * near - (R)0.5 * far) + w2 * ((R)0.5 * (near + other));
 }
 
+// Both WENO3 states of the face between w[1] and w[2] in FP64, from the first
+// differences, as corrections to the value next to the face: 31
+// instructions instead of 46 for the two, which share a difference and its
+// weight, and less rounding (a correction's is that of the differences).
+__device__ inline void weno3_pair(const double *w, double &l, double &r)
+{
+    const double eps = 1.0e-6;
+    const double e1 = w[1] - w[0], e2 = w[2] - w[1], e3 = w[3] - w[2];
+    const double t1 = fma(e1, e1, eps), t2 = fma(e2, e2, eps), t3 = fma(e3, e3, eps);
+    const double T1 = 2.0 * (t1 * t1), T2 = t2 * t2, T3 = 2.0 * (t3 * t3);
+    l = fma(0.5 * fma(T1, e2, T2 * e1), rcp_pos<double>(T2 + T1), w[1]);
+    r = fma(-0.5 * fma(T3, e2, T2 * e3), rcp_pos<double>(T2 + T3), w[2]);
+}
+
 // Roe flux with Harten's entropy fix (delta = 0.06) on a face with metric
 // (mx,my,mz) from primitive left/right states (d,u,v,w,p);
 // sub_inviscid_splitting.f90:65-162.

@@ -109,15 +109,31 @@ int launch_fill(hipStream_t s, double *p, long n, double v)
 // Flux through the face between nodes a and a+1 of one line from the four
 // values w[0..3] = q at a-1, a, a+1, a+2 of every component (alo / ahi are
 // the extended range ends: first order there) and the face metric.
-template <typename R>
+// With SPLIT (FP64, the i and k directions) a face away from the ends branches
+// past the selects, one variable at a time: the compiler otherwise makes one
+// block of the face and moves the loads to its end.  12 blocks of 3.2 M
+// nodes, i / j / k, us: two weno3 states each 106 / 159 / 153, the shared
+// differences of weno3_pair 99 / 148 / 169, with SPLIT 92 / 186 / 137, so the
+// j direction goes without.
+template <typename R, bool SPLIT>
 __device__ inline void face_flux_w(const R (*w)[4], int a, int alo, int ahi, R mx, R my, R mz, R gamma,
                                    R *F)
 {
     R ul[5], ur[5];
 #pragma unroll
     for (int v = 0; v < 5; v++) {
-        ul[v] = a == alo ? w[v][1] : weno3<R>(w[v][0], w[v][1], w[v][2]);
-        ur[v] = a == ahi - 1 ? w[v][2] : weno3<R>(w[v][3], w[v][2], w[v][1]);
+        if constexpr (sizeof(R) == 8) {
+            weno3_pair(w[v], ul[v], ur[v]);
+            if (SPLIT && a > alo && a < ahi - 1) {
+                __asm__ volatile("" : "+v"(ul[v]), "+v"(ur[v]));
+            } else {
+                if (a == alo) ul[v] = w[v][1];
+                if (a == ahi - 1) ur[v] = w[v][2];
+            }
+        } else {
+            ul[v] = a == alo ? w[v][1] : weno3<R>(w[v][0], w[v][1], w[v][2]);
+            ur[v] = a == ahi - 1 ? w[v][2] : weno3<R>(w[v][3], w[v][2], w[v][1]);
+        }
     }
     R pl[5], pr[5];
     cons2prim<R>(ul, pl, gamma);
@@ -168,7 +184,7 @@ __device__ inline void inviscid_i_body(const Ext &e, int bx, int by, int bz, con
     double m[3];
     face_metric(dxidx, inv_j, N, n, 1, 0, m);
     R F[5];
-    face_flux_w<R>(w, a, e.is, e.ie, (R)m[0], (R)m[1], (R)m[2], (R)gamma, F);
+    face_flux_w<R, true>(w, a, e.is, e.ie, (R)m[0], (R)m[1], (R)m[2], (R)gamma, F);
     double Fm[5];
 #pragma unroll
     for (int v = 0; v < 5; v++) Fm[v] = __shfl_up((double)F[v], 1, 64);
@@ -207,9 +223,9 @@ int inviscid_run(long nodes, int precision)
     if (precision == 1) return kInvRunF32;
     return nodes < 100000 ? 1 : nodes < 4000000 ? 4 : nodes < 32000000 ? 8 : 16;
 }
-// Waves per SIMD asked of the k kernel: FP64 it needs 176 VGPRs (two
-// waves); held to 168 with a few values in scratch it runs three, and on
-// the 40-block channel takes 3.84 ms instead of 4.32.  The same bound on
+// Waves per SIMD asked of the k kernel: left to itself its batched FP64 form
+// takes 174 VGPRs (two waves), held to 168 it runs three (when it needed
+// 176, 3.84 ms instead of 4.32 on the 40-block channel).  The same bound on
 // the j kernel (four waves: 22 values in scratch) or four on the k kernel
 // is slower by a third or more.
 constexpr int kInvKWaves = 3;
@@ -257,7 +273,7 @@ __device__ inline void inviscid_jk_body(const Ext &e, int run_, int bx, int by, 
     {
         double m[3];
         face_metric(dxidx, inv_j, N, n, st, c0, m);
-        face_flux_w<R>(w, a0 - 1, alo, ahi, (R)m[0], (R)m[1], (R)m[2], (R)gamma, Fm);
+        face_flux_w<R, AXIS == 2>(w, a0 - 1, alo, ahi, (R)m[0], (R)m[1], (R)m[2], (R)gamma, Fm);
     }
     for (int a = a0; a <= a1; a++) {
         n += st;
@@ -271,7 +287,7 @@ __device__ inline void inviscid_jk_body(const Ext &e, int run_, int bx, int by, 
         }
         double m[3];
         face_metric(dxidx, inv_j, N, n, st, c0, m);
-        face_flux_w<R>(w, a, alo, ahi, (R)m[0], (R)m[1], (R)m[2], (R)gamma, Fp);
+        face_flux_w<R, AXIS == 2>(w, a, alo, ahi, (R)m[0], (R)m[1], (R)m[2], (R)gamma, Fp);
 #pragma unroll
         for (int v = 0; v < 5; v++) {
             rhsi[v * N + n] = rhsi[v * N + n] - ((double)Fp[v] - (double)Fm[v]);
