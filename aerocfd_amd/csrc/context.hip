@@ -674,8 +674,6 @@ int alloc_lu_ws(acfd_ctx *ctx, bool may_pick)
         ctx->lu.ex = (double *)uc_acquire((size_t)ex_n * sizeof(double));
         if (!ctx->lu.ex) return fail(ACFD_EDEVICE, "uncached device memory for the tile exchange is unavailable");
     }
-    // idle lanes of the sweeps read the padding of the layout: defined values
-    HIP_TRY(hipMemsetAsync(ctx->lu.sl, 0, (size_t)sl_n * sizeof(double), ctx->stream));
     HIP_TRY(hipMalloc((void **)&ctx->lu.err, sizeof(int)));
     HIP_TRY(hipMemsetAsync(ctx->lu.err, 0, sizeof(int), ctx->stream));
     ctx->lu_ex_n = ex_n;

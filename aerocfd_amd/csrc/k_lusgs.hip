@@ -631,9 +631,11 @@ __device__ inline double lu_node_radii(const double *op, double *r)
 // 507 -> 350, 40 blocks of 98 M nodes 6.19 -> 6.10 ms (4.7 TB/s).  Tiles of
 // 16 x 16, 16 x 8 and 16 x 4 lines of the one-wavefront form were slower at
 // every one of these sizes and are gone.
-// A lane with nothing to do at a step takes part with rhs, 1/(diag inv_j)
-// and so its products zero (the padding of the sweep layout holds zeros or
-// another block's operands, finite either way), and no lane branches.
+// A lane with nothing to do at a step takes part with zeros, which it is
+// given when the step is prepared (rho 1, every other operand and both
+// reciprocals 0), so that its products are zero and no lane branches.  It
+// takes nothing from its row of the layout: the blocks of a context share
+// the layout, and the row may hold operands of another block, NaN among them.
 constexpr int kPipeRing = 4;    // steps of prepared operands in LDS
 constexpr int kPipeXRing = 16;  // steps of neighbour values in LDS
 constexpr int kPipePrep = 2;    // preparing waves
@@ -728,9 +730,8 @@ __device__ inline void pipe_prepare(const SlGeom &g, int tile, int w, const doub
         const int li = row(s) - t0;
         const bool on = active && li >= 0 && li < g.Li;
         if (!on) {
-            op[kSlQ] = 1.0;
 #pragma unroll
-            for (int x = 0; x < 5; x++) op[kSlOut + x] = 0.0;
+            for (int f = 0; f < kSlF; f++) op[f] = f == kSlQ ? 1.0 : 0.0;
         }
         double rad[3];
         const double ri = 1.0 / op[kSlQ];
