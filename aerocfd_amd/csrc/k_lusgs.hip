@@ -127,19 +127,24 @@ __device__ inline void jac_mv(const double *__restrict__ q, const double *__rest
 }
 
 // A divisor known before its dividends: x / d from y = 1/d (rounded), the
-// quotient estimate x y and one correction by its remainder, in three
-// operations in place of a division's dozen.  The correction step rounds
-// the quotient as the division does (Markstein, IBM J. Res. Dev. 34, 1990),
-// so the sweeps' results are those of the reference's two divisions.  An
-// infinite d (dt = 0) has y = 0 and d held as 0: the quotient is 0.
+// quotient estimate x y, one correction by its remainder and the division's
+// own last instruction, four operations in place of a dozen.  The correction
+// rounds the quotient as the division does (Markstein, IBM J. Res. Dev. 34,
+// 1990), so the sweeps' results are those of the reference's two divisions,
+// for a normal quotient and |x| of at least 2^-969: below that the remainder
+// itself is rounded, and the quotient's last bit can differ.  v_div_fixup
+// gives the quotients of infinities, zeros and NaN, which the estimate makes
+// NaN (an infinite diag, of dt = 0, gives 0); without it, 2 % less time on a
+// block of 33^3 and 0.6 % on 129^3.  One test a step for a NaN, and the
+// divisions then, took 4 and 2 %.
 struct LuDivisor {
     double d, y;
 };
-__device__ inline LuDivisor lu_divisor(double d) { return {isinf(d) ? 0.0 : d, 1.0 / d}; }
+__device__ inline LuDivisor lu_divisor(double d) { return {d, 1.0 / d}; }
 __device__ inline double lu_over(double x, const LuDivisor &b)
 {
     const double q = x * b.y;
-    return fma(fma(-q, b.d, x), b.y, q);
+    return __builtin_amdgcn_div_fixup(fma(fma(-q, b.d, x), b.y, q), b.d, x);
 }
 
 // forward node (:345-365): dq* = (rhs + A+ dq*_i-1 + B+ dq*_j-1 + C+ dq*_k-1)/diag/inv_j
@@ -632,8 +637,8 @@ __device__ inline double lu_node_radii(const double *op, double *r)
 // 16 x 16, 16 x 8 and 16 x 4 lines of the one-wavefront form were slower at
 // every one of these sizes and are gone.
 // A lane with nothing to do at a step takes part with zeros, which it is
-// given when the step is prepared (rho 1, every other operand and both
-// reciprocals 0), so that its products are zero and no lane branches.  It
+// given when the step is prepared (rho 1, every other operand 0, divisors 1
+// with reciprocals 0), so that its products are zero and no lane branches.  It
 // takes nothing from its row of the layout: the blocks of a context share
 // the layout, and the row may hold operands of another block, NaN among them.
 constexpr int kPipeRing = 4;    // steps of prepared operands in LDS
@@ -737,7 +742,7 @@ __device__ inline void pipe_prepare(const SlGeom &g, int tile, int w, const doub
         const double ri = 1.0 / op[kSlQ];
         const LuState t = lu_state(op + kSlQ, ri, op[9], gamma);
         LuDivisor dg = lu_divisor(lu_node_radii(op, rad)), ij = lu_divisor(op[9]);
-        if (!on) dg.d = dg.y = ij.d = ij.y = 0.0;
+        if (!on) dg.d = ij.d = 1.0, dg.y = ij.y = 0.0;
         LuRow m[3];
 #pragma unroll
         for (int d = 0; d < 3; d++) m[d] = lu_row<DIR>(t, op[3 * d], op[3 * d + 1], op[3 * d + 2], rad[d]);
