@@ -21,34 +21,22 @@
 
 namespace acfd {
 
-// x / y for a positive normal y: FP64 through rcp_pos, FP32 divides
-template <typename R>
-__device__ inline R over_pos(R x, R y)
-{
-    return x / y;
-}
-template <>
-__device__ inline double over_pos<double>(double x, double y)
-{
-    return x * rcp_pos<double>(y);
-}
-
 // Steger-Warming split fluxes through the node metric M = grad xi / J.
 template <typename R>
 __device__ inline void sw_split(const R *q, R mx, R my, R mz, R gamma, R *fp, R *fm)
 {
-    const R rho = q[0], ri = rcp_pos<R>(rho);
+    const R rho = q[0], ri = (R)1.0 / rho;
     const R u = q[1] * ri, v = q[2] * ri, w = q[3] * ri;
     const R v2 = u * u + v * v + w * w;
     const R p = (gamma - (R)1.0) * (q[4] - (R)0.5 * rho * v2);
     const R c = sqrt(gamma * p * ri);
     const R mm = sqrt(mx * mx + my * my + mz * mz);
-    const R rm = rcp_pos<R>(mm);
+    const R rm = (R)1.0 / mm;
     const R nx = mx * rm, ny = my * rm, nz = mz * rm;
     const R ut = u * nx + v * ny + w * nz;
-    const R h = over_pos<R>(c * c, gamma - (R)1.0) + (R)0.5 * v2;
+    const R h = c * c / (gamma - (R)1.0) + (R)0.5 * v2;
     const R l[3] = {mm * ut, mm * (ut + c), mm * (ut - c)};
-    const R s = over_pos<R>(rho, (R)2.0 * gamma);
+    const R s = rho / ((R)2.0 * gamma);
 #pragma unroll
     for (int side = 0; side < 2; side++) {
         R lp[3];
