@@ -212,11 +212,13 @@ __global__ void __launch_bounds__(256) k_inviscid_i(Ext e, const double *__restr
 // thousand of them.  Inviscid stage, us, at runs of 1 / 4 / 8 / 16: 33^3 26 /
 // 38 / 57 / 97, 65^3 50 / 47 / 63 / 101, 129^3 375 / 287 / 291 / 317, 193^3
 // 1174 / 893 / 889 / 932, 256^3 - / 1814 / 1729 / 1732, 98 M nodes in 40
-// blocks best at 16.  A run's first face is a second copy of the flux code,
-// rounded in its own way: the rule takes the context's nodes, not a
-// launch's, so that batched and per-block launches cut the same runs, and
-// FP32 fluxes, where an ulp is 1e-7, keep the run of 16 that they were
-// measured with.
+// blocks best at 16.  In FP64 every face goes through the one copy of the
+// flux code in the loop, so a face's value does not depend on the run that
+// holds it, nor a block's residual on what else its context holds (a copy
+// ahead of the loop for the first face, which the compiler contracts in its
+// own way: step 0.5 % faster at 193^3 and 129^3).  FP32 fluxes, where an ulp
+// is 1e-7, keep the run of 16 and the two copies that they were measured
+// with.
 constexpr int kInvRunF32 = 16;
 int inviscid_run(long nodes, int precision)
 {
@@ -269,29 +271,56 @@ __device__ inline void inviscid_jk_body(const Ext &e, int run_, int bx, int by, 
         w[v][2] = (R)qv[st];
         w[v][3] = (R)qv[2 * st];
     }
-    R Fm[5], Fp[5];
-    {
-        double m[3];
-        face_metric(dxidx, inv_j, N, n, st, c0, m);
-        face_flux_w<R, AXIS == 2>(w, a0 - 1, alo, ahi, (R)m[0], (R)m[1], (R)m[2], (R)gamma, Fm);
-    }
-    for (int a = a0; a <= a1; a++) {
-        n += st;
-        const long ahead = a + 2 <= ahi ? 2 * st : st;
-#pragma unroll
-        for (int v = 0; v < 5; v++) {
-            w[v][0] = w[v][1];
-            w[v][1] = w[v][2];
-            w[v][2] = w[v][3];
-            w[v][3] = (R)q[v * N + n + ahead];
+    if constexpr (sizeof(R) == 4) {  // see inviscid_run
+        R Fm[5], Fp[5];
+        {
+            double m[3];
+            face_metric(dxidx, inv_j, N, n, st, c0, m);
+            face_flux_w<R, AXIS == 2>(w, a0 - 1, alo, ahi, (R)m[0], (R)m[1], (R)m[2], (R)gamma, Fm);
         }
-        double m[3];
-        face_metric(dxidx, inv_j, N, n, st, c0, m);
-        face_flux_w<R, AXIS == 2>(w, a, alo, ahi, (R)m[0], (R)m[1], (R)m[2], (R)gamma, Fp);
+        for (int a = a0; a <= a1; a++) {
+            n += st;
+            const long ahead = a + 2 <= ahi ? 2 * st : st;
 #pragma unroll
-        for (int v = 0; v < 5; v++) {
-            rhsi[v * N + n] = rhsi[v * N + n] - ((double)Fp[v] - (double)Fm[v]);
-            Fm[v] = Fp[v];
+            for (int v = 0; v < 5; v++) {
+                w[v][0] = w[v][1];
+                w[v][1] = w[v][2];
+                w[v][2] = w[v][3];
+                w[v][3] = (R)q[v * N + n + ahead];
+            }
+            double m[3];
+            face_metric(dxidx, inv_j, N, n, st, c0, m);
+            face_flux_w<R, AXIS == 2>(w, a, alo, ahi, (R)m[0], (R)m[1], (R)m[2], (R)gamma, Fp);
+#pragma unroll
+            for (int v = 0; v < 5; v++) {
+                rhsi[v * N + n] = rhsi[v * N + n] - ((double)Fp[v] - (double)Fm[v]);
+                Fm[v] = Fp[v];
+            }
+        }
+    } else {
+        R Fm[5] = {0, 0, 0, 0, 0};
+        for (int a = a0 - 1; a <= a1; a++) {
+            double m[3];
+            R Fp[5];
+            face_metric(dxidx, inv_j, N, n, st, c0, m);
+            face_flux_w<R, AXIS == 2>(w, a, alo, ahi, (R)m[0], (R)m[1], (R)m[2], (R)gamma, Fp);
+            if (a >= a0) {
+#pragma unroll
+                for (int v = 0; v < 5; v++) rhsi[v * N + n] = rhsi[v * N + n] - ((double)Fp[v] - (double)Fm[v]);
+            }
+            if (a < a1) {
+                n += st;
+                const long ahead = a + 3 <= ahi ? 2 * st : st;
+#pragma unroll
+                for (int v = 0; v < 5; v++) {
+                    w[v][0] = w[v][1];
+                    w[v][1] = w[v][2];
+                    w[v][2] = w[v][3];
+                    w[v][3] = (R)q[v * N + n + ahead];
+                }
+            }
+#pragma unroll
+            for (int v = 0; v < 5; v++) Fm[v] = Fp[v];
         }
     }
 }
