@@ -188,7 +188,7 @@ struct acfd_ctx {
     // d_res holds the norms of the current rhs, dt and sa_rhs (set by
     // acfd_step, cleared by every call that writes fields)
     bool res_current = false;
-    int *lu_ctr = nullptr;   // ticket counters of the batched sweeps
+    int *lu_ctr = nullptr;   // counters that hand out the sweeps' tiles
     // SA's update runs beside the flow's LU-SGS update on a second stream
     // (batched sweeps, SA): its own exchange slots and ticket counters
     bool sa_concurrent = false;
@@ -678,8 +678,8 @@ int alloc_lu_ws(acfd_ctx *ctx, bool may_pick)
     HIP_TRY(hipMemsetAsync(ctx->lu.err, 0, sizeof(int), ctx->stream));
     ctx->lu_ex_n = ex_n;
     KRN_TRY(launch_fill_sentinel(ctx->stream, ctx->lu.ex, ex_n));
-    HIP_TRY(hipMalloc((void **)&ctx->lu_ctr, 2 * sizeof(int)));
-    HIP_TRY(hipMemsetAsync(ctx->lu_ctr, 0, 2 * sizeof(int), ctx->stream));
+    HIP_TRY(hipMalloc((void **)&ctx->lu_ctr, kTileCounters * sizeof(int)));
+    HIP_TRY(hipMemsetAsync(ctx->lu_ctr, 0, kTileCounters * sizeof(int), ctx->stream));
     ctx->lu.ctr = ctx->lu_ctr;
     lusgs_resident(ctx->lu.resident);
     if (batch) {
@@ -692,8 +692,8 @@ int alloc_lu_ws(acfd_ctx *ctx, bool may_pick)
             ctx->sa_ex = (double *)uc_acquire((size_t)ex_n * sizeof(double));
             if (!ctx->sa_ex) return fail(ACFD_EDEVICE, "uncached device memory for the tile exchange is unavailable");
             KRN_TRY(launch_fill_sentinel(ctx->stream, ctx->sa_ex, ex_n));
-            HIP_TRY(hipMalloc((void **)&ctx->sa_ctr, 2 * sizeof(int)));
-            HIP_TRY(hipMemsetAsync(ctx->sa_ctr, 0, 2 * sizeof(int), ctx->stream));
+            HIP_TRY(hipMalloc((void **)&ctx->sa_ctr, kTileCounters * sizeof(int)));
+            HIP_TRY(hipMemsetAsync(ctx->sa_ctr, 0, kTileCounters * sizeof(int), ctx->stream));
         }
         const char *rc_env = std::getenv("ACFD_RES_CONCURRENT");
         ctx->res_concurrent = ctx->c.solver == 0 && !(rc_env && std::atoi(rc_env) == 0);
@@ -721,12 +721,8 @@ int alloc_lu_ws(acfd_ctx *ctx, bool may_pick)
         if (sa && sa_batch_make(nb, es.data(), fs.data(), ctx->arena, ctx->sa_concurrent ? ctx->sa_ex : ctx->lu.ex,
                                 ctx->sa_sl, &ctx->sab))
             return fail(ACFD_EDEVICE, "batched SA sweep tables: device allocation failed");
-        if (ctx->sa_concurrent) {
-            // two persistent launches share the device: tiles by ticket
-            // (each waits only on tiles that are already running)
-            ctx->lub.resident[0] = ctx->lub.resident[1] = 0;
-            ctx->sab.resident[0] = ctx->sab.resident[1] = 0;
-        }
+        // beside SA's sweeps not all workgroups come together
+        if (ctx->sa_concurrent) ctx->lub.fits[0] = ctx->lub.fits[1] = 0;
     }
     HIP_TRY(hipStreamSynchronize(ctx->stream));
     return 0;
@@ -743,8 +739,8 @@ int tile_error(acfd_ctx *ctx)
         (void)launch_fill_sentinel(ctx->stream, ctx->lu.ex, ctx->lu_ex_n);
         if (ctx->sa_ex) (void)launch_fill_sentinel(ctx->stream, ctx->sa_ex, ctx->lu_ex_n);
         (void)hipMemsetAsync(ctx->lu.err, 0, sizeof(int), ctx->stream);
-        if (ctx->lu_ctr) (void)hipMemsetAsync(ctx->lu_ctr, 0, 2 * sizeof(int), ctx->stream);
-        if (ctx->sa_ctr) (void)hipMemsetAsync(ctx->sa_ctr, 0, 2 * sizeof(int), ctx->stream);
+        if (ctx->lu_ctr) (void)hipMemsetAsync(ctx->lu_ctr, 0, kTileCounters * sizeof(int), ctx->stream);
+        if (ctx->sa_ctr) (void)hipMemsetAsync(ctx->sa_ctr, 0, kTileCounters * sizeof(int), ctx->stream);
         (void)hipStreamSynchronize(ctx->stream);
         return fail(ACFD_EDEVICE, "pipelined LU-SGS sweep timed out waiting for a neighbouring tile");
     }
@@ -1045,7 +1041,8 @@ int st_sa(acfd_ctx *ctx, int m, const double *cfl)
     const Block &b = ctx->blk[m];
     if (ctx->lu_variant != 0 && ctx->lu.ex) {
         // tile sweeps in the flow sweep's exchange slots (idle, sentinel-filled)
-        const SaSweep sw{ctx->sa_ex ? ctx->sa_ex : ctx->lu.ex, ctx->lu.err};
+        const SaSweep sw{ctx->sa_ex ? ctx->sa_ex : ctx->lu.ex, ctx->lu.err,
+                         ctx->sa_ctr ? ctx->sa_ctr : ctx->lu_ctr};
         KRN_TRY(launch_sa(ctx->stream, b.e, b.f, ctx->c, cfl, &sw));
     } else {
         KRN_TRY(launch_sa(ctx->stream, b.e, b.f, ctx->c, cfl));

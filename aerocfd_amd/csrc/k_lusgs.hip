@@ -1010,39 +1010,59 @@ __device__ inline void pipe_body(const SlGeom &g, int tile, double *__restrict__
     }
 }
 
-// Tile numbers.  When every workgroup of the launch fits on the device at
-// once (ctr null), tile = workgroup index: all tiles run together and every
-// wait ends.  Otherwise the tiles are handed out in the order workgroups
+// Tile numbers.  The tiles are handed out in the order in which workgroups
 // start (a ticket counter): a tile then only ever waits on tiles whose
 // workgroups started before it, so the sweep progresses however the launch
-// is dispatched; the last workgroup to finish resets both counters for the
-// next launch.  (The first form is the faster one where it applies: the
-// hardware's placement of consecutive workgroups suits the sweep.)
-__device__ inline int pipe_ticket(int *ctr, int *ticket)
+// is dispatched and whatever else the device runs, other contexts' sweeps
+// among it.  Where tiles by workgroup number are the faster form (fits; the
+// hardware's placement of consecutive workgroups suits the sweep), the
+// workgroups first count themselves: when the last one has come, all are
+// running and every wait ends whatever the order, so each takes the tile of
+// its number; a workgroup that has polled kArrivePolls times without seeing
+// that (the device is shared) switches the launch to tickets, if it can do
+// so before the last one comes.  The last workgroup to finish resets the
+// counters for the next launch.
+constexpr int kByTicket = 1 << 30, kArrivePolls = 32;
+__device__ inline int tile_ticket(int *ctr, int total, bool fits, int *ticket)
 {
-    if (!ctr) return (int)blockIdx.x;
-    if (threadIdx.x == 0) *ticket = __hip_atomic_fetch_add(ctr, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (threadIdx.x == 0) {
+        int here = 0, t = (int)blockIdx.x;
+        if (fits) {
+            here = __hip_atomic_fetch_add(ctr + 2, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1;
+            for (int n = 0; here < total; n++) {
+                if (n < kArrivePolls) {
+                    __builtin_amdgcn_s_sleep(1);
+                    here = __hip_atomic_load(ctr + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                } else if (__hip_atomic_compare_exchange_strong(ctr + 2, &here, here | kByTicket, __ATOMIC_RELAXED,
+                                                                __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
+                    here |= kByTicket;
+                }
+            }
+        }
+        if (here != total) t = __hip_atomic_fetch_add(ctr, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        *ticket = t;
+    }
     __syncthreads();
     return __builtin_amdgcn_readfirstlane(*ticket);
 }
-__device__ inline void pipe_ticket_done(int *ctr, int total)
+__device__ inline void tile_done(int *ctr, int total)
 {
-    if (ctr && threadIdx.x == 0 &&
+    if (threadIdx.x == 0 &&
         __hip_atomic_fetch_add(ctr + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == total - 1) {
-        __hip_atomic_store(ctr, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(ctr + 1, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        for (int x = 0; x < kTileCounters; x++)
+            __hip_atomic_store(ctr + x, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
 }
 
 template <int DIR>
 __global__ void __launch_bounds__(kPipeThreads, 2) k_lu_pipe(SlGeom g, double *__restrict__ sl, double gamma, double *ex,
-                                                             int *err, int *ctr, Ext e, double *q)
+                                                             int *err, int *ctr, int fits, Ext e, double *q)
 {
     __shared__ PipeLds<DIR> L;
     __shared__ int ticket;
-    const int flat = pipe_ticket(ctr, &ticket);
+    const int flat = tile_ticket(ctr, g.ntiles, fits, &ticket);
     pipe_body<DIR>(g, DIR > 0 ? flat : g.ntiles - 1 - flat, sl, gamma, ex, err, L, &e, q);
-    pipe_ticket_done(ctr, g.ntiles);
+    tile_done(ctr, g.ntiles);
 }
 
 // ------------------------------------------------------------ batched tiles
@@ -1094,21 +1114,20 @@ __global__ void __launch_bounds__(kLanes) k_sl_add_batch(const LuBatchEnt *__res
 template <int DIR>
 __global__ void __launch_bounds__(kPipeThreads, 2) k_lu_pipe_batch(const LuBatchEnt *__restrict__ ents,
                                                                    const int *__restrict__ tile_ent, int total,
-                                                                   int resident, double *slb, double *exb,
+                                                                   int fits, double *slb, double *exb,
                                                                    double gamma, int *err, int *ctr, double *arena,
                                                                    int fuse_add)
 {
     __shared__ PipeLds<DIR> L;
     __shared__ int ticket;
-    int *c = resident ? nullptr : ctr;
-    const int flat = pipe_ticket(c, &ticket);
+    const int flat = tile_ticket(ctr, total, fits, &ticket);
     const LuBatchEnt &b = ents[tile_ent[flat]];
     const SlGeom g = b.g;
     const int local = flat - b.tile0;
     const Ext e = b.e;
     pipe_body<DIR>(g, DIR > 0 ? local : g.ntiles - 1 - local, slb + b.sl, gamma, exb + b.ex, err, L, &e,
                    fuse_add ? arena + b.q : nullptr);
-    pipe_ticket_done(c, total);
+    tile_done(ctr, total);
 }
 
 // ------------------------------------------------ scalar sweeps (SA model)
@@ -1289,10 +1308,13 @@ struct SaInPlace {
 template <int DIR>
 __global__ void __launch_bounds__(kLanes) k_sa_tiles(Ext e, SaGeom g, const double *__restrict__ cu,
                                                       const double *__restrict__ rhs, double *__restrict__ dns,
-                                                      double *__restrict__ dn, double *ex, int *err)
+                                                      double *__restrict__ dn, double *ex, int *err, int *ctr)
 {
-    const int tile = DIR > 0 ? (int)blockIdx.x : g.ntiles - 1 - (int)blockIdx.x;
+    __shared__ int ticket;
+    const int flat = tile_ticket(ctr, g.ntiles, false, &ticket);
+    const int tile = DIR > 0 ? flat : g.ntiles - 1 - flat;
     sa_sweep_body<DIR>(g, tile, SaInPlace<DIR>(e, g, tile, cu, rhs, dns, dn), ex, err);
+    tile_done(ctr, g.ntiles);
 }
 
 struct SaBatchEnt {
@@ -1307,16 +1329,11 @@ struct SaBatchEnt {
 template <int DIR>
 __global__ void __launch_bounds__(kLanes) k_sa_tiles_batch(const SaBatchEnt *__restrict__ ents,
                                                             const int *__restrict__ tile_ent, int total,
-                                                            int resident, double *arena, double *exb, int *err,
+                                                            double *arena, double *exb, int *err,
                                                             int *ctr)
 {
     __shared__ int ticket;
-    if (!resident) {
-        if (threadIdx.x == 0)
-            ticket = __hip_atomic_fetch_add(ctr, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __syncthreads();
-    }
-    const int flat = resident ? (int)blockIdx.x : __builtin_amdgcn_readfirstlane(ticket);
+    const int flat = tile_ticket(ctr, total, false, &ticket);
     const SaBatchEnt &b = ents[tile_ent[flat]];
     const Ext e = b.e;
     const SaGeom g = b.g;
@@ -1324,11 +1341,7 @@ __global__ void __launch_bounds__(kLanes) k_sa_tiles_batch(const SaBatchEnt *__r
     sa_sweep_body<DIR>(g, tile,
                        SaInPlace<DIR>(e, g, tile, arena + b.cu, arena + b.rhs, arena + b.dns, arena + b.dn),
                        exb + b.ex, err);
-    if (!resident && threadIdx.x == 0 &&
-        __hip_atomic_fetch_add(ctr + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == total - 1) {
-        __hip_atomic_store(ctr, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(ctr + 1, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
+    tile_done(ctr, total);
 }
 
 // ---- scalar sweeps over an SA sweep layout (every block in one launch)
@@ -1459,26 +1472,17 @@ struct SaRows {
 
 template <int DIR>
 __global__ void __launch_bounds__(kLanes) k_sa_sl_batch(const SaBatchEnt *__restrict__ ents,
-                                                         const int *__restrict__ tile_ent, int total, int resident,
+                                                         const int *__restrict__ tile_ent, int total,
                                                          double *slbase, double *exb, int *err, int *ctr)
 {
     __shared__ int ticket;
-    if (!resident) {
-        if (threadIdx.x == 0)
-            ticket = __hip_atomic_fetch_add(ctr, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __syncthreads();
-    }
-    const int flat = resident ? (int)blockIdx.x : __builtin_amdgcn_readfirstlane(ticket);
+    const int flat = tile_ticket(ctr, total, false, &ticket);
     const SaBatchEnt &b = ents[tile_ent[flat]];
     const SaGeom g = b.g;
     const int local = flat - b.tile0, tile = DIR > 0 ? local : g.ntiles - 1 - local;
     sa_sweep_body<DIR>(g, tile, SaRows<DIR>{slbase + b.sl + sa_slot(g, tile, 0, 0, (int)threadIdx.x), g.nsteps},
                        exb + b.ex, err);
-    if (!resident && threadIdx.x == 0 &&
-        __hip_atomic_fetch_add(ctr + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == total - 1) {
-        __hip_atomic_store(ctr, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(ctr + 1, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
+    tile_done(ctr, total);
 }
 
 static long lusgs_tiles(const Ext &e)
@@ -1597,8 +1601,7 @@ void lusgs_batch_free(LuBatch *b)
     b->nent = b->total = 0;
 }
 
-// whether all `total` workgroups of the sweep kernel fit on the device at once
-// workgroups of the kernel that fit on the device at once (0: unknown)
+// workgroups of the kernel that the device holds (0: unknown)
 template <typename K>
 static int resident_wgs(K kernel, int threads)
 {
@@ -1610,28 +1613,42 @@ static int resident_wgs(K kernel, int threads)
     return cus * per_cu;
 }
 
-void lusgs_resident(int *tiles)
+// ACFD_LU_TICKETS=1: by ticket whatever fits
+static bool tickets_only()
 {
     const char *t = std::getenv("ACFD_LU_TICKETS");
-    const bool tickets = t && std::atoi(t) == 1;
-    tiles[0] = tickets ? 0 : resident_wgs(k_lu_pipe<1>, kPipeThreads);
-    tiles[1] = tickets ? 0 : resident_wgs(k_lu_pipe<-1>, kPipeThreads);
+    return t && std::atoi(t) == 1;
 }
+
+void lusgs_resident(int *wgs)
+{
+    const bool t = tickets_only();
+    wgs[0] = t ? 0 : resident_wgs(k_lu_pipe<1>, kPipeThreads);
+    wgs[1] = t ? 0 : resident_wgs(k_lu_pipe<-1>, kPipeThreads);
+}
+
+// Whether a sweep of `tiles` tiles tries to run them by workgroup number (see
+// tile_ticket).  Forward / backward sweep, us, by ticket, by number after
+// counting and by number at once: 97^3 (169 tiles) 255 / 274, -, 254 / 273;
+// 129^3 (256) 391 / 382, 360 / 359, 358 / 356; 161^3 (400) 584 / 548, 550 /
+// 532, 538 / 519.  Fewer tiles gain nothing by it.  The SA model's sweeps
+// are at least as fast by ticket (both of two blocks of 1.2 M nodes 595 ->
+// 581 us with the passes around them) and always go that way.
+constexpr int kFitsMin = 192;
+static bool tile_fits(int tiles, int resident) { return tiles >= kFitsMin && tiles <= resident; }
 
 static void batch_residency(LuBatch *b)
 {
-    // ACFD_LU_TICKETS=1 hands tiles out by ticket even when all would fit
-    const char *t = std::getenv("ACFD_LU_TICKETS");
-    const bool tickets = t && std::atoi(t) == 1;
-    b->resident[0] = !tickets && resident_wgs(k_lu_pipe_batch<1>, kPipeThreads) >= b->total ? 1 : 0;
-    b->resident[1] = !tickets && resident_wgs(k_lu_pipe_batch<-1>, kPipeThreads) >= b->total ? 1 : 0;
+    if (tickets_only()) return;
+    b->fits[0] = tile_fits(b->total, resident_wgs(k_lu_pipe_batch<1>, kPipeThreads));
+    b->fits[1] = tile_fits(b->total, resident_wgs(k_lu_pipe_batch<-1>, kPipeThreads));
 }
 
 template <int DIR>
 static void launch_pipe_batch(hipStream_t s, const LuBatch &b, double gamma, int *err, int *ctr)
 {
     hipLaunchKernelGGL((k_lu_pipe_batch<DIR>), dim3((unsigned)b.total), dim3(kPipeThreads), 0, s,
-                       (const LuBatchEnt *)b.ents, b.tile_ent, b.total, b.resident[DIR > 0 ? 0 : 1], b.sl, b.ex, gamma,
+                       (const LuBatchEnt *)b.ents, b.tile_ent, b.total, b.fits[DIR > 0 ? 0 : 1], b.sl, b.ex, gamma,
                        err, ctr, b.arena, DIR < 0 && b.fuse_add ? 1 : 0);
 }
 
@@ -1659,29 +1676,17 @@ int launch_lusgs_batch(hipStream_t s, const LuBatch &b, int phase, double gamma,
 }
 
 // ---- scalar sweeps: host side
-template <int DIR>
-static bool sa_fits_resident(int total)
-{
-    int dev = 0, cus = 0, per_cu = 0, per_cu_sl = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_sa_tiles_batch<DIR>, kLanes, 0) !=
-            hipSuccess ||
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu_sl, k_sa_sl_batch<DIR>, kLanes, 0) !=
-            hipSuccess)
-        return false;
-    return (long)cus * std::min(per_cu, per_cu_sl) >= total;
-}
-
 // both SA sweeps of one block (ex: sentinel-filled, at least
 // ntiles * (exj_tile + exk_tile) doubles -- less than the flow sweep's)
 int launch_sa_sweeps(hipStream_t s, const Ext &e, const double *cu, const double *rhs, double *dns,
-                     double *dn, double *ex, int *err)
+                     double *dn, double *ex, int *err, int *ctr)
 {
     const SaGeom g = sa_geom(e);
     if (g.Li <= 0 || g.Lj <= 0 || g.Lk <= 0) return 0;
-    hipLaunchKernelGGL((k_sa_tiles<1>), dim3((unsigned)g.ntiles), dim3(kLanes), 0, s, e, g, cu, rhs, dns, dn, ex, err);
-    hipLaunchKernelGGL((k_sa_tiles<-1>), dim3((unsigned)g.ntiles), dim3(kLanes), 0, s, e, g, cu, rhs, dns, dn, ex, err);
+    hipLaunchKernelGGL((k_sa_tiles<1>), dim3((unsigned)g.ntiles), dim3(kLanes), 0, s, e, g, cu, rhs, dns, dn, ex, err,
+                       ctr);
+    hipLaunchKernelGGL((k_sa_tiles<-1>), dim3((unsigned)g.ntiles), dim3(kLanes), 0, s, e, g, cu, rhs, dns, dn, ex, err,
+                       ctr);
     ACFD_CHECK_LAUNCH();
     return 0;
 }
@@ -1729,10 +1734,6 @@ int sa_batch_make(int nblk, const Ext *e, const Fields *f, double *arena, double
     out->total = (int)te.size();
     for (const SaBatchEnt &b : ents) out->nsteps = std::max(out->nsteps, b.g.nsteps);
     if (ents.empty()) return 0;
-    const char *t = std::getenv("ACFD_LU_TICKETS");
-    const bool tickets = t && std::atoi(t) == 1;
-    out->resident[0] = !tickets && sa_fits_resident<1>(out->total) ? 1 : 0;
-    out->resident[1] = !tickets && sa_fits_resident<-1>(out->total) ? 1 : 0;
     if (hipMalloc(&out->ents, ents.size() * sizeof(SaBatchEnt)) != hipSuccess) return 1;
     if (hipMalloc((void **)&out->tile_ent, te.size() * sizeof(int)) != hipSuccess) return 1;
     if (hipMemcpy(out->ents, ents.data(), ents.size() * sizeof(SaBatchEnt), hipMemcpyHostToDevice) != hipSuccess ||
@@ -1756,10 +1757,10 @@ int launch_sa_sl_batch(hipStream_t s, const LuBatch &b, int *err, int *ctr, int 
     else if (phase == 2)
         hipLaunchKernelGGL((k_sa_layout_batch<false>), gl, dim3(kLanes), 0, s, ents, b.tile_ent, b.arena, b.sl, parts);
     else if (phase == 1)
-        hipLaunchKernelGGL((k_sa_sl_batch<1>), gr, dim3(kLanes), 0, s, ents, b.tile_ent, b.total, b.resident[0], b.sl,
+        hipLaunchKernelGGL((k_sa_sl_batch<1>), gr, dim3(kLanes), 0, s, ents, b.tile_ent, b.total, b.sl,
                            b.ex, err, ctr);
     else
-        hipLaunchKernelGGL((k_sa_sl_batch<-1>), gr, dim3(kLanes), 0, s, ents, b.tile_ent, b.total, b.resident[1], b.sl,
+        hipLaunchKernelGGL((k_sa_sl_batch<-1>), gr, dim3(kLanes), 0, s, ents, b.tile_ent, b.total, b.sl,
                            b.ex, err, ctr);
     ACFD_CHECK_LAUNCH();
     return 0;
@@ -1772,10 +1773,10 @@ int launch_sa_batch(hipStream_t s, const LuBatch &b, int *err, int *ctr, int dir
     const SaBatchEnt *ents = (const SaBatchEnt *)b.ents;
     const dim3 gr((unsigned)b.total);
     if (dir >= 0)
-        hipLaunchKernelGGL((k_sa_tiles_batch<1>), gr, dim3(kLanes), 0, s, ents, b.tile_ent, b.total, b.resident[0],
+        hipLaunchKernelGGL((k_sa_tiles_batch<1>), gr, dim3(kLanes), 0, s, ents, b.tile_ent, b.total,
                            b.arena, b.ex, err, ctr);
     if (dir <= 0)
-        hipLaunchKernelGGL((k_sa_tiles_batch<-1>), gr, dim3(kLanes), 0, s, ents, b.tile_ent, b.total, b.resident[1],
+        hipLaunchKernelGGL((k_sa_tiles_batch<-1>), gr, dim3(kLanes), 0, s, ents, b.tile_ent, b.total,
                            b.arena, b.ex, err, ctr);
     ACFD_CHECK_LAUNCH();
     return 0;
@@ -1793,7 +1794,7 @@ template <int DIR>
 static void launch_pipe(hipStream_t s, const SlGeom &g, const LuWs &ws, double gamma, const Ext &e, double *q)
 {
     hipLaunchKernelGGL((k_lu_pipe<DIR>), dim3((unsigned)g.ntiles), dim3(kPipeThreads), 0, s, g, ws.sl, gamma, ws.ex,
-                       ws.err, g.ntiles > ws.resident[DIR > 0 ? 0 : 1] ? ws.ctr : nullptr, e, q);
+                       ws.err, ws.ctr, tile_fits(g.ntiles, ws.resident[DIR > 0 ? 0 : 1]), e, q);
 }
 
 // Phases of one LU-SGS update:

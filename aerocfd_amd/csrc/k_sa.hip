@@ -506,7 +506,7 @@ int launch_sa(hipStream_t s, const Ext &e, const Fields &f, const Consts &c, con
     if (!rc) {
         if (sweep)
             rc = launch_sa_sweeps(s, e, f.w_dqs, f.sa_rhs, f.w_sa + 8 * e.n, f.w_dq, sweep->ex,
-                                  sweep->err);
+                                  sweep->err, sweep->ctr);
         else
             rc = launch_sa_planes(s, e, f);
     }

@@ -114,8 +114,10 @@ int launch_wall_forces(hipStream_t s, const BlockRec *blks, const WallCell *cell
 // k_lusgs.hip
 // workspace of the tile sweeps: sweep-layout operands (normal memory),
 // exchange slots (uncached memory, sentinel-filled), an error word and the
-// ticket counters; resident: tiles of the forward / backward sweep of one
-// block that fit on the device at once (more are handed out by ticket)
+// kTileCounters counters that hand out tiles (zero between launches);
+// resident: workgroups of the forward / backward sweep of one block that the
+// device holds
+constexpr int kTileCounters = 3;
 struct LuWs {
     double *sl;
     double *ex;
@@ -123,7 +125,7 @@ struct LuWs {
     int *ctr = nullptr;
     int resident[2] = {0, 0};
 };
-void lusgs_resident(int *tiles);
+void lusgs_resident(int *wgs);
 constexpr int kLusgsPhases = 5;
 int launch_lusgs_phase(hipStream_t s, const Ext &e, const Fields &f, const Consts &c, const double *cfl,
                        int variant, const LuWs *ws, int phase, int geo_cached = 0);
@@ -135,7 +137,7 @@ struct LuBatch {
     int *tile_ent = nullptr;  // device, entry of each flat tile number
     double *arena = nullptr, *sl = nullptr, *ex = nullptr;  // bases of the table's offsets
     int nent = 0, total = 0, nsteps = 0;  // nsteps: of the longest sweep
-    int resident[2] = {0, 0};  // forward / backward sweep: every workgroup fits on the device at once
+    int fits[2] = {0, 0};      // forward / backward sweep: tile_fits
     int fuse_add = 0;          // the backward sweep stores q + dq (no add pass)
 };
 void lusgs_batch_ws(int nblk, const Ext *e, long *sl_n, long *ex_n);
@@ -150,7 +152,7 @@ int launch_lusgs_batch(hipStream_t s, const LuBatch &b, int phase, double gamma,
 int launch_fill_sentinel(hipStream_t s, double *p, long n);
 // tile sweeps of the SA model's scalar LU-SGS (cu = a, b, c, diag)
 int launch_sa_sweeps(hipStream_t s, const Ext &e, const double *cu, const double *rhs, double *dns,
-                     double *dn, double *ex, int *err);
+                     double *dn, double *ex, int *err, int *ctr);
 // sl: the SA sweep layout (sa_batch_sl doubles) or null
 void sa_batch_sl(int nblk, const Ext *e, long *sl_n);
 int sa_batch_make(int nblk, const Ext *e, const Fields *f, double *arena, double *ex, double *sl,
@@ -171,7 +173,7 @@ int launch_update_q0(hipStream_t s, const BlockRec *blks, int m0, const Ext &e, 
 // k_sa.hip
 struct SaSweep {
     double *ex;  // sentinel-filled exchange slots
-    int *err;
+    int *err, *ctr;
 };
 int launch_sa(hipStream_t s, const Ext &e, const Fields &f, const Consts &c, const double *cfl,
               const SaSweep *sweep = nullptr);
