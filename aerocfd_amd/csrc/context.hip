@@ -213,10 +213,10 @@ struct acfd_ctx {
     std::vector<BatchGrid> bg_bc;
     bool batch_ready = false;
     double *d_stage = nullptr;     // upload/download staging
-    // large downloads of a resident context (a stateless call's context lives
-    // for one download, which would not repay the threads and pinned memory:
-    // 64^3 inviscid_flux_1 3.6 -> 5.5 ms)
-    HostCopy host_copy;
+    // large downloads of a resident context, from its first one on (a
+    // stateless call's context lives for one download, which would not repay
+    // the threads and pinned memory: 64^3 inviscid_flux_1 3.6 -> 5.5 ms)
+    std::shared_ptr<HostCopy> host_copy;
     bool resident = false;
     long stage_n = 0;
     // pointer tables for the multi-block copy kernels
@@ -1896,10 +1896,12 @@ int acfd_download(acfd_ctx *ctx, int m, int field, double *host)
     if (rc) return rc;
     KRN_TRY(launch_soa_to_aos(ctx->stream, src, ctx->d_stage, b.e.n, nc));
     hipError_t e = hipSuccess;
-    if (ctx->resident && tot * sizeof(double) >= HostCopy::kMinBytes &&
-        ctx->host_copy.fetch(host, ctx->d_stage, tot * sizeof(double), ctx->stream, &e)) {
-        HIP_TRY(e);
-        return 0;
+    if (ctx->resident && HostCopy::worth(host, tot * sizeof(double))) {
+        if (!ctx->host_copy) ctx->host_copy = HostCopy::of_device();
+        if (ctx->host_copy && ctx->host_copy->fetch(host, ctx->d_stage, tot * sizeof(double), ctx->stream, &e)) {
+            HIP_TRY(e);
+            return 0;
+        }
     }
     HIP_TRY(hipMemcpyAsync(host, ctx->d_stage, tot * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
     HIP_TRY(hipStreamSynchronize(ctx->stream));

@@ -7,6 +7,8 @@
 // of their own and copy them out, so the copies out and the faults run side
 // by side with each other and with the link.  A 306 MB field 30.4 -> 11.4 ms
 // (27 GB/s), 24 fields of 12 MB 40 -> 12.8 ms, one of 94 MB 9.2 -> 3.2 ms.
+// A pinned destination goes without: the plain copy has the link's rate
+// there (84 MB: 55 GB/s, through the threads 31).
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -14,6 +16,7 @@
 #include <condition_variable>
 #include <cstring>
 #include <exception>
+#include <memory>
 #include <mutex>
 #include <thread>
 #include <vector>
@@ -22,8 +25,40 @@ namespace acfd {
 
 class HostCopy {
 public:
-    // below this many bytes the plain copy is as fast
-    static constexpr size_t kMinBytes = 2u << 20;
+    // The current device's threads and buffers, which its contexts share; the
+    // last one to let go ends them.  Null without memory.
+    static std::shared_ptr<HostCopy> of_device()
+    {
+        static std::mutex mu;
+        static std::vector<std::weak_ptr<HostCopy>> all;
+        int dev = 0;
+        if (hipGetDevice(&dev) != hipSuccess || dev < 0) return nullptr;
+        try {
+            std::lock_guard<std::mutex> g(mu);
+            if ((size_t)dev >= all.size()) all.resize(dev + 1);
+            std::shared_ptr<HostCopy> h = all[dev].lock();
+            if (!h) all[dev] = h = std::make_shared<HostCopy>();
+            return h;
+        } catch (const std::exception &) {
+            return nullptr;
+        }
+    }
+
+    // whether a copy of bytes to dst gains by it: below 2 MiB, and to pinned
+    // memory, the plain copy is as fast or faster
+    static bool worth(const void *dst, size_t bytes)
+    {
+        if (bytes < kMinBytes) return false;
+        for (const char *p : {(const char *)dst, (const char *)dst + bytes - 1}) {
+            hipPointerAttribute_t a{};
+            if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+                (void)hipGetLastError();  // not known to the runtime: pageable
+                return true;
+            }
+            if (a.type == hipMemoryTypeUnregistered) return true;
+        }
+        return false;
+    }
 
     ~HostCopy()
     {
@@ -40,9 +75,11 @@ public:
 
     // Copy bytes of device memory src, written by work queued on s, to dst
     // and wait for it.  False: nothing was copied (no pinned memory or no
-    // threads to be had); err receives a failed copy's error.
+    // threads to be had); err receives a failed copy's error.  Callers take
+    // turns.
     bool fetch(void *dst, const void *src, size_t bytes, hipStream_t s, hipError_t *err)
     {
+        std::lock_guard<std::mutex> turn(turn_);
         if (!start()) return false;
         std::unique_lock<std::mutex> g(mu_);
         dst_ = (char *)dst;
@@ -59,8 +96,9 @@ public:
     }
 
 private:
+    static constexpr size_t kMinBytes = 2u << 20;
     static constexpr size_t kChunk = 1u << 20;
-    static constexpr int kThreads = 8;
+    static constexpr int kThreads = 8;  // at most, and no more than the process has processors
 
     bool start()
     {
@@ -80,7 +118,8 @@ private:
             }
         try {
             threads_.reserve(kThreads);
-            for (int t = 0; t < kThreads; t++) threads_.emplace_back([this, t] { work(t); });
+            const int n = std::max(1, std::min(kThreads, (int)std::thread::hardware_concurrency()));
+            for (int t = 0; t < n; t++) threads_.emplace_back([this, t] { work(t); });
         } catch (const std::exception &) {
             // fewer threads than asked for: those that run share the chunks
         }
@@ -122,7 +161,10 @@ private:
         for (long c = t; c < n && e == hipSuccess; c += nt, h ^= 1) {
             if (c + nt < n) e = issue(c + nt, h ^ 1);
             const hipError_t w = hipEventSynchronize(ev_[2 * t + h]);
-            if (w != hipSuccess) return w;
+            if (w != hipSuccess) {
+                (void)hipStreamSynchronize(stream_);  // a copy into the other buffer may be under way
+                return w;
+            }
             std::memcpy(dst_ + c * kChunk, pinned_ + (2 * t + h) * kChunk, len(c));
         }
         return e;
@@ -130,7 +172,7 @@ private:
 
     std::vector<std::thread> threads_;
     hipEvent_t ev_[2 * kThreads] = {};
-    std::mutex mu_;
+    std::mutex turn_, mu_;
     std::condition_variable cv_, done_;
     char *pinned_ = nullptr;
     int dev_ = 0;
