@@ -869,12 +869,12 @@ int st_inviscid(acfd_ctx *ctx, int m)
     return 0;
 }
 
-// part 1: the node pass, 2: the difference pass; prep: that pass forms
-// implicit1st's rhs (lu_fold), find_dt: and does the unsteady find_dt
-int st_viscous(acfd_ctx *ctx, int m, int store_aux, int part = -1, bool prep = false, bool find_dt = false)
+// prep: the difference pass forms implicit1st's rhs (lu_fold), find_dt: and
+// does the unsteady find_dt
+int st_viscous(acfd_ctx *ctx, int m, int store_aux, bool prep = false, bool find_dt = false)
 {
     StageTimer t(ctx, ACFD_STAGE_VISCOUS);
-    KRN_TRY(launch_viscous(ctx->stream, ctx->blk[m].e, ctx->blk[m].f, ctx->c, ctx->cfg.precision, store_aux, part,
+    KRN_TRY(launch_viscous(ctx->stream, ctx->blk[m].e, ctx->blk[m].f, ctx->c, ctx->cfg.precision, store_aux, false,
                            prep, find_dt ? ctx->d_cfl : nullptr, find_dt ? ctx->d_cfl_blk + m : nullptr));
     if (prep) ctx->lu_prep_ready = ctx->rhsv_stale = true;
     return 0;
@@ -1202,7 +1202,7 @@ int residual_stage(acfd_ctx *ctx, int m, int store_aux, bool pri_ok = false)
     int rc = pri_ok ? 0 : st_getpri(ctx, m);
     const bool fold = lu_fold(ctx), dt_in = dt_in_diff(ctx);
     if (!rc) rc = st_inviscid(ctx, m);
-    if (!rc && ctx->c.solver == 0) rc = st_viscous(ctx, m, store_aux, -1, fold, dt_in);
+    if (!rc && ctx->c.solver == 0) rc = st_viscous(ctx, m, store_aux, fold, dt_in);
     if (!rc && !dt_in) rc = st_find_dt(ctx, m);
     return rc;
 }
@@ -1260,7 +1260,7 @@ int st_viscous_all(acfd_ctx *ctx, int store_aux, bool fold = false, bool dt_in =
     const int nb = (int)ctx->blk.size();
     if (!batched(ctx)) {
         for (int m = 0; m < nb; m++) {
-            int rc = st_viscous(ctx, m, store_aux, -1, fold, dt_in);
+            int rc = st_viscous(ctx, m, store_aux, fold, dt_in);
             if (rc) return rc;
         }
         return 0;
@@ -1339,7 +1339,7 @@ int rhsv_refresh(acfd_ctx *ctx)
     if (!ctx->rhsv_stale) return 0;
     ctx->rhsv_stale = false;
     if (!batched(ctx)) {
-        for (auto &b : ctx->blk) KRN_TRY(launch_viscous(ctx->stream, b.e, b.f, ctx->c, ctx->cfg.precision, 0, 2));
+        for (auto &b : ctx->blk) KRN_TRY(launch_viscous(ctx->stream, b.e, b.f, ctx->c, ctx->cfg.precision, 0, true));
         return 0;
     }
     KRN_TRY(launch_viscous_batch(ctx->stream, ctx->d_blocks, ctx->bg_visc, ctx->arena, ctx->c, ctx->cfg.precision, 0,

@@ -659,20 +659,19 @@ __global__ void __launch_bounds__(256) k_viscous_diff_batch(const BlockRec *__re
 dim3 viscous_grid(const Ext &e) { return lin_grid(e); }
 
 int launch_viscous(hipStream_t s, const Ext &e, const Fields &f, const Consts &c, int precision,
-                   int store_aux, int part, bool prep, double *cfl, double *cfl_blk)
+                   int store_aux, bool diff_only, bool prep, double *cfl, double *cfl_blk)
 {
     dim3 g = viscous_grid(e), t(64, 4, 1);
     const dim3 gp(g.x + (cfl ? 1 : 0));
     const double *dt = cfl ? f.dt : nullptr;
-    if (part == 2) {
+    if (diff_only) {
     } else if (precision == 1)
         hipLaunchKernelGGL((k_viscous_node<float>), g, t, 0, s, e, c, f.pri, f.amu, f.dxidx, f.inv_j, f.w_flux,
                            f.vor, f.dudx, f.tao, store_aux);
     else
         hipLaunchKernelGGL((k_viscous_node<double>), g, t, 0, s, e, c, f.pri, f.amu, f.dxidx, f.inv_j, f.w_flux,
                            f.vor, f.dudx, f.tao, store_aux);
-    if (part == 1) {
-    } else if (prep && precision == 1)
+    if (prep && precision == 1)
         hipLaunchKernelGGL(k_viscous_diff_prep<float>, gp, t, 0, s, e, f.w_flux, c.re, f.rhsi, f.rhs, f.pri, f.amu,
                            f.dxidx, dt, cfl, cfl_blk);
     else if (prep)

@@ -508,7 +508,12 @@ __global__ void __launch_bounds__(256) k_ext_i(Ext e, const double *__restrict__
 // 565 / 558 / 699, 169^3 6276 / 4548 / 3752 / 3404 / 3430, 1024 x 512 x 4
 // 1344 / 1059 / 993 / 951 / 976; FP32 has its best runs at the same sizes.
 // A face's value does not depend on the run that holds it.  With the
-// sensor the faces counted are those of the runs, which stay at 16.
+// sensor, network each time / decisions reused three times of four, us a
+// stage at runs of 32 / 16: 33^3 362 / 217, 265 / 159; 81^3 397 / 254, 285 /
+// 176; 129^3 572 / 603, 409 / 363; 193^3 2220 / 2170, 1309 / 1309; 1024 x
+// 512 x 4 452 / 386, 267 / 217.  The faces counted are the evaluations, those
+// that two runs make of the same face both: a line longer than 16 nodes
+// counts more than it would in runs of 32 (129^3: 10 %).
 static int ext_run(long nodes, bool sensor)
 {
     if (sensor) return 16;

@@ -382,7 +382,7 @@ __device__ inline void xstore(double *p, double v)
 // ii = 0..CT-1, which are exactly rows t0 + ii of the sweep layout.
 // Natural side: thread x handles ii = x % CT of lines x / CT + m TT/CT,
 // so CT consecutive lanes touch CT consecutive doubles of one line
-// (CT = min(32, 4096/TT)).
+// (CT = kSlCt).
 // Sweep side: thread x is lane x.  LDS holds [CT][TT] doubles per field
 // with the line index XOR-swizzled by ii (no bank conflicts either way).
 // steps a layout kernel transposes at a time
@@ -519,7 +519,7 @@ __device__ inline void sl_add_tile(const Ext &e, const SlGeom &g, int tile, cons
             nat[m] = (t0 + ii_n < g.nsteps && li >= 0 && li < g.Li && sl_line_ok(g, tile, line))
                          ? (int)sl_nat(e, g, tile, line, li) : -1;
         }
-        const int v0 = 2 * fp - kSlOut;  // component of the pair's lower field (-1: diag)
+        const int v0 = 2 * fp - kSlOut;  // component of the pair's lower field (-1: the time term)
         if (me_ok) {
             const double2 *sl2 = reinterpret_cast<const double2 *>(sl);
             double2 d[CT];
@@ -617,8 +617,9 @@ __device__ inline double lu_node_radii(const double *op, double *r)
 //              ds_bpermute (k, formed first) and DPP (j), so no barrier is
 //              on its path.
 //   preparing  step s, s + 1, ... in turn: two steps' loads in flight
-//   waves      each, radii, 1/(diag inv_j) and the scaled metric rows
-//              written to a ring of kPipeRing steps.
+//   waves      each, the state, the metric rows with their radii and the two
+//              divisors with their reciprocals written to a ring of
+//              kPipeRing steps.
 //   last wave  fetches the j and k neighbour tiles' products from the
 //              exchange slots, up to eight steps at a time, into a ring, and
 //              sets the slots back to the sentinel.
@@ -628,8 +629,8 @@ __device__ inline double lu_node_radii(const double *op, double *r)
 // for ring space (wave 0), wave 0 for operands and for slots, the slot
 // wave for the neighbouring tiles with a bounded poll; running out sets
 // *err and `stop`, at which every wait of the workgroup ends.
-// What bounds it: wave 0's instruction issue (about 260 instructions a step,
-// of which 127 are the FP64 arithmetic, at one per four cycles or more:
+// What bounds it: wave 0's instruction issue (about 270 instructions a step,
+// of which 137 are the FP64 arithmetic, at one per four cycles or more:
 // about 0.65 us a step) and 2.6 us a hop; on large batches the HBM traffic.
 // Forward sweep, before (one wavefront a tile) and after: 33^3 184 -> 88 us,
 // 129^3 748 -> 346, 193^3 1218 -> 740, 12 blocks of 3.2 M nodes in all

@@ -12,11 +12,10 @@ int launch_fill(hipStream_t s, double *p, long n, double v);
 // clear: rhsi may not be zero outside the computed range
 int launch_inviscid(hipStream_t s, const Ext &e, const Fields &f, const Consts &c, int precision, int run, bool clear);
 int inviscid_run(long nodes, int precision);
-// part 1, 2: only the node, the difference pass; prep: that pass forms
-// implicit1st's rhs and stores no rhsv, and with cfl given it also does the
-// unsteady find_dt
-int launch_viscous(hipStream_t s, const Ext &e, const Fields &f, const Consts &c, int precision,
-                   int store_aux, int part = -1, bool prep = false, double *cfl = nullptr, double *cfl_blk = nullptr);
+// diff_only: only the difference pass; prep: that pass forms implicit1st's
+// rhs and stores no rhsv, and with cfl given it also does the unsteady find_dt
+int launch_viscous(hipStream_t s, const Ext &e, const Fields &f, const Consts &c, int precision, int store_aux,
+                   bool diff_only = false, bool prep = false, double *cfl = nullptr, double *cfl_blk = nullptr);
 // unsteady: the local cfl of the block's last node goes to *cfl and, when
 // not null, *cfl_blk
 int launch_find_dt(hipStream_t s, const Ext &e, const Fields &f, const Consts &c, double *cfl, double *cfl_blk,

@@ -49,7 +49,11 @@ typedef struct acfd_config {
                                        reference; laminar or Euler) */
     int precision;                  /* 0 = FP64 everywhere; 1 = FP32 reconstruction/splitting/viscous, FP64 update */
     int lusgs_kernel;               /* 0 = the library's choice: the tile sweep per block in a context whose
-                                       device has room for its workspace, else hyperplane launches;
+                                       device has room for its workspace (22 doubles a node of the largest
+                                       block, rounded up to whole tiles of 8 x 8 lines, if that is at
+                                       most a quarter of the free device memory), else
+                                       hyperplane launches, several times slower and without a workspace;
+                                       ACFD_LU_HYPERPLANES=1 in the environment asks for those;
                                        1 = pipelined tile sweep per block, 2 = tile sweeps of all blocks in
                                        one launch (all the same results) */
     int inviscid_scheme;            /* 0 = WENO3 + Roe (the reference's inviscid_flux_1); no counterpart
@@ -116,9 +120,9 @@ int acfd_set_topology(acfd_ctx *ctx, int nblk, const int *dims, const int *nsub,
 int acfd_block_ranges(acfd_ctx *ctx, int m, int *ranges);
 
 /* Copy one field of block m between host (reference AoS layout, extended
- * extents) and the device-resident state.  The batched steady update forms
- * rhs = rhsi + rhsv without storing rhsv; rhsv is then formed again from
- * the viscous node fluxes by the first call that needs it (its download or
+ * extents) and the device-resident state.  A Navier-Stokes step with the
+ * tile sweeps forms rhs = rhsi + rhsv without storing rhsv; rhsv is then
+ * formed again from the viscous node fluxes by the first call that needs it (its download or
  * upload, acfd_run_stage, acfd_grid_metrics), so every call sees the value
  * of the last viscous evaluation. */
 int acfd_upload(acfd_ctx *ctx, int m, int field, const double *host);
@@ -282,7 +286,9 @@ int acfd_sensor_enable(acfd_ctx *ctx, int on, float threshold, int audit_interva
  * The next evaluation of every block runs the network. */
 int acfd_sensor_refresh(acfd_ctx *ctx, int interval);
 /* out[6]: faces evaluated, faces given linear weights, audits, largest
- * audit deviation, blocks fallen back, 0 */
+ * audit deviation, blocks fallen back, 0.  The first two count evaluations:
+ * a face that two threads need counts twice, so they depend on how the
+ * kernels cut a line; their ratio is the share of linear faces */
 int acfd_sensor_stats(acfd_ctx *ctx, double *out);
 /* stateless, for checking the training kernels: mean loss and its
  * gradient over n samples X[n][12], Y[n] */
