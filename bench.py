@@ -117,29 +117,29 @@ HYPERPLANE_BYTES = {  # the hyperplane sweeps read the operands in place
 # counters.  The channel with bump at FP64, batched stages and sweeps
 # (profiles/channel_bump_fp64_hbm_traffic.md).
 MEASURED_TRAFFIC_CHANNEL = {
-    "getpri": 10.035e9,
-    "inviscid_i": 11.019e9,
-    "inviscid_j": 17.098e9,
-    "inviscid_k": 17.812e9,
-    "viscous_node_dt": 29.872e9,
+    "getpri": 10.033e9,
+    "inviscid_i": 11.016e9,
+    "inviscid_j": 17.642e9,
+    "inviscid_k": 20.214e9,
+    "viscous_node_dt": 29.870e9,
     "viscous_diff": 20.764e9,
-    "lusgs_gather": 23.470e9,
-    "lusgs_forward": 28.875e9,
-    "lusgs_backward": 28.883e9,
+    "lusgs_gather": 23.469e9,
+    "lusgs_forward": 28.873e9,
+    "lusgs_backward": 28.874e9,
     "lusgs_add": 9.261e9,
-    "sa_pre": 17.184e9,
-    "sa_pre_b": 24.719e9,
-    "sa_gather": 9.829e9,
-    "sa_forward": 6.183e9,
-    "sa_backward": 6.181e9,
+    "sa_pre": 17.182e9,
+    "sa_pre_b": 24.718e9,
+    "sa_gather": 9.830e9,
+    "sa_forward": 6.178e9,
+    "sa_backward": 6.175e9,
     "sa_add": 3.286e9,
 }
 # The TGV 256^3 block, FP64, tile sweeps (profiles/tgv256_fp64_hbm_traffic.md).
 MEASURED_TRAFFIC_256 = {
     "getpri": 1.687e9,
     "lusgs_gather": 4.090e9,
-    "lusgs_forward": 4.569e9,
-    "lusgs_backward": 4.574e9,
+    "lusgs_forward": 4.579e9,
+    "lusgs_backward": 4.576e9,
     "lusgs_add": 1.578e9,
 }
 
