@@ -168,6 +168,9 @@ struct acfd_ctx {
     // step that did so replays only while it holds.
     bool pri_current = false;
     bool graph_needs_pri = false;
+    // the same for the implicit1st stage, which may follow other stages and
+    // uploads: set by the getpri stage too, cleared by what writes q or pri_v
+    bool pri_of_q = false;
     // the last residual stage also formed implicit1st's rhs (lu_fold): the
     // update that follows skips its preparation pass
     bool lu_prep_ready = false;
@@ -973,11 +976,10 @@ void sl_invalidate(acfd_ctx *ctx)
     ctx->sl_block = -2;
 }
 
-int st_implicit(acfd_ctx *ctx, int m, const double *cfl, bool prep_ready = false)
+int st_implicit(acfd_ctx *ctx, int m, const double *cfl, int variant, bool prep_ready = false)
 {
     StageTimer t(ctx, ACFD_STAGE_IMPLICIT1ST);
     Block &b = ctx->blk[m];
-    const int variant = ctx->lu_variant;
     for (int ph = prep_ready ? 1 : 0; ph < kLusgsPhases; ph++) {
         StageTimer ts(ctx, ph == 2 ? kTimeLuForward : ph == 3 ? kTimeLuBackward
                            : ph == 1 ? kTimeLuGather : ph == 4 ? kTimeLuAdd : kTimeLuOther);
@@ -1005,7 +1007,7 @@ int st_implicit_all(acfd_ctx *ctx, const double *cfl_per_block)
     ctx->lu_prep_ready = false;
     if (ctx->lu_variant != 2) {
         for (int m = 0; m < nb; m++) {
-            int rc = st_implicit(ctx, m, cfl_per_block ? cfl_per_block + m : ctx->d_cfl, prep_ready);
+            int rc = st_implicit(ctx, m, cfl_per_block ? cfl_per_block + m : ctx->d_cfl, ctx->lu_variant, prep_ready);
             if (rc) return rc;
         }
         return 0;
@@ -1408,7 +1410,7 @@ int one_step(acfd_ctx *ctx)
     // getpri is the latest write (a block's q changes only in its own update,
     // after its residual)
     const bool pri_ok = ctx->pri_current;
-    ctx->pri_current = false;
+    ctx->pri_current = ctx->pri_of_q = false;
     if (pri_ok && ctx->capturing && (ctx->cfg.iflag_timeadvance == 2 || ctx->cfg.iflag_timeadvance == 4))
         ctx->graph_needs_pri = true;
     if (ctx->cfg.iflag_timeadvance == 2 && stagewise) {
@@ -1450,7 +1452,7 @@ int one_step(acfd_ctx *ctx)
             rc = residual_stage(ctx, m, aux, pri_ok);
             const bool ready = ctx->lu_prep_ready;
             ctx->lu_prep_ready = false;
-            if (!rc) rc = st_implicit(ctx, m, cfl_of(m), ready);
+            if (!rc) rc = st_implicit(ctx, m, cfl_of(m), ctx->lu_variant, ready);
             if (!rc && sa) rc = st_sa(ctx, m, cfl_of(m));
         }
         if (!rc) rc = refresh(ctx);
@@ -1506,7 +1508,7 @@ int one_step(acfd_ctx *ctx)
     // (its output interval is 1, main.f90:341,575-603); acfd_residual reads
     // them back
     if (!rc) rc = launch_residual_all(ctx) ? ACFD_EDEVICE : 0;
-    if (!rc) ctx->pri_current = true;
+    if (!rc) ctx->pri_current = ctx->pri_of_q = true;
     return rc;
 }
 
@@ -1846,6 +1848,7 @@ int acfd_upload(acfd_ctx *ctx, int m, int field, const double *host)
         return fail(ACFD_EINVAL, "acfd_upload: bad arguments");
     ctx->pri_current = false;
     ctx->res_current = false;
+    if (field == ACFD_Q || field == ACFD_PRI_V) ctx->pri_of_q = false;
     if (field == ACFD_RHSV) {
         int rc = rhsv_refresh(ctx);  // the other blocks' rhsv
         if (rc) return rc;
@@ -1911,7 +1914,11 @@ int acfd_download(acfd_ctx *ctx, int m, int field, double *host)
 int acfd_run_stage(acfd_ctx *ctx, int stage)
 {
     if (!ctx || !ctx->topo) return fail(ACFD_ESTATE, "acfd_run_stage: no topology");
+    const bool pri_of_q = ctx->pri_of_q;
     ctx->pri_current = false;
+    ctx->pri_of_q = stage == ACFD_STAGE_GETPRI ||
+                    (pri_of_q && (stage == ACFD_STAGE_INVISCID || stage == ACFD_STAGE_VISCOUS ||
+                                  stage == ACFD_STAGE_FIND_DT || stage == ACFD_STAGE_SA));
     ctx->res_current = false;
     ctx->lu_prep_ready = false;
     const int nb = (int)ctx->blk.size();
@@ -1932,7 +1939,13 @@ int acfd_run_stage(acfd_ctx *ctx, int stage)
         for (int m = 0; m < nb && !rc; m++) rc = st_find_dt(ctx, m);
         break;
     case ACFD_STAGE_IMPLICIT1ST:
-        rc = st_implicit_all(ctx, nullptr);
+        // the tile sweeps take a node's velocity from q, the hyperplanes, as
+        // the reference, from pri_v: a caller that left the choice to the
+        // library gets the tiles only where the two agree
+        if (ctx->cfg.lusgs_kernel == 0 && !pri_of_q)
+            for (int m = 0; m < nb && !rc; m++) rc = st_implicit(ctx, m, ctx->d_cfl, 0);
+        else
+            rc = st_implicit_all(ctx, nullptr);
         break;
     case ACFD_STAGE_SA:
         if (!(ctx->c.turb == 2 && ctx->c.solver == 0)) return fail(ACFD_EINVAL, "SA stage needs NS + SA");
@@ -1959,7 +1972,7 @@ int acfd_run_stage(acfd_ctx *ctx, int stage)
 int acfd_prepare(acfd_ctx *ctx)
 {
     if (!ctx || !ctx->topo) return fail(ACFD_ESTATE, "acfd_prepare: no topology");
-    ctx->pri_current = false;
+    ctx->pri_current = ctx->pri_of_q = false;
     ctx->res_current = false;
     int rc = refresh(ctx);
     if (rc) return rc;
@@ -1995,7 +2008,7 @@ int acfd_step(acfd_ctx *ctx, int nsteps)
         if (graph && ctx->graph_exec) {
             HIP_TRY(hipGraphLaunch(ctx->graph_exec, ctx->stream));
             ctx->sl_block = ctx->graph_sl_out;
-            ctx->pri_current = true;
+            ctx->pri_current = ctx->pri_of_q = true;
             if (ctx->graph_rhsv) ctx->rhsv_stale = true;
             continue;
         }
