@@ -55,7 +55,7 @@ typedef struct acfd_config {
                                        hyperplane launches, several times slower and without a workspace;
                                        ACFD_LU_HYPERPLANES=1 in the environment asks for those;
                                        1 = pipelined tile sweep per block, 2 = tile sweeps of all blocks in
-                                       one launch (all the same results) */
+                                       one launch (all the same results on finite fields) */
     int inviscid_scheme;            /* 0 = WENO3 + Roe (the reference's inviscid_flux_1); no counterpart
                                        in the reference: 1 = Steger-Warming splitting + WENO5,
                                        2 = WCNS (WENO5 midpoint interpolation + Roe, 6th-order difference) */
@@ -128,7 +128,10 @@ int acfd_block_ranges(acfd_ctx *ctx, int m, int *ranges);
 int acfd_upload(acfd_ctx *ctx, int m, int field, const double *host);
 int acfd_download(acfd_ctx *ctx, int m, int field, double *host);
 
-/* Run one stage over all blocks, in the reference's block order. */
+/* Run one stage over all blocks, in the reference's block order.  implicit1st
+ * takes the velocity in its spectral radii from pri_v with lusgs_kernel 0, as
+ * the reference's routine does, and from q with 1 and 2: the same where pri_v
+ * is getpri of q, as within a step. */
 int acfd_run_stage(acfd_ctx *ctx, int stage);
 /* The boundary refresh before the time loop (main.f90:309-318). */
 int acfd_prepare(acfd_ctx *ctx);
